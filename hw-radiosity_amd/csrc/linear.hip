@@ -342,12 +342,12 @@ __global__ __launch_bounds__(kB) void k_fx64v(const float *__restrict__ F, const
 	}
 }
 
-// out[i][c] = base[i][c] + rho[i][c] * y - beta * xT[c][i], y = the split-K
-// sum of part (FP64, fixed order); base, rho may be null (0 and 1).  Per
+// out[i][c] = base[i][c] + rho[i][c] * y - xT[c][i], y = the split-K sum of
+// part (FP64, fixed order); base, rho and xT may be null (0, 1 and 0).  Per
 // block: sum of squares and max |out|.
 __global__ __launch_bounds__(kB) void k_resid(const double *part, int S, int ld, int rp, int n, int nrhs,
-                                              const double *xT, const double *base, const double *rho, double beta,
-                                              double *out, double *blk)
+                                              const double *xT, const double *base, const double *rho, double *out,
+                                              double *blk)
 {
 	const size_t total = (size_t)n * nrhs;
 	const size_t t = blockIdx.x * (size_t)kB + threadIdx.x;
@@ -356,78 +356,10 @@ __global__ __launch_bounds__(kB) void k_resid(const double *part, int S, int ld,
 		const int i = (int)(t / nrhs), c = (int)(t % nrhs);
 		double y = 0.0;
 		for (int q = 0; q < S; q++) y += part[((size_t)q * ld + i) * rp + c];
-		const double v = (base ? base[t] : 0.0) + (rho ? rho[t] : 1.0) * y - beta * xT[(size_t)c * ld + i];
+		const double v = (base ? base[t] : 0.0) + (rho ? rho[t] : 1.0) * y - (xT ? xT[(size_t)c * ld + i] : 0.0);
 		out[t] = v;
 		ss = v * v;
 		mx = fabs(v);
-	}
-	for (int off = 32; off > 0; off >>= 1) {
-		ss += __shfl_xor(ss, off);
-		mx = fmax(mx, __shfl_xor(mx, off));
-	}
-	__shared__ double r[8];
-	if ((threadIdx.x & 63) == 0) {
-		r[2 * (threadIdx.x >> 6)] = ss;
-		r[2 * (threadIdx.x >> 6) + 1] = mx;
-	}
-	__syncthreads();
-	if (threadIdx.x == 0) {
-		blk[2 * blockIdx.x] = r[0] + r[2] + r[4] + r[6];
-		blk[2 * blockIdx.x + 1] = fmax(fmax(r[1], r[3]), fmax(r[5], r[7]));
-	}
-}
-
-// Transposed product split over row chunks, for nrhs <= 4:
-//   part[s][j][c] = sum over rows i of chunk s of F[i][j] * rho[i][c] * x[i][c]
-template <typename T>
-__global__ __launch_bounds__(kB) void k_ftx(const float *__restrict__ F, int ld, int n, int nrhs, const T *__restrict__ x,
-                                            const T *__restrict__ rho, int rows_per_split, T *part)
-{
-	// four consecutive columns per lane (one 16-byte load per row; ld is a
-	// multiple of 256, so the load stays in the zero-padded row)
-	const int j4 = (blockIdx.x * kB + threadIdx.x) * 4;
-	const int s = blockIdx.y, i0 = s * rows_per_split, i1 = min(n, i0 + rows_per_split);
-	if (j4 >= n) return;
-	T acc[4][4];
-#pragma unroll
-	for (int q = 0; q < 4; q++)
-#pragma unroll
-		for (int c = 0; c < 4; c++) acc[q][c] = 0;
-	constexpr int kRowsUnrolled = sizeof(T) == 8 ? 4 : 1;  // measured: helps the FP64 form only
-#pragma unroll kRowsUnrolled
-	for (int i = i0; i < i1; i++) {
-		const float4 f = *(const float4 *)(F + (size_t)i * ld + j4);
-		const float fq[4] = {f.x, f.y, f.z, f.w};
-		T w[4];
-#pragma unroll
-		for (int c = 0; c < 4; c++) w[c] = c < nrhs ? rho[(size_t)i * nrhs + c] * x[(size_t)i * nrhs + c] : (T)0;
-#pragma unroll
-		for (int q = 0; q < 4; q++)
-#pragma unroll
-			for (int c = 0; c < 4; c++)
-				if (c < nrhs) acc[q][c] += (T)fq[q] * w[c];
-	}
-#pragma unroll
-	for (int q = 0; q < 4; q++)
-		if (j4 + q < n)
-			for (int c = 0; c < nrhs; c++) part[((size_t)s * n + j4 + q) * nrhs + c] = acc[q][c];
-}
-
-// out = base + sum_s part - beta * x; per block sum of squares and max |out|
-template <typename T>
-__global__ __launch_bounds__(kB) void k_ftx_finish(const T *part, int S, int n, int nrhs, const T *base, const T *x,
-                                                   T beta, T *out, double *blk)
-{
-	const size_t total = (size_t)n * nrhs;
-	const size_t t = blockIdx.x * (size_t)kB + threadIdx.x;
-	double ss = 0.0, mx = 0.0;
-	if (t < total) {
-		T y = 0;
-		for (int s = 0; s < S; s++) y += part[(size_t)s * total + t];
-		const T v = base[t] + y - beta * x[t];
-		out[t] = v;
-		ss = (double)v * (double)v;
-		mx = fabs((double)v);
 	}
 	for (int off = 32; off > 0; off >>= 1) {
 		ss += __shfl_xor(ss, off);
@@ -457,16 +389,26 @@ __global__ void k_scale(const double *r64, double inv_s, size_t total, int nrhs,
 	}
 }
 
-// xT[c][i] += s * d[i][c]
-__global__ void k_axpy_t(double *xT, int ld, const float *d, double s, int n, int nrhs)
+// xT[c][i] += s * d[i][c]; with wT, wT[c][i] <- rho[i][c] * xT[c][i] (the
+// adjoint's product input)
+__global__ void k_axpy_t(double *xT, int ld, const float *d, double s, int n, int nrhs, double *wT = nullptr,
+                         const double *rho = nullptr)
+{
+	const size_t total = (size_t)n * nrhs;
+	for (size_t t = blockIdx.x * (size_t)kB + threadIdx.x; t < total; t += (size_t)gridDim.x * kB) {
+		const size_t q = (size_t)(t % nrhs) * ld + t / nrhs;
+		const double x = xT[q] + s * (double)d[t];
+		xT[q] = x;
+		if (wT) wT[q] = rho[t] * x;
+	}
+}
+
+// out[i][c] = xT[c][i]
+__global__ void k_rows(const double *xT, int ld, int n, int nrhs, double *out)
 {
 	const size_t total = (size_t)n * nrhs;
 	for (size_t t = blockIdx.x * (size_t)kB + threadIdx.x; t < total; t += (size_t)gridDim.x * kB)
-		xT[(size_t)(t % nrhs) * ld + t / nrhs] += s * (double)d[t];
-}
-__global__ void k_axpy(double *x, const float *d, double s, size_t total)
-{
-	for (size_t t = blockIdx.x * (size_t)kB + threadIdx.x; t < total; t += (size_t)gridDim.x * kB) x[t] += s * (double)d[t];
+		out[t] = xT[(size_t)(t % nrhs) * ld + t / nrhs];
 }
 
 // per block: sum (x - ref)^2 and sum ref^2 (x transposed [c][ld] or row-major)
@@ -721,21 +663,21 @@ struct Fx64 {
 	// at most 4 columns: the vector-unit kernel (ld is a multiple of 256:
 	// whole chunks of 1024 or 256 k, whole blocks of 4 kFxRows rows)
 	bool vec() const { return nrhs <= 4 && rp >= 4 && ld % 256 == 0 && ld % (4 * kFxRows) == 0; }
-	// out = base + rho o (F x) - beta x; returns (sum of squares, max |out|)
-	int run(const float *F, const double *xT, const double *base, const double *rho, double beta, double *out,
+	// out = base + rho o (F w) - x (xT null: 0); returns (sum of squares, max |out|)
+	int run(const float *F, const double *wT, const double *base, const double *rho, const double *xT, double *out,
 	        hipStream_t st, double &ss, double &mx, bool want_stats, std::string &err)
 	{
 		const dim3 grid(ld / (64 * rt), rp / (16 * ct), S);
 		const int kchunk = ld / S;
 		if (vec() && ld % 1024 == 0)
-			hipLaunchKernelGGL(k_fx64v<1024>, dim3(ld / (4 * kFxRows)), dim3(kB), 0, st, F, xT, part.p, ld, rp);
+			hipLaunchKernelGGL(k_fx64v<1024>, dim3(ld / (4 * kFxRows)), dim3(kB), 0, st, F, wT, part.p, ld, rp);
 		else if (vec())
-			hipLaunchKernelGGL(k_fx64v<256>, dim3(ld / (4 * kFxRows)), dim3(kB), 0, st, F, xT, part.p, ld, rp);
-		else if (ct == 4) hipLaunchKernelGGL((k_fx64m<2, 4>), grid, dim3(kB), 0, st, F, xT, part.p, ld, rp, kchunk);
-		else if (ct == 2) hipLaunchKernelGGL((k_fx64m<4, 2>), grid, dim3(kB), 0, st, F, xT, part.p, ld, rp, kchunk);
-		else hipLaunchKernelGGL((k_fx64m<4, 1>), grid, dim3(kB), 0, st, F, xT, part.p, ld, rp, kchunk);
+			hipLaunchKernelGGL(k_fx64v<256>, dim3(ld / (4 * kFxRows)), dim3(kB), 0, st, F, wT, part.p, ld, rp);
+		else if (ct == 4) hipLaunchKernelGGL((k_fx64m<2, 4>), grid, dim3(kB), 0, st, F, wT, part.p, ld, rp, kchunk);
+		else if (ct == 2) hipLaunchKernelGGL((k_fx64m<4, 2>), grid, dim3(kB), 0, st, F, wT, part.p, ld, rp, kchunk);
+		else hipLaunchKernelGGL((k_fx64m<4, 1>), grid, dim3(kB), 0, st, F, wT, part.p, ld, rp, kchunk);
 		hipLaunchKernelGGL(k_resid, dim3((unsigned)nblk), dim3(kB), 0, st, part.p, S, ld, rp, n, nrhs, xT, base, rho,
-		                   beta, out, blk.p);
+		                   out, blk.p);
 		HIP_OK(hipGetLastError(), "FP64 product");
 		ss = mx = 0.0;
 		if (!want_stats) return 0;
@@ -1054,7 +996,7 @@ int LinearSystem::multiply(int prec, int nrhs, const double *X, double *Y, std::
 		if (xT.alloc(xt.size(), err) || out.alloc(total, err)) return -1;
 		HIP_OK(hipMemcpyAsync(xT.p, xt.data(), xt.size() * 8, hipMemcpyHostToDevice, st), "upload");
 		double ss, mx;
-		if (fx.run(d.F32.p, xT.p, nullptr, nullptr, 0.0, out.p, st, ss, mx, false, err)) return -1;
+		if (fx.run(d.F32.p, xT.p, nullptr, nullptr, nullptr, out.p, st, ss, mx, false, err)) return -1;
 		HIP_OK(hipMemcpyAsync(Y, out.p, total * 8, hipMemcpyDeviceToHost, st), "download");
 		HIP_OK(hipStreamSynchronize(st), "multiply");
 		return 0;
@@ -1191,7 +1133,7 @@ int LinearSystem::gather(int prec, int nrhs, const double *rho, const double *E,
 			HIP_OK(hipMemcpyAsync(r64.p, E64.p, total * 8, hipMemcpyDeviceToDevice, st), "residual");
 			ss = ss0;
 			mx = mx0;
-		} else if (fx.run(d.F32.p, xT.p, E64.p, rho64.p, 1.0, r64.p, st, ss, mx, true, err)) {
+		} else if (fx.run(d.F32.p, xT.p, E64.p, rho64.p, xT.p, r64.p, st, ss, mx, true, err)) {
 			return -1;
 		}
 		if (!std::isfinite(ss)) {
@@ -1229,7 +1171,7 @@ int LinearSystem::gather(int prec, int nrhs, const double *rho, const double *E,
 			}
 			total_sweeps++;
 		}
-		hipLaunchKernelGGL(k_axpy_t, dim3(g), dim3(kB), 0, st, xT.p, ld, d32.p, s, n, nrhs);
+		hipLaunchKernelGGL(k_axpy_t, dim3(g), dim3(kB), 0, st, xT.p, ld, d32.p, s, n, nrhs, nullptr, nullptr);
 		HIP_OK(hipGetLastError(), "sweep launch");
 	}
 	const double ms = ms_since(t0) - check_ms;
@@ -1367,7 +1309,7 @@ int LinearSystem::shoot(int nrhs, const double *rho, const double *E, const doub
 	return 0;
 }
 
-int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const double *g, double tol, int max_outer,
+int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const double *gin, double tol, int max_outer,
                           int sweeps, double *lambda, double *drho, double *info, std::string &err)
 {
 	Impl &d = *d_;
@@ -1390,38 +1332,35 @@ int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const do
 	int rt, Sg;
 	tile_config(nrhs, PREC_F16, &rt, &Sg);
 	const float inv = 1.0f / d.s16;
-	const int S = std::max(1, std::min(64, n / 256));
-	const int rows_per_split = (n + S - 1) / S;
-	const int fin_blocks = (int)((total + kB - 1) / kB);
-	Buf<double> rho64, g64, x64, r64, part64, blk, B64T, fb;
+	const int g = grid_for(total);
+	Buf<double> rho64, g64, xT, wT, r64, out, B64T, fb;
 	Fx64 fx;
 	if (fx.setup(n, ld, nrhs, err)) return -1;
 	Buf<float> rho32, r32, l32, part16;
 	Buf<_Float16> XT16;
 	const size_t xts = (size_t)rp * ld;
-	if (rho64.alloc(total, err) || g64.alloc(total, err) || x64.alloc(total, err) || r64.alloc(total, err) ||
-	    part64.alloc((size_t)S * total, err) || rho32.alloc(total, err) || r32.alloc(total, err) ||
+	const size_t xtn = (size_t)fx.rp * ld;
+	if (rho64.alloc(total, err) || g64.alloc(total, err) || xT.alloc(xtn, err) || wT.alloc(xtn, err) ||
+	    r64.alloc(total, err) || out.alloc(total, err) || rho32.alloc(total, err) || r32.alloc(total, err) ||
 	    l32.alloc(total, err) || part16.alloc((size_t)Sg * ld * rp, err) || XT16.alloc(xts, err) ||
-	    blk.alloc((size_t)std::max(fin_blocks, 8192) * 2, err) || B64T.alloc((size_t)fx.rp * ld, err) ||
-	    fb.alloc(total, err))
+	    B64T.alloc(xtn, err) || fb.alloc(total, err))
 		return -1;
 	hipLaunchKernelGGL(k_fill<_Float16>, dim3(grid_for(xts)), dim3(kB), 0, st, XT16.p, xts, (_Float16)0.f);
 	std::vector<float> h(total);
 	for (size_t t = 0; t < total; t++) h[t] = (float)rho[t];
 	HIP_OK(hipMemcpyAsync(rho32.p, h.data(), total * 4, hipMemcpyHostToDevice, st), "upload");
 	HIP_OK(hipMemcpyAsync(rho64.p, rho, total * 8, hipMemcpyHostToDevice, st), "upload");
-	HIP_OK(hipMemcpyAsync(g64.p, g, total * 8, hipMemcpyHostToDevice, st), "upload");
-	hipLaunchKernelGGL(k_fill<double>, dim3(grid_for(total)), dim3(kB), 0, st, x64.p, total, 0.0);
-	const dim3 tgrid(((n + 3) / 4 + kB - 1) / kB, S);  // four columns per lane
-	std::vector<double> hb((size_t)fin_blocks * 2);
+	HIP_OK(hipMemcpyAsync(g64.p, gin, total * 8, hipMemcpyHostToDevice, st), "upload");
+	hipLaunchKernelGGL(k_fill<double>, dim3(grid_for(xtn)), dim3(kB), 0, st, xT.p, xtn, 0.0);
+	hipLaunchKernelGGL(k_fill<double>, dim3(grid_for(xtn)), dim3(kB), 0, st, wT.p, xtn, 0.0);
 	HIP_OK(hipStreamSynchronize(st), "upload");
 	const auto t0 = std::chrono::steady_clock::now();
 	double enorm = -1.0, rel = 0.0;
 	int outer = 0, total_sweeps = 0;
 	double ss0 = 0.0, mx0 = 0.0;  // lambda = 0 at the start: the first residual is g
 	for (size_t t = 0; t < total; t++) {
-		ss0 += g[t] * g[t];
-		mx0 = std::max(mx0, std::fabs(g[t]));
+		ss0 += gin[t] * gin[t];
+		mx0 = std::max(mx0, std::fabs(gin[t]));
 	}
 	for (;; outer++) {
 		double ss = 0.0, mx = 0.0;
@@ -1429,19 +1368,12 @@ int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const do
 			HIP_OK(hipMemcpyAsync(r64.p, g64.p, total * 8, hipMemcpyDeviceToDevice, st), "residual");
 			ss = ss0;
 			mx = mx0;
-		} else {
-			// r = g + F^T (rho o x) - x in FP64
-			hipLaunchKernelGGL(k_ftx<double>, tgrid, dim3(kB), 0, st, d.F32.p, ld, n, nrhs, x64.p, rho64.p,
-			                   rows_per_split, part64.p);
-			hipLaunchKernelGGL(k_ftx_finish<double>, dim3(fin_blocks), dim3(kB), 0, st, part64.p, S, n, nrhs, g64.p,
-			                   x64.p, 1.0, r64.p, blk.p);
-			HIP_OK(hipGetLastError(), "adjoint residual");
-			HIP_OK(hipMemcpyAsync(hb.data(), blk.p, hb.size() * 8, hipMemcpyDeviceToHost, st), "reduce");
-			HIP_OK(hipStreamSynchronize(st), "reduce");
-			for (int b = 0; b < fin_blocks; b++) {
-				ss += hb[2 * b];
-				mx = std::max(mx, hb[2 * b + 1]);
-			}
+		} else if (fx.run(d.Ft.p, wT.p, g64.p, nullptr, xT.p, r64.p, st, ss, mx, true, err)) {
+			// r = g + F^T (rho o x) - x in FP64 over the transposed copy that
+			// the FP16 one is made from: its rows are read whole, where
+			// F's columns, split over row chunks, ran at a sixth of the
+			// rate (n = 6001: 151 + 8.6 -> 64 + 4 us)
+			return -1;
 		}
 		if (!std::isfinite(ss)) {
 			err = "adjoint diverged (non-finite residual)";
@@ -1450,20 +1382,19 @@ int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const do
 		if (enorm < 0) enorm = std::sqrt(ss);
 		rel = enorm > 0 ? std::sqrt(ss) / enorm : 0.0;
 		if (rel <= tol || outer >= max_outer || mx == 0.0) break;
-		const int gg = grid_for(total);
 		// d <- r (scaled), then sweeps d <- r + F^T (rho o d) with XT = rho o d
-		hipLaunchKernelGGL(k_scale<_Float16>, dim3(gg), dim3(kB), 0, st, r64.p, 1.0 / mx, total, nrhs, ld, r32.p,
+		hipLaunchKernelGGL(k_scale<_Float16>, dim3(g), dim3(kB), 0, st, r64.p, 1.0 / mx, total, nrhs, ld, r32.p,
 		                   XT16.p, rho32.p);
 		for (int m = 0; m < sweeps; m++) {
 			if (launch_gemm<_Float16>(rt, ct, d.FT16.p, XT16.p, part16.p, ld, rp, Sg, st)) {
 				err = "adjoint: no kernel for this tile";
 				return -1;
 			}
-			hipLaunchKernelGGL((k_jacobi<_Float16, true>), dim3(gg), dim3(kB), 0, st, part16.p, Sg, ld, rp, n, nrhs,
+			hipLaunchKernelGGL((k_jacobi<_Float16, true>), dim3(g), dim3(kB), 0, st, part16.p, Sg, ld, rp, n, nrhs,
 			                   inv, r32.p, rho32.p, l32.p, XT16.p);
 			total_sweeps++;
 		}
-		hipLaunchKernelGGL(k_axpy, dim3(gg), dim3(kB), 0, st, x64.p, l32.p, mx, total);
+		hipLaunchKernelGGL(k_axpy_t, dim3(g), dim3(kB), 0, st, xT.p, ld, l32.p, mx, n, nrhs, wT.p, rho64.p);
 		HIP_OK(hipGetLastError(), "adjoint sweep");
 	}
 	// dL/drho = lambda o (F B), F B in FP64
@@ -1473,10 +1404,11 @@ int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const do
 	HIP_OK(hipMemcpyAsync(B64T.p, bt.data(), bt.size() * 8, hipMemcpyHostToDevice, st), "upload");
 	{
 		double ss, mx;
-		if (fx.run(d.F32.p, B64T.p, nullptr, nullptr, 0.0, fb.p, st, ss, mx, false, err)) return -1;
+		if (fx.run(d.F32.p, B64T.p, nullptr, nullptr, nullptr, fb.p, st, ss, mx, false, err)) return -1;
 	}
+	hipLaunchKernelGGL(k_rows, dim3(g), dim3(kB), 0, st, xT.p, ld, n, nrhs, out.p);
 	std::vector<double> hfb(total);
-	HIP_OK(hipMemcpyAsync(lambda, x64.p, total * 8, hipMemcpyDeviceToHost, st), "download");
+	HIP_OK(hipMemcpyAsync(lambda, out.p, total * 8, hipMemcpyDeviceToHost, st), "download");
 	HIP_OK(hipMemcpyAsync(hfb.data(), fb.p, total * 8, hipMemcpyDeviceToHost, st), "download");
 	HIP_OK(hipStreamSynchronize(st), "adjoint");
 	const double ms = ms_since(t0);
