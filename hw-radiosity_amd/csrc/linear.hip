@@ -266,79 +266,120 @@ __global__ __launch_bounds__(kB) void k_fx64m(const float *__restrict__ F, const
 	                  s * kchunk, (s + 1) * kchunk);
 }
 
-// The same FP64 product for at most 4 right-hand sides on the vector FP64
+// The whole FP64 residual for NC <= 4 right-hand sides on the vector FP64
 // units, where a 16-column MFMA would spend 13 of its 16 columns on padding:
-// wave w of block b owns the kFxRows rows from kFxRows (4 b + w) over the whole K; per
-// step each lane takes 4 consecutive k of each row (one 16-byte load per
-// row, the next step's loads in flight) against x staged through LDS in
-// chunks of kFxChunk k (1024 or 256; 4 columns, FP64), then a butterfly
-// sums the lanes.
-// Writes part[row][c] (S = 1), c < 4; columns >= nrhs of xT are zero.
+// out[i][c] = base[i][c] + rho[i][c] * (F w)[i][c] - xT[c][i] (base, rho and xT
+// may be null: 0, 1 and 0) and, per block, the sum of squares and max |out|.
+// A wave owns kFxRows rows; per step each lane takes 4 consecutive k of each
+// row (one 16-byte load per row, the next step's loads in flight) against w
+// staged through LDS in chunks of 1024 k, column-major, so that a lane's 4
+// values are two 16-byte reads.  KS of the block's four waves share rows, each
+// taking every KS-th step of 256 k: a block is 32 / KS rows.  The 64 lane
+// partials of the 8 NC sums are combined by a reduce-scatter (the exchanges
+// over lane bits 5, 4, 3 halve the set each time and leave lane l with row
+// l >> 3), then the KS waves' in a fixed order.
+// Bound by HBM: 6.0-6.6 TB/s from n = 8192 up, FP64 work about half of that.
+// Against the form with one block size (32 rows), 32-way LDS conflicts, 4
+// columns for any NC and a second kernel for the residual (3 columns, us,
+// first kernel alone): n = 1024 10.8 -> 4.7, 4096 30.5 -> 16.6, 9216 88.7 ->
+// 61.9, 20224 290 -> 247, 32768 696 -> 643.
 constexpr int kFxRows = 8;
-template <int kFxChunk>
-__global__ __launch_bounds__(kB) void k_fx64v(const float *__restrict__ F, const double *__restrict__ xT,
-                                              double *__restrict__ part, int ld, int rp)
+constexpr int kFxChunk = 1024;
+template <int NC, int KS>
+__global__ __launch_bounds__(kB) void k_fx64v(const float *__restrict__ F, const double *__restrict__ wT, int ld, int n,
+                                              const double *xT, const double *base, const double *rho, double *out,
+                                              double *blk)
 {
 	typedef float fv4 __attribute__((ext_vector_type(4)));
-	__shared__ double xs[kFxChunk * 4];
+	typedef double dv2 __attribute__((ext_vector_type(2)));
+	constexpr int ROWS = 4 / KS * kFxRows, STEPS = kFxChunk / 256;
+	static_assert(kFxRows == 8 && ROWS * NC <= kB, "the reduce-scatter assumes 8 rows; one thread per result");
+	__shared__ double xs[NC * kFxChunk];
+	__shared__ double red[KS][ROWS * NC];
+	__shared__ double stat[8];
 	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-	const int r0 = (blockIdx.x * 4 + w) * kFxRows;
-	double acc[kFxRows][4];
+	const int rg = w / KS, ks = w % KS;
+	const float *Fr = F + (size_t)(blockIdx.x * ROWS + rg * kFxRows) * ld + 4 * lane;
+	const int ns = ld / 256;
+	double v[kFxRows * NC];
 #pragma unroll
-	for (int r = 0; r < kFxRows; r++)
-#pragma unroll
-		for (int c = 0; c < 4; c++) acc[r][c] = 0.0;
-	const float *Fr = F + (size_t)r0 * ld + 4 * lane;
+	for (int i = 0; i < kFxRows * NC; i++) v[i] = 0.0;
 	fv4 a[kFxRows], an[kFxRows];
 #pragma unroll
-	for (int r = 0; r < kFxRows; r++) a[r] = __builtin_nontemporal_load((const fv4 *)(Fr + (size_t)r * ld));
-	for (int k0 = 0; k0 < ld; k0 += kFxChunk) {
+	for (int r = 0; r < kFxRows; r++)
+		a[r] = __builtin_nontemporal_load((const fv4 *)(Fr + (size_t)r * ld + min(ks, ns - 1) * 256));
+	for (int s0 = 0; s0 < ns; s0 += STEPS) {
+		const int cnt = min(STEPS, ns - s0);
 		__syncthreads();  // the previous chunk's reads are done
-		for (int i = threadIdx.x; i < kFxChunk * 4; i += kB) {
-			const int c = i / kFxChunk, kk = i % kFxChunk;
-			xs[kk * 4 + c] = xT[(size_t)c * ld + k0 + kk];
-		}
+		for (int i = threadIdx.x; i < cnt * 128; i += kB)
+#pragma unroll
+			for (int c = 0; c < NC; c++)
+				*(dv2 *)(xs + c * kFxChunk + 2 * i) = *(const dv2 *)(wT + (size_t)c * ld + s0 * 256 + 2 * i);
 		__syncthreads();
 #pragma unroll 1
-		for (int st = 0; st < kFxChunk; st += 256) {
-			const int k = k0 + st;
-			if (k + 256 < ld) {
+		for (int q = ks; q < cnt; q += KS) {
+			const int sn = min(s0 + q + KS, ns - 1);  // clamped: the last load of a wave is not used
 #pragma unroll
-				for (int r = 0; r < kFxRows; r++)
-					an[r] = __builtin_nontemporal_load((const fv4 *)(Fr + (size_t)r * ld + k + 256));
-			}
-			const double *xl = xs + (st + 4 * lane) * 4;
+			for (int r = 0; r < kFxRows; r++)
+				an[r] = __builtin_nontemporal_load((const fv4 *)(Fr + (size_t)r * ld + sn * 256));
+			double x[NC][4];
 #pragma unroll
-			for (int j = 0; j < 4; j++) {
-				const double x0 = xl[4 * j], x1 = xl[4 * j + 1], x2 = xl[4 * j + 2], x3 = xl[4 * j + 3];
+			for (int c = 0; c < NC; c++)
+#pragma unroll
+				for (int j = 0; j < 4; j++) x[c][j] = xs[c * kFxChunk + q * 256 + 4 * lane + j];
+#pragma unroll
+			for (int j = 0; j < 4; j++)
 #pragma unroll
 				for (int r = 0; r < kFxRows; r++) {
 					const double f = (double)a[r][j];
-					acc[r][0] = __builtin_fma(f, x0, acc[r][0]);
-					acc[r][1] = __builtin_fma(f, x1, acc[r][1]);
-					acc[r][2] = __builtin_fma(f, x2, acc[r][2]);
-					acc[r][3] = __builtin_fma(f, x3, acc[r][3]);
+#pragma unroll
+					for (int c = 0; c < NC; c++) v[r * NC + c] = __builtin_fma(f, x[c][j], v[r * NC + c]);
 				}
-			}
 #pragma unroll
 			for (int r = 0; r < kFxRows; r++) a[r] = an[r];
 		}
 	}
 #pragma unroll
-	for (int r = 0; r < kFxRows; r++)
+	for (int half = kFxRows * NC / 2, bit = 32; bit >= 8; half >>= 1, bit >>= 1) {
+		const bool upper = (lane & bit) != 0;
 #pragma unroll
-		for (int c = 0; c < 4; c++) {
-			double v = acc[r][c];
-			for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off);
-			acc[r][c] = v;
+		for (int i = 0; i < half; i++) {
+			const double lo = v[i], hi = v[half + i];
+			v[i] = (upper ? hi : lo) + __shfl_xor(upper ? lo : hi, bit);
 		}
-	if (lane < kFxRows * 4) {
-		const int r = lane >> 2, c = lane & 3;
-		double v = 0.0;
+	}
 #pragma unroll
-		for (int q = 0; q < kFxRows * 4; q++)
-			if (q == lane) v = acc[q >> 2][q & 3];
-		part[(size_t)(r0 + r) * rp + c] = v;
+	for (int bit = 4; bit > 0; bit >>= 1)
+#pragma unroll
+		for (int c = 0; c < NC; c++) v[c] += __shfl_xor(v[c], bit);
+	if ((lane & 7) == 0)
+#pragma unroll
+		for (int c = 0; c < NC; c++) red[ks][(rg * kFxRows + (lane >> 3)) * NC + c] = v[c];
+	__syncthreads();
+	double ss = 0.0, mx = 0.0;
+	const int e = threadIdx.x, i = blockIdx.x * ROWS + e / NC, c = e % NC;
+	if (e < ROWS * NC && i < n) {
+		double y = red[0][e];
+#pragma unroll
+		for (int k = 1; k < KS; k++) y += red[k][e];
+		const size_t t = (size_t)i * NC + c;
+		const double o = (base ? base[t] : 0.0) + (rho ? rho[t] : 1.0) * y - (xT ? xT[(size_t)c * ld + i] : 0.0);
+		out[t] = o;
+		ss = o * o;
+		mx = fabs(o);
+	}
+	for (int off = 32; off > 0; off >>= 1) {
+		ss += __shfl_xor(ss, off);
+		mx = fmax(mx, __shfl_xor(mx, off));
+	}
+	if (lane == 0) {
+		stat[2 * w] = ss;
+		stat[2 * w + 1] = mx;
+	}
+	__syncthreads();
+	if (threadIdx.x == 0) {
+		blk[2 * blockIdx.x] = stat[0] + stat[2] + stat[4] + stat[6];
+		blk[2 * blockIdx.x + 1] = fmax(fmax(stat[1], stat[3]), fmax(stat[5], stat[7]));
 	}
 }
 
@@ -634,10 +675,10 @@ double power_sum(const std::vector<float> &a, const double *v, int n, int nrhs)
 
 }  // namespace
 
-// FP64 residual machinery: the caller's xT holds rp x ld doubles with rows
+// FP64 residual machinery: the caller's wT holds rp x ld doubles with rows
 // >= nrhs and columns >= n zero; split-K partials; per-block stats.
 struct Fx64 {
-	int n = 0, ld = 0, nrhs = 0, rp = 0, rt = 4, ct = 1, S = 1;
+	int n = 0, ld = 0, nrhs = 0, rp = 0, rt = 4, ct = 1, S = 1, ks = 1;
 	Buf<double> part, blk;
 	size_t nblk = 0;
 	std::vector<double> hb;
@@ -653,31 +694,61 @@ struct Fx64 {
 		rp = (nct + ct - 1) / ct * ct * 16;  // whole column groups: every tile the grid covers exists
 		const int tiles = (ld / (64 * rt)) * (rp / (16 * ct));
 		S = 1;
-		if (!vec())
+		if (vec()) {
+			// waves per row group (32 / ks rows a block): four below 8192 rows,
+			// where fewer leave CUs without a block (n = 6144: 33.6, 31.8 and
+			// 29.3 us at 1, 2 and 4; 4096: 22.5, 19.7, 16.6); above, as few as
+			// fill the last round of 256 CUs to 95 % (less traffic of w per
+			// row; us at 1, 2, 4: 8192 49.8, 59.1, 63.7; 9216 71.4, 67.6,
+			// 61.9; 12288 102.4, 98.0, 98.5; 20224 259.7, 246.8, 262.5;
+			// 32768 643, 667, 694)
+			ks = 4;
+			for (int k = 1; ld >= 8192 && k < 4; k *= 2) {
+				const int blocks = ld / 32 * k, full = (blocks + 255) / 256 * 256;
+				if (100 * blocks >= 95 * full) {
+					ks = k;
+					break;
+				}
+			}
+			nblk = (size_t)ld / 32 * ks;
+		} else {
 			while (S < 8 && tiles * S < 512 && (ld / (2 * S)) % 32 == 0) S *= 2;
-		nblk = ((size_t)n * nrhs + kB - 1) / kB;
-		if (part.alloc((size_t)S * ld * rp, err) || blk.alloc(std::max<size_t>(nblk, 8192) * 2, err)) return -1;
+			nblk = ((size_t)n * nrhs + kB - 1) / kB;
+			if (part.alloc((size_t)S * ld * rp, err)) return -1;
+		}
+		if (blk.alloc(nblk * 2, err)) return -1;
 		hb.assign(nblk * 2, 0.0);
 		return 0;
 	}
 	// at most 4 columns: the vector-unit kernel (ld is a multiple of 256:
-	// whole chunks of 1024 or 256 k, whole blocks of 4 kFxRows rows)
-	bool vec() const { return nrhs <= 4 && rp >= 4 && ld % 256 == 0 && ld % (4 * kFxRows) == 0; }
+	// whole steps of 256 k, whole blocks of 32 rows)
+	bool vec() const { return nrhs <= 4 && ld % 256 == 0; }
+	template <int NC> void launch_vec(const float *F, const double *wT, const double *base, const double *rho,
+	                                  const double *xT, double *out, hipStream_t st)
+	{
+		const dim3 g((unsigned)nblk), b(kB);
+		if (ks == 1) hipLaunchKernelGGL((k_fx64v<NC, 1>), g, b, 0, st, F, wT, ld, n, xT, base, rho, out, blk.p);
+		else if (ks == 2) hipLaunchKernelGGL((k_fx64v<NC, 2>), g, b, 0, st, F, wT, ld, n, xT, base, rho, out, blk.p);
+		else hipLaunchKernelGGL((k_fx64v<NC, 4>), g, b, 0, st, F, wT, ld, n, xT, base, rho, out, blk.p);
+	}
 	// out = base + rho o (F w) - x (xT null: 0); returns (sum of squares, max |out|)
 	int run(const float *F, const double *wT, const double *base, const double *rho, const double *xT, double *out,
 	        hipStream_t st, double &ss, double &mx, bool want_stats, std::string &err)
 	{
-		const dim3 grid(ld / (64 * rt), rp / (16 * ct), S);
-		const int kchunk = ld / S;
-		if (vec() && ld % 1024 == 0)
-			hipLaunchKernelGGL(k_fx64v<1024>, dim3(ld / (4 * kFxRows)), dim3(kB), 0, st, F, wT, part.p, ld, rp);
-		else if (vec())
-			hipLaunchKernelGGL(k_fx64v<256>, dim3(ld / (4 * kFxRows)), dim3(kB), 0, st, F, wT, part.p, ld, rp);
-		else if (ct == 4) hipLaunchKernelGGL((k_fx64m<2, 4>), grid, dim3(kB), 0, st, F, wT, part.p, ld, rp, kchunk);
-		else if (ct == 2) hipLaunchKernelGGL((k_fx64m<4, 2>), grid, dim3(kB), 0, st, F, wT, part.p, ld, rp, kchunk);
-		else hipLaunchKernelGGL((k_fx64m<4, 1>), grid, dim3(kB), 0, st, F, wT, part.p, ld, rp, kchunk);
-		hipLaunchKernelGGL(k_resid, dim3((unsigned)nblk), dim3(kB), 0, st, part.p, S, ld, rp, n, nrhs, xT, base, rho,
-		                   out, blk.p);
+		if (vec()) {
+			if (nrhs == 1) launch_vec<1>(F, wT, base, rho, xT, out, st);
+			else if (nrhs == 2) launch_vec<2>(F, wT, base, rho, xT, out, st);
+			else if (nrhs == 3) launch_vec<3>(F, wT, base, rho, xT, out, st);
+			else launch_vec<4>(F, wT, base, rho, xT, out, st);
+		} else {
+			const dim3 grid(ld / (64 * rt), rp / (16 * ct), S);
+			const int kchunk = ld / S;
+			if (ct == 4) hipLaunchKernelGGL((k_fx64m<2, 4>), grid, dim3(kB), 0, st, F, wT, part.p, ld, rp, kchunk);
+			else if (ct == 2) hipLaunchKernelGGL((k_fx64m<4, 2>), grid, dim3(kB), 0, st, F, wT, part.p, ld, rp, kchunk);
+			else hipLaunchKernelGGL((k_fx64m<4, 1>), grid, dim3(kB), 0, st, F, wT, part.p, ld, rp, kchunk);
+			hipLaunchKernelGGL(k_resid, dim3((unsigned)nblk), dim3(kB), 0, st, part.p, S, ld, rp, n, nrhs, xT, base, rho,
+			                   out, blk.p);
+		}
 		HIP_OK(hipGetLastError(), "FP64 product");
 		ss = mx = 0.0;
 		if (!want_stats) return 0;
@@ -1372,7 +1443,7 @@ int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const do
 			// r = g + F^T (rho o x) - x in FP64 over the transposed copy that
 			// the FP16 one is made from: its rows are read whole, where
 			// F's columns, split over row chunks, ran at a sixth of the
-			// rate (n = 6001: 151 + 8.6 -> 64 + 4 us)
+			// rate (n = 6001: 151 + 8.6 -> 29 us)
 			return -1;
 		}
 		if (!std::isfinite(ss)) {
