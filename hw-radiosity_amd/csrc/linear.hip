@@ -18,9 +18,10 @@
 // A[l%16][8*(l/16)+j] and B[8*(l/16)+j][l%16], j = 0..7, and receives
 // D[4*(l/16)+j][l%16], j = 0..3.  A wave owns 16*RT rows and all 16*CT
 // right-hand-side columns, so F is read from HBM once per sweep; split-K S
-// spreads the K loop over S blocks whose partial tiles the epilogue sums in a
-// fixed order (results do not depend on timing).  (RT, S) per (CT, precision)
-// come from the autotuner, which times GEMM + epilogue for each candidate.
+// spreads the K loop over S waves of a block (over S blocks for 8 or 12 column
+// tiles), whose partial tiles are summed in a fixed order (results do not
+// depend on timing).  (RT, S) go by the size (sweep_tile); for 8 or 12 column
+// tiles the autotuner times a whole sweep for each candidate.
 #include "linear.h"
 
 #include <hip/hip_runtime.h>
@@ -30,6 +31,7 @@
 #include <cmath>
 #include <cstring>
 #include <map>
+#include <type_traits>
 #include <vector>
 
 namespace rgpu {
@@ -37,14 +39,127 @@ namespace {
 
 #include "lin_common.h"
 
-// part[s][row][col] = sum over the s-th K chunk of A[row][k] X[k][col]
+// What becomes of a low-precision product y = (A X)[i][c]: with y given, the
+// product itself, y[i][c] = inv y.  Else one Jacobi sweep, v = rhs + rho o (inv
+// y) and XTn <- v (fragment order); with rho_in (the adjoint's sweep v <- r +
+// F^T (rho o v)) v = rhs + inv y and XTn <- rho o v.  Padding of XTn (rows >=
+// nrhs, k >= n) is never written and stays zero.  With xT (the last sweep of a
+// refinement) the FP64 iterate takes the correction, xT[c][i] += s v, and wT
+// (the adjoint's product input) becomes rho64 o xT.
+template <typename E> struct SweepOut {
+	int n, nrhs;
+	float inv;
+	bool rho_in;
+	const float *rhs, *rho;
+	E *XTn;
+	double *xT, s, *wT;
+	const double *rho64;
+	float *y;
+
+	__device__ __forceinline__ void put(int i, int c, int ld, float sum) const
+	{
+		const size_t t = (size_t)i * nrhs + c;
+		if (y) {
+			y[t] = sum * inv;
+			return;
+		}
+		const float v = rho_in ? rhs[t] + sum * inv : rhs[t] + rho[t] * (sum * inv);
+		XTn[frag_index(c, i, ld)] = (E)(rho_in ? rho[t] * v : v);
+		if (xT) {
+			const size_t q = (size_t)c * ld + i;
+			const double x = xT[q] + s * (double)v;
+			xT[q] = x;
+			if (wT) wT[q] = rho64[t] * x;
+		}
+	}
+};
+
+// One sweep in one launch.  A block is eight waves: 8 / S row groups of 16 RT
+// rows, the K range of each split over S waves.  Each wave streams its A
+// fragments (two register sets of two k-blocks, one loading while the other
+// feeds the MFMAs; the index is clamped past the chunk's end, those k-blocks
+// are not multiplied), the partial tiles meet in LDS and are summed in chunk
+// order, and the block's threads finish their rows (SweepOut).  The next
+// iterate goes to a second buffer, as other blocks still read this one.
+// A is read without the non-temporal policy where it stays in the 256 MB
+// last-level cache from sweep to sweep (cached).
+// Bound by that cache or HBM: the split inside the block keeps every CU busy
+// where a block per row group and a second kernel for the sweep's update left
+// CUs idle and paid a launch (one column tile, us per sweep, before -> now:
+// n = 1024 8.0 -> 3.2, 4096 12.5 -> 5.3, 6144 20 -> 12.5, 9216 39 -> 25.0,
+// 20224 187 -> 137 (6.0 TB/s), 32768 313 -> 302 (7.1 TB/s)).
+constexpr int kSweepWaves = 8;
 template <typename E, int RT, int CT>
-__global__ __launch_bounds__(kB) void k_gemm(const E *__restrict__ A, const E *__restrict__ XT, float *__restrict__ part,
-                                             int ld, int rp, int kchunk)
+__global__ __launch_bounds__(kSweepWaves * 64) void k_sweep(const E *__restrict__ A, const E *__restrict__ XT, int ld,
+                                                            int S, bool cached, SweepOut<E> o)
 {
-	const int w = threadIdx.x >> 6;
-	const int s = blockIdx.y, kb0 = s * (kchunk >> 5);
-	gemm_tile<E, RT, CT>(A, XT, part + (size_t)s * ld * rp, ld, rp, (blockIdx.x * 4 + w) * RT, kb0, kb0 + (kchunk >> 5));
+	typedef typename VecOf<E>::type V;
+	constexpr int U = 2;
+	__shared__ f4 red[kSweepWaves * RT * CT * 64];
+	const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const int WR = kSweepWaves / S, wr = w % WR, s = w / WR;
+	const int nkb = ld >> 5, cnt = nkb / S, nrt = ld >> 4;  // ld is a multiple of 256: nkb of 8
+	const int rt0 = (blockIdx.x * WR + wr) * RT;
+	const V *Ap[RT];
+#pragma unroll
+	for (int r = 0; r < RT; r++) Ap[r] = (const V *)A + ((size_t)min(rt0 + r, nrt - 1) * nkb + s * cnt) * 64 + lane;
+	const V *Bp = (const V *)XT + (size_t)(s * cnt) * 64 + lane;
+	f4 acc[RT][CT];
+#pragma unroll
+	for (int r = 0; r < RT; r++)
+#pragma unroll
+		for (int c = 0; c < CT; c++) acc[r][c] = f4{0.f, 0.f, 0.f, 0.f};
+	V a[2][U][RT], b[2][U][CT];
+	auto run = [&](auto nt) {
+		auto load = [&](int p, int k0) {
+#pragma unroll
+			for (int u = 0; u < U; u++) {
+				const size_t k = (size_t)min(k0 + u, cnt - 1);
+#pragma unroll
+				for (int r = 0; r < RT; r++) {
+					if constexpr (decltype(nt)::value) a[p][u][r] = __builtin_nontemporal_load(Ap[r] + k * 64);
+					else a[p][u][r] = Ap[r][k * 64];
+				}
+#pragma unroll
+				for (int c = 0; c < CT; c++) b[p][u][c] = Bp[((size_t)c * nkb + k) * 64];
+			}
+		};
+		auto mma = [&](int p, int k0) {
+#pragma unroll
+			for (int u = 0; u < U; u++)
+				if (k0 + u < cnt) {
+#pragma unroll
+					for (int r = 0; r < RT; r++)
+#pragma unroll
+						for (int c = 0; c < CT; c++) acc[r][c] = mfma(a[p][u][r], b[p][u][c], acc[r][c]);
+				}
+		};
+		load(0, 0);
+		for (int k = 0; k < cnt; k += 2 * U) {
+			load(1, k + U);
+			mma(0, k);
+			load(0, k + 2 * U);
+			mma(1, k + U);
+		}
+	};
+	if (cached) run(std::integral_constant<bool, false>{});
+	else run(std::integral_constant<bool, true>{});
+#pragma unroll
+	for (int r = 0; r < RT; r++)
+#pragma unroll
+		for (int c = 0; c < CT; c++) red[(((s * WR + wr) * RT + r) * CT + c) * 64 + lane] = acc[r][c];
+	__syncthreads();
+	// element (row, column) of a 16 x 16 tile: lane 16 (row / 4) + column, value row % 4
+	const float *rf = (const float *)red;
+	const int rows = WR * RT * 16, row0 = blockIdx.x * rows, part = WR * RT * CT * 256;
+	for (int e = threadIdx.x; e < rows * o.nrhs; e += kSweepWaves * 64) {
+		const int rl = e / o.nrhs, c = e - rl * o.nrhs;
+		if (row0 + rl >= o.n) break;
+		const float *q = rf + ((rl >> 4) * CT + (c >> 4)) * 256 + (((rl & 15) >> 2) * 16 + (c & 15)) * 4 + (rl & 3);
+		float y = 0.f;
+		for (int k = 0; k < S; k++) y += q[k * part];
+		o.put(row0 + rl, c, ld, y);
+	}
 }
 
 // Wide right-hand sides (NCT = 8 or 12 column tiles) with the operands
@@ -235,22 +350,15 @@ __global__ __launch_bounds__(512) void k_gemm_dma(const E *__restrict__ A, const
 			}
 }
 
-// d = rhs + rho o (inv_s * sum_s part); XT <- d (fragment order).
-// Padding of XT (rows >= nrhs, k >= n) is never written and stays zero.
-// RHO_IN (the adjoint's sweep d <- r + F^T (rho o d)): v = rhs + inv_s * sum
-// part and XT <- rho o v instead.
-template <typename E, bool RHO_IN = false>
-__global__ void k_jacobi(const float *part, int S, int ld, int rp, int n, int nrhs, float inv_s, const float *rhs,
-                         const float *rho, float *d, E *XT)
+// The sweep's second half after k_gemm_dma: its split-K partials summed in order
+template <typename E> __global__ void k_finish(const float *part, int S, int ld, int rp, SweepOut<E> o)
 {
-	const size_t total = (size_t)n * nrhs;
+	const size_t total = (size_t)o.n * o.nrhs;
 	for (size_t t = blockIdx.x * (size_t)kB + threadIdx.x; t < total; t += (size_t)gridDim.x * kB) {
-		const int i = (int)(t / nrhs), c = (int)(t % nrhs);
+		const int i = (int)(t / o.nrhs), c = (int)(t % o.nrhs);
 		float y = 0.f;
 		for (int s = 0; s < S; s++) y += part[((size_t)s * ld + i) * rp + c];
-		const float v = RHO_IN ? rhs[t] + y * inv_s : rhs[t] + rho[t] * (y * inv_s);
-		d[t] = v;
-		XT[frag_index(c, i, ld)] = (E)(RHO_IN ? rho[t] * v : v);
+		o.put(i, c, ld, y);
 	}
 }
 
@@ -430,20 +538,6 @@ __global__ void k_scale(const double *r64, double inv_s, size_t total, int nrhs,
 	}
 }
 
-// xT[c][i] += s * d[i][c]; with wT, wT[c][i] <- rho[i][c] * xT[c][i] (the
-// adjoint's product input)
-__global__ void k_axpy_t(double *xT, int ld, const float *d, double s, int n, int nrhs, double *wT = nullptr,
-                         const double *rho = nullptr)
-{
-	const size_t total = (size_t)n * nrhs;
-	for (size_t t = blockIdx.x * (size_t)kB + threadIdx.x; t < total; t += (size_t)gridDim.x * kB) {
-		const size_t q = (size_t)(t % nrhs) * ld + t / nrhs;
-		const double x = xT[q] + s * (double)d[t];
-		xT[q] = x;
-		if (wT) wT[q] = rho[t] * x;
-	}
-}
-
 // out[i][c] = xT[c][i]
 __global__ void k_rows(const double *xT, int ld, int n, int nrhs, double *out)
 {
@@ -611,55 +705,72 @@ int pick_ct(int nrhs)
 	return -1;
 }
 
-template <typename E>
-int launch_gemm(int rt, int ct, const E *A, const E *XT, float *part, int ld, int rp, int S, hipStream_t st)
+// the wide kernels' tiles: split-K over blocks, partials in part
+bool dma_tile(int rt, int ct) { return ct >= 8 && rt >= 2; }
+
+// the matrix's 16-bit copy stays in the 256 MB last-level cache between
+// sweeps: up to 11.5k rows (us per sweep, cached against non-temporal: n = 4096
+// 5.3, 8.0; 9216 25.0, 37.1; 12288 48.9, 50.6; 16384 95.6, 82.9; 20224 144.5,
+// 136.5)
+bool stays_cached(int ld) { return 2 * (size_t)ld * ld <= (size_t)256 << 20; }
+
+// The sweep's tile for ct <= 4 where none was tuned or forced: the smallest
+// row group whose blocks fit the 256 CUs in one round (16, 32, 64 rows a block
+// with every wave on the same rows, or 128).  Of the twelve tiles, timed at 21
+// sizes from 512 to 32768 rows, this one is the fastest or within 6 % of it
+// (one column tile, us: n = 4096 (1, 8) 5.4, (2, 8) 6.2; 6144 (1, 8) 13.7, (2,
+// 8) 12.5; 9216 (2, 8) 30.7, (4, 8) 24.7; four column tiles: 20224 (4, 8)
+// 205.3, (4, 4) 197.6).  Past 16384 rows one column tile does better with more
+// blocks of 32 rows (20224: 136.3 against 142.2).
+void sweep_tile(int ct, int ld, int &rt, int &S)
 {
-	const dim3 grid(ld / (64 * rt), S), blk(kB);
-	const int kchunk = ld / S;
-#define G(R, C) hipLaunchKernelGGL((k_gemm<E, R, C>), grid, blk, 0, st, A, XT, part, ld, rp, kchunk)
-#define GR(R)                 \
-	switch (ct) {             \
-	case 1: G(R, 1); break;   \
-	case 2: G(R, 2); break;   \
-	case 4: G(R, 4); break;   \
-	case 8: G(R, 8); break;   \
-	case 12: G(R, 12); break; \
-	default: return -1;       \
+	rt = ld <= 4096 ? 1 : ld <= 8192 ? 2 : 4;
+	S = 8;
+	if (ld > 16384) {
+		rt = ct == 1 ? 2 : 4;
+		S = ct == 1 ? 8 : 4;
 	}
-	if (rt == 1) {
-		GR(1)
-	} else if (rt == 2 && ct == 8) {
-		hipLaunchKernelGGL((k_gemm_dma<E, 8, 2, 1>), dim3(ld / 256, S), dim3(512), 0, st, A, XT, part, ld, rp, kchunk);
-	} else if (rt == 2 && ct == 12) {
-		hipLaunchKernelGGL((k_gemm_dma<E, 12, 2, 1>), dim3(ld / 256, S), dim3(512), 0, st, A, XT, part, ld, rp, kchunk);
-	} else if (rt == 2) {
-		GR(2)
-	} else if (rt == 4 && ct <= 4) {
-		switch (ct) {
-		case 1: G(4, 1); break;
-		case 2: G(4, 2); break;
-		case 4: G(4, 4); break;
-		default: return -1;
-		}
-	} else if (rt == 4 && ct == 8) {
-		hipLaunchKernelGGL((k_gemm_dma<E, 8, 4, 2>), dim3(ld / 256, S), dim3(512), 0, st, A, XT, part, ld, rp, kchunk);
-	} else if (rt == 4 && ct == 12) {
-		hipLaunchKernelGGL((k_gemm_dma<E, 12, 4, 2>), dim3(ld / 256, S), dim3(512), 0, st, A, XT, part, ld, rp, kchunk);
-	} else {
-		return -1;
-	}
-#undef GR
-#undef G
-	return 0;
 }
 
+// One product with the tile (rt, S) and what follows it (o).  finish = false:
+// the wide tiles' product only (for timing it alone).
+template <typename E>
+int launch_sweep(int rt, int ct, int S, const E *A, const E *XT, float *part, int ld, int rp, const SweepOut<E> &o,
+                 hipStream_t st, bool finish = true)
+{
+	if (dma_tile(rt, ct)) {
+		const dim3 grid(ld / 256, S), blk(512);
+		const int kchunk = ld / S;
+		if (rt == 2 && ct == 8) hipLaunchKernelGGL((k_gemm_dma<E, 8, 2, 1>), grid, blk, 0, st, A, XT, part, ld, rp, kchunk);
+		else if (rt == 2 && ct == 12) hipLaunchKernelGGL((k_gemm_dma<E, 12, 2, 1>), grid, blk, 0, st, A, XT, part, ld, rp, kchunk);
+		else if (rt == 4 && ct == 8) hipLaunchKernelGGL((k_gemm_dma<E, 8, 4, 2>), grid, blk, 0, st, A, XT, part, ld, rp, kchunk);
+		else if (rt == 4 && ct == 12) hipLaunchKernelGGL((k_gemm_dma<E, 12, 4, 2>), grid, blk, 0, st, A, XT, part, ld, rp, kchunk);
+		else return -1;
+		if (finish)
+			hipLaunchKernelGGL(k_finish<E>, dim3(grid_for((size_t)o.n * o.nrhs)), dim3(kB), 0, st, part, S, ld, rp, o);
+		return 0;
+	}
+	const int wr = kSweepWaves / S * rt;  // row tiles per block
+	const dim3 grid((ld / 16 + wr - 1) / wr), blk(kSweepWaves * 64);
+	const bool cached = stays_cached(ld);
+#define G(R, C) \
+	if (rt == R && ct == C) { \
+		hipLaunchKernelGGL((k_sweep<E, R, C>), grid, blk, 0, st, A, XT, ld, S, cached, o); \
+		return 0; \
+	}
+	G(1, 1) G(1, 2) G(1, 4) G(1, 8) G(1, 12)
+	G(2, 1) G(2, 2) G(2, 4)
+	G(4, 1) G(4, 2) G(4, 4)
+#undef G
+	return -1;
+}
+
+// tiles set_tile takes: whole blocks of 64 rt rows (256 for the wide kernels),
+// whole chunks of 32 k, and per chunk a multiple of 8 k-blocks (4 for 8 or 12
+// column tiles at rt = 1; any for the wide kernels)
 bool valid_tile(int rt, int ct, int S, int ld)
 {
-	// k-blocks per pipelined loop trip: 2 * GemmUnroll<ct>::U, 2 * U of the
-	// four-wave LDS kernel (8 or 12 column tiles, rt = 4: U = 4 or 2), or 1
-	// for the eight-wave LDS DMA kernel (8 or 12 column tiles, rt = 2);
-	// rows per block: 64 rt, or 256 for the eight-wave kernel
-	const bool dma = ct >= 8 && (rt == 2 || rt == 4);
+	const bool dma = dma_tile(rt, ct);
 	const int u2 = dma ? 1 : 2 * (ct <= 4 ? 4 : 2);
 	const int rows = dma ? 256 : 64 * rt;
 	return ld % rows == 0 && ld % (32 * S) == 0 && (ld / 32 / S) % u2 == 0 && ld / 32 / S >= 1;
@@ -830,6 +941,152 @@ struct LinearSystem::Impl {
 		havet16 = true;
 		return 0;
 	}
+
+	// the tile of a solve: tuned or forced, else by rule, tuned here for the
+	// wide tiles
+	int solve_tile(LinearSystem &L, int nrhs, int prec, int &rt, int &S, std::string &err)
+	{
+		const int ct = pick_ct(nrhs);
+		if (!tiles.count({ct, prec})) {
+			if (ct <= 4) {
+				sweep_tile(ct, L.ld(), rt, S);
+				return 0;
+			}
+			if (L.autotune(nrhs, prec, err)) return -1;
+		}
+		L.tile_config(nrhs, prec, &rt, &S);
+		return 0;
+	}
+
+	// the iterate's two buffers (rp x ld, fragment order), zeroed
+	template <typename E> int iterates(Buf<E> (&X)[2], size_t count, std::string &err)
+	{
+		for (Buf<E> &x : X) {
+			if (x.alloc(count, err)) return -1;
+			hipLaunchKernelGGL(k_fill<E>, dim3(grid_for(count)), dim3(kB), 0, st, x.p, count, (E)0.f);
+		}
+		return 0;
+	}
+
+	// times one sweep for every (rows per wave, split-K) and keeps the fastest
+	template <typename E> int tune(const E *A, int n, int ld, int nrhs, int prec, std::string &err)
+	{
+		const int ct = pick_ct(nrhs), rp = ct * 16;
+		const size_t total = (size_t)n * nrhs;
+		Buf<E> X[2];
+		Buf<float> part, r32, rho;
+		if (iterates(X, (size_t)rp * ld, err) || r32.alloc(total, err) || rho.alloc(total, err) ||
+		    (ct >= 8 && part.alloc((size_t)8 * ld * rp, err)))
+			return -1;
+		hipLaunchKernelGGL(k_fill<float>, dim3(grid_for(total)), dim3(kB), 0, st, r32.p, total, 1.0f);
+		hipLaunchKernelGGL(k_fill<float>, dim3(grid_for(total)), dim3(kB), 0, st, rho.p, total, 0.5f);
+		SweepOut<E> o{};
+		o.n = n, o.nrhs = nrhs, o.inv = 1.0f, o.rhs = r32.p, o.rho = rho.p, o.XTn = X[1].p;
+		double best = 1e30;
+		int brt = 0, bs = 0;
+		for (int rt : {1, 2, 4}) {
+			for (int S : {1, 2, 4, 8}) {
+				if (dma_tile(rt, ct) && !valid_tile(rt, ct, S, ld)) continue;
+				if (launch_sweep<E>(rt, ct, S, A, X[0].p, part.p, ld, rp, o, st)) continue;  // warm-up
+				HIP_OK(hipEventRecord(e0, st), "event");
+				for (int k = 0; k < 3; k++) launch_sweep<E>(rt, ct, S, A, X[0].p, part.p, ld, rp, o, st);
+				HIP_OK(hipEventRecord(e1, st), "event");
+				HIP_OK(hipEventSynchronize(e1), "event");
+				float ms = 0;
+				HIP_OK(hipEventElapsedTime(&ms, e0, e1), "event");
+				if (ms < best) {
+					best = ms;
+					brt = rt;
+					bs = S;
+				}
+			}
+		}
+		HIP_OK(hipGetLastError(), "autotune");
+		HIP_OK(hipStreamSynchronize(st), "autotune");
+		if (!brt) {
+			err = "autotune: no valid tile";
+			return -1;
+		}
+		tiles[{ct, prec}] = {brt, bs};
+		return 0;
+	}
+
+	template <typename E>
+	int time_product(const E *A, int n, int ld, int nrhs, int prec, int reps, double *ms, std::string &err)
+	{
+		const int ct = pick_ct(nrhs), rp = ct * 16;
+		const auto [rt, S] = tiles.at({ct, prec});
+		const size_t total = (size_t)n * nrhs, xts = (size_t)rp * ld;
+		Buf<E> x;
+		Buf<float> part, y;
+		if (x.alloc(xts, err) || y.alloc(total, err) || (dma_tile(rt, ct) && part.alloc((size_t)S * ld * rp, err)))
+			return -1;
+		hipLaunchKernelGGL(k_fill<E>, dim3(grid_for(xts)), dim3(kB), 0, st, x.p, xts, (E)1.f);
+		SweepOut<E> o{};
+		o.n = n, o.nrhs = nrhs, o.inv = 1.0f, o.y = y.p;
+		launch_sweep<E>(rt, ct, S, A, x.p, part.p, ld, rp, o, st, false);
+		HIP_OK(hipEventRecord(e0, st), "event");
+		for (int k = 0; k < reps; k++) launch_sweep<E>(rt, ct, S, A, x.p, part.p, ld, rp, o, st, false);
+		HIP_OK(hipEventRecord(e1, st), "event");
+		HIP_OK(hipEventSynchronize(e1), "event");
+		HIP_OK(hipGetLastError(), "gemm_ms");
+		float t = 0;
+		HIP_OK(hipEventElapsedTime(&t, e0, e1), "event");
+		*ms = t / reps;
+		return 0;
+	}
+
+	// Y = F X in prec; the tuned or forced tile, else one wave per 16 rows
+	template <typename E>
+	int product(const E *A, float inv, int n, int ld, int nrhs, int prec, const double *X, double *Y, std::string &err)
+	{
+		const int ct = pick_ct(nrhs), rp = ct * 16;
+		int rt = 1, S = 1;
+		if (const auto it = tiles.find({ct, prec}); it != tiles.end()) {
+			rt = it->second.first;
+			S = it->second.second;
+		}
+		const size_t total = (size_t)n * nrhs, xts = (size_t)rp * ld;
+		Buf<E> x;
+		Buf<float> part, y;
+		Buf<double> x64;
+		if (x.alloc(xts, err) || y.alloc(total, err) || x64.alloc(total, err) ||
+		    (dma_tile(rt, ct) && part.alloc((size_t)S * ld * rp, err)))
+			return -1;
+		HIP_OK(hipMemcpyAsync(x64.p, X, total * 8, hipMemcpyHostToDevice, st), "upload");
+		hipLaunchKernelGGL(k_fill<E>, dim3(grid_for(xts)), dim3(kB), 0, st, x.p, xts, (E)0.f);
+		hipLaunchKernelGGL(k_scale<E>, dim3(grid_for(total)), dim3(kB), 0, st, x64.p, 1.0, total, nrhs, ld, y.p, x.p);
+		SweepOut<E> o{};
+		o.n = n, o.nrhs = nrhs, o.inv = inv, o.y = y.p;
+		if (launch_sweep<E>(rt, ct, S, A, x.p, part.p, ld, rp, o, st)) {
+			err = "multiply: no kernel for this tile";
+			return -1;
+		}
+		HIP_OK(hipGetLastError(), "multiply");
+		std::vector<float> hy(total);
+		HIP_OK(hipMemcpyAsync(hy.data(), y.p, total * 4, hipMemcpyDeviceToHost, st), "download");
+		HIP_OK(hipStreamSynchronize(st), "multiply");
+		for (size_t t = 0; t < total; t++) Y[t] = hy[t];
+		return 0;
+	}
+
+	// the sweeps of one refinement (v <- rhs + .. from X[0]); the last one
+	// adds the correction to the iterate
+	template <typename E>
+	int sweep(const E *A, Buf<E> (&X)[2], float *part, int ct, int rt, int S, int ld, int sweeps, SweepOut<E> o,
+	          std::string &err)
+	{
+		double *xT = o.xT;
+		for (int m = 0; m < sweeps; m++) {
+			o.XTn = X[(m + 1) & 1].p;
+			o.xT = m == sweeps - 1 ? xT : nullptr;
+			if (launch_sweep<E>(rt, ct, S, A, X[m & 1].p, part, ld, ct * 16, o, st)) {
+				err = "no kernel for this tile";
+				return -1;
+			}
+		}
+		return 0;
+	}
 };
 
 LinearSystem::~LinearSystem()
@@ -945,65 +1202,12 @@ int LinearSystem::autotune(int nrhs, int prec, std::string &err)
 		err = "autotune: nrhs must be 1..192 and precision FP16 or BF16";
 		return -1;
 	}
-	const int rp = ct * 16, ld = np_, n = n_;
-	if (d.ensure_lowp(prec, ld, err)) return -1;
-	const size_t total = (size_t)n * nrhs;
-	Buf<_Float16> xt16;
-	Buf<__bf16> xtb;
-	Buf<float> part, r32, d32, rho;
-	if (part.alloc((size_t)8 * ld * rp, err) || r32.alloc(total, err) || d32.alloc(total, err) || rho.alloc(total, err))
-		return -1;
-	const int g = grid_for(total);
-	const size_t xts = (size_t)rp * ld;
-	hipLaunchKernelGGL(k_fill<float>, dim3(g), dim3(kB), 0, d.st, r32.p, total, 1.0f);
-	hipLaunchKernelGGL(k_fill<float>, dim3(g), dim3(kB), 0, d.st, rho.p, total, 0.5f);
-	if (prec == PREC_F16) {
-		if (xt16.alloc(xts, err)) return -1;
-		hipLaunchKernelGGL(k_fill<_Float16>, dim3(grid_for(xts)), dim3(kB), 0, d.st, xt16.p, xts, (_Float16)0.f);
-	} else {
-		if (xtb.alloc(xts, err)) return -1;
-		hipLaunchKernelGGL(k_fill<__bf16>, dim3(grid_for(xts)), dim3(kB), 0, d.st, xtb.p, xts, (__bf16)0.f);
-	}
-	auto sweep = [&](int rt, int S) -> int {
-		if (prec == PREC_F16) {
-			if (launch_gemm<_Float16>(rt, ct, d.F16.p, xt16.p, part.p, ld, rp, S, d.st)) return -1;
-			hipLaunchKernelGGL(k_jacobi<_Float16>, dim3(g), dim3(kB), 0, d.st, part.p, S, ld, rp, n, nrhs, 1.0f, r32.p,
-			                   rho.p, d32.p, xt16.p);
-		} else {
-			if (launch_gemm<__bf16>(rt, ct, d.FB16.p, xtb.p, part.p, ld, rp, S, d.st)) return -1;
-			hipLaunchKernelGGL(k_jacobi<__bf16>, dim3(g), dim3(kB), 0, d.st, part.p, S, ld, rp, n, nrhs, 1.0f, r32.p,
-			                   rho.p, d32.p, xtb.p);
-		}
-		return 0;
-	};
-	double best = 1e30;
-	int brt = 0, bs = 0;
-	for (int rt : {1, 2, 4}) {
-		for (int S : {1, 2, 4, 8}) {
-			if (!valid_tile(rt, ct, S, ld)) continue;
-			if (sweep(rt, S)) continue;  // warm-up
-			HIP_OK(hipEventRecord(d.e0, d.st), "event");
-			for (int k = 0; k < 3; k++) sweep(rt, S);
-			HIP_OK(hipEventRecord(d.e1, d.st), "event");
-			HIP_OK(hipEventSynchronize(d.e1), "event");
-			float ms = 0;
-			HIP_OK(hipEventElapsedTime(&ms, d.e0, d.e1), "event");
-			if (ms < best) {
-				best = ms;
-				brt = rt;
-				bs = S;
-			}
-		}
-	}
-	HIP_OK(hipGetLastError(), "autotune");
-	HIP_OK(hipStreamSynchronize(d.st), "autotune");
-	if (!brt) {
-		err = "autotune: no valid tile";
-		return -1;
-	}
-	d.tiles[{ct, prec}] = {brt, bs};
-	return 0;
+	if (d.ensure_lowp(prec, np_, err)) return -1;
+	const int rc = prec == PREC_F16 ? d.tune<_Float16>(d.F16.p, n_, np_, nrhs, prec, err)
+	                                : d.tune<__bf16>(d.FB16.p, n_, np_, nrhs, prec, err);
+	return rc;
 }
+
 
 int LinearSystem::gemm_ms(int nrhs, int prec, int reps, double *ms, std::string &err)
 {
@@ -1014,36 +1218,9 @@ int LinearSystem::gemm_ms(int nrhs, int prec, int reps, double *ms, std::string 
 		return -1;
 	}
 	if (!d.tiles.count({ct, prec}) && autotune(nrhs, prec, err)) return -1;
-	int rt, S;
-	tile_config(nrhs, prec, &rt, &S);
-	const int rp = ct * 16, ld = np_;
-	if (d.ensure_lowp(prec, ld, err)) return -1;
-	Buf<_Float16> xt16;
-	Buf<__bf16> xtb;
-	Buf<float> part;
-	const size_t xts = (size_t)rp * ld;
-	if (part.alloc((size_t)S * ld * rp, err)) return -1;
-	if (prec == PREC_F16) {
-		if (xt16.alloc(xts, err)) return -1;
-		hipLaunchKernelGGL(k_fill<_Float16>, dim3(grid_for(xts)), dim3(kB), 0, d.st, xt16.p, xts, (_Float16)1.f);
-	} else {
-		if (xtb.alloc(xts, err)) return -1;
-		hipLaunchKernelGGL(k_fill<__bf16>, dim3(grid_for(xts)), dim3(kB), 0, d.st, xtb.p, xts, (__bf16)1.f);
-	}
-	auto one = [&]() {
-		if (prec == PREC_F16) launch_gemm<_Float16>(rt, ct, d.F16.p, xt16.p, part.p, ld, rp, S, d.st);
-		else launch_gemm<__bf16>(rt, ct, d.FB16.p, xtb.p, part.p, ld, rp, S, d.st);
-	};
-	one();
-	HIP_OK(hipEventRecord(d.e0, d.st), "event");
-	for (int k = 0; k < reps; k++) one();
-	HIP_OK(hipEventRecord(d.e1, d.st), "event");
-	HIP_OK(hipEventSynchronize(d.e1), "event");
-	HIP_OK(hipGetLastError(), "gemm_ms");
-	float t = 0;
-	HIP_OK(hipEventElapsedTime(&t, d.e0, d.e1), "event");
-	*ms = t / reps;
-	return 0;
+	if (d.ensure_lowp(prec, np_, err)) return -1;
+	return prec == PREC_F16 ? d.time_product<_Float16>(d.F16.p, n_, np_, nrhs, prec, reps, ms, err)
+	                        : d.time_product<__bf16>(d.FB16.p, n_, np_, nrhs, prec, reps, ms, err);
 }
 
 int LinearSystem::multiply(int prec, int nrhs, const double *X, double *Y, std::string &err)
@@ -1054,7 +1231,7 @@ int LinearSystem::multiply(int prec, int nrhs, const double *X, double *Y, std::
 		err = "multiply: nrhs must be 1..192";
 		return -1;
 	}
-	const int n = n_, ld = np_, rp = ct * 16;
+	const int n = n_, ld = np_;
 	const size_t total = (size_t)n * nrhs;
 	hipStream_t st = d.st;
 	if (prec == PREC_F32) {
@@ -1073,51 +1250,8 @@ int LinearSystem::multiply(int prec, int nrhs, const double *X, double *Y, std::
 		return 0;
 	}
 	if (d.ensure_lowp(prec, ld, err)) return -1;
-	int rt, S;
-	tile_config(nrhs, prec, &rt, &S);
-	if (!rt) {
-		rt = 1;
-		S = 1;
-	}
-	Buf<float> part, zero, ones, y;
-	Buf<double> x64;
-	Buf<_Float16> xt16;
-	Buf<__bf16> xtb;
-	if (part.alloc((size_t)S * ld * rp, err) || zero.alloc(total, err) || ones.alloc(total, err) || y.alloc(total, err) ||
-	    x64.alloc(total, err))
-		return -1;
-	const int g = grid_for(total);
-	const size_t xts = (size_t)rp * ld;
-	hipLaunchKernelGGL(k_fill<float>, dim3(g), dim3(kB), 0, st, zero.p, total, 0.0f);
-	hipLaunchKernelGGL(k_fill<float>, dim3(g), dim3(kB), 0, st, ones.p, total, 1.0f);
-	HIP_OK(hipMemcpyAsync(x64.p, X, total * 8, hipMemcpyHostToDevice, st), "upload");
-	const float inv = 1.0f / (prec == PREC_F16 ? d.s16 : d.sb16);
-	int rc;
-	if (prec == PREC_F16) {
-		if (xt16.alloc(xts, err)) return -1;
-		hipLaunchKernelGGL(k_fill<_Float16>, dim3(grid_for(xts)), dim3(kB), 0, st, xt16.p, xts, (_Float16)0.f);
-		hipLaunchKernelGGL(k_scale<_Float16>, dim3(g), dim3(kB), 0, st, x64.p, 1.0, total, nrhs, ld, y.p, xt16.p);
-		rc = launch_gemm<_Float16>(rt, ct, d.F16.p, xt16.p, part.p, ld, rp, S, st);
-		hipLaunchKernelGGL(k_jacobi<_Float16>, dim3(g), dim3(kB), 0, st, part.p, S, ld, rp, n, nrhs, inv, zero.p, ones.p,
-		                   y.p, xt16.p);
-	} else {
-		if (xtb.alloc(xts, err)) return -1;
-		hipLaunchKernelGGL(k_fill<__bf16>, dim3(grid_for(xts)), dim3(kB), 0, st, xtb.p, xts, (__bf16)0.f);
-		hipLaunchKernelGGL(k_scale<__bf16>, dim3(g), dim3(kB), 0, st, x64.p, 1.0, total, nrhs, ld, y.p, xtb.p);
-		rc = launch_gemm<__bf16>(rt, ct, d.FB16.p, xtb.p, part.p, ld, rp, S, st);
-		hipLaunchKernelGGL(k_jacobi<__bf16>, dim3(g), dim3(kB), 0, st, part.p, S, ld, rp, n, nrhs, inv, zero.p, ones.p,
-		                   y.p, xtb.p);
-	}
-	if (rc) {
-		err = "multiply: no kernel for this tile";
-		return -1;
-	}
-	HIP_OK(hipGetLastError(), "multiply");
-	std::vector<float> hy(total);
-	HIP_OK(hipMemcpyAsync(hy.data(), y.p, total * 4, hipMemcpyDeviceToHost, st), "download");
-	HIP_OK(hipStreamSynchronize(st), "multiply");
-	for (size_t t = 0; t < total; t++) Y[t] = hy[t];
-	return 0;
+	return prec == PREC_F16 ? d.product<_Float16>(d.F16.p, 1.0f / d.s16, n, ld, nrhs, prec, X, Y, err)
+	                        : d.product<__bf16>(d.FB16.p, 1.0f / d.sb16, n, ld, nrhs, prec, X, Y, err);
 }
 
 int LinearSystem::gather(int prec, int nrhs, const double *rho, const double *E, double tol, int max_outer, int sweeps,
@@ -1138,32 +1272,25 @@ int LinearSystem::gather(int prec, int nrhs, const double *rho, const double *E,
 		return -1;
 	}
 	if (d.ensure_lowp(prec, np_, err)) return -1;
-	if (!d.tiles.count({ct, prec}) && autotune(nrhs, prec, err)) return -1;
 	int rt, S;
-	tile_config(nrhs, prec, &rt, &S);
+	if (d.solve_tile(*this, nrhs, prec, rt, S, err)) return -1;
 	const int n = n_, ld = np_, rp = ct * 16;
 	const size_t total = (size_t)n * nrhs;
 	const float inv = 1.0f / (prec == PREC_F16 ? d.s16 : d.sb16);
 	hipStream_t st = d.st;
-	Buf<float> rho32, r32, d32, part;
+	Buf<float> rho32, r32, part;
 	Buf<double> rho64, E64, xT, r64, blk, Bref64;
-	Buf<_Float16> XT16;
-	Buf<__bf16> XTb;
+	Buf<_Float16> XT16[2];
+	Buf<__bf16> XTb[2];
 	Fx64 fx;
 	if (fx.setup(n, ld, nrhs, err)) return -1;
 	const size_t xtn = (size_t)fx.rp * ld;
-	if (rho32.alloc(total, err) || r32.alloc(total, err) || d32.alloc(total, err) ||
-	    part.alloc((size_t)S * ld * rp, err) || rho64.alloc(total, err) || E64.alloc(total, err) ||
+	if (rho32.alloc(total, err) || r32.alloc(total, err) ||
+	    (dma_tile(rt, ct) && part.alloc((size_t)S * ld * rp, err)) || rho64.alloc(total, err) || E64.alloc(total, err) ||
 	    xT.alloc(xtn, err) || r64.alloc(total, err) || blk.alloc(8192 * 2, err))
 		return -1;
 	const size_t xts = (size_t)rp * ld;
-	if (prec == PREC_F16) {
-		if (XT16.alloc(xts, err)) return -1;
-		hipLaunchKernelGGL(k_fill<_Float16>, dim3(grid_for(xts)), dim3(kB), 0, st, XT16.p, xts, (_Float16)0.f);
-	} else {
-		if (XTb.alloc(xts, err)) return -1;
-		hipLaunchKernelGGL(k_fill<__bf16>, dim3(grid_for(xts)), dim3(kB), 0, st, XTb.p, xts, (__bf16)0.f);
-	}
+	if (prec == PREC_F16 ? d.iterates(XT16, xts, err) : d.iterates(XTb, xts, err)) return -1;
 	std::vector<float> h32(total);
 	for (size_t t = 0; t < total; t++) h32[t] = (float)rho[t];
 	HIP_OK(hipMemcpyAsync(rho32.p, h32.data(), total * 4, hipMemcpyHostToDevice, st), "upload");
@@ -1221,28 +1348,18 @@ int LinearSystem::gather(int prec, int nrhs, const double *rho, const double *E,
 		}
 		if (rel <= tol || outer >= max_outer || mx == 0.0) break;
 		const double s = mx;
-		if (prec == PREC_F16)
-			hipLaunchKernelGGL(k_scale<_Float16>, dim3(g), dim3(kB), 0, st, r64.p, 1.0 / s, total, nrhs, ld, r32.p, XT16.p);
-		else
-			hipLaunchKernelGGL(k_scale<__bf16>, dim3(g), dim3(kB), 0, st, r64.p, 1.0 / s, total, nrhs, ld, r32.p, XTb.p);
-		for (int m = 0; m < sweeps; m++) {
-			int rc;
-			if (prec == PREC_F16) {
-				rc = launch_gemm<_Float16>(rt, ct, d.F16.p, XT16.p, part.p, ld, rp, S, st);
-				hipLaunchKernelGGL(k_jacobi<_Float16>, dim3(g), dim3(kB), 0, st, part.p, S, ld, rp, n, nrhs, inv, r32.p,
-				                   rho32.p, d32.p, XT16.p);
-			} else {
-				rc = launch_gemm<__bf16>(rt, ct, d.FB16.p, XTb.p, part.p, ld, rp, S, st);
-				hipLaunchKernelGGL(k_jacobi<__bf16>, dim3(g), dim3(kB), 0, st, part.p, S, ld, rp, n, nrhs, inv, r32.p,
-				                   rho32.p, d32.p, XTb.p);
-			}
-			if (rc) {
-				err = "gather: no kernel for this tile";
-				return -1;
-			}
-			total_sweeps++;
-		}
-		hipLaunchKernelGGL(k_axpy_t, dim3(g), dim3(kB), 0, st, xT.p, ld, d32.p, s, n, nrhs, nullptr, nullptr);
+		int rc;
+		auto refine = [&](const auto *A, auto &X) {
+			typedef std::remove_cv_t<std::remove_pointer_t<decltype(A)>> T;
+			hipLaunchKernelGGL(k_scale<T>, dim3(g), dim3(kB), 0, st, r64.p, 1.0 / s, total, nrhs, ld, r32.p, X[0].p);
+			SweepOut<T> o{};
+			o.n = n, o.nrhs = nrhs, o.inv = inv, o.rhs = r32.p, o.rho = rho32.p, o.xT = xT.p, o.s = s;
+			rc = d.sweep(A, X, part.p, ct, rt, S, ld, sweeps, o, err);
+		};
+		if (prec == PREC_F16) refine(d.F16.p, XT16);
+		else refine(d.FB16.p, XTb);
+		if (rc) return -1;
+		total_sweeps += sweeps;
 		HIP_OK(hipGetLastError(), "sweep launch");
 	}
 	const double ms = ms_since(t0) - check_ms;
@@ -1399,24 +1516,21 @@ int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const do
 	// the transposed fragment copy); the residual stays FP64 over FP32 F
 	const int ct = pick_ct(nrhs), rp = ct * 16;
 	if (d.ensure_t16(ld, err)) return -1;
-	if (!d.tiles.count({ct, PREC_F16}) && autotune(nrhs, PREC_F16, err)) return -1;
 	int rt, Sg;
-	tile_config(nrhs, PREC_F16, &rt, &Sg);
+	if (d.solve_tile(*this, nrhs, PREC_F16, rt, Sg, err)) return -1;
 	const float inv = 1.0f / d.s16;
 	const int g = grid_for(total);
 	Buf<double> rho64, g64, xT, wT, r64, out, B64T, fb;
 	Fx64 fx;
 	if (fx.setup(n, ld, nrhs, err)) return -1;
-	Buf<float> rho32, r32, l32, part16;
-	Buf<_Float16> XT16;
+	Buf<float> rho32, r32;
+	Buf<_Float16> XT16[2];
 	const size_t xts = (size_t)rp * ld;
 	const size_t xtn = (size_t)fx.rp * ld;
 	if (rho64.alloc(total, err) || g64.alloc(total, err) || xT.alloc(xtn, err) || wT.alloc(xtn, err) ||
 	    r64.alloc(total, err) || out.alloc(total, err) || rho32.alloc(total, err) || r32.alloc(total, err) ||
-	    l32.alloc(total, err) || part16.alloc((size_t)Sg * ld * rp, err) || XT16.alloc(xts, err) ||
-	    B64T.alloc(xtn, err) || fb.alloc(total, err))
+	    d.iterates(XT16, xts, err) || B64T.alloc(xtn, err) || fb.alloc(total, err))
 		return -1;
-	hipLaunchKernelGGL(k_fill<_Float16>, dim3(grid_for(xts)), dim3(kB), 0, st, XT16.p, xts, (_Float16)0.f);
 	std::vector<float> h(total);
 	for (size_t t = 0; t < total; t++) h[t] = (float)rho[t];
 	HIP_OK(hipMemcpyAsync(rho32.p, h.data(), total * 4, hipMemcpyHostToDevice, st), "upload");
@@ -1455,17 +1569,12 @@ int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const do
 		if (rel <= tol || outer >= max_outer || mx == 0.0) break;
 		// d <- r (scaled), then sweeps d <- r + F^T (rho o d) with XT = rho o d
 		hipLaunchKernelGGL(k_scale<_Float16>, dim3(g), dim3(kB), 0, st, r64.p, 1.0 / mx, total, nrhs, ld, r32.p,
-		                   XT16.p, rho32.p);
-		for (int m = 0; m < sweeps; m++) {
-			if (launch_gemm<_Float16>(rt, ct, d.FT16.p, XT16.p, part16.p, ld, rp, Sg, st)) {
-				err = "adjoint: no kernel for this tile";
-				return -1;
-			}
-			hipLaunchKernelGGL((k_jacobi<_Float16, true>), dim3(g), dim3(kB), 0, st, part16.p, Sg, ld, rp, n, nrhs,
-			                   inv, r32.p, rho32.p, l32.p, XT16.p);
-			total_sweeps++;
-		}
-		hipLaunchKernelGGL(k_axpy_t, dim3(g), dim3(kB), 0, st, xT.p, ld, l32.p, mx, n, nrhs, wT.p, rho64.p);
+		                   XT16[0].p, rho32.p);
+		SweepOut<_Float16> o{};
+		o.n = n, o.nrhs = nrhs, o.inv = inv, o.rho_in = true, o.rhs = r32.p, o.rho = rho32.p;
+		o.xT = xT.p, o.s = mx, o.wT = wT.p, o.rho64 = rho64.p;
+		if (d.sweep(d.FT16.p, XT16, nullptr, ct, rt, Sg, ld, sweeps, o, err)) return -1;
+		total_sweeps += sweeps;
 		HIP_OK(hipGetLastError(), "adjoint sweep");
 	}
 	// dL/drho = lambda o (F B), F B in FP64

@@ -24,3 +24,24 @@ def test_f64_product_few_columns(n, nrhs):
     F64 = F.astype(np.float64)
     # any order of summation stays within (n + 1) u of the sum of magnitudes; the reference's own order likewise
     assert (np.abs(Y - F64 @ X) <= 2 * (n + 1) * U64 * (F64 @ np.abs(X))).all()
+
+
+# sweeps at the edges of the tile rule (16, 32, 64 and 128 or 32 rows a block:
+# padded sizes up to 4096, 8192, 16384, beyond) and ragged ends; the solution
+# satisfies the system in float64
+@pytest.mark.parametrize("n,nrhs", [(1, 1), (17, 3), (256, 16), (4096, 3), (4097, 17), (8193, 3), (8193, 33), (16500, 1),
+                                    (16500, 17)])
+@pytest.mark.parametrize("prec", ["f16", "bf16"])
+def test_gather_tile_rule(n, nrhs, prec):
+    rng = np.random.default_rng(n)
+    F = rng.random((n, n), np.float32) * np.float32(1.8 / n)  # rows sum to about 0.9
+    rho = rng.uniform(0.2, 0.7, (n, nrhs))
+    E = rng.uniform(0.0, 1.0, (n, nrhs))
+    tol = 1e-9
+    with radgpu.LinearSystem(n) as lin:
+        lin.set_matrix(F)
+        B, info = lin.gather(rho, E, prec=prec, tol=tol, max_outer=40, sweeps=5)
+    assert info["rel_res"] <= tol
+    r = E + rho * (F.astype(np.float64) @ B) - B
+    # the solver's own residual and this one differ by rounding in float64 only
+    assert np.linalg.norm(r) <= tol * np.linalg.norm(E) + 1e-12 * np.linalg.norm(B)
