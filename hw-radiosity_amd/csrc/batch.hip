@@ -19,6 +19,8 @@
 #include "batch.h"
 #include "linear.h"
 
+#include "pack.h"
+
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -31,6 +33,7 @@ namespace rgpu {
 namespace {
 
 #include "lin_common.h"
+#include "stage.h"
 
 constexpr int NR = 3;           // right-hand sides per scene (RGB)
 constexpr int kKChunk = 2048;   // k per residual tile
@@ -249,6 +252,23 @@ __global__ __launch_bounds__(kB) void k_bjacobi(const int2 *etiles, int e0, int 
 	}
 }
 
+// rho in FP32
+__global__ void k_brho(const double *rho, size_t total, float *rho32)
+{
+	for (size_t t = blockIdx.x * (size_t)kB + threadIdx.x; t < total; t += (size_t)gridDim.x * kB) rho32[t] = (float)rho[t];
+}
+
+// out = x, the scenes' rows in the caller's order
+__global__ __launch_bounds__(kB) void k_brows(const int2 *etiles, int ne, const BMeta *meta, const double *xT, double *out)
+{
+	for (int t = blockIdx.x; t < ne; t += gridDim.x) {
+		const int2 et = etiles[t];
+		const BMeta m = meta[et.x];
+		const int idx = et.y + threadIdx.x;
+		if (idx < m.n * NR) out[m.voff + idx] = xT[m.xoff + (size_t)(idx % NR) * m.ld + idx / NR];
+	}
+}
+
 // x += scale * d
 __global__ __launch_bounds__(kB) void k_baxpy(const int2 *etiles, int e0, int e1, const BMeta *meta,
                                               const int *active, const double *scale, const float *d, double *xT)
@@ -276,6 +296,8 @@ struct SceneBatch::Impl {
 	bool forced = false;    // set_tile overrides the autotuner
 	hipStream_t st = nullptr;
 	hipEvent_t e0 = nullptr, e1 = nullptr;
+	Stage stage;
+	Buf<double> out;  // the answer as the caller takes it
 	Buf<float> F32, r32, d32, rho32, part32;
 	Buf<_Float16> F16, X16;
 	Buf<__bf16> FB, XB;
@@ -557,7 +579,7 @@ SceneBatch *SceneBatch::create(int count, const int *n, std::string &err)
 	}
 	const size_t V = d.vsize;
 	if (d.F32.alloc(d.fsize, e) || d.r32.alloc(V, e) || d.d32.alloc(V, e) || d.rho32.alloc(V, e) ||
-	    d.part32.alloc(d.gsize, e) || d.E64.alloc(V, e) || d.rho64.alloc(V, e) || d.r64.alloc(V, e) ||
+	    d.part32.alloc(d.gsize, e) || d.E64.alloc(V, e) || d.rho64.alloc(V, e) || d.r64.alloc(V, e) || d.out.alloc(V, e) || d.stage.init(e) ||
 	    d.xT.alloc(d.xsize, e) || d.part64.alloc(d.psize, e) || d.blk.alloc((size_t)d.netiles * 2, e) ||
 	    d.enorm.alloc(count, e) || d.rel.alloc(count, e) || d.scale.alloc(count, e) || d.active.alloc(count, e) ||
 	    d.d_tb.alloc(count, e) || d.d_te.alloc(count, e) || d.d_etb.alloc(count, e) || d.d_ete.alloc(count, e) ||
@@ -652,11 +674,10 @@ int SceneBatch::solve(int prec, bool graph, const double *rho, const double *E, 
 		if (b.rt == 0 ? autotune(prec, got, err) : d.set_sched(b, err)) return -1;
 	}
 	const size_t V = d.vsize;
-	std::vector<float> h(V);
-	for (size_t t = 0; t < V; t++) h[t] = (float)rho[t];
-	HIP_OK(hipMemcpyAsync(d.rho32.p, h.data(), V * 4, hipMemcpyHostToDevice, d.st), "upload");
-	HIP_OK(hipMemcpyAsync(d.rho64.p, rho, V * 8, hipMemcpyHostToDevice, d.st), "upload");
-	HIP_OK(hipMemcpyAsync(d.E64.p, E, V * 8, hipMemcpyHostToDevice, d.st), "upload");
+	HIP_OK(hipStreamSynchronize(d.st), "batch solve");  // nothing of an earlier call is in flight
+	d.stage.begin();
+	if (d.stage.up(d.rho64.p, rho, V * 8, d.st, err) || d.stage.up(d.E64.p, E, V * 8, d.st, err)) return -1;
+	hipLaunchKernelGGL(k_brho, dim3(grid_for(V)), dim3(kB), 0, d.st, d.rho64.p, V, d.rho32.p);
 	HIP_OK(hipStreamSynchronize(d.st), "upload");
 	const float inv = prec == PREC_F16 ? 1.0f / d.s16 : 1.0f;
 	double build_ms = 0.0;
@@ -710,21 +731,17 @@ int SceneBatch::solve(int prec, bool graph, const double *rho, const double *E, 
 		HIP_OK(hipEventRecord(d.e1, d.st), "event");
 	}
 	HIP_OK(hipGetLastError(), "batch launch");
-	HIP_OK(hipEventSynchronize(d.e1), "batch solve");
+	hipLaunchKernelGGL(k_brows, dim3(std::max(1, std::min(kPersist * 4, d.netiles))), dim3(kB), 0, d.st, d.etiles.p,
+	                   d.netiles, d.d_meta.p, d.xT.p, d.out.p);
+	HIP_OK(hipGetLastError(), "batch launch");
+	std::vector<int> act(d.count);
+	if (d.stage.down(Bout, d.out.p, V * 8, d.st, err) || d.stage.down(rel_res, d.rel.p, (size_t)d.count * 8, d.st, err) ||
+	    d.stage.down(act.data(), d.active.p, (size_t)d.count * 4, d.st, err))
+		return -1;
 	float ms = 0.f;
 	HIP_OK(hipEventElapsedTime(&ms, d.e0, d.e1), "event");
-	std::vector<double> hx(d.xsize);
-	std::vector<int> act(d.count);
-	HIP_OK(hipMemcpy(hx.data(), d.xT.p, d.xsize * 8, hipMemcpyDeviceToHost), "download");
-	HIP_OK(hipMemcpy(rel_res, d.rel.p, d.count * 8, hipMemcpyDeviceToHost), "download");
-	HIP_OK(hipMemcpy(act.data(), d.active.p, d.count * 4, hipMemcpyDeviceToHost), "download");
 	int above = 0;
-	for (int s = 0; s < d.count; s++) {
-		const BMeta &m = d.meta[s];
-		for (int i = 0; i < m.n; i++)
-			for (int c = 0; c < NR; c++) Bout[(size_t)m.voff + (size_t)i * NR + c] = hx[(size_t)m.xoff + (size_t)c * m.ld + i];
-		above += act[s];
-	}
+	for (int s = 0; s < d.count; s++) above += act[s];
 	if (info) {
 		info[0] = ms;
 		info[1] = build_ms;

@@ -79,6 +79,8 @@ public:
 
 private:
 	DeviceEngine() = default;
+	int run_cast(int n, const RayIn *rays, void *dray, int *o, int *hit, int *cells, int *tests, bool grow,
+	             std::string &err);
 	struct Impl;
 	Impl *d_ = nullptr;
 	double shoot_ms_ = 0, kernel_ms_ = 0, cast_ms_ = 0;

@@ -1490,6 +1490,8 @@ void launch_cast(hipStream_t st, const DScene &S, const RayIn *rays, int n, int 
 // the rays and their three results for up to kStaticRays rays per call.  One
 // array per GPU, held until the process ends; every call on a GPU shares it.
 constexpr int kStaticRays = RAD_CAST_STATIC_MAX;
+// rays whose buffers (44 bytes each) rad_cast keeps between calls
+constexpr int kCastKeep = 1 << 22;
 constexpr size_t kStaticRayBytes = (size_t)kStaticRays * sizeof(RayIn);
 constexpr size_t kStaticBytes = kStaticRayBytes + (size_t)3 * kStaticRays * sizeof(int);
 static __device__ __align__(256) unsigned char scratch[kStaticBytes];
@@ -2055,6 +2057,8 @@ template <typename T> __global__ void k_fill_n(T *p, size_t n, T v)
 		}                                                                         \
 	} while (0)
 
+#include "stage.h"
+
 // A device array of n elements; the allocation is kept and reused while
 // later sizes fit in it.
 template <typename T> struct DevBuf {
@@ -2071,6 +2075,12 @@ template <typename T> struct DevBuf {
 		HIP_OK(hipMalloc(&p, count * sizeof(T)), "hipMalloc");
 		cap = count;
 		return 0;
+	}
+	void release()
+	{
+		if (p) (void)hipFree(p);
+		p = nullptr;
+		n = cap = 0;
 	}
 	int put(const T *src, size_t count, hipStream_t s, std::string &err)
 	{
@@ -2175,6 +2185,9 @@ struct DeviceEngine::Impl {
 	DevBuf<float> v3ff;
 	DevBuf<unsigned char> v3act;
 	hipEvent_t ev0 = nullptr, ev1 = nullptr;
+	Stage stage;
+	DevBuf<RayIn> cast_rays;  // rad_cast: rays, then hit, cells and tests (kept for the next call up to kCastKeep rays)
+	DevBuf<int> cast_out;
 	void *scratch = nullptr;  // this device's address of the static scratch (rad_cast_static)
 	// kGraphIters shooting iterations captured once per upload and replayed
 	hipGraphExec_t graph_exec = nullptr;
@@ -2229,7 +2242,7 @@ DeviceEngine *DeviceEngine::create(std::string &err)
 			delete e;
 			return nullptr;
 		}
-	if (scratch_address(&e->d_->scratch, err)) {
+	if (e->d_->stage.init(err) || scratch_address(&e->d_->scratch, err)) {
 		delete e;
 		return nullptr;
 	}
@@ -2683,19 +2696,39 @@ int DeviceEngine::cast(int n, const RayIn *rays, int *hit, int *cells, int *test
 {
 	Impl &d = *d_;
 	if (n <= 0) return 0;
-	DevBuf<RayIn> dr;
-	DevBuf<int> dh, dc, dt;
+	if (d.cast_rays.alloc(n, err) || d.cast_out.alloc((size_t)3 * n, err)) return -1;
+	if (run_cast(n, rays, d.cast_rays.p, d.cast_out.p, hit, cells, tests, true, err)) return -1;
+	if (n > kCastKeep) {
+		d.cast_rays.release();
+		d.cast_out.release();
+	}
+	return 0;
+}
+
+// n rays through dray, their hit, cells and tests through o (3 n ints): one
+// copy back; grow: as Stage's
+int DeviceEngine::run_cast(int n, const RayIn *rays, void *dray, int *o, int *hit, int *cells, int *tests, bool grow,
+                           std::string &err)
+{
+	Impl &d = *d_;
 	hipStream_t st = d.stream;
-	if (dr.put(rays, n, st, err) || dh.alloc(n, err) || dc.alloc(n, err) || dt.alloc(n, err)) return -1;
+	RayIn *dr = static_cast<RayIn *>(dray);
+	HIP_OK(hipStreamSynchronize(st), "cast");  // nothing of an earlier call is in flight
+	d.stage.begin();
+	if (d.stage.up(dr, rays, (size_t)n * sizeof(RayIn), st, err, grow)) return -1;
 	HIP_OK(hipEventRecord(d.ev0, st), "event");
-	if (d.fma) launch_cast<true>(st, d.S, dr.p, n, dh.p, dc.p, dt.p);
-	else launch_cast<false>(st, d.S, dr.p, n, dh.p, dc.p, dt.p);
+	if (d.fma) launch_cast<true>(st, d.S, dr, n, o, o + n, o + 2 * (size_t)n);
+	else launch_cast<false>(st, d.S, dr, n, o, o + n, o + 2 * (size_t)n);
 	HIP_OK(hipGetLastError(), "cast launch");
 	HIP_OK(hipEventRecord(d.ev1, st), "event");
-	HIP_OK(hipMemcpyAsync(hit, dh.p, n * sizeof(int), hipMemcpyDeviceToHost, st), "cast");
-	if (cells) HIP_OK(hipMemcpyAsync(cells, dc.p, n * sizeof(int), hipMemcpyDeviceToHost, st), "cast");
-	if (tests) HIP_OK(hipMemcpyAsync(tests, dt.p, n * sizeof(int), hipMemcpyDeviceToHost, st), "cast");
-	HIP_OK(hipStreamSynchronize(st), "cast");
+	const size_t b = (size_t)n * sizeof(int);
+	if (cells && tests) {
+		const Stage::Part parts[3] = {{hit, b}, {cells, b}, {tests, b}};
+		if (d.stage.down_parts(o, parts, 3, st, err, grow)) return -1;
+	} else if (d.stage.down(hit, o, b, st, err, grow) || (cells && d.stage.down(cells, o + n, b, st, err, grow)) ||
+	           (tests && d.stage.down(tests, o + 2 * (size_t)n, b, st, err, grow))) {
+		return -1;
+	}
 	float ms = 0;
 	if (hipEventElapsedTime(&ms, d.ev0, d.ev1) == hipSuccess) cast_ms_ = ms;
 	return 0;
@@ -2757,26 +2790,10 @@ int DeviceEngine::cast_static(int n, const RayIn *rays, int *hit, int *cells, in
 		err = "rad_cast_static: no static scratch on this device";
 		return -1;
 	}
-	// staging in this device's scratch: rays, then hit, cells and tests;
-	// k_cast writes every result, so nothing needs clearing
+	// in this device's scratch: rays, then hit, cells and tests; k_cast writes
+	// every result, so nothing needs clearing
 	unsigned char *base = static_cast<unsigned char *>(d.scratch);
-	RayIn *dr = reinterpret_cast<RayIn *>(base);
-	int *dh = reinterpret_cast<int *>(base + kStaticRayBytes);
-	int *dc = dh + kStaticRays, *dt = dc + kStaticRays;
-	hipStream_t st = d.stream;
-	HIP_OK(hipMemcpyAsync(dr, rays, (size_t)n * sizeof(RayIn), hipMemcpyHostToDevice, st), "upload");
-	HIP_OK(hipEventRecord(d.ev0, st), "event");
-	if (d.fma) launch_cast<true>(st, d.S, dr, n, dh, dc, dt);
-	else launch_cast<false>(st, d.S, dr, n, dh, dc, dt);
-	HIP_OK(hipGetLastError(), "cast launch");
-	HIP_OK(hipEventRecord(d.ev1, st), "event");
-	HIP_OK(hipMemcpyAsync(hit, dh, (size_t)n * sizeof(int), hipMemcpyDeviceToHost, st), "cast");
-	if (cells) HIP_OK(hipMemcpyAsync(cells, dc, (size_t)n * sizeof(int), hipMemcpyDeviceToHost, st), "cast");
-	if (tests) HIP_OK(hipMemcpyAsync(tests, dt, (size_t)n * sizeof(int), hipMemcpyDeviceToHost, st), "cast");
-	HIP_OK(hipStreamSynchronize(st), "cast");
-	float ms = 0;
-	if (hipEventElapsedTime(&ms, d.ev0, d.ev1) == hipSuccess) cast_ms_ = ms;
-	return 0;
+	return run_cast(n, rays, base, reinterpret_cast<int *>(base + kStaticRayBytes), hit, cells, tests, false, err);
 }
 
 int DeviceEngine::ff_pairs(int n, const int *pairs, float *ff3, std::string &err)

@@ -24,6 +24,8 @@
 // tiles the autotuner times a whole sweep for each candidate.
 #include "linear.h"
 
+#include "pack.h"
+
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -38,18 +40,19 @@ namespace rgpu {
 namespace {
 
 #include "lin_common.h"
+#include "stage.h"
 
 // What becomes of a low-precision product y = (A X)[i][c]: with y given, the
 // product itself, y[i][c] = inv y.  Else one Jacobi sweep, v = rhs + rho o (inv
 // y) and XTn <- v (fragment order); with rho_in (the adjoint's sweep v <- r +
 // F^T (rho o v)) v = rhs + inv y and XTn <- rho o v.  Padding of XTn (rows >=
 // nrhs, k >= n) is never written and stays zero.  With xT (the last sweep of a
-// refinement) the FP64 iterate takes the correction, xT[c][i] += s v, and wT
-// (the adjoint's product input) becomes rho64 o xT.
+// refinement) the FP64 iterate takes the correction, xT[c][i] += s v (first:
+// xT[c][i] = s v), and wT (the adjoint's product input) becomes rho64 o xT.
 template <typename E> struct SweepOut {
 	int n, nrhs;
 	float inv;
-	bool rho_in;
+	bool rho_in, first;
 	const float *rhs, *rho;
 	E *XTn;
 	double *xT, s, *wT;
@@ -67,7 +70,7 @@ template <typename E> struct SweepOut {
 		XTn[frag_index(c, i, ld)] = (E)(rho_in ? rho[t] * v : v);
 		if (xT) {
 			const size_t q = (size_t)c * ld + i;
-			const double x = xT[q] + s * (double)v;
+			const double x = (first ? 0.0 : xT[q]) + s * (double)v;
 			xT[q] = x;
 			if (wT) wT[q] = rho64[t] * x;
 		}
@@ -538,13 +541,78 @@ __global__ void k_scale(const double *r64, double inv_s, size_t total, int nrhs,
 	}
 }
 
-// out[i][c] = xT[c][i]
-__global__ void k_rows(const double *xT, int ld, int n, int nrhs, double *out)
+// rho32 <- rho and per block (grid-stride): sum of squares and max of |E|, the
+// power sum_i area_i E_i
+constexpr int kStatBlocks = 1024;
+__global__ __launch_bounds__(kB) void k_prep(const double *rho, const double *E, const float *area, unsigned total,
+                                             unsigned nrhs, float *rho32, double *stat)
 {
-	const size_t total = (size_t)n * nrhs;
-	for (size_t t = blockIdx.x * (size_t)kB + threadIdx.x; t < total; t += (size_t)gridDim.x * kB)
-		out[t] = xT[(size_t)(t % nrhs) * ld + t / nrhs];
+	double ss = 0.0, mx = 0.0, pw = 0.0;
+	for (unsigned t = blockIdx.x * kB + threadIdx.x; t < total; t += gridDim.x * kB) {
+		const double e = E[t];
+		rho32[t] = (float)rho[t];
+		ss += e * e;
+		mx = fmax(mx, fabs(e));
+		pw += (double)area[t / nrhs] * e;
+	}
+	for (int off = 32; off > 0; off >>= 1) {
+		ss += __shfl_xor(ss, off);
+		mx = fmax(mx, __shfl_xor(mx, off));
+		pw += __shfl_xor(pw, off);
+	}
+	__shared__ double r[12];
+	if ((threadIdx.x & 63) == 0) {
+		r[3 * (threadIdx.x >> 6)] = ss;
+		r[3 * (threadIdx.x >> 6) + 1] = mx;
+		r[3 * (threadIdx.x >> 6) + 2] = pw;
+	}
+	__syncthreads();
+	if (threadIdx.x == 0) {
+		stat[3 * blockIdx.x] = r[0] + r[3] + r[6] + r[9];
+		stat[3 * blockIdx.x + 1] = fmax(fmax(r[1], r[4]), fmax(r[7], r[10]));
+		stat[3 * blockIdx.x + 2] = r[2] + r[5] + r[8] + r[11];
+	}
 }
+
+// xT[c][i] = in[i][c], and out[i][c] = (mul ? mul[i][c] : 1) * xT[c][i] with,
+// per block (pw given), the power sum_i area_i xT[.][i]: 64 rows by up to 64
+// columns a block, turned through LDS so that both sides are contiguous
+constexpr int kTurn = 64;
+__global__ __launch_bounds__(kB) void k_cols(const double *in, int ld, int n, int nrhs, double *xT)
+{
+	__shared__ double tile[kTurn][kTurn + 1];
+	const int i0 = blockIdx.x * kTurn, c0 = blockIdx.y * kTurn, nc = min(kTurn, nrhs - c0), ni = min(kTurn, n - i0);
+	for (int e = threadIdx.x; e < ni * nc; e += kB) tile[e / nc][e % nc] = in[(size_t)(i0 + e / nc) * nrhs + c0 + e % nc];
+	__syncthreads();
+	for (int e = threadIdx.x; e < kTurn * nc; e += kB)
+		if (e % kTurn < ni) xT[(size_t)(c0 + e / kTurn) * ld + i0 + e % kTurn] = tile[e % kTurn][e / kTurn];
+}
+__global__ __launch_bounds__(kB) void k_rows(const double *xT, int ld, int n, int nrhs, const double *mul, double *out,
+                                             const float *area, double *pw)
+{
+	__shared__ double tile[kTurn][kTurn + 1];
+	const int i0 = blockIdx.x * kTurn, c0 = blockIdx.y * kTurn, nc = min(kTurn, nrhs - c0), ni = min(kTurn, n - i0);
+	double p = 0.0;
+	for (int e = threadIdx.x; e < kTurn * nc; e += kB)
+		if (e % kTurn < ni) {
+			const double x = xT[(size_t)(c0 + e / kTurn) * ld + i0 + e % kTurn];
+			tile[e % kTurn][e / kTurn] = x;
+			if (pw) p += (double)area[i0 + e % kTurn] * x;
+		}
+	__syncthreads();
+	for (int e = threadIdx.x; e < ni * nc; e += kB) {
+		const size_t t = (size_t)(i0 + e / nc) * nrhs + c0 + e % nc;
+		const double x = tile[e / nc][e % nc];
+		out[t] = mul ? x * mul[t] : x;
+	}
+	if (!pw) return;
+	for (int off = 32; off > 0; off >>= 1) p += __shfl_xor(p, off);
+	__shared__ double r[4];
+	if ((threadIdx.x & 63) == 0) r[threadIdx.x >> 6] = p;
+	__syncthreads();
+	if (threadIdx.x == 0) pw[blockIdx.y * gridDim.x + blockIdx.x] = r[0] + r[1] + r[2] + r[3];
+}
+dim3 turn_grid(int n, int nrhs) { return dim3((n + kTurn - 1) / kTurn, (nrhs + kTurn - 1) / kTurn); }
 
 // per block: sum (x - ref)^2 and sum ref^2 (x transposed [c][ld] or row-major)
 __global__ void k_err(const double *x, int transposed, int ld, const double *ref, int n, int nrhs, double *blk)
@@ -790,11 +858,11 @@ double power_sum(const std::vector<float> &a, const double *v, int n, int nrhs)
 // >= nrhs and columns >= n zero; split-K partials; per-block stats.
 struct Fx64 {
 	int n = 0, ld = 0, nrhs = 0, rp = 0, rt = 4, ct = 1, S = 1, ks = 1;
-	Buf<double> part, blk;
+	Buf<double> part;
 	size_t nblk = 0;
-	std::vector<double> hb;
+	double *blk = nullptr;  // the blocks' statistics, in host memory (Stage)
 
-	int setup(int n_, int ld_, int nrhs_, std::string &err)
+	int setup(int n_, int ld_, int nrhs_, Stage &stage, std::string &err)
 	{
 		n = n_;
 		ld = ld_;
@@ -827,8 +895,8 @@ struct Fx64 {
 			nblk = ((size_t)n * nrhs + kB - 1) / kB;
 			if (part.alloc((size_t)S * ld * rp, err)) return -1;
 		}
-		if (blk.alloc(nblk * 2, err)) return -1;
-		hb.assign(nblk * 2, 0.0);
+		if (stage.stat_room(std::max<size_t>(nblk * 2, 3 * kStatBlocks), err)) return -1;
+		blk = stage.stats;
 		return 0;
 	}
 	// at most 4 columns: the vector-unit kernel (ld is a multiple of 256:
@@ -838,9 +906,9 @@ struct Fx64 {
 	                                  const double *xT, double *out, hipStream_t st)
 	{
 		const dim3 g((unsigned)nblk), b(kB);
-		if (ks == 1) hipLaunchKernelGGL((k_fx64v<NC, 1>), g, b, 0, st, F, wT, ld, n, xT, base, rho, out, blk.p);
-		else if (ks == 2) hipLaunchKernelGGL((k_fx64v<NC, 2>), g, b, 0, st, F, wT, ld, n, xT, base, rho, out, blk.p);
-		else hipLaunchKernelGGL((k_fx64v<NC, 4>), g, b, 0, st, F, wT, ld, n, xT, base, rho, out, blk.p);
+		if (ks == 1) hipLaunchKernelGGL((k_fx64v<NC, 1>), g, b, 0, st, F, wT, ld, n, xT, base, rho, out, blk);
+		else if (ks == 2) hipLaunchKernelGGL((k_fx64v<NC, 2>), g, b, 0, st, F, wT, ld, n, xT, base, rho, out, blk);
+		else hipLaunchKernelGGL((k_fx64v<NC, 4>), g, b, 0, st, F, wT, ld, n, xT, base, rho, out, blk);
 	}
 	// out = base + rho o (F w) - x (xT null: 0); returns (sum of squares, max |out|)
 	int run(const float *F, const double *wT, const double *base, const double *rho, const double *xT, double *out,
@@ -858,24 +926,37 @@ struct Fx64 {
 			else if (ct == 2) hipLaunchKernelGGL((k_fx64m<4, 2>), grid, dim3(kB), 0, st, F, wT, part.p, ld, rp, kchunk);
 			else hipLaunchKernelGGL((k_fx64m<4, 1>), grid, dim3(kB), 0, st, F, wT, part.p, ld, rp, kchunk);
 			hipLaunchKernelGGL(k_resid, dim3((unsigned)nblk), dim3(kB), 0, st, part.p, S, ld, rp, n, nrhs, xT, base, rho,
-			                   out, blk.p);
+			                   out, blk);
 		}
 		HIP_OK(hipGetLastError(), "FP64 product");
 		ss = mx = 0.0;
 		if (!want_stats) return 0;
-		HIP_OK(hipMemcpyAsync(hb.data(), blk.p, nblk * 2 * 8, hipMemcpyDeviceToHost, st), "reduce");
 		HIP_OK(hipStreamSynchronize(st), "residual");
 		for (size_t b = 0; b < nblk; b++) {
-			ss += hb[2 * b];
-			mx = std::max(mx, hb[2 * b + 1]);
+			ss += blk[2 * b];
+			mx = std::max(mx, blk[2 * b + 1]);
 		}
 		return 0;
 	}
 };
 
+// What a solve works in, kept between calls (grown where a wider one needs
+// it).  Rows past the right-hand sides of xT, wT, X16 and Xb may hold an
+// earlier call's columns, which touch only their own; columns past n are
+// never written and stay zero.
+struct Work {
+	Buf<float> rho32, r32, part;
+	Buf<double> rho64, E64, xT, wT, r64, out, fb, Bref64, blk;
+	Buf<_Float16> X16[2];
+	Buf<__bf16> Xb[2];
+	Fx64 fx;
+};
+
 struct LinearSystem::Impl {
 	hipStream_t st = nullptr;
 	hipEvent_t e0 = nullptr, e1 = nullptr;
+	Stage stage;
+	Work work;
 	Buf<float> F32, Ft, area;
 	Buf<_Float16> F16, FT16;  // FT16: s16 * F^T in fragment order (the adjoint's sweeps)
 	Buf<__bf16> FB16;
@@ -958,14 +1039,37 @@ struct LinearSystem::Impl {
 		return 0;
 	}
 
-	// the iterate's two buffers (rp x ld, fragment order), zeroed
+	// the start of a call: nothing of an earlier one (which may have ended in
+	// an error) is in flight
+	int begin(std::string &err)
+	{
+		HIP_OK(hipStreamSynchronize(st), "stream");
+		stage.begin();
+		return 0;
+	}
+	// room for count elements, zero where it was allocated anew
+	template <typename T> int zeroed(Buf<T> &b, size_t count, std::string &err)
+	{
+		if (b.p && count <= b.n) return 0;
+		if (b.alloc(count, err)) return -1;
+		hipLaunchKernelGGL(k_fill<T>, dim3(grid_for(count)), dim3(kB), 0, st, b.p, count, (T)0.f);
+		return 0;
+	}
+	// the iterate's two buffers (rp x ld, fragment order)
 	template <typename E> int iterates(Buf<E> (&X)[2], size_t count, std::string &err)
 	{
-		for (Buf<E> &x : X) {
-			if (x.alloc(count, err)) return -1;
-			hipLaunchKernelGGL(k_fill<E>, dim3(grid_for(count)), dim3(kB), 0, st, x.p, count, (E)0.f);
-		}
-		return 0;
+		return zeroed(X[0], count, err) || zeroed(X[1], count, err) ? -1 : 0;
+	}
+	template <typename E> Buf<E> (&iterate_of())[2]
+	{
+		if constexpr (std::is_same_v<E, _Float16>) return work.X16;
+		else return work.Xb;
+	}
+	double power(size_t blocks) const
+	{
+		double p = 0.0;
+		for (size_t b = 0; b < blocks; b++) p += stage.stats[b];
+		return p;
 	}
 
 	// times one sweep for every (rows per wave, split-K) and keeps the fastest
@@ -1047,25 +1151,21 @@ struct LinearSystem::Impl {
 			S = it->second.second;
 		}
 		const size_t total = (size_t)n * nrhs, xts = (size_t)rp * ld;
-		Buf<E> x;
-		Buf<float> part, y;
-		Buf<double> x64;
-		if (x.alloc(xts, err) || y.alloc(total, err) || x64.alloc(total, err) ||
-		    (dma_tile(rt, ct) && part.alloc((size_t)S * ld * rp, err)))
+		Work &w = work;
+		Buf<E>(&x)[2] = iterate_of<E>();
+		if (begin(err) || iterates(x, xts, err) || w.r32.alloc(total, err) || w.E64.alloc(total, err) ||
+		    (dma_tile(rt, ct) && w.part.alloc((size_t)S * ld * rp, err)) || stage.up(w.E64.p, X, total * 8, st, err))
 			return -1;
-		HIP_OK(hipMemcpyAsync(x64.p, X, total * 8, hipMemcpyHostToDevice, st), "upload");
-		hipLaunchKernelGGL(k_fill<E>, dim3(grid_for(xts)), dim3(kB), 0, st, x.p, xts, (E)0.f);
-		hipLaunchKernelGGL(k_scale<E>, dim3(grid_for(total)), dim3(kB), 0, st, x64.p, 1.0, total, nrhs, ld, y.p, x.p);
+		hipLaunchKernelGGL(k_scale<E>, dim3(grid_for(total)), dim3(kB), 0, st, w.E64.p, 1.0, total, nrhs, ld, w.r32.p, x[0].p);
 		SweepOut<E> o{};
-		o.n = n, o.nrhs = nrhs, o.inv = inv, o.y = y.p;
-		if (launch_sweep<E>(rt, ct, S, A, x.p, part.p, ld, rp, o, st)) {
+		o.n = n, o.nrhs = nrhs, o.inv = inv, o.y = w.r32.p;
+		if (launch_sweep<E>(rt, ct, S, A, x[0].p, w.part.p, ld, rp, o, st)) {
 			err = "multiply: no kernel for this tile";
 			return -1;
 		}
 		HIP_OK(hipGetLastError(), "multiply");
 		std::vector<float> hy(total);
-		HIP_OK(hipMemcpyAsync(hy.data(), y.p, total * 4, hipMemcpyDeviceToHost, st), "download");
-		HIP_OK(hipStreamSynchronize(st), "multiply");
+		if (stage.down(hy.data(), w.r32.p, total * 4, st, err)) return -1;
 		for (size_t t = 0; t < total; t++) Y[t] = hy[t];
 		return 0;
 	}
@@ -1124,6 +1224,10 @@ LinearSystem *LinearSystem::create(int n, std::string &err)
 	}
 	if (L->d_->F32.alloc(np * np, err) || hipMemset(L->d_->F32.p, 0, np * np * sizeof(float)) != hipSuccess) {
 		if (err.empty()) err = "matrix clear failed";
+		delete L;
+		return nullptr;
+	}
+	if (L->d_->stage.init(err)) {
 		delete L;
 		return nullptr;
 	}
@@ -1235,19 +1339,14 @@ int LinearSystem::multiply(int prec, int nrhs, const double *X, double *Y, std::
 	const size_t total = (size_t)n * nrhs;
 	hipStream_t st = d.st;
 	if (prec == PREC_F32) {
-		Fx64 fx;
-		if (fx.setup(n, ld, nrhs, err)) return -1;
-		std::vector<double> xt((size_t)fx.rp * ld, 0.0);
-		for (int i = 0; i < n; i++)
-			for (int c = 0; c < nrhs; c++) xt[(size_t)c * ld + i] = X[(size_t)i * nrhs + c];
-		Buf<double> xT, out;
-		if (xT.alloc(xt.size(), err) || out.alloc(total, err)) return -1;
-		HIP_OK(hipMemcpyAsync(xT.p, xt.data(), xt.size() * 8, hipMemcpyHostToDevice, st), "upload");
+		Work &w = d.work;
+		if (d.begin(err) || w.fx.setup(n, ld, nrhs, d.stage, err) || d.zeroed(w.xT, (size_t)w.fx.rp * ld, err) ||
+		    w.E64.alloc(total, err) || w.out.alloc(total, err) || d.stage.up(w.E64.p, X, total * 8, st, err))
+			return -1;
+		hipLaunchKernelGGL(k_cols, turn_grid(n, nrhs), dim3(kB), 0, st, w.E64.p, ld, n, nrhs, w.xT.p);
 		double ss, mx;
-		if (fx.run(d.F32.p, xT.p, nullptr, nullptr, nullptr, out.p, st, ss, mx, false, err)) return -1;
-		HIP_OK(hipMemcpyAsync(Y, out.p, total * 8, hipMemcpyDeviceToHost, st), "download");
-		HIP_OK(hipStreamSynchronize(st), "multiply");
-		return 0;
+		if (w.fx.run(d.F32.p, w.xT.p, nullptr, nullptr, nullptr, w.out.p, st, ss, mx, false, err)) return -1;
+		return d.stage.down(Y, w.out.p, total * 8, st, err);
 	}
 	if (d.ensure_lowp(prec, ld, err)) return -1;
 	return prec == PREC_F16 ? d.product<_Float16>(d.F16.p, 1.0f / d.s16, n, ld, nrhs, prec, X, Y, err)
@@ -1278,35 +1377,33 @@ int LinearSystem::gather(int prec, int nrhs, const double *rho, const double *E,
 	const size_t total = (size_t)n * nrhs;
 	const float inv = 1.0f / (prec == PREC_F16 ? d.s16 : d.sb16);
 	hipStream_t st = d.st;
-	Buf<float> rho32, r32, part;
-	Buf<double> rho64, E64, xT, r64, blk, Bref64;
-	Buf<_Float16> XT16[2];
-	Buf<__bf16> XTb[2];
-	Fx64 fx;
-	if (fx.setup(n, ld, nrhs, err)) return -1;
-	const size_t xtn = (size_t)fx.rp * ld;
-	if (rho32.alloc(total, err) || r32.alloc(total, err) ||
-	    (dma_tile(rt, ct) && part.alloc((size_t)S * ld * rp, err)) || rho64.alloc(total, err) || E64.alloc(total, err) ||
-	    xT.alloc(xtn, err) || r64.alloc(total, err) || blk.alloc(8192 * 2, err))
-		return -1;
+	Work &w = d.work;
 	const size_t xts = (size_t)rp * ld;
-	if (prec == PREC_F16 ? d.iterates(XT16, xts, err) : d.iterates(XTb, xts, err)) return -1;
-	std::vector<float> h32(total);
-	for (size_t t = 0; t < total; t++) h32[t] = (float)rho[t];
-	HIP_OK(hipMemcpyAsync(rho32.p, h32.data(), total * 4, hipMemcpyHostToDevice, st), "upload");
-	HIP_OK(hipMemcpyAsync(rho64.p, rho, total * 8, hipMemcpyHostToDevice, st), "upload");
-	HIP_OK(hipMemcpyAsync(E64.p, E, total * 8, hipMemcpyHostToDevice, st), "upload");
-	hipLaunchKernelGGL(k_fill<double>, dim3(grid_for(xtn)), dim3(kB), 0, st, xT.p, xtn, 0.0);
-	if (Bref) {
-		if (Bref64.alloc(total, err)) return -1;
-		HIP_OK(hipMemcpyAsync(Bref64.p, Bref, total * 8, hipMemcpyHostToDevice, st), "upload");
-	}
+	if (d.begin(err) || w.fx.setup(n, ld, nrhs, d.stage, err) || w.rho32.alloc(total, err) || w.r32.alloc(total, err) ||
+	    (dma_tile(rt, ct) && w.part.alloc((size_t)S * ld * rp, err)) || w.rho64.alloc(total, err) ||
+	    w.E64.alloc(total, err) || d.zeroed(w.xT, (size_t)w.fx.rp * ld, err) || w.r64.alloc(total, err) ||
+	    w.out.alloc(total, err) || (prec == PREC_F16 ? d.iterates(w.X16, xts, err) : d.iterates(w.Xb, xts, err)) ||
+	    d.stage.up(w.rho64.p, rho, total * 8, st, err) || d.stage.up(w.E64.p, E, total * 8, st, err))
+		return -1;
+	if (Bref && (w.Bref64.alloc(total, err) || w.blk.alloc(8192 * 2, err) ||
+	             d.stage.up(w.Bref64.p, Bref, total * 8, st, err)))
+		return -1;
+	const int g = grid_for(total), gs = std::min(g, kStatBlocks);
+	hipLaunchKernelGGL(k_prep, dim3(gs), dim3(kB), 0, st, w.rho64.p, w.E64.p, d.area.p, (unsigned)total, (unsigned)nrhs,
+	                   w.rho32.p, d.stage.stats);
+	HIP_OK(hipGetLastError(), "upload");
 	HIP_OK(hipStreamSynchronize(st), "upload");
-	std::vector<double> hb(8192 * 2);
-	const int g = grid_for(total);
+	// x = 0 at the start, so the first residual is E itself
+	double ss0 = 0.0, mx0 = 0.0, power_E = 0.0;
+	for (int k = 0; k < gs; k++) {
+		ss0 += d.stage.stats[3 * k];
+		mx0 = std::max(mx0, d.stage.stats[3 * k + 1]);
+		power_E += d.stage.stats[3 * k + 2];
+	}
+	std::vector<double> hb(Bref ? 8192 * 2 : 0);
 	auto err_vs_ref = [&](double &e) -> int {
-		hipLaunchKernelGGL(k_err, dim3(g), dim3(kB), 0, st, xT.p, 1, ld, Bref64.p, n, nrhs, blk.p);
-		HIP_OK(hipMemcpyAsync(hb.data(), blk.p, (size_t)g * 2 * 8, hipMemcpyDeviceToHost, st), "err");
+		hipLaunchKernelGGL(k_err, dim3(g), dim3(kB), 0, st, w.xT.p, 1, ld, w.Bref64.p, n, nrhs, w.blk.p);
+		HIP_OK(hipMemcpyAsync(hb.data(), w.blk.p, (size_t)g * 2 * 8, hipMemcpyDeviceToHost, st), "err");
 		HIP_OK(hipStreamSynchronize(st), "err");
 		double a = 0.0, b = 0.0;
 		for (int k = 0; k < g; k++) {
@@ -1319,21 +1416,9 @@ int LinearSystem::gather(int prec, int nrhs, const double *rho, const double *E,
 	const auto t0 = std::chrono::steady_clock::now();
 	double enorm = -1.0, rel = 0.0, ms_target = -1.0, errv = -1.0, check_ms = 0.0;
 	int outer = 0, total_sweeps = 0;
-	// x = 0 at the start, so the first residual is E itself
-	double ss0 = 0.0, mx0 = 0.0;
-	for (size_t t = 0; t < total; t++) {
-		ss0 += E[t] * E[t];
-		mx0 = std::max(mx0, std::fabs(E[t]));
-	}
 	for (;; outer++) {
-		double ss = 0.0, mx = 0.0;
-		if (outer == 0) {
-			HIP_OK(hipMemcpyAsync(r64.p, E64.p, total * 8, hipMemcpyDeviceToDevice, st), "residual");
-			ss = ss0;
-			mx = mx0;
-		} else if (fx.run(d.F32.p, xT.p, E64.p, rho64.p, xT.p, r64.p, st, ss, mx, true, err)) {
-			return -1;
-		}
+		double ss = ss0, mx = mx0;
+		if (outer > 0 && w.fx.run(d.F32.p, w.xT.p, w.E64.p, w.rho64.p, w.xT.p, w.r64.p, st, ss, mx, true, err)) return -1;
 		if (!std::isfinite(ss)) {
 			err = "gather diverged (non-finite residual): the iteration needs spectral radius of diag(rho) F below 1";
 			return -1;
@@ -1351,33 +1436,37 @@ int LinearSystem::gather(int prec, int nrhs, const double *rho, const double *E,
 		int rc;
 		auto refine = [&](const auto *A, auto &X) {
 			typedef std::remove_cv_t<std::remove_pointer_t<decltype(A)>> T;
-			hipLaunchKernelGGL(k_scale<T>, dim3(g), dim3(kB), 0, st, r64.p, 1.0 / s, total, nrhs, ld, r32.p, X[0].p);
+			hipLaunchKernelGGL(k_scale<T>, dim3(g), dim3(kB), 0, st, outer ? w.r64.p : w.E64.p, 1.0 / s, total, nrhs, ld,
+			                   w.r32.p, X[0].p);
 			SweepOut<T> o{};
-			o.n = n, o.nrhs = nrhs, o.inv = inv, o.rhs = r32.p, o.rho = rho32.p, o.xT = xT.p, o.s = s;
-			rc = d.sweep(A, X, part.p, ct, rt, S, ld, sweeps, o, err);
+			o.n = n, o.nrhs = nrhs, o.inv = inv, o.rhs = w.r32.p, o.rho = w.rho32.p;
+			o.xT = w.xT.p, o.s = s, o.first = outer == 0;
+			rc = d.sweep(A, X, w.part.p, ct, rt, S, ld, sweeps, o, err);
 		};
-		if (prec == PREC_F16) refine(d.F16.p, XT16);
-		else refine(d.FB16.p, XTb);
+		if (prec == PREC_F16) refine(d.F16.p, w.X16);
+		else refine(d.FB16.p, w.Xb);
 		if (rc) return -1;
 		total_sweeps += sweeps;
 		HIP_OK(hipGetLastError(), "sweep launch");
 	}
 	const double ms = ms_since(t0) - check_ms;
-	std::vector<double> hx((size_t)nrhs * ld);
-	HIP_OK(hipMemcpy(hx.data(), xT.p, hx.size() * 8, hipMemcpyDeviceToHost), "download");  // rows < nrhs
-	for (int i = 0; i < n; i++)
-		for (int c = 0; c < nrhs; c++) B[(size_t)i * nrhs + c] = hx[(size_t)c * ld + i];
+	if (outer == 0)  // no refinement: the iterate is the zero it started from
+		hipLaunchKernelGGL(k_fill<double>, dim3(grid_for(w.xT.n)), dim3(kB), 0, st, w.xT.p, w.xT.n, 0.0);
+	const dim3 tg = turn_grid(n, nrhs);
+	const size_t blocks = (size_t)tg.x * tg.y;
+	if (d.stage.stat_room(blocks, err)) return -1;  // the residual's were read
+	hipLaunchKernelGGL(k_rows, tg, dim3(kB), 0, st, w.xT.p, ld, n, nrhs, nullptr, w.out.p, d.area.p, d.stage.stats);
+	HIP_OK(hipGetLastError(), "download");
+	if (d.stage.down(B, w.out.p, total * 8, st, err)) return -1;
 	if (info) {
-		std::vector<float> a(n);
-		HIP_OK(hipMemcpy(a.data(), d.area.p, n * 4, hipMemcpyDeviceToHost), "area");
 		info[INFO_OUTER] = outer;
 		info[INFO_SWEEPS] = total_sweeps;
 		info[INFO_REL_RES] = rel;
 		info[INFO_MS] = ms;
 		info[INFO_MS_TARGET] = ms_target;
 		info[INFO_ERR] = errv;
-		info[INFO_POWER_E] = power_sum(a, E, n, nrhs);
-		info[INFO_POWER_B] = power_sum(a, B, n, nrhs);
+		info[INFO_POWER_E] = power_E;
+		info[INFO_POWER_B] = d.power(blocks);
 	}
 	return 0;
 }
@@ -1519,47 +1608,35 @@ int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const do
 	int rt, Sg;
 	if (d.solve_tile(*this, nrhs, PREC_F16, rt, Sg, err)) return -1;
 	const float inv = 1.0f / d.s16;
-	const int g = grid_for(total);
-	Buf<double> rho64, g64, xT, wT, r64, out, B64T, fb;
-	Fx64 fx;
-	if (fx.setup(n, ld, nrhs, err)) return -1;
-	Buf<float> rho32, r32;
-	Buf<_Float16> XT16[2];
-	const size_t xts = (size_t)rp * ld;
-	const size_t xtn = (size_t)fx.rp * ld;
-	if (rho64.alloc(total, err) || g64.alloc(total, err) || xT.alloc(xtn, err) || wT.alloc(xtn, err) ||
-	    r64.alloc(total, err) || out.alloc(total, err) || rho32.alloc(total, err) || r32.alloc(total, err) ||
-	    d.iterates(XT16, xts, err) || B64T.alloc(xtn, err) || fb.alloc(total, err))
+	const int g = grid_for(total), gs = std::min(g, kStatBlocks);
+	Work &w = d.work;
+	if (d.begin(err) || w.fx.setup(n, ld, nrhs, d.stage, err)) return -1;
+	const size_t xtn = (size_t)w.fx.rp * ld;
+	// out: lambda, then dL/drho
+	if (w.rho64.alloc(total, err) || w.E64.alloc(total, err) || d.zeroed(w.xT, xtn, err) || d.zeroed(w.wT, xtn, err) ||
+	    w.r64.alloc(total, err) || w.out.alloc(2 * total, err) || w.rho32.alloc(total, err) || w.r32.alloc(total, err) ||
+	    w.fb.alloc(total, err) || d.iterates(w.X16, (size_t)rp * ld, err) ||
+	    d.stage.up(w.rho64.p, rho, total * 8, st, err) || d.stage.up(w.E64.p, gin, total * 8, st, err))
 		return -1;
-	std::vector<float> h(total);
-	for (size_t t = 0; t < total; t++) h[t] = (float)rho[t];
-	HIP_OK(hipMemcpyAsync(rho32.p, h.data(), total * 4, hipMemcpyHostToDevice, st), "upload");
-	HIP_OK(hipMemcpyAsync(rho64.p, rho, total * 8, hipMemcpyHostToDevice, st), "upload");
-	HIP_OK(hipMemcpyAsync(g64.p, gin, total * 8, hipMemcpyHostToDevice, st), "upload");
-	hipLaunchKernelGGL(k_fill<double>, dim3(grid_for(xtn)), dim3(kB), 0, st, xT.p, xtn, 0.0);
-	hipLaunchKernelGGL(k_fill<double>, dim3(grid_for(xtn)), dim3(kB), 0, st, wT.p, xtn, 0.0);
+	hipLaunchKernelGGL(k_prep, dim3(gs), dim3(kB), 0, st, w.rho64.p, w.E64.p, d.area.p, (unsigned)total, (unsigned)nrhs,
+	                   w.rho32.p, d.stage.stats);
+	HIP_OK(hipGetLastError(), "upload");
 	HIP_OK(hipStreamSynchronize(st), "upload");
 	const auto t0 = std::chrono::steady_clock::now();
 	double enorm = -1.0, rel = 0.0;
 	int outer = 0, total_sweeps = 0;
 	double ss0 = 0.0, mx0 = 0.0;  // lambda = 0 at the start: the first residual is g
-	for (size_t t = 0; t < total; t++) {
-		ss0 += gin[t] * gin[t];
-		mx0 = std::max(mx0, std::fabs(gin[t]));
+	for (int k = 0; k < gs; k++) {
+		ss0 += d.stage.stats[3 * k];
+		mx0 = std::max(mx0, d.stage.stats[3 * k + 1]);
 	}
 	for (;; outer++) {
-		double ss = 0.0, mx = 0.0;
-		if (outer == 0) {
-			HIP_OK(hipMemcpyAsync(r64.p, g64.p, total * 8, hipMemcpyDeviceToDevice, st), "residual");
-			ss = ss0;
-			mx = mx0;
-		} else if (fx.run(d.Ft.p, wT.p, g64.p, nullptr, xT.p, r64.p, st, ss, mx, true, err)) {
-			// r = g + F^T (rho o x) - x in FP64 over the transposed copy that
-			// the FP16 one is made from: its rows are read whole, where
-			// F's columns, split over row chunks, ran at a sixth of the
-			// rate (n = 6001: 151 + 8.6 -> 29 us)
-			return -1;
-		}
+		double ss = ss0, mx = mx0;
+		// r = g + F^T (rho o x) - x in FP64 over the transposed copy that the
+		// FP16 one is made from: its rows are read whole, where F's columns,
+		// split over row chunks, ran at a sixth of the rate (n = 6001: 151 +
+		// 8.6 -> 29 us)
+		if (outer > 0 && w.fx.run(d.Ft.p, w.wT.p, w.E64.p, nullptr, w.xT.p, w.r64.p, st, ss, mx, true, err)) return -1;
 		if (!std::isfinite(ss)) {
 			err = "adjoint diverged (non-finite residual)";
 			return -1;
@@ -1568,31 +1645,31 @@ int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const do
 		rel = enorm > 0 ? std::sqrt(ss) / enorm : 0.0;
 		if (rel <= tol || outer >= max_outer || mx == 0.0) break;
 		// d <- r (scaled), then sweeps d <- r + F^T (rho o d) with XT = rho o d
-		hipLaunchKernelGGL(k_scale<_Float16>, dim3(g), dim3(kB), 0, st, r64.p, 1.0 / mx, total, nrhs, ld, r32.p,
-		                   XT16[0].p, rho32.p);
+		hipLaunchKernelGGL(k_scale<_Float16>, dim3(g), dim3(kB), 0, st, outer ? w.r64.p : w.E64.p, 1.0 / mx, total, nrhs,
+		                   ld, w.r32.p, w.X16[0].p, w.rho32.p);
 		SweepOut<_Float16> o{};
-		o.n = n, o.nrhs = nrhs, o.inv = inv, o.rho_in = true, o.rhs = r32.p, o.rho = rho32.p;
-		o.xT = xT.p, o.s = mx, o.wT = wT.p, o.rho64 = rho64.p;
-		if (d.sweep(d.FT16.p, XT16, nullptr, ct, rt, Sg, ld, sweeps, o, err)) return -1;
+		o.n = n, o.nrhs = nrhs, o.inv = inv, o.rho_in = true, o.rhs = w.r32.p, o.rho = w.rho32.p;
+		o.xT = w.xT.p, o.s = mx, o.first = outer == 0, o.wT = w.wT.p, o.rho64 = w.rho64.p;
+		if (d.sweep(d.FT16.p, w.X16, nullptr, ct, rt, Sg, ld, sweeps, o, err)) return -1;
 		total_sweeps += sweeps;
 		HIP_OK(hipGetLastError(), "adjoint sweep");
 	}
-	// dL/drho = lambda o (F B), F B in FP64
-	std::vector<double> bt((size_t)fx.rp * ld, 0.0);
-	for (int i = 0; i < n; i++)
-		for (int c = 0; c < nrhs; c++) bt[(size_t)c * ld + i] = B[(size_t)i * nrhs + c];
-	HIP_OK(hipMemcpyAsync(B64T.p, bt.data(), bt.size() * 8, hipMemcpyHostToDevice, st), "upload");
+	if (outer == 0)  // no refinement: lambda is the zero it started from
+		hipLaunchKernelGGL(k_fill<double>, dim3(grid_for(w.xT.n)), dim3(kB), 0, st, w.xT.p, w.xT.n, 0.0);
+	// dL/drho = lambda o (F B), F B in FP64 (wT takes B)
+	if (d.stage.up(w.r64.p, B, total * 8, st, err)) return -1;
+	const dim3 tg = turn_grid(n, nrhs);
+	hipLaunchKernelGGL(k_cols, tg, dim3(kB), 0, st, w.r64.p, ld, n, nrhs, w.wT.p);
 	{
 		double ss, mx;
-		if (fx.run(d.F32.p, B64T.p, nullptr, nullptr, nullptr, fb.p, st, ss, mx, false, err)) return -1;
+		if (w.fx.run(d.F32.p, w.wT.p, nullptr, nullptr, nullptr, w.fb.p, st, ss, mx, false, err)) return -1;
 	}
-	hipLaunchKernelGGL(k_rows, dim3(g), dim3(kB), 0, st, xT.p, ld, n, nrhs, out.p);
-	std::vector<double> hfb(total);
-	HIP_OK(hipMemcpyAsync(lambda, out.p, total * 8, hipMemcpyDeviceToHost, st), "download");
-	HIP_OK(hipMemcpyAsync(hfb.data(), fb.p, total * 8, hipMemcpyDeviceToHost, st), "download");
-	HIP_OK(hipStreamSynchronize(st), "adjoint");
+	hipLaunchKernelGGL(k_rows, tg, dim3(kB), 0, st, w.xT.p, ld, n, nrhs, nullptr, w.out.p, nullptr, nullptr);
+	hipLaunchKernelGGL(k_rows, tg, dim3(kB), 0, st, w.xT.p, ld, n, nrhs, w.fb.p, w.out.p + total, nullptr, nullptr);
+	HIP_OK(hipGetLastError(), "adjoint");
+	const Stage::Part parts[2] = {{lambda, total * 8}, {drho, total * 8}};
+	if (d.stage.down_parts(w.out.p, parts, 2, st, err)) return -1;
 	const double ms = ms_since(t0);
-	for (size_t t = 0; t < total; t++) drho[t] = lambda[t] * hfb[t];
 	if (info) {
 		for (int k = 0; k < INFO_N; k++) info[k] = -1;
 		info[INFO_OUTER] = outer;

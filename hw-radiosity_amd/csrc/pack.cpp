@@ -42,4 +42,19 @@ void spatial_order(const Patch *pool, int n, const float *G0, const float *G1, i
 	for (int i = 0; i < n; i++) order[i] = (int)(uint32_t)key[i];
 }
 
+void copy_bytes(void *dst, const void *src, size_t bytes)
+{
+	constexpr size_t kSlice = (size_t)128 << 10;
+	if (bytes < 2 * kSlice) {
+		std::memcpy(dst, src, bytes);
+		return;
+	}
+	const long slices = (long)((bytes + kSlice - 1) / kSlice);
+#pragma omp parallel for schedule(static) num_threads(slices < 8 ? (int)slices : 8)
+	for (long k = 0; k < slices; k++) {
+		const size_t o = (size_t)k * kSlice;
+		std::memcpy((char *)dst + o, (const char *)src + o, bytes - o < kSlice ? bytes - o : kSlice);
+	}
+}
+
 }  // namespace rgpu

@@ -222,7 +222,7 @@ class Engine:
     def cast(self, rays):
         rays = np.ascontiguousarray(rays, RAY_DTYPE)
         n = len(rays)
-        hit, cells, tests = (np.zeros(n, np.int32) for _ in range(3))
+        hit, cells, tests = (np.empty(n, np.int32) for _ in range(3))
         self._ok(library().rad_cast(self.h, n, _p(rays), _p(hit), _p(cells), _p(tests)))
         return hit, cells, tests
 
@@ -231,7 +231,7 @@ class Engine:
         CAST_STATIC_MAX rays)."""
         rays = np.ascontiguousarray(rays, RAY_DTYPE)
         n = len(rays)
-        hit, cells, tests = (np.zeros(n, np.int32) for _ in range(3))
+        hit, cells, tests = (np.empty(n, np.int32) for _ in range(3))
         self._ok(library().rad_cast_static(self.h, n, _p(rays), _p(hit), _p(cells), _p(tests)))
         return hit, cells, tests
 
@@ -342,7 +342,7 @@ class LinearSystem:
 
     def multiply(self, X, prec="f32"):
         X = _rhs(X, self.n)
-        Y = np.zeros_like(X)
+        Y = np.empty_like(X)
         self._ok(library().rad_lin_multiply(self.h, _prec(prec), X.shape[1], _p(X), _p(Y)))
         return Y
 
@@ -351,7 +351,7 @@ class LinearSystem:
         rho = _rhs(rho, self.n)
         assert rho.shape == E.shape
         ref = None if Bref is None else _rhs(Bref, self.n)
-        B = np.zeros_like(E)
+        B = np.empty_like(E)
         info = np.zeros(8, np.float64)
         self._ok(library().rad_lin_gather(self.h, _prec(prec), E.shape[1], _p(rho), _p(E), float(tol),
                                           int(max_outer), int(sweeps), _p(ref), float(target), _p(B), _p(info)))
@@ -362,7 +362,7 @@ class LinearSystem:
         rho = _rhs(rho, self.n)
         assert rho.shape == E.shape
         ref = None if Bref is None else _rhs(Bref, self.n)
-        B = np.zeros_like(E)
+        B = np.empty_like(E)
         info = np.zeros(8, np.float64)
         self._ok(library().rad_lin_shoot(self.h, E.shape[1], _p(rho), _p(E), _p(ref), float(target),
                                          int(max_shots), _p(B), _p(info)))
@@ -374,7 +374,7 @@ class LinearSystem:
         rho = _rhs(rho, self.n)
         g = _rhs(dLdB, self.n)
         assert rho.shape == B.shape == g.shape
-        dE, drho = np.zeros_like(B), np.zeros_like(B)
+        dE, drho = np.empty_like(B), np.empty_like(B)
         info = np.zeros(8, np.float64)
         self._ok(library().rad_lin_adjoint(self.h, B.shape[1], _p(rho), _p(B), _p(g), float(tol), int(max_outer),
                                            int(sweeps), _p(dE), _p(drho), _p(info)))
@@ -439,7 +439,7 @@ class SceneBatch:
         rho = np.ascontiguousarray(rho, np.float64)
         E = np.ascontiguousarray(E, np.float64)
         assert rho.shape == E.shape == (int(self.offsets[-1]), 3)
-        B = np.zeros_like(E)
+        B = np.empty_like(E)
         rel = np.zeros(len(self.sizes), np.float64)
         info = np.zeros(4, np.float64)
         self._ok(library().rad_batch_solve(self.h, _prec(prec), 1 if graph else 0, _p(rho), _p(E), float(tol),
