@@ -686,6 +686,211 @@ __device__ __forceinline__ void block_record(unsigned long long key, const float
 		for (int c = 0; c < nrhs; c++) rec->dB[c] = row[c];
 }
 
+// The same shots in one launch, where one block's registers hold the system:
+// 1024 threads, R patches each (i = thread + 1024 r), C >= nrhs columns, with
+// R (3 C + 3) <= kOneState values a thread (radiosity, unshot, reflectance, area
+// and two matrix columns).  Per shot the patches' keys are reduced over the wave's
+// lanes (DPP), the wave's largest and its dB row meet the others' in LDS (two
+// sets by parity: one barrier a shot), and every wave takes the block's
+// largest from there.  The runner-up's column is loaded while the source's is
+// on its way: mostly it is the next source.
+// Bound by that dependent chain (an HBM or cache latency where the guess
+// fails, two reductions, a barrier) and, from about 4000 patches, by one CU's
+// loads and updates.  us per shot for 3 columns, a launch per shot -> now: n =
+// 500 4.00 -> 0.85, 2000 4.23 -> 1.16, 4000 4.32 -> 1.55, 8000 4.41 -> 2.87;
+// 1 column, n = 12000 3.71 -> 2.25.  16 patches a thread (1 column, n = 16000)
+// spill: 4.82 against 3.74, so twelve is the most.
+constexpr int kOneThreads = 1024;
+constexpr int kOneState = 100;
+
+// maximum over the wave (row_shr 1, 2, 4, 8, then row_bcast 15 and 31; lanes
+// without a source give 0), in every lane
+__device__ __forceinline__ uint32_t row_max(uint32_t x)
+{
+	x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false));
+	x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false));
+	x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false));
+	x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false));
+	return x;  // lane 15 of each row of 16 holds the row's
+}
+__device__ __forceinline__ uint32_t lane_max(uint32_t x)
+{
+	x = row_max(x);
+	x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false));
+	x = max(x, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false));
+	return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+// the lane of `who` with the lowest idx (who != 0)
+__device__ __forceinline__ int lowest(unsigned long long who, int idx)
+{
+	int l = __ffsll((long long)who) - 1;
+	int best = __builtin_amdgcn_readlane(idx, l);
+	for (who &= who - 1; who; who &= who - 1) {  // ties only
+		const int m = __ffsll((long long)who) - 1, i = __builtin_amdgcn_readlane(idx, m);
+		if (i < best) {
+			best = i;
+			l = m;
+		}
+	}
+	return l;
+}
+
+template <int R, int C>
+__global__ __launch_bounds__(kOneThreads) void k_lshoot_one(const float *__restrict__ Ft, int ld, const float *rho,
+                                                            const float *area, float *B, float *dB, int n, int nrhs,
+                                                            int shots, int *done)
+{
+	constexpr int NW = kOneThreads / 64;
+	static_assert(NW == 16, "one row of 16 lanes reduces the waves' records");
+	// per parity and wave: its largest power, that patch, its dB row; the power
+	// and patch of its second largest
+	__shared__ uint32_t pw[2][NW], pw2[2][NW];
+	__shared__ int ix[2][NW], ix2[2][NW];
+	__shared__ float row[2][NW][C];
+	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+	float b[R][C], d[R][C], rh[R][C], ar[R], f[R], g[R];
+#pragma unroll
+	for (int r = 0; r < R; r++) {
+		const int i = threadIdx.x + kOneThreads * r;
+		ar[r] = i < n ? area[i] : 0.f;
+#pragma unroll
+		for (int c = 0; c < C; c++) {
+			const bool in = i < n && c < nrhs;
+			const size_t t = (size_t)i * nrhs + c;
+			b[r][c] = in ? B[t] : 0.f;
+			d[r][c] = in ? dB[t] : 0.f;
+			rh[r][c] = in ? rho[t] : 0.f;
+		}
+		g[r] = 0.f;
+	}
+	int guess = -1;  // the patch whose column g holds
+	int k = 0;
+	for (; k < shots; k++) {
+		const int q = k & 1;
+		// this thread's two largest (the lower patch on ties)
+		uint32_t p1 = 0, p2 = 0;
+		int i1 = 0, i2 = 0, r1 = 0;
+#pragma unroll
+		for (int r = 0; r < R; r++) {
+			float p = 0.f;
+#pragma unroll
+			for (int c = 0; c < C; c++) p += d[r][c];
+			p *= ar[r];
+			const uint32_t u = p > 0.f ? __float_as_uint(p) : 0u;
+			const int i = threadIdx.x + kOneThreads * r;
+			if (u > p1) {
+				p2 = p1, i2 = i1;
+				p1 = u, i1 = i, r1 = r;
+			} else if (u > p2) {
+				p2 = u, i2 = i;
+			}
+		}
+		// the wave's: its winner's lane also gives the runner-up up for the rest
+		const uint32_t wm = lane_max(p1);
+		const int wl = wm ? lowest(__ballot(p1 == wm), i1) : 0;
+		const uint32_t s1 = lane == wl ? p2 : p1;
+		const int si = lane == wl ? i2 : i1;
+		const uint32_t wm2 = lane_max(s1);
+		const int wl2 = wm2 ? __ffsll((long long)__ballot(s1 == wm2)) - 1 : 0;
+		if (lane == wl) {
+			pw[q][w] = wm;
+			ix[q][w] = i1;
+#pragma unroll
+			for (int r = 0; r < R; r++)
+				if (r == r1)
+#pragma unroll
+					for (int c = 0; c < C; c++) row[q][w][c] = d[r][c];
+		}
+		if (lane == wl2) {
+			pw2[q][w] = wm2;
+			ix2[q][w] = si;
+		}
+		__syncthreads();
+		// the block's, in every wave
+		const uint32_t bp = pw[q][lane & 15], bp2 = pw2[q][lane & 15];
+		const int bi = ix[q][lane & 15], bi2 = ix2[q][lane & 15];
+		const uint32_t best = (uint32_t)__builtin_amdgcn_readlane((int)row_max(bp), 15);
+		if (best == 0) break;  // nothing left to shoot
+		const int ws = lowest(__ballot(bp == best) & 0xffffull, bi);
+		const int j = __builtin_amdgcn_readlane(bi, ws);
+		const float *col = Ft + (size_t)j * ld;
+		if (j != guess) {
+#pragma unroll
+			for (int r = 0; r < R; r++) f[r] = col[min((int)threadIdx.x + kOneThreads * r, n - 1)];
+		} else {
+#pragma unroll
+			for (int r = 0; r < R; r++) f[r] = g[r];
+		}
+		// the runner-up: the largest of the other waves' first and this one's second
+		const uint32_t t1 = (lane & 15) == ws ? bp2 : bp;
+		const int ti = (lane & 15) == ws ? bi2 : bi;
+		const uint32_t second = (uint32_t)__builtin_amdgcn_readlane((int)row_max(t1), 15);
+		guess = -1;
+		if (second) {
+			guess = __builtin_amdgcn_readlane(ti, __ffsll((long long)(__ballot(t1 == second) & 0xffffull)) - 1);
+			const float *c2 = Ft + (size_t)guess * ld;
+#pragma unroll
+			for (int r = 0; r < R; r++) g[r] = c2[min((int)threadIdx.x + kOneThreads * r, n - 1)];
+		}
+		float src[C];
+#pragma unroll
+		for (int c = 0; c < C; c++) src[c] = row[q][ws][c];
+#pragma unroll
+		for (int r = 0; r < R; r++) {
+			const bool self = (int)threadIdx.x + kOneThreads * r == j;
+#pragma unroll
+			for (int c = 0; c < C; c++) {
+				const float v = rh[r][c] * f[r] * src[c];
+				b[r][c] += v;
+				d[r][c] = (self ? 0.f : d[r][c]) + v;
+			}
+		}
+	}
+#pragma unroll
+	for (int r = 0; r < R; r++) {
+		const int i = threadIdx.x + kOneThreads * r;
+#pragma unroll
+		for (int c = 0; c < C; c++)
+			if (i < n && c < nrhs) {
+				B[(size_t)i * nrhs + c] = b[r][c];
+				dB[(size_t)i * nrhs + c] = d[r][c];
+			}
+	}
+	if (threadIdx.x == 0) *done += k;
+}
+
+// launches k_lshoot_one for the system, or returns false where it is too large
+// for one block
+bool launch_shoot_one(const float *Ft, int ld, const float *rho, const float *area, float *B, float *dB, int n,
+                      int nrhs, int shots, int *done, hipStream_t st)
+{
+	const int r = (n + kOneThreads - 1) / kOneThreads;
+	bool ok = false;
+	auto go = [&](auto rc, auto cc) {
+		constexpr int R = decltype(rc)::value, C = decltype(cc)::value;
+		if constexpr (R * (3 * C + 3) <= kOneState) {
+			if (ok || r > R || nrhs > C) return;
+			hipLaunchKernelGGL((k_lshoot_one<R, C>), dim3(1), dim3(kOneThreads), 0, st, Ft, ld, rho, area, B, dB, n, nrhs,
+			                   shots, done);
+			ok = true;
+		}
+	};
+	auto rows = [&](auto cc) {
+		go(std::integral_constant<int, 1>{}, cc);
+		go(std::integral_constant<int, 2>{}, cc);
+		go(std::integral_constant<int, 4>{}, cc);
+		go(std::integral_constant<int, 6>{}, cc);
+		go(std::integral_constant<int, 8>{}, cc);
+		go(std::integral_constant<int, 12>{}, cc);
+	};
+	if (nrhs <= 1) rows(std::integral_constant<int, 1>{});
+	else if (nrhs <= 3) rows(std::integral_constant<int, 3>{});
+	else if (nrhs <= 6) rows(std::integral_constant<int, 6>{});
+	else if (nrhs <= 12) rows(std::integral_constant<int, 12>{});
+	else rows(std::integral_constant<int, 16>{});
+	return ok;
+}
+
 // records of the initial dB (launch 0's input)
 __global__ __launch_bounds__(kB) void k_lsel(const float *dB, const float *area, int n, int nrhs, ShotRec *rout)
 {
@@ -1523,9 +1728,10 @@ int LinearSystem::shoot(int nrhs, const double *rho, const double *E, const doub
 		hipLaunchKernelGGL(k_lshoot, dim3(nb), dim3(kB), 0, st, d.Ft.p, ld, rho32.p, d.area.p, B32.p, dB32.p, n, nrhs,
 		                   rec.p + (size_t)(k & 1) * nb, rec.p + (size_t)((k + 1) & 1) * nb, shots_d.p);
 	};
-	// A shot needs the previous one's argmax, so plain shooting is bound by
-	// launch latency: runs of kGraphShots shots (an even number, so parities
-	// repeat) are captured once into a HIP graph and replayed.
+	// Where one block holds the system, a launch makes many shots; else a shot
+	// needs the previous launch's argmax and plain shooting is bound by launch
+	// latency: runs of kGraphShots shots (an even number, so parities repeat)
+	// are captured once into a HIP graph and replayed.
 	constexpr int kGraphShots = 64;
 	struct GraphGuard {
 		hipGraph_t g = nullptr;
@@ -1536,21 +1742,34 @@ int LinearSystem::shoot(int nrhs, const double *rho, const double *E, const doub
 			if (g) (void)hipGraphDestroy(g);
 		}
 	} run;
-	HIP_OK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal), "shot capture");
-	for (int k = 0; k < kGraphShots; k++) launch_shot(k);
-	HIP_OK(hipStreamEndCapture(st, &run.g), "shot capture");
-	HIP_OK(hipGraphInstantiate(&run.x, run.g, nullptr, nullptr, 0), "shot graph");
+	auto one = [&](int shots) {
+		return launch_shoot_one(d.Ft.p, ld, rho32.p, d.area.p, B32.p, dB32.p, n, nrhs, shots, shots_d.p, st);
+	};
+	const bool single = one(0);  // no shot: whether there is a kernel for the size
+	if (!single) {
+		HIP_OK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal), "shot capture");
+		for (int k = 0; k < kGraphShots; k++) launch_shot(k);
+		HIP_OK(hipStreamEndCapture(st, &run.g), "shot capture");
+		HIP_OK(hipGraphInstantiate(&run.x, run.g, nullptr, nullptr, 0), "shot graph");
+	}
 	const auto t0 = std::chrono::steady_clock::now();
-	hipLaunchKernelGGL(k_lsel, dim3(nb), dim3(kB), 0, st, dB32.p, d.area.p, n, nrhs, rec.p);
+	if (!single)
+		hipLaunchKernelGGL(k_lsel, dim3(nb), dim3(kB), 0, st, dB32.p, d.area.p, n, nrhs, rec.p);
 	double check_ms = 0.0, ms_target = -1.0, errv = -1.0;
-	int launched = 0, chunk = 64, done_shots = 0;
+	// shots per look at the state: as many as the error against Bref may be
+	// late by; with none to check, a launch of the one-block kernel ends by itself
+	int launched = 0, chunk = single && !Bref ? 4096 : 64, done_shots = 0;
 	for (;;) {
 		const int b = std::min(chunk, max_shots - launched);
 		if (b <= 0) break;
-		int k = 0;
-		if ((launched & 1) == 0)
-			for (; k + kGraphShots <= b; k += kGraphShots) HIP_OK(hipGraphLaunch(run.x, st), "shot graph launch");
-		for (; k < b; k++) launch_shot(launched + k);
+		if (single) {
+			one(b);
+		} else {
+			int k = 0;
+			if ((launched & 1) == 0)
+				for (; k + kGraphShots <= b; k += kGraphShots) HIP_OK(hipGraphLaunch(run.x, st), "shot graph launch");
+			for (; k < b; k++) launch_shot(launched + k);
+		}
 		launched += b;
 		HIP_OK(hipGetLastError(), "shoot launch");
 		HIP_OK(hipMemcpyAsync(&done_shots, shots_d.p, sizeof(int), hipMemcpyDeviceToHost, st), "state");

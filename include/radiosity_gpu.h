@@ -235,7 +235,8 @@ rad_status rad_lin_gather(rad_lin *lin, int prec, int nrhs, const double *rho, c
 /* Plain FP32 progressive shooting on the same system, the reference's method
  * (source = largest unshot power area_j * sum_c dB_j, ties to the lowest
  * index as MaxDeltaRad, rad.cpp:359-386; update rho_i F_ij dB_j as
- * CalRadiosity, shade.cpp:244-259), one device launch per shot.  Stops when
+ * CalRadiosity, shade.cpp:244-259), many shots a launch where one block holds
+ * the system (8192 patches x 3 columns, 12288 x 1), else one.  Stops when
  * no unshot power is left, after max_shots, or when the error against Bref
  * (if given) reaches target.  nrhs 1..16. */
 rad_status rad_lin_shoot(rad_lin *lin, int nrhs, const double *rho, const double *E, const double *Bref,

@@ -1,9 +1,15 @@
 """The device products of the explicit-matrix solvers at the edges of their
 tiles and dispatch rules, against plain float64."""
+import os
+import sys
+
 import numpy as np
 import pytest
 
 import radgpu
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oracle"))
+import linear as lo  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 U64 = 2.0 ** -53
@@ -45,3 +51,21 @@ def test_gather_tile_rule(n, nrhs, prec):
     r = E + rho * (F.astype(np.float64) @ B) - B
     # the solver's own residual and this one differ by rounding in float64 only
     assert np.linalg.norm(r) <= tol * np.linalg.norm(E) + 1e-12 * np.linalg.norm(B)
+
+
+# plain shooting in one block (every patches-per-thread and column form, the
+# ragged ends, equal powers) and past its limits, bit for bit
+@pytest.mark.parametrize("n,nrhs", [(1, 1), (63, 2), (1024, 1), (1025, 3), (2049, 3), (4097, 5), (5000, 3), (8192, 3), (8193, 3),
+                                    (1500, 12), (1024, 16), (1025, 16), (3000, 6), (12288, 1), (12289, 1)])
+def test_shooting_bits(n, nrhs):
+    rng = np.random.default_rng(n + nrhs)
+    F = rng.random((n, n), np.float32) * np.float32(1.6 / n)
+    rho = rng.uniform(0.2, 0.8, (n, nrhs))
+    E = np.where(rng.random((n, 1)) < 0.1, np.round(rng.uniform(0, 4, (n, nrhs))), 0.0)  # many ties
+    shots = 150
+    with radgpu.LinearSystem(n) as lin:
+        lin.set_matrix(F)
+        B, info = lin.shoot(rho, E, max_shots=shots)
+    want, _, src = lo.shoot32(F, rho, E, np.ones(n), shots)
+    assert info["outer"] == len(src)
+    assert np.array_equal(B.astype(np.float32), want)
