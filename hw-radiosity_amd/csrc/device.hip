@@ -62,6 +62,7 @@
 #include "../../include/radiosity_gpu.h"
 #include "octree_gpu.h"
 #include "pack.h"
+#include "segindex.h"
 
 namespace rgpu {
 namespace {
@@ -1219,76 +1220,78 @@ __global__ __launch_bounds__(kBlock) void k_ff_rows(DScene S, DRecv R, int n, in
 
 // ---- explicit matrix with segment visibility -------------------------------
 // The gathering matrix asks whether anything blocks the open segment between
-// two centroids.  Point location is geometric (the 2^D grid of the deepest
-// octree level, each cell mapped to its leaf), the walk is Amanatides-Woo over
-// that grid (at most 3 * 2^D steps), and each leaf's complete list is tested
-// once (a leaf is a box, so its cells are consecutive along a segment).  The
-// test of one original is TriHitted's plane and side-plane arithmetic with the
-// segment's parameter range (1e-4, 1 - 1e-4).
+// two centroids: whether the test of any original but their own accepts it.
+// The test is TriHitted's plane and side-plane arithmetic with the segment's
+// parameter range (1e-4, 1 - 1e-4).  The walk goes through the cells of
+// SegIndex's grid (Amanatides-Woo, a bit per cell in LDS saying whether it
+// lists any triangle) and tests the lists it meets; which triangles those are
+// does not matter to the answer as long as none is missed that would accept.
 constexpr float kSegLo = 0.0001f, kSegHi = 0.9999f;
 
-struct DFine {
-	const int *__restrict__ leaf;        // R^3 cell -> leaf
-	const int *__restrict__ begin;       // leaf -> first record, n_leaves + 1
-	const float4 *__restrict__ nc;       // 2 per record: {n, c.x}, {c.y, c.z, id, -}
+struct DSeg {
+	const unsigned *__restrict__ mask;   // bit per cell: lists any triangle
+	const int *__restrict__ begin;       // cell -> first record
+	const float4 *__restrict__ nc;       // 2 per record: {n, c.x}, {c.y, c.z, id, cull radius}
 	const float4 *__restrict__ se;       // 3 per record: side planes
-	int r;
+	int ny, nz, words;                   // cells per axis (border included), words of mask
+	int inner[3];                        // cells per axis without the border
 	float g0[3], h[3], inv[3];
+	float cull_cl;                       // DScene's
 };
 
+// The cells are walked along wp + t wv, the tests run along (px, ..) + t (vx,
+// ..): the same segment, in the same direction or the other.
 template <bool F>
-__device__ bool seg_occluded(const DFine &G, float px, float py, float pz, float vx, float vy, float vz, int ban0,
-                             int ban1, Cnt &c)
+__device__ __forceinline__ bool seg_occluded(const DSeg &G, const unsigned *mask, const float (&wp)[3], const float (&wv)[3],
+                                             float px, float py, float pz, float vx, float vy, float vz, int ban0,
+                                             int ban1, Cnt &c)
 {
-	const int R = G.r;
-	const float p[3] = {px, py, pz}, v[3] = {vx, vy, vz};
-	int cell[3], step[3];
-	float tmax[3], tdelta[3];
+	const int stride[3] = {G.ny * G.nz, G.nz, 1};
+	int idx = 0, step[3];
+	float tn[3], td[3];  // parameter of the next cell wall of each axis, and between walls
 #pragma unroll
 	for (int k = 0; k < 3; k++) {
-		const float rel = p[k] - G.g0[k];
-		int ck = (int)floorf(rel * G.inv[k]);
-		ck = ck < 0 ? 0 : (ck >= R ? R - 1 : ck);
-		cell[k] = ck;
-		if (v[k] > 0.0f) {
-			step[k] = 1;
-			tmax[k] = ((float)(ck + 1) * G.h[k] - rel) / v[k];
-			tdelta[k] = G.h[k] / v[k];
-		} else if (v[k] < 0.0f) {
-			step[k] = -1;
-			tmax[k] = ((float)ck * G.h[k] - rel) / v[k];
-			tdelta[k] = -G.h[k] / v[k];
-		} else {
-			step[k] = 0;
-			tmax[k] = tdelta[k] = __builtin_inff();
-		}
+		const float rel = wp[k] - G.g0[k];
+		const int ck = min(max((int)floorf(rel * G.inv[k]), 0), G.inner[k] - 1);
+		idx += (ck + 1) * stride[k];
+		const bool up = wv[k] > 0.0f, still = wv[k] == 0.0f;
+		const float iv = 1.0f / wv[k];
+		step[k] = up ? stride[k] : -stride[k];
+		tn[k] = still ? __builtin_inff() : ((float)(up ? ck + 1 : ck) * G.h[k] - rel) * iv;
+		td[k] = still ? 0.0f : G.h[k] * fabsf(iv);
 	}
+	// test_entry's cull margin
+	const float vl = (fabsf(vx) + fabsf(vy) + fabsf(vz)) * 0x1p-11f;
+	const float cb = (fabsf(px) + fabsf(py) + fabsf(pz) + G.cull_cl) * 0x1p-12f;
 	c.rays++;
-	int last = -1;
 	for (;;) {
-		const int leaf = G.leaf[(cell[0] * R + cell[1]) * R + cell[2]];  // R^3 < 2^31
-		if (leaf != last) {
-			last = leaf;
+		if ((mask[idx >> 5] >> (idx & 31)) & 1u) {
 			c.cells++;
-			const int e0 = G.begin[leaf], e1 = G.begin[leaf + 1];
-			// the whole 32-byte record at once, the next one in flight; the
-			// load is not conditional (the index is clamped to the list), so
-			// that the wait before a test covers only the loads it needs
-			float4 na = make_float4(0.f, 0.f, 0.f, 0.f), nb = na;
-			if (e0 < e1) {
-				na = G.nc[2 * e0];
-				nb = G.nc[2 * e0 + 1];
-			}
+			const int e0 = G.begin[idx], e1 = G.begin[idx + 1];
+			// the next record in flight; the load is not conditional (the index
+			// is clamped to the list), so that the wait before a test covers only
+			// the loads it needs
+			float4 na = G.nc[2 * e0], nb = G.nc[2 * e0 + 1];
 			for (int e = e0; e < e1; e++) {
 				const float4 a = na, b = nb;
 				const int en = min(e + 1, e1 - 1);
 				na = G.nc[2 * en];
 				nb = G.nc[2 * en + 1];
 				const int id = __float_as_int(b.z);
-				if (id == ban0 || id == ban1) continue;
-				c.tests++;
+				const bool own = (id == ban0) | (id == ban1);
+				c.tests += own ? 0 : 1;
 				const float a1 = dot3<F>(vx, vy, vz, a.x, a.y, a.z);
 				const float a2 = dot3<F>(a.w - px, b.x - py, b.y - pz, a.x, a.y, a.z);
+				// test_entry's exact rejections from the quotient's estimate
+				const float fa1 = fabsf(a1);
+				const bool est = (fa1 >= 0x1p-100f) & (fa1 <= 0x1p100f) & (fabsf(a2) <= 0x1p100f);
+				const float ta = a2 * __builtin_amdgcn_rcpf(a1);
+				const float qx = __builtin_fmaf(ta, vx, px) - a.w, qy = __builtin_fmaf(ta, vy, py) - b.x,
+				            qz = __builtin_fmaf(ta, vz, pz) - b.y;
+				const float d2 = __builtin_fmaf(qz, qz, __builtin_fmaf(qy, qy, qx * qx));
+				const float lim = __builtin_fmaf(b.w, 1.0f + 0x1p-11f, __builtin_fmaf(fabsf(ta), vl, cb));
+				const bool rej = est & ((ta < kSegLo * kGuardDown) | (ta > kSegHi * kGuardUp) | (d2 > lim * lim));
+				if (own | rej) continue;
 				const float tt = a2 / a1;
 				if (!(tt > kSegLo && tt < kSegHi)) continue;
 				const float hx = axpy<F>(tt, vx, px), hy = axpy<F>(tt, vy, py), hz = axpy<F>(tt, vz, pz);
@@ -1300,21 +1303,35 @@ __device__ bool seg_occluded(const DFine &G, float px, float py, float pz, float
 					return true;
 			}
 		}
-		const int ax = tmax[0] <= tmax[1] ? (tmax[0] <= tmax[2] ? 0 : 2) : (tmax[1] <= tmax[2] ? 1 : 2);
-		if (tmax[ax] >= 1.0f) return false;
-		cell[ax] += step[ax];
-		if ((unsigned)cell[ax] >= (unsigned)R) return false;
-		tmax[ax] += tdelta[ax];
+		const float t = fminf(fminf(tn[0], tn[1]), tn[2]);
+		if (!(t < 1.0f)) return false;
+		const bool ax = tn[0] == t, ay = !ax & (tn[1] == t), az = !(ax | ay);
+		idx += ax ? step[0] : ay ? step[1] : step[2];
+		tn[0] += ax ? td[0] : 0.0f;
+		tn[1] += ay ? td[1] : 0.0f;
+		tn[2] += az ? td[2] : 0.0f;
 	}
 }
 
-// Visibility of every unordered pair, once: tile (ti <= tj) of 64 x 64 pairs
-// per block; wave w takes rows ti*64 + 16w .. +15, lane l column tj*64 + l,
-// so a wave's 64 rays at a time leave one centroid for 64 neighbouring ones.
-// The segment runs from the lower slot index to the higher; pairs that do
-// not face each other (CalFF's sign test, which is symmetric) are left 0.
-// vis[i * nt + j/64] bit j%64 = 1 when i and j see each other; the block
-// writes its tile and, transposed through LDS, the mirror tile.
+// Visibility of every unordered pair, once.  Patches are taken in R.order (a
+// Z-order curve of their centroids), so that 64 consecutive ones are one
+// neighbourhood: tile (ti <= tj) of 64 x 64 positions, RB of its rows per block
+// (64, or fewer where a block a tile would leave CUs idle); wave w takes RB / 4
+// rows, lane l column tj*64 + l, so a wave's 64 segments at a time fan out
+// narrowly from one centroid, meet the same cells and read the same records.
+// Each is tested from the lower slot index to the higher whichever way it is
+// walked; pairs that do not face each other (CalFF's sign test, which is
+// symmetric) are left 0.  vis[a * nt + b/64] bit b%64 = 1 when the patches at
+// positions a and b see each other; the block writes its rows and, transposed
+// through LDS, its RB bits of the mirror tile's words.
+// Bound by VALU issue with the lanes' lists of different lengths (7 tests a
+// segment on average, several times that for the longest of 64).  Rooms of
+// 1000, 3000, 9000, 20000 patches, ms with k_ff_seg: 2.08, 4.11, 16.6, 71.2
+// over the octree's leaves with every original listed and slots in order
+// (17 leaves and 54 tests a segment); 1.12, 2.24, 6.4, 26.5 without the walls;
+// 0.11, 0.64, 4.9, 19.8 on the grid of segindex.h; 0.10, 0.61, 2.9, 12.6 in
+// Z-order.  Trying the record that blocked the lane's last segment first: the
+// same (few segments are blocked).
 __device__ __forceinline__ int tri_tile(int t, int nt, int &tj)
 {
 	// t -> (ti, tj) over ti <= tj, row by row: row r starts at
@@ -1328,52 +1345,80 @@ __device__ __forceinline__ int tri_tile(int t, int nt, int &tj)
 	return ti;
 }
 
-template <bool F>
-__global__ __launch_bounds__(kBlock) void k_vis_tiles(DFine G, DRecv R, int n, int nt,
-                                                      unsigned long long *vis, long long *bcnt)
+template <bool F, int RB>
+__global__ __launch_bounds__(kBlock) void k_vis_tiles(DSeg G, DRecv R, int n, int nt, unsigned char *vis,
+                                                      long long *bcnt)
 {
-	__shared__ unsigned long long rowbits[64];
+	extern __shared__ unsigned mask[];
+	__shared__ unsigned long long rowbits[RB];
+	constexpr int PER = 64 / RB;  // blocks per tile
 	int tj;
-	const int ti = tri_tile(blockIdx.x, nt, tj);
+	const int ti = tri_tile(blockIdx.x / PER, nt, tj), row0 = blockIdx.x % PER * RB;
 	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-	const int j = tj * 64 + lane;
+	for (int k = threadIdx.x; k < G.words; k += kBlock) mask[k] = G.mask[k];
+	const int pb = tj * 64 + lane;
+	const int b = pb < n ? R.order[pb] : -1;
 	Cnt c = {0, 0, 0, 0, 0, 0, 0};
-	float4 nj = make_float4(0.f, 0.f, 0.f, 0.f), cj = nj;
-	int pj = -1;
-	if (j < n) {
-		nj = R.nrm[j];
-		cj = R.cA[j];
-		pj = __float_as_int(nj.w);
-	}
-	for (int q = 0; q < 16; q++) {
-		const int i = ti * 64 + w * 16 + q;  // wave-uniform
-		bool see = false;
-		if (i < n && j < n && i < j && pj >= 0) {
-			const float4 ni = R.nrm[i], ci = R.cA[i];
-			const int pi = __float_as_int(ni.w);
-			const float dx = cj.x - ci.x, dy = cj.y - ci.y, dz = cj.z - ci.z;
-			const float ds = dot3<F>(dx, dy, dz, nj.x, nj.y, nj.z);
-			const float dd = -dot3<F>(dx, dy, dz, ni.x, ni.y, ni.z);
-			if (pi >= 0 && (ds < 0) == (dd < 0) && ds != 0.0f && dd != 0.0f)
-				see = !seg_occluded<F>(G, ci.x, ci.y, ci.z, dx, dy, dz, pi, pj, c);
-		}
-		const unsigned long long bits = __ballot(see);
-		if (lane == 0) rowbits[w * 16 + q] = bits;
+	float4 nb = make_float4(0.f, 0.f, 0.f, 0.f), cb = nb;
+	int parb = -1;
+	if (b >= 0) {
+		nb = R.nrm[b];
+		cb = R.cA[b];
+		parb = __float_as_int(nb.w);
 	}
 	__syncthreads();
+	for (int q = 0; q < RB / 4; q++) {
+		const int pa = ti * 64 + row0 + w * (RB / 4) + q;  // wave-uniform
+		bool see = false;
+		if (pa < n && b >= 0 && pa < pb && parb >= 0) {
+			const int a = __builtin_amdgcn_readfirstlane(R.order[pa]);
+			const float4 na = R.nrm[a], ca = R.cA[a];
+			const int para = __float_as_int(na.w);
+			const bool fwd = a < b;  // the tested segment starts at a
+			const float wx = cb.x - ca.x, wy = cb.y - ca.y, wz = cb.z - ca.z;
+			const float dx = fwd ? wx : -wx, dy = fwd ? wy : -wy, dz = fwd ? wz : -wz;
+			const float sa = dot3<F>(dx, dy, dz, na.x, na.y, na.z), sb = dot3<F>(dx, dy, dz, nb.x, nb.y, nb.z);
+			const float ds = fwd ? sb : sa, dd = fwd ? -sa : -sb;
+			if (para >= 0 && (ds < 0) == (dd < 0) && ds != 0.0f && dd != 0.0f) {
+				const float wp[3] = {ca.x, ca.y, ca.z}, wv[3] = {wx, wy, wz};
+				see = !seg_occluded<F>(G, mask, wp, wv, fwd ? ca.x : cb.x, fwd ? ca.y : cb.y, fwd ? ca.z : cb.z, dx, dy, dz,
+				                       para, parb, c);
+			}
+		}
+		const unsigned long long bits = __ballot(see);
+		if (lane == 0) rowbits[w * (RB / 4) + q] = bits;
+	}
+	__syncthreads();
+	// a row of the matrix is nt words of 8 bytes, and the block's RB bits of a
+	// word are RB / 8 of them, from byte row0 / 8
+	constexpr int NB = RB / 8;
 	if (threadIdx.x < 64) {
 		const int r = threadIdx.x;
-		if (ti * 64 + r < n) vis[(size_t)(ti * 64 + r) * nt + tj] = rowbits[r];
-		// mirror: row tj*64 + r, bits over the tile's rows
-		unsigned long long m = 0;
-		for (int q = 0; q < 64; q++) m |= ((rowbits[q] >> r) & 1ull) << q;
-		if (tj * 64 + r < n) {
-			if (ti == tj) m |= rowbits[r];  // diagonal tile: both halves in one word
-			vis[(size_t)(tj * 64 + r) * nt + ti] = m;
+		unsigned long long m = 0;  // mirror: row tj*64 + r, bits over the block's rows
+		for (int q = 0; q < RB; q++) m |= ((rowbits[q] >> r) & 1ull) << q;
+		const bool mine = r >= row0 && r < row0 + RB;
+		if (ti == tj && mine) m |= (rowbits[r - row0] >> row0) & (RB == 64 ? ~0ull : (1ull << (RB & 63)) - 1);
+		// a diagonal tile's row holds its own bits from its block on and the
+		// mirrored ones of the blocks before
+		const bool put = ti != tj || r >= row0;
+		if (tj * 64 + r < n && put) {
+			unsigned char *o = vis + ((size_t)(tj * 64 + r) * nt + ti) * 8 + row0 / 8;
+			for (int k = 0; k < NB; k++) o[k] = (unsigned char)(m >> (8 * k));
+		}
+		if (mine && ti * 64 + r < n) {
+			unsigned char *o = vis + ((size_t)(ti * 64 + r) * nt + tj) * 8;
+			const unsigned long long b = rowbits[r - row0];
+			for (int k = ti == tj ? row0 / 8 + NB : 0; k < 8; k++) o[k] = (unsigned char)(b >> (8 * k));
 		}
 	}
 	const int vals[8] = {c.rays, c.ref_rays, c.cells, c.tests, c.levels, c.precision, c.stalled, 0};
 	add_block_counters(vals, bcnt);
+}
+
+__global__ __launch_bounds__(kBlock) void k_positions(const int *order, int n, int *pos)
+{
+	const int p = blockIdx.x * kBlock + threadIdx.x;
+	if (p < n) pos[order[p]] = p;
 }
 
 // Row i (one block): F[i][j] = CalFF's value from the centroid of i to the
@@ -1382,7 +1427,7 @@ __global__ __launch_bounds__(kBlock) void k_vis_tiles(DFine G, DRecv R, int n, i
 // when its double sum (fixed reduction order) exceeds 1.
 template <bool F>
 __global__ __launch_bounds__(kBlock) void k_ff_seg(DRecv R, int n, int ld, int nt, const unsigned long long *vis,
-                                                   float *Fm)
+                                                   const int *pos, float *Fm)
 {
 	__shared__ double wsum[kWavesPerBlock];
 	const int i = blockIdx.x;
@@ -1391,13 +1436,16 @@ __global__ __launch_bounds__(kBlock) void k_ff_seg(DRecv R, int n, int ld, int n
 	const int pi = __float_as_int(ni.w);
 	const float nlen_i = __builtin_sqrtf(dot3<F>(ni.x, ni.y, ni.z, ni.x, ni.y, ni.z));
 	float *row = Fm + (size_t)i * ld;
-	const unsigned long long *vrow = vis + (size_t)i * nt;
+	// its visibility bits, by position (pos[slot])
+	extern __shared__ unsigned long long vrow[];
+	for (int k = threadIdx.x; k < nt; k += kBlock) vrow[k] = vis[(size_t)pos[i] * nt + k];
+	__syncthreads();
 	double sum = 0.0;
 	for (int j = threadIdx.x; j < n; j += kBlock) {
 		float ff = 0.0f;
 		const float4 nj = R.nrm[j], cj = R.cA[j];
 		const int pj = __float_as_int(nj.w);
-		if (j != i && pi >= 0 && pj >= 0 && ((vrow[j >> 6] >> (j & 63)) & 1ull)) {
+		if (j != i && pi >= 0 && pj >= 0 && ((vrow[pos[j] >> 6] >> (pos[j] & 63)) & 1ull)) {
 			SrcPatch sp;
 			sp.c[0] = cj.x; sp.c[1] = cj.y; sp.c[2] = cj.z;
 			sp.n[0] = nj.x; sp.n[1] = nj.y; sp.n[2] = nj.z;
@@ -2154,10 +2202,13 @@ struct DeviceEngine::Impl {
 	DevBuf<float4> lnc, lse, leaf_box, nrm, cA, rho, acc, dacc, dB;
 	DevBuf<int> cell_leaf;
 	DevBuf<float> vx, vy, vz;
-	DevBuf<int> fine_leaf, seg_begin;  // segment-visibility index (explicit matrix)
+	SegIndex seg;                      // segment visibility of the explicit matrix, on the host
+	DevBuf<unsigned> seg_mask;         // ... and on the device
+	DevBuf<int> seg_begin, pos;        // pos: each slot's position in order
 	DevBuf<unsigned long long> vis;    // pair visibility bits of the explicit matrix
 	DevBuf<float4> seg_nc, seg_se;
 	bool have_seg = false;
+	float seg_cl = 0.f;                // bound on |c|_1 of the records with a cull radius
 	DevBuf<Loop> loop;
 	DevBuf<long long> bcnt;
 	DevBuf<unsigned long long> cand;
@@ -2839,29 +2890,39 @@ int DeviceEngine::form_factors(float *dF, int n, int ld, int vis, FlatOctree &t,
 			      " slots, " + std::to_string(s.n_orig) + " originals)";
 			return -1;
 		}
-		if (build_segment_index(t, s.pool.data(), s.n_orig, s.G0, s.G1, err)) return -1;
-		const size_t ne = t.seg_items.size();
-		if (ne >= ((size_t)1 << 29) || (size_t)t.fine_r * t.fine_r * t.fine_r >= ((size_t)1 << 31)) {
-			err = "segment index too large for 32-bit record and cell indices";  // the walk indexes in int
+		// originals only: upload's cull radii are theirs
+		std::vector<float> rad((size_t)s.n_orig + 1);
+		d.seg_cl = cull_radii(s, rad.data());
+		build_segment_index(d.seg, s.pool.data(), s.n_orig, rad.data());
+		const size_t ne = d.seg.items.size();
+		if (ne >= ((size_t)1 << 29)) {
+			err = "segment index too large for 32-bit record indices";  // the walk indexes in int
 			return -1;
 		}
-		std::vector<float4> nc(2 * ne), se(3 * ne);
+		std::vector<float4> nc(2 * ne + 2), se(3 * ne + 3);
 		for (size_t e = 0; e < ne; e++) {
-			const Patch &p = s.pool[t.seg_items[e]];
+			const int id = d.seg.items[e];
+			const Patch &p = s.pool[id];
 			float idf;
-			std::memcpy(&idf, &t.seg_items[e], 4);
+			std::memcpy(&idf, &id, 4);
 			nc[2 * e] = make_float4(p.n[0], p.n[1], p.n[2], p.c[0]);
-			nc[2 * e + 1] = make_float4(p.c[1], p.c[2], idf, 0.f);
+			nc[2 * e + 1] = make_float4(p.c[1], p.c[2], idf, rad[id]);
 			for (int q = 0; q < 3; q++) se[3 * e + q] = make_float4(p.se[q][0], p.se[q][1], p.se[q][2], p.se[q][3]);
 		}
-		if (d.fine_leaf.put(t.fine_leaf.data(), t.fine_leaf.size(), st, err) ||
-		    d.seg_begin.put(t.seg_begin.data(), t.seg_begin.size(), st, err) ||
+		if (d.seg_mask.put(d.seg.mask.data(), d.seg.mask.size(), st, err) ||
+		    d.seg_begin.put(d.seg.begin.data(), d.seg.begin.size(), st, err) ||
 		    d.seg_nc.put(nc.data(), nc.size(), st, err) || d.seg_se.put(se.data(), se.size(), st, err))
 			return -1;
 		HIP_OK(hipStreamSynchronize(st), "segment index upload");
 		d.have_seg = true;
 	}
-	const size_t nblk_ff = std::max<size_t>((size_t)n, (size_t)((n + 63) / 64) * ((n + 63) / 64 + 1) / 2);
+	// rows of a 64 x 64 tile per block: fewer than 64 while that leaves less
+	// than eight blocks per CU
+	const int nt = (n + 63) / 64;
+	const long long tiles = (long long)nt * (nt + 1) / 2;
+	int rb = 64;
+	while (rb > 8 && tiles * (64 / rb) < 2048) rb /= 2;
+	const size_t nblk_ff = std::max<size_t>((size_t)n, (size_t)tiles * (64 / rb));
 	if (d.bcnt.n < nblk_ff * 8) {  // the largest grid of the two kernels indexes bcnt
 		std::vector<long long> zeros(nblk_ff * 8, 0);
 		if (d.bcnt.put(zeros.data(), zeros.size(), st, err)) return -1;
@@ -2869,24 +2930,35 @@ int DeviceEngine::form_factors(float *dF, int n, int ld, int vis, FlatOctree &t,
 	}
 	HIP_OK(hipEventRecord(d.ev0, st), "event");
 	if (vis == VIS_SEGMENT) {
-		DFine G;
-		G.leaf = d.fine_leaf.p;
+		const SegIndex &g = d.seg;
+		DSeg G;
+		G.mask = d.seg_mask.p;
 		G.begin = d.seg_begin.p;
 		G.nc = d.seg_nc.p;
 		G.se = d.seg_se.p;
-		G.r = t.fine_r;
+		G.ny = g.r[1];
+		G.nz = g.r[2];
+		G.words = (int)g.mask.size();
+		G.cull_cl = d.seg_cl;
 		for (int k = 0; k < 3; k++) {
-			G.g0[k] = s.G0[k];
-			G.h[k] = (s.G1[k] - s.G0[k]) / (float)t.fine_r;
-			G.inv[k] = (float)t.fine_r / (s.G1[k] - s.G0[k]);
+			G.inner[k] = g.r[k] - 2;
+			G.g0[k] = g.g0[k];
+			G.h[k] = g.h[k];
+			G.inv[k] = 1.0f / g.h[k];
 		}
-		const int nt = (n + 63) / 64;
-		const long long tiles = (long long)nt * (nt + 1) / 2;
-		if (d.vis.alloc((size_t)n * nt, err)) return -1;
-		if (d.fma) hipLaunchKernelGGL(k_vis_tiles<true>, dim3((unsigned)tiles), dim3(kBlock), 0, st, G, d.R, n, nt, d.vis.p, d.bcnt.p);
-		else hipLaunchKernelGGL(k_vis_tiles<false>, dim3((unsigned)tiles), dim3(kBlock), 0, st, G, d.R, n, nt, d.vis.p, d.bcnt.p);
-		if (d.fma) hipLaunchKernelGGL(k_ff_seg<true>, dim3(n), dim3(kBlock), 0, st, d.R, n, ld, nt, d.vis.p, dF);
-		else hipLaunchKernelGGL(k_ff_seg<false>, dim3(n), dim3(kBlock), 0, st, d.R, n, ld, nt, d.vis.p, dF);
+		if (d.vis.alloc((size_t)n * nt, err) || d.pos.alloc(n, err)) return -1;
+		hipLaunchKernelGGL(k_positions, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, d.order.p, n, d.pos.p);
+		const dim3 vg((unsigned)(tiles * (64 / rb)));
+		const size_t lds = (size_t)G.words * sizeof(unsigned);
+#define VIS(RB)                                                                                                        \
+	if (rb == RB) {                                                                                                    \
+		if (d.fma) hipLaunchKernelGGL((k_vis_tiles<true, RB>), vg, dim3(kBlock), lds, st, G, d.R, n, nt, (unsigned char *)d.vis.p, d.bcnt.p); \
+		else hipLaunchKernelGGL((k_vis_tiles<false, RB>), vg, dim3(kBlock), lds, st, G, d.R, n, nt, (unsigned char *)d.vis.p, d.bcnt.p);      \
+	}
+		VIS(64) VIS(32) VIS(16) VIS(8)
+#undef VIS
+		if (d.fma) hipLaunchKernelGGL(k_ff_seg<true>, dim3(n), dim3(kBlock), (size_t)nt * 8, st, d.R, n, ld, nt, d.vis.p, d.pos.p, dF);
+		else hipLaunchKernelGGL(k_ff_seg<false>, dim3(n), dim3(kBlock), (size_t)nt * 8, st, d.R, n, ld, nt, d.vis.p, d.pos.p, dF);
 	} else {
 		if (d.fma) hipLaunchKernelGGL(k_ff_rows<true>, dim3(n), dim3(kBlock), 0, st, d.S, d.R, n, ld, dF, d.bcnt.p);
 		else hipLaunchKernelGGL(k_ff_rows<false>, dim3(n), dim3(kBlock), 0, st, d.S, d.R, n, ld, dF, d.bcnt.p);

@@ -196,7 +196,8 @@ const char *rad_lin_last_error(const rad_lin *lin);
  *   RAD_VIS_SEGMENT    nothing crosses the open segment between the two
  *                      centroids (parameter in (1e-4, 1 - 1e-4), walked from
  *                      the lower slot index to the higher, so symmetric),
- *                      found by a grid walk over complete octree leaf lists;
+ *                      found by a grid walk over complete lists of the
+ *                      triangles that can block any segment;
  *                      needs a scene that pre-partition left unsplit
  *   RAD_VIS_REFERENCE  RayHitted from the centroid returns j
  *                      (raycast.cpp:335-360), blind spots included
