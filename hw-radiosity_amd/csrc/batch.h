@@ -12,9 +12,9 @@
 
 namespace rgpu {
 
-// Schedule of the batched sweep product: each wave owns 16*rt rows (a tile
-// is 64*rt rows of one scene), a tile spans kc of k, and grid persistent
-// blocks walk the tile list.
+// Schedule of the batched sweep: each wave owns 16*rt rows, a block's eight
+// waves split K into chunks of kc or more (at most eight) and take as many row
+// groups as that leaves, and grid persistent blocks walk the tile list.
 struct BatchTile {
 	int rt, kc, grid;
 };
@@ -30,12 +30,13 @@ public:
 	float *matrix32(int s);  // device, ld(s) x ld(s) row-major, zero padded
 	int set_matrix(int s, const float *F, std::string &err);
 	// Times one sweep for every candidate schedule on the current matrices
-	// and keeps the fastest for precision prec; solve does it on first use
-	// unless set_tile fixed the schedule.
+	// and keeps the fastest for precision prec; without it or set_tile the
+	// schedule goes by the batch's size.
 	int autotune(int prec, BatchTile &out, std::string &err);
 	int set_tile(const BatchTile &t, std::string &err);
 	// rho, E, B: (total() x 3) row-major, scenes concatenated in order.
-	// graph = true: one HIP graph launch for everything; false: the same
+	// graph = true: a HIP graph launch per refinement of all scenes, until none
+	// is above tol; false: the same
 	// kernels launched scene after scene (the unbatched reference schedule,
 	// bit-identical results).  rel_res[count] = each scene's final FP64
 	// relative residual.  info[4]: device ms of the solve, ms to build the

@@ -4,18 +4,15 @@
 //   F32   ld_s^2 floats at off[s], row-major (the matrix of record)
 //   F16 / BF16  ld_s^2 at off[s], MFMA fragment order, one power-of-two scale
 //         for the whole batch (FP16)
-//   rows  n_s * 3 at voff[s]: rho, E, residual, scaled residual, correction
+//   rows  n_s * 3 at voff[s]: rho, E, residual, scaled residual, answer
 //   xT    16 x ld_s at xoff[s]: FP64 iterate (rows 0..2 used), and its
-//         low-precision copy in fragment order for the MFMA B operand
-//   part64  ceil(ld_s / 2048) x ld_s x 16 at poff[s]: split-K partials of
-//         the FP64 residual product
-//   part32  ceil(ld_s / kc) x ld_s x 16 at goff[s] (room for kc = 1024):
-//         split-K partials of the sweep product
-// Work lists, sorted by scene: residual tiles {scene, 256-row block, k range
-// of 2048}; sweep-product tiles {scene, 64*rt-row block, k range of kc},
-// whose shape (rt, kc) and persistent grid come from the autotuner; element
-// tiles {scene, first element} of 256 elements, never straddling a scene, so
-// per-scene norms are sums over a fixed range of tile partials.
+//         low-precision copies (two, read and written in turn) in fragment
+//         order for the MFMA B operand
+// Work lists, sorted by scene: residual tiles {scene, block of 32 / KS rows};
+// sweep tiles {scene, block of 16 rt 8 / S rows, S}, whose shape goes by the
+// schedule; element tiles {scene, first element} of 256 elements, never
+// straddling a scene, so that per-scene norms are sums over a fixed range of
+// tile statistics.
 #include "batch.h"
 #include "linear.h"
 
@@ -36,142 +33,67 @@ namespace {
 #include "stage.h"
 
 constexpr int NR = 3;           // right-hand sides per scene (RGB)
-constexpr int kKChunk = 2048;   // k per residual tile
-constexpr int kPersist = 1024;  // blocks of the element-walking kernels
-constexpr int kMinKc = 1024;    // smallest k chunk of a sweep-product tile
+constexpr int kPersist = 4096;  // blocks of the element-walking kernels
 
 struct BMeta {
-	int n, ld, nk;  // nk = k chunks of the residual product
-	int nkg;        // k chunks of the sweep product (its kc)
-	long long off, voff, xoff, poff, goff;
+	int n, ld;
+	long long off, voff, xoff;
 };
 
-// low-precision sweep product, one tile per block per step of the walk: the
-// block's 4 waves own 16*RT rows each of the tile's 64*RT, over k-blocks
-// [z, w) (kcb = kc / 32 per chunk)
+// one sweep of every active scene: block after block of the list (sweep_rows)
+// in a persistent grid
 template <typename E, int RT>
-__global__ __launch_bounds__(kB) void k_bgemm(const int4 *tiles, int t0, int t1, const BMeta *meta, const int *active,
-                                              const E *F16, const E *XT, float *part, int kcb)
+__global__ __launch_bounds__(kSweepWaves * 64) void k_bsweep(const int4 *tiles, int t0, int t1, const BMeta *meta,
+                                                             const int *active, const E *F, const E *X, bool cached,
+                                                             float inv, const float *r32, const float *rho, E *Xn,
+                                                             double *xT, const double *scale)
 {
+	__shared__ f4 red[kSweepWaves * RT * 64];
 	for (int t = t0 + blockIdx.x; t < t1; t += gridDim.x) {
-		const int4 tl = tiles[t];  // scene, row block, k-blocks [z, w)
+		const int4 tl = tiles[t];  // scene, block, S
 		if (!active[tl.x]) continue;
 		const BMeta m = meta[tl.x];
-		gemm_tile<E, RT, 1>(F16 + m.off, XT + m.xoff, part + m.goff + (size_t)(tl.z / kcb) * m.ld * 16, m.ld, 16,
-		                    tl.y * 4 * RT + (threadIdx.x >> 6) * RT, tl.z, tl.w);
+		SweepOut<E> o{};
+		o.n = m.n, o.nrhs = NR, o.inv = inv, o.rhs = r32 + m.voff, o.rho = rho + m.voff, o.XTn = Xn + m.xoff;
+		if (xT) o.xT = xT + m.xoff, o.s = scale[tl.x];
+		sweep_rows<E, RT, 1>(F + m.off, X + m.xoff, m.ld, tl.z, cached, tl.y, red, o);
+		__syncthreads();  // red is read to the end
 	}
 }
 
-// FP64 residual product on the vector FP64 units, same tiles (three columns:
-// a 16-column FP64 MFMA would spend 13 of them on padding).  Per tile the
-// block stages x over the tile's k range (at most kKChunk, a multiple of 256)
-// in LDS, column-major, then walks the 256-row block in passes of 32 rows:
-// wave w takes kBRows rows, each lane 4 consecutive k per step of 256 (one
-// 16-byte load per row, the next step's loads in flight).  The 64 lane
-// partials of the 24 sums are combined by a reduce-scatter: the exchanges
-// over lane bits 5, 4, 3 halve the set each time (12, 6, 3 shuffles) and
-// leave lane l with row l >> 3; bits 2, 1, 0 then sum those 3 in full.
-// Writes part[kc][row][c], c < 3 (rows up to ld; F is zero past n).
-constexpr int kBRows = 8;
-__global__ __launch_bounds__(kB) void k_bfx64v(const int4 *tiles, int t0, int t1, const BMeta *meta, const int *active,
-                                               const float *__restrict__ F32, const double *__restrict__ xT,
-                                               double *__restrict__ part)
+// FP64 residual r = E + rho o (F x) - x of every active scene, with the norms
+// of each tile
+template <int KS>
+__global__ __launch_bounds__(kB) void k_bfx(const int2 *tiles, int t0, int t1, const BMeta *meta, const int *active,
+                                            const float *__restrict__ F32, const double *xT, const double *E,
+                                            const double *rho, double *r, double *blk)
 {
-	typedef float fv4 __attribute__((ext_vector_type(4)));
-	static_assert(kBRows == 8 && NR == 3, "the reduce-scatter assumes 8 rows of 3 columns");
-	__shared__ double xs[NR * kKChunk];
-	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+	__shared__ FxShared<NR, KS> sh;
 	for (int t = t0 + blockIdx.x; t < t1; t += gridDim.x) {
-		const int4 tl = tiles[t];  // scene, 256-row block, k-blocks [z, w)
+		const int2 tl = tiles[t];
 		if (!active[tl.x]) continue;
 		const BMeta m = meta[tl.x];
-		const int k0 = tl.z * 32, nkk = (tl.w - tl.z) * 32;
-		__syncthreads();  // the previous tile's reads of xs are done
-		for (int i = threadIdx.x; i < NR * nkk; i += kB) {
-			const int c = i / nkk, kk = i - c * nkk;
-			xs[c * kKChunk + kk] = xT[m.xoff + (size_t)c * m.ld + k0 + kk];
-		}
+		const double *x = xT + m.xoff;
+		fx64_rows<NR, KS>(F32 + m.off, x, m.ld, m.n, tl.y, sh, x, E + m.voff, rho + m.voff, r + m.voff, blk + 2 * t);
 		__syncthreads();
-		const float *F = F32 + m.off;
-		double *P = part + m.poff + (size_t)(tl.z / (kKChunk / 32)) * m.ld * 16;
-#pragma unroll 1
-		for (int g = 0; g < 256 / (4 * kBRows); g++) {
-			const int r0 = tl.y * 256 + (g * 4 + w) * kBRows;
-			const float *Fr = F + (size_t)r0 * m.ld + k0 + 4 * lane;
-			double v[kBRows * NR];
-#pragma unroll
-			for (int i = 0; i < kBRows * NR; i++) v[i] = 0.0;
-			fv4 a[kBRows], an[kBRows];
-#pragma unroll
-			for (int r = 0; r < kBRows; r++) a[r] = __builtin_nontemporal_load((const fv4 *)(Fr + (size_t)r * m.ld));
-#pragma unroll 1
-			for (int st = 0; st < nkk; st += 256) {
-				if (st + 256 < nkk) {
-#pragma unroll
-					for (int r = 0; r < kBRows; r++)
-						an[r] = __builtin_nontemporal_load((const fv4 *)(Fr + (size_t)r * m.ld + st + 256));
-				}
-				double x[NR][4];
-#pragma unroll
-				for (int c = 0; c < NR; c++)
-#pragma unroll
-					for (int j = 0; j < 4; j++) x[c][j] = xs[c * kKChunk + st + 4 * lane + j];
-#pragma unroll
-				for (int j = 0; j < 4; j++)
-#pragma unroll
-					for (int r = 0; r < kBRows; r++) {
-						const double f = (double)a[r][j];
-#pragma unroll
-						for (int c = 0; c < NR; c++) v[r * NR + c] = __builtin_fma(f, x[c][j], v[r * NR + c]);
-					}
-#pragma unroll
-				for (int r = 0; r < kBRows; r++) a[r] = an[r];
-			}
-#pragma unroll
-			for (int half = kBRows * NR / 2, bit = 32; half >= NR; half >>= 1, bit >>= 1) {
-				const bool upper = (lane & bit) != 0;
-#pragma unroll
-				for (int i = 0; i < half; i++) {
-					const double lo = v[i], hi = v[half + i];
-					v[i] = (upper ? hi : lo) + __shfl_xor(upper ? lo : hi, bit);
-				}
-			}
-#pragma unroll
-			for (int bit = 4; bit > 0; bit >>= 1)
-#pragma unroll
-				for (int c = 0; c < NR; c++) v[c] += __shfl_xor(v[c], bit);
-			if ((lane & 7) == 0) {
-				double *o = P + (size_t)(r0 + (lane >> 3)) * 16;
-#pragma unroll
-				for (int c = 0; c < NR; c++) o[c] = v[c];
-			}
-		}
 	}
 }
 
-// r = E + rho o (F x) - x (FP64; part == null: x = 0, r = E); per element
-// tile: sum of squares and max |r|
-__global__ __launch_bounds__(kB) void k_bresid(const int2 *etiles, int e0, int e1, const BMeta *meta,
-                                               const int *active, const double *part, const double *xT,
-                                               const double *E, const double *rho, double *r, double *blk)
+// the first residual (x = 0): r = E, rho in FP32, and each element tile's norms
+__global__ __launch_bounds__(kB) void k_binit(const int2 *etiles, int e0, int e1, const BMeta *meta, const double *E,
+                                              const double *rho, double *r, float *rho32, double *blk)
 {
 	__shared__ double red[8];
 	for (int t = e0 + blockIdx.x; t < e1; t += gridDim.x) {
 		const int2 et = etiles[t];
-		if (!active[et.x]) continue;
 		const BMeta m = meta[et.x];
 		const int idx = et.y + threadIdx.x;
 		double ss = 0.0, mx = 0.0;
 		if (idx < m.n * NR) {
-			const int i = idx / NR, c = idx % NR;
 			const size_t g = m.voff + idx;
-			double v = E[g];
-			if (part) {
-				double y = 0.0;
-				for (int q = 0; q < m.nk; q++) y += part[m.poff + ((size_t)q * m.ld + i) * 16 + c];
-				v += rho[g] * y - xT[m.xoff + (size_t)c * m.ld + i];
-			}
+			const double v = E[g];
 			r[g] = v;
+			rho32[g] = (float)rho[g];
 			ss = v * v;
 			mx = fabs(v);
 		}
@@ -192,23 +114,36 @@ __global__ __launch_bounds__(kB) void k_bresid(const int2 *etiles, int e0, int e
 	}
 }
 
-// per scene (one block each): norms from its element tiles in order;
-// relative residual, scale for the next correction, still active?
-__global__ void k_bnorm(int sc0, const int *etb, const int *ete, const double *blk, int *active, double *enorm,
-                        double *rel, double *scale, double tol, int first)
+// per scene (one wave each): norms from its tiles [tb, te) in a fixed order;
+// relative residual, scale for the next correction, still active?  state (host
+// memory): the residual and the flag for the host's own look
+struct BState {
+	double rel;
+	int active, pad;
+};
+__global__ void k_bnorm(int sc0, const int *tb, const int *te, const double *blk, int *active, double *enorm,
+                        double *scale, BState *state, double tol, int first)
 {
 	const int s = sc0 + blockIdx.x;
-	if (threadIdx.x != 0 || !active[s]) return;
+	if (!active[s]) return;
 	double ss = 0.0, mx = 0.0;
-	for (int t = etb[s]; t < ete[s]; t++) {
+	for (int t = tb[s] + threadIdx.x; t < te[s]; t += 64) {
 		ss += blk[2 * t];
 		mx = fmax(mx, blk[2 * t + 1]);
 	}
-	if (first) enorm[s] = sqrt(ss);
-	const double r = enorm[s] > 0.0 ? sqrt(ss) / enorm[s] : 0.0;
-	rel[s] = r;
+	for (int off = 32; off > 0; off >>= 1) {
+		ss += __shfl_xor(ss, off);
+		mx = fmax(mx, __shfl_xor(mx, off));
+	}
+	if (threadIdx.x != 0) return;
+	const double e = first ? sqrt(ss) : enorm[s];
+	if (first) enorm[s] = e;
+	const double r = e > 0.0 ? sqrt(ss) / e : 0.0;
+	const int act = (r > tol && mx > 0.0) ? 1 : 0;
 	scale[s] = mx;
-	active[s] = (r > tol && mx > 0.0) ? 1 : 0;
+	active[s] = act;
+	state[s].rel = r;
+	state[s].active = act;
 }
 
 // r32 = r / scale; XT <- r32 (fragment order)
@@ -230,34 +165,6 @@ __global__ __launch_bounds__(kB) void k_bscale(const int2 *etiles, int e0, int e
 	}
 }
 
-// d = r32 + rho o (inv_s * sum part); XT <- d
-template <typename E>
-__global__ __launch_bounds__(kB) void k_bjacobi(const int2 *etiles, int e0, int e1, const BMeta *meta,
-                                                const int *active, const float *part, float inv_s, const float *r32,
-                                                const float *rho, float *d, E *XT)
-{
-	for (int t = e0 + blockIdx.x; t < e1; t += gridDim.x) {
-		const int2 et = etiles[t];
-		if (!active[et.x]) continue;
-		const BMeta m = meta[et.x];
-		const int idx = et.y + threadIdx.x;
-		if (idx >= m.n * NR) continue;
-		const int i = idx / NR, c = idx % NR;
-		const size_t g = m.voff + idx;
-		float y = 0.f;
-		for (int q = 0; q < m.nkg; q++) y += part[m.goff + ((size_t)q * m.ld + i) * 16 + c];
-		const float v = r32[g] + rho[g] * (y * inv_s);
-		d[g] = v;
-		XT[m.xoff + frag_index(c, i, m.ld)] = (E)v;
-	}
-}
-
-// rho in FP32
-__global__ void k_brho(const double *rho, size_t total, float *rho32)
-{
-	for (size_t t = blockIdx.x * (size_t)kB + threadIdx.x; t < total; t += (size_t)gridDim.x * kB) rho32[t] = (float)rho[t];
-}
-
 // out = x, the scenes' rows in the caller's order
 __global__ __launch_bounds__(kB) void k_brows(const int2 *etiles, int ne, const BMeta *meta, const double *xT, double *out)
 {
@@ -269,59 +176,51 @@ __global__ __launch_bounds__(kB) void k_brows(const int2 *etiles, int ne, const 
 	}
 }
 
-// x += scale * d
-__global__ __launch_bounds__(kB) void k_baxpy(const int2 *etiles, int e0, int e1, const BMeta *meta,
-                                              const int *active, const double *scale, const float *d, double *xT)
-{
-	for (int t = e0 + blockIdx.x; t < e1; t += gridDim.x) {
-		const int2 et = etiles[t];
-		if (!active[et.x]) continue;
-		const BMeta m = meta[et.x];
-		const int idx = et.y + threadIdx.x;
-		if (idx >= m.n * NR) continue;
-		xT[m.xoff + (size_t)(idx % NR) * m.ld + idx / NR] += scale[et.x] * (double)d[m.voff + idx];
-	}
-}
-
 }  // namespace
 
 struct SceneBatch::Impl {
 	int count = 0;
 	std::vector<int> n, ld, tb, te, gtb, gte, etb, ete;
 	std::vector<BMeta> meta;
-	size_t fsize = 0, vsize = 0, xsize = 0, psize = 0, gsize = 0;
+	size_t fsize = 0, vsize = 0, xsize = 0;
 	int ntiles = 0, ngtiles = 0, netiles = 0, total = 0;
-	BatchTile gs{0, 0, 0};  // current sweep-product schedule
+	int ks = 4;             // waves per row group of the residual (32 / ks rows a tile)
+	BatchTile gs{0, -1, 0}; // current sweep schedule; kc = 0: S = 8 whatever the size
 	BatchTile best[2] = {{0, 0, 0}, {0, 0, 0}};  // autotuned, per precision
 	bool forced = false;    // set_tile overrides the autotuner
 	hipStream_t st = nullptr;
 	hipEvent_t e0 = nullptr, e1 = nullptr;
 	Stage stage;
 	Buf<double> out;  // the answer as the caller takes it
-	Buf<float> F32, r32, d32, rho32, part32;
-	Buf<_Float16> F16, X16;
-	Buf<__bf16> FB, XB;
-	Buf<double> E64, rho64, r64, xT, part64, blk, enorm, rel, scale;
+	Buf<float> F32, r32, rho32;
+	Buf<_Float16> F16, X16[2];
+	Buf<__bf16> FB, XB[2];
+	Buf<double> E64, rho64, r64, xT, blk, enorm, scale;
 	Buf<int> active, d_tb, d_te, d_etb, d_ete;
-	Buf<int4> tiles, gtiles;
-	Buf<int2> etiles;
+	Buf<int4> gtiles;
+	Buf<int2> tiles, etiles;
 	Buf<BMeta> d_meta;
 	Buf<unsigned> umax;
 	bool have16 = false, haveb = false;
 	float s16 = 1.f;
-	hipGraphExec_t exec = nullptr;
-	hipGraph_t graph = nullptr;
-	int g_prec = -1, g_outer = -1, g_sweeps = -1, g_nodes = 0;
+	// captured once and replayed: the start (clears, first norms) and one
+	// refinement
+	hipGraphExec_t exec[2] = {};
+	hipGraph_t graph[2] = {};
+	int g_prec = -1, g_sweeps = -1, g_nodes[2] = {};
 	double g_tol = -1.0;
 
 	void drop_graph()
 	{
-		if (exec) (void)hipGraphExecDestroy(exec);
-		if (graph) (void)hipGraphDestroy(graph);
-		exec = nullptr;
-		graph = nullptr;
+		for (int k = 0; k < 2; k++) {
+			if (exec[k]) (void)hipGraphExecDestroy(exec[k]);
+			if (graph[k]) (void)hipGraphDestroy(graph[k]);
+			exec[k] = nullptr;
+			graph[k] = nullptr;
+		}
 		g_prec = -1;
 	}
+	BState *state() { return reinterpret_cast<BState *>(stage.stats); }
 	int ensure_lowp(int prec, std::string &err)
 	{
 		if ((prec == PREC_F16 && have16) || (prec == PREC_BF16 && haveb)) return 0;
@@ -359,15 +258,25 @@ struct SceneBatch::Impl {
 		return 0;
 	}
 
+	// the default schedule: every wave of a block on the same rows, 16 of them,
+	// 32 from four blocks of 16 per CU up, 64 from sixty-four (ms per solve at 16,
+	// 32, 64: 8 rooms of 500 to 1000 patches 0.312, 0.305, 0.332; 48 of 500 to
+	// 4000 2.45, 2.26, 2.27; 64 of 3000 to 8000 22.5, 20.5, 20.1)
+	BatchTile rule() const
+	{
+		size_t rows = 0;
+		for (int l : ld) rows += l;
+		return BatchTile{rows / 16 < 1024 ? 1 : rows / 16 < 16384 ? 2 : 4, 0, 16384};
+	}
 	static bool valid_tile(const BatchTile &g)
 	{
 		return (g.rt == 1 || g.rt == 2 || g.rt == 4) &&
 		       (g.kc == 1024 || g.kc == 2048 || g.kc == 4096 || g.kc == 8192) && g.grid >= 64 && g.grid <= 16384;
 	}
-	// rebuilds the sweep-product tile list and chunk counts for schedule g
+	// rebuilds the sweep's tile list for schedule g (g.kc = 0: rule())
 	int set_sched(const BatchTile &g, std::string &err)
 	{
-		if (!valid_tile(g)) {
+		if (g.kc != 0 && !valid_tile(g)) {
 			err = "batch tile: rt in {1, 2, 4}, kc in {1024, 2048, 4096, 8192}, grid 64..16384";
 			return -1;
 		}
@@ -381,65 +290,55 @@ struct SceneBatch::Impl {
 		gtb.assign(count, 0);
 		gte.assign(count, 0);
 		for (const int s : ord) {
-			BMeta &m = meta[s];
-			m.nkg = (m.ld + g.kc - 1) / g.kc;
+			int S = kSweepWaves;  // K split: chunks of at least kc
+			while (g.kc && S > 1 && (S - 1) * g.kc >= ld[s]) S /= 2;
 			gtb[s] = (int)tl.size();
-			for (int rb = 0; rb < m.ld / (64 * g.rt); rb++)
-				for (int q = 0; q < m.nkg; q++) {
-					const int kb0 = q * (g.kc / 32), kb1 = std::min(m.ld / 32, kb0 + g.kc / 32);
-					tl.push_back(make_int4(s, rb, kb0, kb1));
-				}
+			const int wr = kSweepWaves / S * g.rt;  // row tiles per block
+			for (int b = 0; b < (ld[s] / 16 + wr - 1) / wr; b++) tl.push_back(make_int4(s, b, S, 0));
 			gte[s] = (int)tl.size();
 		}
 		ngtiles = (int)tl.size();
 		HIP_OK(hipStreamSynchronize(st), "batch tile");
 		if (gtiles.alloc(tl.size(), err)) return -1;
 		HIP_OK(hipMemcpyAsync(gtiles.p, tl.data(), tl.size() * sizeof(int4), hipMemcpyHostToDevice, st), "batch tile");
-		HIP_OK(hipMemcpyAsync(d_meta.p, meta.data(), count * sizeof(BMeta), hipMemcpyHostToDevice, st), "batch tile");
 		HIP_OK(hipStreamSynchronize(st), "batch tile");
 		gs = g;
 		drop_graph();
 		return 0;
 	}
-	template <typename E> void launch_gemm(const E *Fl, const E *X, int g0, int g1)
+	// one sweep over tiles [g0, g1); last: it adds the correction to x
+	template <typename E> void sweep(const E *F, const E *X, E *Xn, int g0, int g1, float inv, bool last)
 	{
-		const dim3 grid(std::max(1, std::min(gs.grid, g1 - g0)));
-		const int kcb = gs.kc / 32;
-		if (gs.rt == 1)
-			hipLaunchKernelGGL((k_bgemm<E, 1>), grid, dim3(kB), 0, st, gtiles.p, g0, g1, d_meta.p, active.p, Fl, X,
-			                   part32.p, kcb);
-		else if (gs.rt == 2)
-			hipLaunchKernelGGL((k_bgemm<E, 2>), grid, dim3(kB), 0, st, gtiles.p, g0, g1, d_meta.p, active.p, Fl, X,
-			                   part32.p, kcb);
-		else
-			hipLaunchKernelGGL((k_bgemm<E, 4>), grid, dim3(kB), 0, st, gtiles.p, g0, g1, d_meta.p, active.p, Fl, X,
-			                   part32.p, kcb);
+		const dim3 grid(std::max(1, std::min(gs.grid, g1 - g0))), blk(kSweepWaves * 64);
+		const bool cached = stays_cached(fsize);
+		double *x = last ? xT.p : nullptr;
+#define G(R)                                                                                                           \
+	hipLaunchKernelGGL((k_bsweep<E, R>), grid, blk, 0, st, gtiles.p, g0, g1, d_meta.p, active.p, F, X, cached, inv,     \
+	                   r32.p, rho32.p, Xn, x, scale.p)
+		if (gs.rt == 1) G(1);
+		else if (gs.rt == 2) G(2);
+		else G(4);
+#undef G
 	}
-	// times one sweep (product + Jacobi update, every scene active) for each
-	// candidate schedule on this batch's matrices and keeps the fastest
-	template <typename E> int tune(const E *Fl, E *X, float inv, BatchTile &out, std::string &err)
+	// times one sweep (every scene active) for each candidate schedule on this
+	// batch's matrices and keeps the fastest
+	template <typename E> int tune(const E *Fl, Buf<E> (&X)[2], float inv, BatchTile &out, std::string &err)
 	{
 		const size_t V = vsize;
 		hipLaunchKernelGGL(k_fill<int>, dim3(grid_for((size_t)count)), dim3(kB), 0, st, active.p, (size_t)count, 1);
 		hipLaunchKernelGGL(k_fill<float>, dim3(grid_for(V)), dim3(kB), 0, st, r32.p, V, 0.f);
 		hipLaunchKernelGGL(k_fill<float>, dim3(grid_for(V)), dim3(kB), 0, st, rho32.p, V, 0.f);
-		hipLaunchKernelGGL(k_fill<E>, dim3(grid_for(xsize)), dim3(kB), 0, st, X, xsize, (E)0.f);
 		HIP_OK(hipGetLastError(), "tune");
-		const int q0 = etb[0], q1 = ete[count - 1];
-		const int ge = std::max(1, std::min(kPersist * 4, q1 - q0));
 		double best_ms = 1e300;
 		BatchTile pick = gs;
 		for (int rt : {1, 2, 4})
 			for (int kc : {1024, 2048, 4096, 8192})
 				for (int grid : {512, 1024, 2048, 4096}) {
 					if (set_sched(BatchTile{rt, kc, grid}, err)) return -1;
-					const int g0 = 0, g1 = ngtiles;
 					constexpr int kReps = 3;
 					for (int r = 0; r <= kReps; r++) {
 						if (r == 1) HIP_OK(hipEventRecord(e0, st), "tune");
-						launch_gemm<E>(Fl, X, g0, g1);
-						hipLaunchKernelGGL(k_bjacobi<E>, dim3(ge), dim3(kB), 0, st, etiles.p, q0, q1, d_meta.p,
-						                   active.p, part32.p, inv, r32.p, rho32.p, d32.p, X);
+						sweep<E>(Fl, X[0].p, X[1].p, 0, ngtiles, inv, false);
 					}
 					HIP_OK(hipEventRecord(e1, st), "tune");
 					HIP_OK(hipEventSynchronize(e1), "tune");
@@ -453,53 +352,113 @@ struct SceneBatch::Impl {
 		out = pick;
 		return set_sched(pick, err);
 	}
-
-	// the solve's kernel sequence for scenes [sc0, sc1) (one scene, or all:
-	// the sweep-product list is in its own scene order); returns the number
-	// of launches
-	template <typename E>
-	int enqueue(const E *Fl, E *X, int sc0, int sc1, int outer, int sweeps, double tol, float inv)
+	// the iterate's two buffers: padding zero, never written
+	template <typename E> int iterates(Buf<E> (&X)[2], std::string &err)
 	{
-		int launches = 0;
+		for (Buf<E> &x : X)
+			if (!x.p) {
+				if (x.alloc(xsize, err)) return -1;
+				hipLaunchKernelGGL(k_fill<E>, dim3(grid_for(xsize)), dim3(kB), 0, st, x.p, xsize, (E)0.f);
+			}
+		return 0;
+	}
+
+	// The solve's kernels for scenes [sc0, sc1) (one scene, or all: the sweep
+	// list is in its own scene order); both return the number of launches.
+	// start: x = 0, the first residual and its norms
+	int start(int sc0, int sc1, double tol)
+	{
+		const int q0 = etb[sc0], q1 = ete[sc1 - 1];
+		hipLaunchKernelGGL(k_binit, dim3(std::max(1, std::min(kPersist, q1 - q0))), dim3(kB), 0, st, etiles.p, q0, q1,
+		                   d_meta.p, E64.p, rho64.p, r64.p, rho32.p, blk.p);
+		hipLaunchKernelGGL(k_bnorm, dim3(sc1 - sc0), dim3(64), 0, st, sc0, d_etb.p, d_ete.p, blk.p, active.p, enorm.p,
+		                   scale.p, state(), tol, 1);
+		return 2;
+	}
+	// one refinement: the scaled residual, sweeps, the new residual and norms
+	template <typename E> int refine(const E *F, Buf<E> (&X)[2], int sc0, int sc1, int sweeps, double tol, float inv)
+	{
 		const int t0 = tb[sc0], t1 = te[sc1 - 1], q0 = etb[sc0], q1 = ete[sc1 - 1];
 		const bool all = sc0 == 0 && sc1 == count;
 		const int g0 = all ? 0 : gtb[sc0], g1 = all ? ngtiles : gte[sc0];  // else sc1 = sc0 + 1
-		const int gt = std::max(1, std::min(kPersist, t1 - t0)), ge = std::max(1, std::min(kPersist * 4, q1 - q0));
-		for (int o = 0; o <= outer; o++) {
-			if (o > 0) {
-				hipLaunchKernelGGL(k_bfx64v, dim3(gt), dim3(kB), 0, st, tiles.p, t0, t1, d_meta.p, active.p, F32.p, xT.p,
-				                   part64.p);
-				launches++;
-			}
-			hipLaunchKernelGGL(k_bresid, dim3(ge), dim3(kB), 0, st, etiles.p, q0, q1, d_meta.p, active.p,
-			                   o > 0 ? (const double *)part64.p : (const double *)nullptr, xT.p, E64.p, rho64.p, r64.p,
-			                   blk.p);
-			hipLaunchKernelGGL(k_bnorm, dim3(sc1 - sc0), dim3(64), 0, st, sc0, d_etb.p, d_ete.p, blk.p, active.p,
-			                   enorm.p, rel.p, scale.p, tol, o == 0 ? 1 : 0);
-			launches += 2;
-			if (o == outer) break;
-			hipLaunchKernelGGL(k_bscale<E>, dim3(ge), dim3(kB), 0, st, etiles.p, q0, q1, d_meta.p, active.p, r64.p,
-			                   scale.p, r32.p, X);
-			launches++;
-			for (int m = 0; m < sweeps; m++) {
-				launch_gemm<E>(Fl, X, g0, g1);
-				hipLaunchKernelGGL(k_bjacobi<E>, dim3(ge), dim3(kB), 0, st, etiles.p, q0, q1, d_meta.p, active.p,
-				                   part32.p, inv, r32.p, rho32.p, d32.p, X);
-				launches += 2;
-			}
-			hipLaunchKernelGGL(k_baxpy, dim3(ge), dim3(kB), 0, st, etiles.p, q0, q1, d_meta.p, active.p, scale.p, d32.p,
-			                   xT.p);
-			launches++;
-		}
-		return launches;
+		hipLaunchKernelGGL(k_bscale<E>, dim3(std::max(1, std::min(kPersist, q1 - q0))), dim3(kB), 0, st, etiles.p, q0, q1,
+		                   d_meta.p, active.p, r64.p, scale.p, r32.p, X[0].p);
+		for (int m = 0; m < sweeps; m++) sweep<E>(F, X[m & 1].p, X[(m + 1) & 1].p, g0, g1, inv, m == sweeps - 1);
+		const dim3 gt(t1 - t0);
+		if (ks == 1)
+			hipLaunchKernelGGL(k_bfx<1>, gt, dim3(kB), 0, st, tiles.p, t0, t1, d_meta.p, active.p, F32.p, xT.p, E64.p,
+			                   rho64.p, r64.p, blk.p);
+		else
+			hipLaunchKernelGGL(k_bfx<4>, gt, dim3(kB), 0, st, tiles.p, t0, t1, d_meta.p, active.p, F32.p, xT.p, E64.p,
+			                   rho64.p, r64.p, blk.p);
+		hipLaunchKernelGGL(k_bnorm, dim3(sc1 - sc0), dim3(64), 0, st, sc0, d_tb.p, d_te.p, blk.p, active.p, enorm.p,
+		                   scale.p, state(), tol, 0);
+		return 3 + sweeps;
 	}
-
-	template <typename E> int fills(E *X)
+	int clears()
 	{
 		hipLaunchKernelGGL(k_fill<double>, dim3(grid_for(xsize)), dim3(kB), 0, st, xT.p, xsize, 0.0);
-		hipLaunchKernelGGL(k_fill<E>, dim3(grid_for(xsize)), dim3(kB), 0, st, X, xsize, (E)0.f);
 		hipLaunchKernelGGL(k_fill<int>, dim3(grid_for((size_t)count)), dim3(kB), 0, st, active.p, (size_t)count, 1);
-		return 3;
+		return 2;
+	}
+	// what record launches, as graph k
+	template <typename L> int capture(int k, L record, std::string &err)
+	{
+		HIP_OK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal), "capture");
+		const int l = record();
+		hipGraph_t g = nullptr;
+		const hipError_t ce = hipStreamEndCapture(st, &g);
+		if (ce != hipSuccess || !g) {
+			err = std::string("graph capture: ") + hipGetErrorString(ce);
+			return -1;
+		}
+		graph[k] = g;
+		HIP_OK(hipGraphInstantiate(&exec[k], graph[k], nullptr, nullptr, 0), "graph instantiate");
+		g_nodes[k] = l;
+		return 0;
+	}
+	// the whole solve; launches and graph build time out
+	template <typename E>
+	int run(const E *F, Buf<E> (&X)[2], int prec, bool use_graph, int outer, int sweeps, double tol, float inv,
+	        int &launches, double &build_ms, std::string &err)
+	{
+		if (!use_graph) {  // scene after scene
+			HIP_OK(hipEventRecord(e0, st), "event");
+			launches += clears();
+			for (int s = 0; s < count; s++) {
+				launches += start(s, s + 1, tol);
+				for (int o = 0; o < outer; o++) launches += refine<E>(F, X, s, s + 1, sweeps, tol, inv);
+			}
+			HIP_OK(hipEventRecord(e1, st), "event");
+			return 0;
+		}
+		if (!(exec[0] && exec[1] && g_prec == prec && g_sweeps == sweeps && g_tol == tol)) {
+			drop_graph();
+			const auto c0 = std::chrono::steady_clock::now();
+			if (capture(0, [&] { return clears() + start(0, count, tol); }, err) ||
+			    capture(1, [&] { return refine<E>(F, X, 0, count, sweeps, tol, inv); }, err)) {
+				drop_graph();
+				return -1;
+			}
+			g_prec = prec;
+			g_sweeps = sweeps;
+			g_tol = tol;
+			build_ms = ms_since(c0);
+		}
+		HIP_OK(hipEventRecord(e0, st), "event");
+		HIP_OK(hipGraphLaunch(exec[0], st), "graph launch");
+		launches += g_nodes[0];
+		for (int o = 0; o < outer; o++) {
+			// a graph launch per refinement, until no scene is above tol
+			HIP_OK(hipStreamSynchronize(st), "batch solve");
+			bool any = false;
+			for (int s = 0; s < count && !any; s++) any = state()[s].active != 0;
+			if (!any) break;
+			HIP_OK(hipGraphLaunch(exec[1], st), "graph launch");
+			launches += g_nodes[1];
+		}
+		HIP_OK(hipEventRecord(e1, st), "event");
+		return 0;
 	}
 };
 
@@ -535,33 +494,28 @@ SceneBatch *SceneBatch::create(int count, const int *n, std::string &err)
 	B->d_ = new Impl();
 	Impl &d = *B->d_;
 	d.count = count;
-	std::vector<int4> tl;
-	std::vector<int2> el;
+	size_t rows = 0;
+	for (int s = 0; s < count; s++) rows += (n[s] + 255) / 256 * 256;
+	// residual rows per tile: 32, or 8 while that leaves CUs without a block (ms
+	// per solve at 32 and 8: 20 rooms of 500 to 2000 patches 0.508, 0.548; 48 of
+	// 500 to 4000 2.12, 2.26; 8 of 500 to 1000 0.306, 0.305)
+	d.ks = rows / 32 < 256 ? 4 : 1;
+	std::vector<int2> tl, el;
 	for (int s = 0; s < count; s++) {
 		BMeta m;
 		m.n = n[s];
 		m.ld = (n[s] + 255) / 256 * 256;
-		m.nk = (m.ld + kKChunk - 1) / kKChunk;
-		m.nkg = 0;
 		m.off = (long long)d.fsize;
 		m.voff = (long long)d.vsize;
 		m.xoff = (long long)d.xsize;
-		m.poff = (long long)d.psize;
-		m.goff = (long long)d.gsize;
 		d.fsize += (size_t)m.ld * m.ld;
 		d.vsize += (size_t)m.n * NR;
 		d.xsize += (size_t)16 * m.ld;
-		d.psize += (size_t)m.nk * m.ld * 16;
-		d.gsize += (size_t)((m.ld + kMinKc - 1) / kMinKc) * m.ld * 16;
 		d.n.push_back(m.n);
 		d.ld.push_back(m.ld);
 		d.meta.push_back(m);
 		d.tb.push_back((int)tl.size());
-		for (int rb = 0; rb < m.ld / 256; rb++)
-			for (int kc = 0; kc < m.nk; kc++) {
-				const int kb0 = kc * (kKChunk / 32), kb1 = std::min(m.ld / 32, kb0 + kKChunk / 32);
-				tl.push_back(make_int4(s, rb, kb0, kb1));
-			}
+		for (int b = 0; b < m.ld / 32 * d.ks; b++) tl.push_back(make_int2(s, b));
 		d.te.push_back((int)tl.size());
 		d.etb.push_back((int)el.size());
 		for (int e = 0; e < m.n * NR; e += kB) el.push_back(make_int2(s, e));
@@ -578,20 +532,23 @@ SceneBatch *SceneBatch::create(int count, const int *n, std::string &err)
 		return nullptr;
 	}
 	const size_t V = d.vsize;
-	if (d.F32.alloc(d.fsize, e) || d.r32.alloc(V, e) || d.d32.alloc(V, e) || d.rho32.alloc(V, e) ||
-	    d.part32.alloc(d.gsize, e) || d.E64.alloc(V, e) || d.rho64.alloc(V, e) || d.r64.alloc(V, e) || d.out.alloc(V, e) || d.stage.init(e) ||
-	    d.xT.alloc(d.xsize, e) || d.part64.alloc(d.psize, e) || d.blk.alloc((size_t)d.netiles * 2, e) ||
-	    d.enorm.alloc(count, e) || d.rel.alloc(count, e) || d.scale.alloc(count, e) || d.active.alloc(count, e) ||
-	    d.d_tb.alloc(count, e) || d.d_te.alloc(count, e) || d.d_etb.alloc(count, e) || d.d_ete.alloc(count, e) ||
-	    d.tiles.alloc(tl.size(), e) || d.etiles.alloc(el.size(), e) || d.d_meta.alloc(count, e)) {
+	if (d.F32.alloc(d.fsize, e) || d.r32.alloc(V, e) || d.rho32.alloc(V, e) || d.E64.alloc(V, e) ||
+	    d.rho64.alloc(V, e) || d.r64.alloc(V, e) || d.out.alloc(V, e) || d.stage.init(e) ||
+	    d.stage.stat_room((size_t)count * (sizeof(BState) / sizeof(double)), e) || d.xT.alloc(d.xsize, e) ||
+	    d.blk.alloc((size_t)std::max(d.netiles, d.ntiles) * 2, e) || d.enorm.alloc(count, e) || d.scale.alloc(count, e) ||
+	    d.active.alloc(count, e) || d.d_tb.alloc(count, e) || d.d_te.alloc(count, e) || d.d_etb.alloc(count, e) ||
+	    d.d_ete.alloc(count, e) || d.tiles.alloc(tl.size(), e) || d.etiles.alloc(el.size(), e) ||
+	    d.d_meta.alloc(count, e)) {
 		err = e;
 		delete B;
 		return nullptr;
 	}
 	if (hipMemsetAsync(d.F32.p, 0, d.fsize * 4, d.st) != hipSuccess ||
-	    hipMemcpyAsync(d.tiles.p, tl.data(), tl.size() * sizeof(int4), hipMemcpyHostToDevice, d.st) != hipSuccess ||
+	    hipMemcpyAsync(d.tiles.p, tl.data(), tl.size() * sizeof(int2), hipMemcpyHostToDevice, d.st) != hipSuccess ||
 	    hipMemcpyAsync(d.etiles.p, el.data(), el.size() * sizeof(int2), hipMemcpyHostToDevice, d.st) != hipSuccess ||
 	    hipMemcpyAsync(d.d_meta.p, d.meta.data(), count * sizeof(BMeta), hipMemcpyHostToDevice, d.st) != hipSuccess ||
+	    hipMemcpyAsync(d.d_tb.p, d.tb.data(), count * 4, hipMemcpyHostToDevice, d.st) != hipSuccess ||
+	    hipMemcpyAsync(d.d_te.p, d.te.data(), count * 4, hipMemcpyHostToDevice, d.st) != hipSuccess ||
 	    hipMemcpyAsync(d.d_etb.p, d.etb.data(), count * 4, hipMemcpyHostToDevice, d.st) != hipSuccess ||
 	    hipMemcpyAsync(d.d_ete.p, d.ete.data(), count * 4, hipMemcpyHostToDevice, d.st) != hipSuccess ||
 	    hipStreamSynchronize(d.st) != hipSuccess) {
@@ -599,7 +556,7 @@ SceneBatch *SceneBatch::create(int count, const int *n, std::string &err)
 		delete B;
 		return nullptr;
 	}
-	if (d.set_sched(BatchTile{4, kKChunk, kPersist}, err)) {
+	if (d.set_sched(d.rule(), err)) {
 		delete B;
 		return nullptr;
 	}
@@ -639,9 +596,9 @@ int SceneBatch::autotune(int prec, BatchTile &out, std::string &err)
 	if (d.ensure_lowp(prec, err)) return -1;
 	const int pi = prec == PREC_F16 ? 0 : 1;
 	if (prec == PREC_F16) {
-		if (d.X16.alloc(d.xsize, err) || d.tune<_Float16>(d.F16.p, d.X16.p, 1.0f / d.s16, d.best[pi], err)) return -1;
+		if (d.iterates(d.X16, err) || d.tune<_Float16>(d.F16.p, d.X16, 1.0f / d.s16, d.best[pi], err)) return -1;
 	} else {
-		if (d.XB.alloc(d.xsize, err) || d.tune<__bf16>(d.FB.p, d.XB.p, 1.0f, d.best[pi], err)) return -1;
+		if (d.iterates(d.XB, err) || d.tune<__bf16>(d.FB.p, d.XB, 1.0f, d.best[pi], err)) return -1;
 	}
 	d.forced = false;
 	out = d.best[pi];
@@ -668,80 +625,33 @@ int SceneBatch::solve(int prec, bool graph, const double *rho, const double *E, 
 		return -1;
 	}
 	if (d.ensure_lowp(prec, err)) return -1;
-	if (!d.forced) {
+	if (!d.forced) {  // the tuned schedule, or the rule's
 		const BatchTile &b = d.best[prec == PREC_F16 ? 0 : 1];
-		BatchTile got;
-		if (b.rt == 0 ? autotune(prec, got, err) : d.set_sched(b, err)) return -1;
+		if (d.set_sched(b.rt == 0 ? d.rule() : b, err)) return -1;
 	}
 	const size_t V = d.vsize;
 	HIP_OK(hipStreamSynchronize(d.st), "batch solve");  // nothing of an earlier call is in flight
 	d.stage.begin();
 	if (d.stage.up(d.rho64.p, rho, V * 8, d.st, err) || d.stage.up(d.E64.p, E, V * 8, d.st, err)) return -1;
-	hipLaunchKernelGGL(k_brho, dim3(grid_for(V)), dim3(kB), 0, d.st, d.rho64.p, V, d.rho32.p);
-	HIP_OK(hipStreamSynchronize(d.st), "upload");
 	const float inv = prec == PREC_F16 ? 1.0f / d.s16 : 1.0f;
 	double build_ms = 0.0;
 	int launches = 0;
-	auto run_all = [&](void) -> int {
-		int l = 0;
-		if (prec == PREC_F16) {
-			l += d.fills(d.X16.p);
-			l += d.enqueue<_Float16>(d.F16.p, d.X16.p, 0, d.count, outer, sweeps, tol, inv);
-		} else {
-			l += d.fills(d.XB.p);
-			l += d.enqueue<__bf16>(d.FB.p, d.XB.p, 0, d.count, outer, sweeps, tol, inv);
-		}
-		return l;
-	};
-	if (prec == PREC_F16 ? d.X16.alloc(d.xsize, err) : d.XB.alloc(d.xsize, err)) return -1;
-	if (graph) {
-		if (!(d.exec && d.g_prec == prec && d.g_outer == outer && d.g_sweeps == sweeps && d.g_tol == tol)) {
-			d.drop_graph();
-			const auto c0 = std::chrono::steady_clock::now();
-			HIP_OK(hipStreamBeginCapture(d.st, hipStreamCaptureModeThreadLocal), "capture");
-			const int l = run_all();
-			hipGraph_t g = nullptr;
-			const hipError_t ce = hipStreamEndCapture(d.st, &g);
-			if (ce != hipSuccess || !g) {
-				err = std::string("graph capture: ") + hipGetErrorString(ce);
-				return -1;
-			}
-			d.graph = g;
-			HIP_OK(hipGraphInstantiate(&d.exec, d.graph, nullptr, nullptr, 0), "graph instantiate");
-			d.g_prec = prec;
-			d.g_outer = outer;
-			d.g_sweeps = sweeps;
-			d.g_tol = tol;
-			d.g_nodes = l;
-			build_ms = ms_since(c0);
-		}
-		launches = d.g_nodes;
-		HIP_OK(hipEventRecord(d.e0, d.st), "event");
-		HIP_OK(hipGraphLaunch(d.exec, d.st), "graph launch");
-		HIP_OK(hipEventRecord(d.e1, d.st), "event");
-	} else {
-		HIP_OK(hipEventRecord(d.e0, d.st), "event");
-		launches += prec == PREC_F16 ? d.fills(d.X16.p) : d.fills(d.XB.p);
-		for (int s = 0; s < d.count; s++) {
-			if (prec == PREC_F16)
-				launches += d.enqueue<_Float16>(d.F16.p, d.X16.p, s, s + 1, outer, sweeps, tol, inv);
-			else
-				launches += d.enqueue<__bf16>(d.FB.p, d.XB.p, s, s + 1, outer, sweeps, tol, inv);
-		}
-		HIP_OK(hipEventRecord(d.e1, d.st), "event");
-	}
-	HIP_OK(hipGetLastError(), "batch launch");
+	if (prec == PREC_F16 ? d.iterates(d.X16, err) || d.run<_Float16>(d.F16.p, d.X16, prec, graph, outer, sweeps, tol, inv,
+	                                                                 launches, build_ms, err)
+	                     : d.iterates(d.XB, err) || d.run<__bf16>(d.FB.p, d.XB, prec, graph, outer, sweeps, tol, inv,
+	                                                              launches, build_ms, err))
+		return -1;
 	hipLaunchKernelGGL(k_brows, dim3(std::max(1, std::min(kPersist * 4, d.netiles))), dim3(kB), 0, d.st, d.etiles.p,
 	                   d.netiles, d.d_meta.p, d.xT.p, d.out.p);
 	HIP_OK(hipGetLastError(), "batch launch");
-	std::vector<int> act(d.count);
-	if (d.stage.down(Bout, d.out.p, V * 8, d.st, err) || d.stage.down(rel_res, d.rel.p, (size_t)d.count * 8, d.st, err) ||
-	    d.stage.down(act.data(), d.active.p, (size_t)d.count * 4, d.st, err))
-		return -1;
+	if (d.stage.down(Bout, d.out.p, V * 8, d.st, err)) return -1;
 	float ms = 0.f;
 	HIP_OK(hipEventElapsedTime(&ms, d.e0, d.e1), "event");
 	int above = 0;
-	for (int s = 0; s < d.count; s++) above += act[s];
+	for (int s = 0; s < d.count; s++) {
+		rel_res[s] = d.state()[s].rel;
+		above += d.state()[s].active;
+	}
 	if (info) {
 		info[0] = ms;
 		info[1] = build_ms;

@@ -1,6 +1,6 @@
 // Device building blocks shared by the explicit-matrix solvers (linear.hip)
 // and the batched solver (batch.hip): MFMA fragment layout, the
-// low-precision GEMM tile, the FP64 MFMA product tile, buffers.
+// sweep, the FP64 residual, the FP64 MFMA product tile, buffers.
 // Included inside an anonymous namespace of each translation unit.
 #pragma once
 
@@ -52,76 +52,255 @@ template <typename T> __global__ void k_fill(T *p, size_t count, T v)
 	for (size_t i = blockIdx.x * (size_t)kB + threadIdx.x; i < count; i += (size_t)gridDim.x * kB) p[i] = v;
 }
 
-template <typename E, int RT, int CT, int U> struct GemmRegs {
-	typedef typename VecOf<E>::type V;
-	V a[U][RT], b[U][CT];
+// What becomes of a low-precision product y = (A X)[i][c]: with y given, the
+// product itself, y[i][c] = inv y.  Else one Jacobi sweep, v = rhs + rho o (inv
+// y) and XTn <- v (fragment order); with rho_in (the adjoint's sweep v <- r +
+// F^T (rho o v)) v = rhs + inv y and XTn <- rho o v.  Padding of XTn (rows >=
+// nrhs, k >= n) is never written and stays zero.  With xT (the last sweep of a
+// refinement) the FP64 iterate takes the correction, xT[c][i] += s v (first:
+// xT[c][i] = s v), and wT (the adjoint's product input) becomes rho64 o xT.
+template <typename E> struct SweepOut {
+	int n, nrhs;
+	float inv;
+	bool rho_in, first;
+	const float *rhs, *rho;
+	E *XTn;
+	double *xT, s, *wT;
+	const double *rho64;
+	float *y;
+
+	__device__ __forceinline__ void put(int i, int c, int ld, float sum) const
+	{
+		const size_t t = (size_t)i * nrhs + c;
+		if (y) {
+			y[t] = sum * inv;
+			return;
+		}
+		const float v = rho_in ? rhs[t] + sum * inv : rhs[t] + rho[t] * (sum * inv);
+		XTn[frag_index(c, i, ld)] = (E)(rho_in ? rho[t] * v : v);
+		if (xT) {
+			const size_t q = (size_t)c * ld + i;
+			const double x = (first ? 0.0 : xT[q]) + s * (double)v;
+			xT[q] = x;
+			if (wT) wT[q] = rho64[t] * x;
+		}
+	}
 };
 
-template <typename E, int RT, int CT, int U>
-__device__ __forceinline__ void gemm_load(GemmRegs<E, RT, CT, U> &g, const typename VecOf<E>::type *Ap,
-                                          const typename VecOf<E>::type *Bp, int rb0, int nkb, int kb)
-{
-#pragma unroll
-	for (int u = 0; u < U; u++) {
-#pragma unroll
-		for (int r = 0; r < RT; r++) g.a[u][r] = __builtin_nontemporal_load(Ap + ((size_t)(rb0 + r) * nkb + kb + u) * 64);
-#pragma unroll
-		for (int c = 0; c < CT; c++) g.b[u][c] = Bp[((size_t)c * nkb + kb + u) * 64];
-	}
-}
-
-template <typename E, int RT, int CT, int U>
-__device__ __forceinline__ void gemm_mma(const GemmRegs<E, RT, CT, U> &g, f4 (&acc)[RT][CT])
-{
-#pragma unroll
-	for (int u = 0; u < U; u++)
-#pragma unroll
-		for (int r = 0; r < RT; r++)
-#pragma unroll
-			for (int c = 0; c < CT; c++) acc[r][c] = mfma(g.a[u][r], g.b[u][c], acc[r][c]);
-}
-
-template <int CT> struct GemmUnroll { static constexpr int U = CT <= 4 ? 4 : 2; };
-
-// One wave's share of part[s] = A X over k-blocks [kb0, kb1) (32 k each):
-// rows 16*rb0 .. 16*(rb0+RT)-1, all 16*CT columns.  A and XT are fragment
-// ordered with ld columns; the loop is software pipelined (two register sets
-// of U k-blocks, one loading while the other feeds the MFMAs), so kb1 - kb0
-// must be a multiple of 2U.
+// One block's rows of a sweep (block blk of the matrix; red: kSweepWaves RT CT
+// 64 entries of LDS).  A block is eight waves: 8 / S row groups of 16 RT rows,
+// the K range of each split over S waves.  Each wave streams its A
+// fragments (two register sets of two k-blocks, one loading while the other
+// feeds the MFMAs; the index is clamped past the chunk's end, those k-blocks
+// are not multiplied), the partial tiles meet in LDS and are summed in chunk
+// order, and the block's threads finish their rows (SweepOut).  The next
+// iterate goes to a second buffer, as other blocks still read this one.
+// A is read without the non-temporal policy where it stays in the 256 MB
+// last-level cache from sweep to sweep (cached).
+// Bound by that cache or HBM: the split inside the block keeps every CU busy
+// where a block per row group and a second kernel for the sweep's update left
+// CUs idle and paid a launch (one column tile, us per sweep, before -> now:
+// n = 1024 8.0 -> 3.2, 4096 12.5 -> 5.3, 6144 20 -> 12.5, 9216 39 -> 25.0,
+// 20224 187 -> 137 (6.0 TB/s), 32768 313 -> 302 (7.1 TB/s)).
+constexpr int kSweepWaves = 8;
 template <typename E, int RT, int CT>
-__device__ __forceinline__ void gemm_tile(const E *__restrict__ A, const E *__restrict__ XT, float *__restrict__ part,
-                                          int ld, int rp, int rb0, int kb0, int kb1)
+__device__ __forceinline__ void sweep_rows(const E *__restrict__ A, const E *__restrict__ XT, int ld, int S, bool cached,
+                                           int blk, f4 *red, const SweepOut<E> &o)
 {
 	typedef typename VecOf<E>::type V;
-	constexpr int U = GemmUnroll<CT>::U;
-	const int lane = threadIdx.x & 63;
-	const int nkb = ld >> 5;
-	const V *Ap = (const V *)A + lane;
-	const V *Bp = (const V *)XT + lane;
+	constexpr int U = 2;
+	const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const int WR = kSweepWaves / S, wr = w % WR, s = w / WR;
+	const int nkb = ld >> 5, cnt = nkb / S, nrt = ld >> 4;  // ld is a multiple of 256: nkb of 8
+	const int rt0 = (blk * WR + wr) * RT;
+	const V *Ap[RT];
+#pragma unroll
+	for (int r = 0; r < RT; r++) Ap[r] = (const V *)A + ((size_t)min(rt0 + r, nrt - 1) * nkb + s * cnt) * 64 + lane;
+	const V *Bp = (const V *)XT + (size_t)(s * cnt) * 64 + lane;
 	f4 acc[RT][CT];
 #pragma unroll
 	for (int r = 0; r < RT; r++)
 #pragma unroll
 		for (int c = 0; c < CT; c++) acc[r][c] = f4{0.f, 0.f, 0.f, 0.f};
-	GemmRegs<E, RT, CT, U> g0, g1;
-	gemm_load(g0, Ap, Bp, rb0, nkb, kb0);
-	for (int kb = kb0; kb < kb1; kb += 2 * U) {
-		gemm_load(g1, Ap, Bp, rb0, nkb, kb + U);
-		gemm_mma(g0, acc);
-		if (kb + 2 * U < kb1) gemm_load(g0, Ap, Bp, rb0, nkb, kb + 2 * U);
-		gemm_mma(g1, acc);
-	}
-	const int lr = lane & 15;
+	V a[2][U][RT], b[2][U][CT];
+	auto run = [&](auto nt) {
+		auto load = [&](int p, int k0) {
+#pragma unroll
+			for (int u = 0; u < U; u++) {
+				const size_t k = (size_t)min(k0 + u, cnt - 1);
+#pragma unroll
+				for (int r = 0; r < RT; r++) {
+					if constexpr (decltype(nt)::value) a[p][u][r] = __builtin_nontemporal_load(Ap[r] + k * 64);
+					else a[p][u][r] = Ap[r][k * 64];
+				}
+#pragma unroll
+				for (int c = 0; c < CT; c++) b[p][u][c] = Bp[((size_t)c * nkb + k) * 64];
+			}
+		};
+		auto mma = [&](int p, int k0) {
+#pragma unroll
+			for (int u = 0; u < U; u++)
+				if (k0 + u < cnt) {
+#pragma unroll
+					for (int r = 0; r < RT; r++)
+#pragma unroll
+						for (int c = 0; c < CT; c++) acc[r][c] = mfma(a[p][u][r], b[p][u][c], acc[r][c]);
+				}
+		};
+		load(0, 0);
+		for (int k = 0; k < cnt; k += 2 * U) {
+			load(1, k + U);
+			mma(0, k);
+			load(0, k + 2 * U);
+			mma(1, k + U);
+		}
+	};
+	if (cached) run(std::integral_constant<bool, false>{});
+	else run(std::integral_constant<bool, true>{});
 #pragma unroll
 	for (int r = 0; r < RT; r++)
 #pragma unroll
-		for (int c = 0; c < CT; c++)
-#pragma unroll
-			for (int j = 0; j < 4; j++) {
-				const int row = (rb0 + r) * 16 + (lane >> 4) * 4 + j;
-				part[(size_t)row * rp + c * 16 + lr] = acc[r][c][j];
-			}
+		for (int c = 0; c < CT; c++) red[(((s * WR + wr) * RT + r) * CT + c) * 64 + lane] = acc[r][c];
+	__syncthreads();
+	// element (row, column) of a 16 x 16 tile: lane 16 (row / 4) + column, value row % 4
+	const float *rf = (const float *)red;
+	const int rows = WR * RT * 16, row0 = blk * rows, part = WR * RT * CT * 256;
+	for (int e = threadIdx.x; e < rows * o.nrhs; e += kSweepWaves * 64) {
+		const int rl = e / o.nrhs, c = e - rl * o.nrhs;
+		if (row0 + rl >= o.n) break;
+		const float *q = rf + ((rl >> 4) * CT + (c >> 4)) * 256 + (((rl & 15) >> 2) * 16 + (c & 15)) * 4 + (rl & 3);
+		float y = 0.f;
+		for (int k = 0; k < S; k++) y += q[k * part];
+		o.put(row0 + rl, c, ld, y);
+	}
 }
+
+// One block's rows (block blk of the matrix) of the whole FP64 residual for NC
+// <= 4 right-hand sides on the vector FP64 units, where a 16-column MFMA would spend 13 of its 16 columns on padding:
+// out[i][c] = base[i][c] + rho[i][c] * (F w)[i][c] - xT[c][i] (base, rho and xT
+// may be null: 0, 1 and 0) and, into st, the sum of squares and max |out|.
+// A wave owns kFxRows rows; per step each lane takes 4 consecutive k of each
+// row (one 16-byte load per row, the next step's loads in flight) against w
+// staged through LDS in chunks of 1024 k, column-major, so that a lane's 4
+// values are two 16-byte reads.  KS of the block's four waves share rows, each
+// taking every KS-th step of 256 k: a block is 32 / KS rows.  The 64 lane
+// partials of the 8 NC sums are combined by a reduce-scatter (the exchanges
+// over lane bits 5, 4, 3 halve the set each time and leave lane l with row
+// l >> 3), then the KS waves' in a fixed order.
+// Bound by HBM: 6.0-6.6 TB/s from n = 8192 up, FP64 work about half of that.
+// Against the form with one block size (32 rows), 32-way LDS conflicts, 4
+// columns for any NC and a second kernel for the residual (3 columns, us,
+// first kernel alone): n = 1024 10.8 -> 4.7, 4096 30.5 -> 16.6, 9216 88.7 ->
+// 61.9, 20224 290 -> 247, 32768 696 -> 643.
+constexpr int kFxRows = 8;
+constexpr int kFxChunk = 1024;
+template <int NC, int KS> struct FxShared {
+	double xs[NC * kFxChunk];
+	double red[KS][4 / KS * kFxRows * NC];
+	double stat[8];
+};
+template <int NC, int KS>
+__device__ __forceinline__ void fx64_rows(const float *__restrict__ F, const double *__restrict__ wT, int ld, int n,
+                                          int blk, FxShared<NC, KS> &sh, const double *xT, const double *base,
+                                          const double *rho, double *out, double *st)
+{
+	typedef float fv4 __attribute__((ext_vector_type(4)));
+	typedef double dv2 __attribute__((ext_vector_type(2)));
+	constexpr int ROWS = 4 / KS * kFxRows, STEPS = kFxChunk / 256;
+	static_assert(kFxRows == 8 && ROWS * NC <= kB, "the reduce-scatter assumes 8 rows; one thread per result");
+	double *xs = sh.xs, *stat = sh.stat;
+	auto &red = sh.red;
+	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+	const int rg = w / KS, ks = w % KS;
+	const float *Fr = F + (size_t)(blk * ROWS + rg * kFxRows) * ld + 4 * lane;
+	const int ns = ld / 256;
+	double v[kFxRows * NC];
+#pragma unroll
+	for (int i = 0; i < kFxRows * NC; i++) v[i] = 0.0;
+	fv4 a[kFxRows], an[kFxRows];
+#pragma unroll
+	for (int r = 0; r < kFxRows; r++)
+		a[r] = __builtin_nontemporal_load((const fv4 *)(Fr + (size_t)r * ld + min(ks, ns - 1) * 256));
+	for (int s0 = 0; s0 < ns; s0 += STEPS) {
+		const int cnt = min(STEPS, ns - s0);
+		__syncthreads();  // the previous chunk's reads are done
+		for (int i = threadIdx.x; i < cnt * 128; i += kB)
+#pragma unroll
+			for (int c = 0; c < NC; c++)
+				*(dv2 *)(xs + c * kFxChunk + 2 * i) = *(const dv2 *)(wT + (size_t)c * ld + s0 * 256 + 2 * i);
+		__syncthreads();
+#pragma unroll 1
+		for (int q = ks; q < cnt; q += KS) {
+			const int sn = min(s0 + q + KS, ns - 1);  // clamped: the last load of a wave is not used
+#pragma unroll
+			for (int r = 0; r < kFxRows; r++)
+				an[r] = __builtin_nontemporal_load((const fv4 *)(Fr + (size_t)r * ld + sn * 256));
+			double x[NC][4];
+#pragma unroll
+			for (int c = 0; c < NC; c++)
+#pragma unroll
+				for (int j = 0; j < 4; j++) x[c][j] = xs[c * kFxChunk + q * 256 + 4 * lane + j];
+#pragma unroll
+			for (int j = 0; j < 4; j++)
+#pragma unroll
+				for (int r = 0; r < kFxRows; r++) {
+					const double f = (double)a[r][j];
+#pragma unroll
+					for (int c = 0; c < NC; c++) v[r * NC + c] = __builtin_fma(f, x[c][j], v[r * NC + c]);
+				}
+#pragma unroll
+			for (int r = 0; r < kFxRows; r++) a[r] = an[r];
+		}
+	}
+#pragma unroll
+	for (int half = kFxRows * NC / 2, bit = 32; bit >= 8; half >>= 1, bit >>= 1) {
+		const bool upper = (lane & bit) != 0;
+#pragma unroll
+		for (int i = 0; i < half; i++) {
+			const double lo = v[i], hi = v[half + i];
+			v[i] = (upper ? hi : lo) + __shfl_xor(upper ? lo : hi, bit);
+		}
+	}
+#pragma unroll
+	for (int bit = 4; bit > 0; bit >>= 1)
+#pragma unroll
+		for (int c = 0; c < NC; c++) v[c] += __shfl_xor(v[c], bit);
+	if ((lane & 7) == 0)
+#pragma unroll
+		for (int c = 0; c < NC; c++) red[ks][(rg * kFxRows + (lane >> 3)) * NC + c] = v[c];
+	__syncthreads();
+	double ss = 0.0, mx = 0.0;
+	const int e = threadIdx.x, i = blk * ROWS + e / NC, c = e % NC;
+	if (e < ROWS * NC && i < n) {
+		double y = red[0][e];
+#pragma unroll
+		for (int k = 1; k < KS; k++) y += red[k][e];
+		const size_t t = (size_t)i * NC + c;
+		const double o = (base ? base[t] : 0.0) + (rho ? rho[t] : 1.0) * y - (xT ? xT[(size_t)c * ld + i] : 0.0);
+		out[t] = o;
+		ss = o * o;
+		mx = fabs(o);
+	}
+	for (int off = 32; off > 0; off >>= 1) {
+		ss += __shfl_xor(ss, off);
+		mx = fmax(mx, __shfl_xor(mx, off));
+	}
+	if (lane == 0) {
+		stat[2 * w] = ss;
+		stat[2 * w + 1] = mx;
+	}
+	__syncthreads();
+	if (threadIdx.x == 0) {
+		st[0] = stat[0] + stat[2] + stat[4] + stat[6];
+		st[1] = fmax(fmax(stat[1], stat[3]), fmax(stat[5], stat[7]));
+	}
+}
+
+// the matrix's 16-bit copy stays in the 256 MB last-level cache between
+// sweeps: up to 11.5k rows (us per sweep, cached against non-temporal: n = 4096
+// 5.3, 8.0; 9216 25.0, 37.1; 12288 48.9, 50.6; 16384 95.6, 82.9; 20224 144.5,
+// 136.5)
+bool stays_cached(size_t elements) { return 2 * elements <= (size_t)256 << 20; }
 
 // One wave's share of the FP64 product with an FP32 matrix on the FP64 MFMA
 // (v_mfma_f64_16x16x4_f64: lane l supplies A[l%16][l/16] and B[l/16][l%16],

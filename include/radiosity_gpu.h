@@ -256,9 +256,9 @@ rad_status rad_lin_adjoint(rad_lin *lin, int nrhs, const double *rho, const doub
  * count independent systems B_s = E_s + diag(rho_s) F_s B_s with three
  * columns (RGB) each, solved by the mixed-precision gather above with every
  * step of every scene in one kernel (tile lists spanning the scenes, grids
- * sized to the machine, converged scenes dropping out), the whole schedule
- * captured once into a HIP graph and replayed with one launch.  No reference
- * counterpart (the reference solves one scene per process). */
+ * sized to the machine, converged scenes dropping out), a refinement of all
+ * scenes captured once into a HIP graph and replayed until no scene is above
+ * tol.  No reference counterpart (the reference solves one scene per process). */
 typedef struct rad_batch rad_batch;
 
 rad_status rad_batch_create(rad_batch **out, int count, const int *n);
@@ -271,14 +271,15 @@ rad_status rad_batch_set_matrix(rad_batch *batch, int scene, const float *F);
 /* Picks the schedule of the batched sweep product -- rows per wave rt*16
  * (rt in {1, 2, 4}), k per tile kc (1024..8192) and the persistent grid
  * (512..4096 blocks) -- by timing one sweep of every candidate on this
- * batch; solve does it on first use for each precision. */
+ * batch; without it solve goes by the batch's size. */
 rad_status rad_batch_autotune(rad_batch *batch, int prec, int *rt, int *kc, int *grid);
 /* Forces that schedule instead (rt in {1, 2, 4}, kc in {1024, 2048, 4096,
  * 8192}, grid 64..16384); a later rad_batch_autotune hands the choice back. */
 rad_status rad_batch_set_tile(rad_batch *batch, int rt, int kc, int grid);
 /* rho, E, B: (sum of n) x 3 row-major, scenes concatenated in order.
  * `outer` refinements of `sweeps` sweeps each, a scene stopping once its
- * FP64 relative residual is <= tol.  use_graph = 1: one graph launch;
+ * FP64 relative residual is <= tol.  use_graph = 1: a graph launch per
+ * refinement, none once every scene is there;
  * 0: the same kernels scene after scene (bit-identical results).
  * rel_res[count] = final relative residuals; info4 = {device ms, graph
  * build ms (0 when reused), kernel launches, scenes still above tol}. */

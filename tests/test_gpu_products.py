@@ -69,3 +69,33 @@ def test_shooting_bits(n, nrhs):
     want, _, src = lo.shoot32(F, rho, E, np.ones(n), shots)
     assert info["outer"] == len(src)
     assert np.array_equal(B.astype(np.float32), want)
+
+
+# batches on each side of the residual's and the sweep's size rules (8192 and
+# 16384 padded rows), one scene above all; tolerances met and missed
+@pytest.mark.parametrize("sizes", [[1], [256, 257, 1, 40], [700] * 11, [1500] * 12, [8200, 64]])
+@pytest.mark.parametrize("prec", ["f16", "bf16"])
+def test_batch_size_rules(sizes, prec):
+    rng = np.random.default_rng(len(sizes))
+    tol = 1e-10
+    with radgpu.SceneBatch(sizes) as b:
+        Fs = [rng.random((n, n), np.float32) * np.float32(1.8 / n) for n in sizes]
+        for s, F in enumerate(Fs):
+            b.set_matrix(s, F)
+        total = sum(sizes)
+        rho = rng.uniform(0.2, 0.7, (total, 3))
+        E = rng.uniform(0.0, 1.0, (total, 3))
+        E[-64:] = 0.0  # the last scene starts converged where that is all of it
+        B, rel, info = b.solve(rho, E, prec=prec, graph=True, tol=tol, outer=20, sweeps=5)
+        Bs, rels, _ = b.solve(rho, E, prec=prec, graph=False, tol=tol, outer=20, sweeps=5)
+        assert np.array_equal(B, Bs) and np.array_equal(rel, rels)
+        assert info["above_tol"] == 0 and np.all(rel <= tol)
+        o = 0
+        for n, F in zip(sizes, Fs):
+            r = E[o:o + n] + rho[o:o + n] * (F.astype(np.float64) @ B[o:o + n]) - B[o:o + n]
+            assert np.linalg.norm(r) <= tol * np.linalg.norm(E[o:o + n]) + 1e-12 * np.linalg.norm(B[o:o + n])
+            o += n
+        # two refinements do not reach it
+        _, rel2, info2 = b.solve(rho, E, prec=prec, graph=True, tol=1e-14, outer=2, sweeps=2)
+        lit = [i for i, n in enumerate(sizes) if E[sum(sizes[:i]):sum(sizes[:i + 1])].any()]
+        assert info2["above_tol"] == len(lit) and np.all(rel2[lit] > 1e-14)
