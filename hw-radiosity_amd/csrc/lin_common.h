@@ -1,6 +1,6 @@
 // Device building blocks shared by the explicit-matrix solvers (linear.hip)
 // and the batched solver (batch.hip): MFMA fragment layout, the
-// sweep, the FP64 residual, the FP64 MFMA product tile, buffers.
+// sweep, the FP64 residual of few columns, buffers.
 // Included inside an anonymous namespace of each translation unit.
 #pragma once
 
@@ -301,67 +301,6 @@ __device__ __forceinline__ void fx64_rows(const float *__restrict__ F, const dou
 // 5.3, 8.0; 9216 25.0, 37.1; 12288 48.9, 50.6; 16384 95.6, 82.9; 20224 144.5,
 // 136.5)
 bool stays_cached(size_t elements) { return 2 * elements <= (size_t)256 << 20; }
-
-// One wave's share of the FP64 product with an FP32 matrix on the FP64 MFMA
-// (v_mfma_f64_16x16x4_f64: lane l supplies A[l%16][l/16] and B[l/16][l%16],
-// receives D[l/16 + 4*j][l%16], j = 0..3 -- rows interleaved, unlike the
-// 16-bit MFMAs): rows 16*rb0 .. 16*(rb0+RT)-1, columns
-// 16*cb0 .. 16*(cb0+CT)-1, k in [k0, k1) (a multiple of 32).  Per 32 k each
-// lane loads 8 consecutive F entries (converted exactly to FP64) and 8
-// consecutive X entries, then runs 8 MFMAs, step s pairing k = kk + 8*(l/16)
-// + s in both operands, so every k is summed once.  part is row-major, rp
-// columns.
-template <int RT, int CT>
-__device__ __forceinline__ void fx64_tile(const float *__restrict__ F, const double *__restrict__ xT,
-                                          double *__restrict__ part, int ld, int rp, int rb0, int cb0, int k0, int k1)
-{
-	typedef double d4 __attribute__((ext_vector_type(4)));
-	typedef float fv4 __attribute__((ext_vector_type(4)));
-	const int lane = threadIdx.x & 63;
-	const int lr = lane & 15, g8 = (lane >> 4) * 8;
-	d4 acc[RT][CT];
-#pragma unroll
-	for (int r = 0; r < RT; r++)
-#pragma unroll
-		for (int c = 0; c < CT; c++) acc[r][c] = d4{0.0, 0.0, 0.0, 0.0};
-	for (int kk = k0; kk < k1; kk += 32) {
-		float a[RT][8];
-		double b[CT][8];
-#pragma unroll
-		for (int r = 0; r < RT; r++) {
-			const fv4 *pa = (const fv4 *)(F + (size_t)((rb0 + r) * 16 + lr) * ld + kk + g8);
-			const fv4 u = __builtin_nontemporal_load(pa), v = __builtin_nontemporal_load(pa + 1);
-			a[r][0] = u[0]; a[r][1] = u[1]; a[r][2] = u[2]; a[r][3] = u[3];
-			a[r][4] = v[0]; a[r][5] = v[1]; a[r][6] = v[2]; a[r][7] = v[3];
-		}
-#pragma unroll
-		for (int c = 0; c < CT; c++) {
-			const double2 *pb = (const double2 *)(xT + (size_t)((cb0 + c) * 16 + lr) * ld + kk + g8);
-#pragma unroll
-			for (int q = 0; q < 4; q++) {
-				const double2 t = pb[q];
-				b[c][2 * q] = t.x;
-				b[c][2 * q + 1] = t.y;
-			}
-		}
-#pragma unroll
-		for (int st = 0; st < 8; st++)
-#pragma unroll
-			for (int r = 0; r < RT; r++)
-#pragma unroll
-				for (int c = 0; c < CT; c++)
-					acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)a[r][st], b[c][st], acc[r][c], 0, 0, 0);
-	}
-#pragma unroll
-	for (int r = 0; r < RT; r++)
-#pragma unroll
-		for (int c = 0; c < CT; c++)
-#pragma unroll
-			for (int j = 0; j < 4; j++) {
-				const int row = (rb0 + r) * 16 + (lane >> 4) + 4 * j;
-				part[(size_t)row * rp + (cb0 + c) * 16 + lr] = acc[r][c][j];
-			}
-}
 
 #define HIP_OK(expr, what)                                          \
 	do {                                                            \

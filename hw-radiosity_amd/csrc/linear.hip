@@ -252,15 +252,103 @@ template <typename E> __global__ void k_finish(const float *part, int S, int ld,
 }
 
 // Split-K partials part[s][row][col] (FP64) of F X, summed in a fixed order
-// by k_resid.
-template <int RT, int CT>
-__global__ __launch_bounds__(kB) void k_fx64m(const float *__restrict__ F, const double *__restrict__ xT,
-                                              double *__restrict__ part, int ld, int rp, int kchunk)
+// by k_resid, on the FP64 MFMA (v_mfma_f64_16x16x4_f64: lane l supplies
+// A[l%16][l/16] and B[l/16][l%16], receives D[l/16 + 4*j][l%16], j = 0..3 --
+// rows interleaved, unlike the 16-bit MFMAs).  A block is W waves of 16 RT rows
+// each over the same 16 CT columns, whose 32 k per step they stage in LDS (two
+// buffers, columns 34 doubles apart: a lane's 16-byte reads of 16 columns fall
+// on all 64 banks); a lane loads 8 consecutive F entries of its row per step
+// (converted exactly to FP64), the next step's on their way, and step s pairs
+// k = kk + 8*(l/16) + s in both operands, so every k is summed once.
+// Bound by the FP64 matrix units (73 TFLOP/s in a large library product); with
+// each wave reading its own X from L2 it was that traffic (12 TB/s).  us at n =
+// 7936, 16, 32, 64, 192 columns: 67, 103, 172, 486 -> 45, 75, 131, 382 (63
+// TFLOP/s); n = 1024, 16 and 64: 9.2, 13.2 -> 4.6, 9.2; n = 16384, 192: 1850 ->
+// 1513 (68 TFLOP/s).
+template <int RT, int CT, int W>
+__global__ __launch_bounds__(W * 64) void k_fx64m(const float *__restrict__ F, const double *__restrict__ xT,
+                                                  double *__restrict__ part, int ld, int rp, int kchunk)
 {
-	const int w = threadIdx.x >> 6;
-	const int s = blockIdx.z;
-	fx64_tile<RT, CT>(F, xT, part + (size_t)s * ld * rp, ld, rp, (blockIdx.x * 4 + w) * RT, blockIdx.y * CT,
-	                  s * kchunk, (s + 1) * kchunk);
+	typedef double d4 __attribute__((ext_vector_type(4)));
+	typedef double dv2 __attribute__((ext_vector_type(2)));
+	typedef float fv4 __attribute__((ext_vector_type(4)));
+	constexpr int PAD = 34, NL = CT * 16 * 16 / (W * 64);  // 16-byte loads of X per thread and step
+	static_assert(NL * W * 64 == CT * 16 * 16, "whole loads");
+	__shared__ double bs[2][CT * 16 * PAD];
+	const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, lr = lane & 15, g8 = (lane >> 4) * 8;
+	const int rb0 = (blockIdx.x * W + w) * RT, cb0 = blockIdx.y * CT;
+	const int k0 = blockIdx.z * kchunk, k1 = k0 + kchunk;
+	const float *Fr[RT];
+#pragma unroll
+	for (int r = 0; r < RT; r++) Fr[r] = F + (size_t)((rb0 + r) * 16 + lr) * ld + g8;
+	d4 acc[RT][CT];
+#pragma unroll
+	for (int r = 0; r < RT; r++)
+#pragma unroll
+		for (int c = 0; c < CT; c++) acc[r][c] = d4{0.0, 0.0, 0.0, 0.0};
+	fv4 a[RT][2], an[RT][2];
+	dv2 sb[NL];
+	auto load_x = [&](int kk) {
+#pragma unroll
+		for (int i = 0; i < NL; i++) {
+			const int e = threadIdx.x + i * W * 64;  // 16 loads per column
+			sb[i] = *(const dv2 *)(xT + (size_t)(cb0 * 16 + e / 16) * ld + kk + 2 * (e % 16));
+		}
+	};
+	auto store_x = [&](int p) {
+#pragma unroll
+		for (int i = 0; i < NL; i++) {
+			const int e = threadIdx.x + i * W * 64;
+			*(dv2 *)(&bs[p][(e / 16) * PAD + 2 * (e % 16)]) = sb[i];
+		}
+	};
+	auto load_f = [&](fv4 (&x)[RT][2], int kk) {
+#pragma unroll
+		for (int r = 0; r < RT; r++) {
+			x[r][0] = ((const fv4 *)(Fr[r] + kk))[0];
+			x[r][1] = ((const fv4 *)(Fr[r] + kk))[1];
+		}
+	};
+	load_x(k0);
+	load_f(a, k0);
+	store_x(0);
+	__syncthreads();
+	int p = 0;
+	for (int kk = k0; kk < k1; kk += 32) {
+		const int kn = kk + 32 < k1 ? kk + 32 : kk;  // the last step's loads are not used
+		load_x(kn);
+		load_f(an, kn);
+#pragma unroll
+		for (int h = 0; h < 4; h++) {
+			dv2 b[CT];
+#pragma unroll
+			for (int c = 0; c < CT; c++) b[c] = *(const dv2 *)(&bs[p][(c * 16 + lr) * PAD + g8 + 2 * h]);
+#pragma unroll
+			for (int u = 0; u < 2; u++)
+#pragma unroll
+				for (int r = 0; r < RT; r++) {
+					const double f = (double)a[r][h >> 1][(h & 1) * 2 + u];
+#pragma unroll
+					for (int c = 0; c < CT; c++) acc[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(f, b[c][u], acc[r][c], 0, 0, 0);
+				}
+		}
+		store_x(p ^ 1);  // its readers are past the previous step's barrier
+		__syncthreads();
+		p ^= 1;
+#pragma unroll
+		for (int r = 0; r < RT; r++) {
+			a[r][0] = an[r][0];
+			a[r][1] = an[r][1];
+		}
+	}
+	double *P = part + (size_t)blockIdx.z * ld * rp;
+#pragma unroll
+	for (int r = 0; r < RT; r++)
+#pragma unroll
+		for (int c = 0; c < CT; c++)
+#pragma unroll
+			for (int j = 0; j < 4; j++)
+				P[(size_t)((rb0 + r) * 16 + (lane >> 4) + 4 * j) * rp + (cb0 + c) * 16 + lr] = acc[r][c][j];
 }
 
 template <int NC, int KS>
@@ -834,7 +922,7 @@ double power_sum(const std::vector<float> &a, const double *v, int n, int nrhs)
 // FP64 residual machinery: the caller's wT holds rp x ld doubles with rows
 // >= nrhs and columns >= n zero; split-K partials; per-block stats.
 struct Fx64 {
-	int n = 0, ld = 0, nrhs = 0, rp = 0, rt = 4, ct = 1, S = 1, ks = 1;
+	int n = 0, ld = 0, nrhs = 0, rp = 0, rt = 1, ct = 1, W = 4, S = 1, ks = 1;
 	Buf<double> part;
 	size_t nblk = 0;
 	double *blk = nullptr;  // the blocks' statistics, in host memory (Stage)
@@ -846,10 +934,10 @@ struct Fx64 {
 		nrhs = nrhs_;
 		const int nct = (nrhs + 15) / 16;
 		ct = nct >= 4 ? 4 : (nct >= 2 ? 2 : 1);
-		rt = ct == 4 ? 2 : 4;
 		rp = (nct + ct - 1) / ct * ct * 16;  // whole column groups: every tile the grid covers exists
-		const int tiles = (ld / (64 * rt)) * (rp / (16 * ct));
-		S = 1;
+		rt = 1;
+		W = 4;
+		S = 8;
 		if (vec()) {
 			// waves per row group (32 / ks rows a block): four below 8192 rows,
 			// where fewer leave CUs without a block (n = 6144: 33.6, 31.8 and
@@ -868,13 +956,42 @@ struct Fx64 {
 			}
 			nblk = (size_t)ld / 32 * ks;
 		} else {
-			while (S < 8 && tiles * S < 512 && (ld / (2 * S)) % 32 == 0) S *= 2;
+			tile();
 			nblk = ((size_t)n * nrhs + kB - 1) / kB;
 			if (part.alloc((size_t)S * ld * rp, err)) return -1;
 		}
 		if (stage.stat_room(std::max<size_t>(nblk * 2, 3 * kStatBlocks), err)) return -1;
 		blk = stage.stats;
 		return 0;
+	}
+	// Row tiles per wave, waves per block and split-K of k_fx64m (ld is a
+	// multiple of 256: every choice divides it).  Four column tiles: blocks of
+	// 256 rows with the least split whose last round of 256 CUs is 85 % full, else
+	// of 128 rows, else (small matrices) 64 rows split eight ways; fewer column
+	// tiles: 128 rows from 4096 rows up for two, 64 rows for one, whose split
+	// keeps the grid at 1024 blocks.  us at (rows per block, split), 64 columns, n
+	// = 7936: (256, 8) 131, (128, 8) 149, (64, 8) 166; 192 columns, n = 4096: (256,
+	// 8), a last round half full, 134, (128, 8) 103, (64, 8) 115; n = 1024: 21.5,
+	// 14.1, 14.2; 32 columns, n = 2048: 12.0 at 128, 8.9 at 64.
+	void tile()
+	{
+		const int groups = rp / (16 * ct);
+		if (ct == 1) {
+			while (S > 1 && ld / 64 * S > 1024) S /= 2;
+		} else if (ct == 2) {
+			W = ld >= 4096 ? 8 : 4;
+		} else {
+			for (int r = 2; r >= 1; r--)
+				for (int s = 1; s <= 8; s *= 2) {
+					const int blocks = ld / (128 * r) * groups * s, full = (blocks + 255) / 256 * 256;
+					if (blocks >= 240 && 100 * blocks >= 85 * full) {
+						rt = r;
+						W = 8;
+						S = s;
+						return;
+					}
+				}
+		}
 	}
 	// at most 4 columns: the vector-unit kernel (ld is a multiple of 256:
 	// whole steps of 256 k, whole blocks of 32 rows)
@@ -897,11 +1014,14 @@ struct Fx64 {
 			else if (nrhs == 3) launch_vec<3>(F, wT, base, rho, xT, out, st);
 			else launch_vec<4>(F, wT, base, rho, xT, out, st);
 		} else {
-			const dim3 grid(ld / (64 * rt), rp / (16 * ct), S);
+			const dim3 grid(ld / (16 * rt * W), rp / (16 * ct), S), threads(64 * W);
 			const int kchunk = ld / S;
-			if (ct == 4) hipLaunchKernelGGL((k_fx64m<2, 4>), grid, dim3(kB), 0, st, F, wT, part.p, ld, rp, kchunk);
-			else if (ct == 2) hipLaunchKernelGGL((k_fx64m<4, 2>), grid, dim3(kB), 0, st, F, wT, part.p, ld, rp, kchunk);
-			else hipLaunchKernelGGL((k_fx64m<4, 1>), grid, dim3(kB), 0, st, F, wT, part.p, ld, rp, kchunk);
+			if (ct == 1) hipLaunchKernelGGL((k_fx64m<1, 1, 4>), grid, threads, 0, st, F, wT, part.p, ld, rp, kchunk);
+			else if (ct == 2 && W == 4) hipLaunchKernelGGL((k_fx64m<1, 2, 4>), grid, threads, 0, st, F, wT, part.p, ld, rp, kchunk);
+			else if (ct == 2) hipLaunchKernelGGL((k_fx64m<1, 2, 8>), grid, threads, 0, st, F, wT, part.p, ld, rp, kchunk);
+			else if (W == 4) hipLaunchKernelGGL((k_fx64m<1, 4, 4>), grid, threads, 0, st, F, wT, part.p, ld, rp, kchunk);
+			else if (rt == 1) hipLaunchKernelGGL((k_fx64m<1, 4, 8>), grid, threads, 0, st, F, wT, part.p, ld, rp, kchunk);
+			else hipLaunchKernelGGL((k_fx64m<2, 4, 8>), grid, threads, 0, st, F, wT, part.p, ld, rp, kchunk);
 			hipLaunchKernelGGL(k_resid, dim3((unsigned)nblk), dim3(kB), 0, st, part.p, S, ld, rp, n, nrhs, xT, base, rho,
 			                   out, blk);
 		}

@@ -99,3 +99,18 @@ def test_batch_size_rules(sizes, prec):
         _, rel2, info2 = b.solve(rho, E, prec=prec, graph=True, tol=1e-14, outer=2, sweeps=2)
         lit = [i for i, n in enumerate(sizes) if E[sum(sizes[:i]):sum(sizes[:i + 1])].any()]
         assert info2["above_tol"] == len(lit) and np.all(rel2[lit] > 1e-14)
+
+
+# the FP64 MFMA product at each of its tiles: one, two and four column tiles,
+# 64, 128 and 256 rows a block, split-K 1 to 8, ragged ends
+@pytest.mark.parametrize("n,nrhs", [(1, 5), (250, 16), (300, 17), (300, 40), (1024, 64), (2049, 192), (4100, 30), (4100, 64),
+                                    (4096, 192), (7900, 65), (9000, 16), (8192, 129)])
+def test_f64_product_many_columns(n, nrhs):
+    rng = np.random.default_rng(n + nrhs)
+    F = rng.random((n, n), np.float32)
+    X = rng.standard_normal((n, nrhs))
+    with radgpu.LinearSystem(n) as lin:
+        lin.set_matrix(F)
+        Y = lin.multiply(X, "f32")
+    F64 = F.astype(np.float64)
+    assert (np.abs(Y - F64 @ X) <= 2 * (n + 1) * U64 * (F64 @ np.abs(X))).all()
