@@ -205,10 +205,18 @@ __device__ __forceinline__ unsigned long long wave_max(unsigned long long k)
 	}
 	return k;
 }
+// sum over the wave, in every lane: prefix sums within rows of 16 lanes (DPP
+// row_shr 1, 2, 4, 8; lanes without a source add 0), then across the rows
+// (row_bcast 15 and 31), and lane 63's total read back
 __device__ __forceinline__ int wave_sum(int x)
 {
-	for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
-	return x;
+	x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+	x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+	x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+	x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+	x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+	x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+	return __builtin_amdgcn_readlane(x, 63);
 }
 // (int)(((double)q - G0) / MinGridLen) of TreeNodeNum (raycast.cpp:263),
 // from the product with the reciprocal unless its fraction is within 1e-9
@@ -445,6 +453,166 @@ __device__ int walk(const DScene &S, float px, float py, float pz, float vx, flo
 		qy = axpy<F>(tm, vy, py);
 		qz = axpy<F>(tm, vz, pz);
 		t = tm;
+	}
+}
+
+// walk() for launches of a wave or two per SIMD, where a step's instructions
+// and loads are one dependent chain: the eight lanes of a group walk one ray as
+// walk<F, 8> does, with the same result and counts, but
+//  - lane a of each quad takes axis a of the step (the exit plane's quotient,
+//    the next point's coordinate and cell), combined over the quad by DPP, and
+//    lane 3 the record's list bounds: a third of the instructions;
+//  - the exit point, which does not depend on the hits, is taken first, and
+//    the next leaf's cell and record are on their way while this leaf's list
+//    is tested;
+//  - the hits are combined by DPP, and only where a lane has one.
+// The 2120-slot room, 5 leaves a ray and up to 17 in a launch: k_trace_direct
+// 24.2 -> 17.2 us with it (that needs its 90 VGPRs: held to 80 it spills and
+// gains nothing), 3001 rays cast 23.7 -> 16.9 us. Where waves enough are in
+// flight to hide the chain it gives nothing: the hall's k_trace 195 us with
+// walk, 198 with this, 98000 rays there at four lanes 91 and 100 us.
+
+// x of the lane that differs in bit 0, in bit 1, or (where quads agree) in bit
+// 2 of the group
+template <int O, typename T> __device__ __forceinline__ T group_other(T x)
+{
+	static_assert(sizeof(T) == 4, "32 bits");
+	constexpr int ctrl = O == 1 ? 0xB1 : O == 2 ? 0x4E : 0x141;  // quad_perm [1,0,3,2], [2,3,0,1], row_half_mirror
+	return __builtin_bit_cast(T, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), ctrl, 0xf, 0xf, true));
+}
+// lane 3 of the quad's x
+__device__ __forceinline__ int quad_last(float x)
+{
+	return __builtin_amdgcn_mov_dpp(__float_as_int(x), 0xFF, 0xf, 0xf, true);
+}
+template <int O> __device__ __forceinline__ void group_nearest(float &tmin, int &best, int &best_e, int &redo)
+{
+	const float t2 = group_other<O>(tmin);
+	const int b2 = group_other<O>(best), e2 = group_other<O>(best_e);
+	redo |= group_other<O>(redo);
+	if (b2 >= 0 && (best < 0 || t2 < tmin || (t2 == tmin && e2 < best_e))) {
+		tmin = t2;
+		best = b2;
+		best_e = e2;
+	}
+}
+// This lane's axis of a walk; lane 3 of a quad has none (its coordinate stays
+// on the grid's corner and adds nothing).
+struct Axis {
+	float p, v, lo, hi;
+	int mul;   // of the cell index
+	bool use;  // NextPoint steps along it
+};
+// the cell of p + t v: -1 outside the grid, -2 outside the tabulated descent
+template <bool F> __device__ __forceinline__ int quad_cell(const DScene &S, const Axis &A, float t, bool at_p)
+{
+	const float q = at_p ? A.p : axpy<F>(t, A.v, A.p);
+	int g = cell_coord(q, A.lo, S);
+	// outside: bit 30 (grid) or 29 (descent) set in some lane; cells are < 2^30
+	const int out = (q < A.lo || q > A.hi) ? 2 : (unsigned)g >= (unsigned)S.gt ? 1 : 0;
+	g = out ? 0 : g * A.mul;
+	g += group_other<1>(g);
+	g += group_other<2>(g);
+	int o = out | group_other<1>(out);
+	o |= group_other<2>(o);
+	return o == 0 ? g : (o & 2) ? -1 : -2;
+}
+template <bool F>
+__device__ int walk_ahead(const DScene &S, float px, float py, float pz, float vx, float vy, float vz, int ban, Cnt &c,
+                          int sub)
+{
+	constexpr int L = 8;
+	const int ax = sub & 3;
+	Axis A;
+	A.p = ax == 0 ? px : ax == 1 ? py : ax == 2 ? pz : S.g0x;
+	A.v = ax == 0 ? vx : ax == 1 ? vy : ax == 2 ? vz : 0.0f;
+	A.lo = ax == 1 ? S.g0y : ax == 2 ? S.g0z : S.g0x;
+	A.hi = ax == 1 ? S.g1y : ax == 2 ? S.g1z : S.g1x;
+	A.mul = ax == 0 ? S.gt * S.gt : ax == 1 ? S.gt : ax == 2 ? 1 : 0;
+	A.use = fabsf(A.v) > S.thr_v;
+	const float *box = reinterpret_cast<const float *>(S.leaf_box) + ax;
+	float t = 0.f;
+	int prev = -1, tort = -1, power = 1, lam = 0;  // Brent's cycle detection, as walk's
+	const float ck = (fabsf(vx) + fabsf(vy) + fabsf(vz)) * 0x1p-11f;
+	const float cb = (fabsf(px) + fabsf(py) + fabsf(pz) + S.cull_cl) * 0x1p-12f;
+	int cell = quad_cell<F>(S, A, 0.0f, true);
+	int leaf = S.cell_leaf[max(cell, 0)];
+	float b0 = box[8 * leaf], b1 = box[8 * leaf + 4];  // this axis of the leaf's box; lane 3: first item, count | depth << 24
+	for (int steps = 0;;) {
+		if (cell == -1) return -1;
+		if (cell < 0 || ++steps > kMaxWalk) { c.stalled++; return -2; }
+		if (leaf == prev) {
+			c.precision++;
+			const float nt = (float)((double)t + 1.0);
+			if (nt == t) { c.stalled++; return -2; }  // the reference loops forever here
+			t = nt;
+			cell = quad_cell<F>(S, A, t, false);
+			leaf = S.cell_leaf[max(cell, 0)];
+			b0 = box[8 * leaf];
+			b1 = box[8 * leaf + 4];
+			continue;
+		}
+		const int begin = quad_last(b0), cd = quad_last(b1), cnt = cd & 0xffffff;
+		const int my = cnt > sub ? (cnt - sub + L - 1) / L : 0;  // this lane's share of the list
+		const float4 *nc = S.lnc + 2 * (size_t)begin;
+		const float4 *se = S.lse + 3 * (size_t)begin;
+		float4 ea = make_float4(0.f, 0.f, 0.f, 0.f), eb = ea;
+		if (my > 0) {
+			ea = nc[2 * sub];
+			eb = nc[2 * sub + 1];
+		}
+		c.cells++;
+		c.levels += cd >> 24;
+		// the way out (NextPoint), and the next point's cell
+		float tm = 1000000.0f;
+		if (A.use) {
+			const float s = ((A.v > 0 ? b1 : b0) - A.p) / A.v;
+			tm = s < tm ? s : tm;
+		}
+		tm = fminf(tm, group_other<1>(tm));
+		tm = fminf(tm, group_other<2>(tm));
+		tm = (float)((double)tm + 0.1);
+		const int ncell = quad_cell<F>(S, A, tm, false);
+		const int nleaf = S.cell_leaf[max(ncell, 0)];
+		float tmin = 1000000.0f, tmin_hi = 1000000.0f * kGuardUp;
+		int best = -1, best_e = 0;
+		bool nan_hit = false;
+		if (my > 0)
+			test_entry<F, true>(S, ea, eb, se + 3 * sub, px, py, pz, vx, vy, vz, ban, ck, cb, tmin, tmin_hi, best, sub,
+			                    best_e, nan_hit, c);
+		const float n0 = box[8 * nleaf], n1 = box[8 * nleaf + 4];
+		for (int m = 1; m < my; m++) {
+			const int e = sub + L * m;
+			test_entry<F, true>(S, nc[2 * e], nc[2 * e + 1], se + 3 * e, px, py, pz, vx, vy, vz, ban, ck, cb, tmin, tmin_hi,
+			                    best, e, best_e, nan_hit, c);
+		}
+		// the group's nearest hit (the earliest entry on ties), if any lane has one
+		const unsigned long long any = __ballot(best >= 0);
+		if ((any >> ((int)(threadIdx.x & 63) & ~(L - 1))) & 0xffull) {
+			int redo = nan_hit;
+			group_nearest<1>(tmin, best, best_e, redo);
+			group_nearest<2>(tmin, best, best_e, redo);
+			group_nearest<4>(tmin, best, best_e, redo);
+			if (redo) {
+				// a NaN quotient was accepted: the whole list in order, in every
+				// lane of the group (its tests were counted by the shares)
+				Cnt tmp = c;
+				tmin = 1000000.0f;
+				tmin_hi = 1000000.0f * kGuardUp;
+				best = -1;
+				test_list<F, 1>(S, begin, cnt, 0, px, py, pz, vx, vy, vz, ban, ck, cb, tmin, tmin_hi, best, best_e, nan_hit,
+				                tmp);
+			}
+			if (best >= 0) return best;
+		}
+		if (leaf == tort) { c.stalled++; return -2; }
+		if (++lam == power) { tort = leaf; power <<= 1; lam = 0; }
+		prev = leaf;
+		t = tm;
+		cell = ncell;
+		leaf = nleaf;
+		b0 = n0;
+		b1 = n1;
 	}
 }
 
@@ -708,20 +876,27 @@ template <int G> struct RecvMap {
 	}
 };
 
-template <int W = kWavesPerBlock> __device__ void add_block_counters(const int (&vals_in)[8], long long *bcnt)
+// adds a block's counters to its own slots: one lane per counter, so that they
+// are read and written together (one after the other took 2 us of a small
+// launch's last wave)
+template <int W = kWavesPerBlock> __device__ void add_block_counters(const int (&vals)[8], long long *bcnt)
 {
-	__shared__ int wcnt[W][8];
-	int vals[8];
-	for (int k = 0; k < 8; k++) vals[k] = wave_sum(vals_in[k]);
-	if ((threadIdx.x & 63) == 0)
-		for (int k = 0; k < 8; k++) wcnt[threadIdx.x >> 6][k] = vals[k];
-	__syncthreads();
-	if (threadIdx.x == 0)
-		for (int k = 0; k < 8; k++) {
-			long long sum = 0;
-			for (int w = 0; w < W; w++) sum += wcnt[w][k];
-			if (sum) bcnt[(size_t)blockIdx.x * 8 + k] += sum;
-		}
+	const int lane = threadIdx.x & 63;
+	int mine = 0;  // lane k: the wave's sum of counter k
+#pragma unroll
+	for (int k = 0; k < 8; k++) {
+		const int t = wave_sum(vals[k]);
+		mine = lane == k ? t : mine;
+	}
+	if (W > 1) {
+		__shared__ int wcnt[W][8];
+		if (lane < 8) wcnt[threadIdx.x >> 6][lane] = mine;
+		__syncthreads();
+		mine = 0;
+		if (lane < 8)
+			for (int w = 0; w < W; w++) mine += wcnt[w][lane];
+	}
+	if (threadIdx.x < 8 && mine != 0) bcnt[(size_t)blockIdx.x * 8 + threadIdx.x] += mine;
 }
 
 // Source k's rays, part 1: which receivers take part (fixed at the first
@@ -952,7 +1127,8 @@ __global__ __launch_bounds__(kBlock) void k_ray_keys(DScene S, DRecv R, int nv, 
 // fewer would leave most of the machine's wave slots idle: measured on the
 // hall against one lane per ray (242 us) and four (239 us), two take 227 us,
 // the list loop's lanes being busier than the walk's doubled steps cost; on
-// the 2120-slot room eight lanes take an iteration from 49.4 to 48.4 us.
+// the 2120-slot room eight lanes took an iteration from 49.4 to 48.4 us (its
+// launches now go to k_trace_direct).
 __host__ __device__ __forceinline__ int lanes_per_ray(int nr)
 {
 	return 8LL * nr <= kTraceSlots ? 8 : 4LL * nr <= kTraceSlots ? 4 : 2;
@@ -1057,7 +1233,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(6, 
 // what k_compact does besides (the key and the source's deltaB with PREP)
 // block 0 does here.
 template <bool F>
-__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(6, 8))) void k_trace_direct(
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_trace_direct(
 	DScene S, DRecv R, Loop *L, int k, float *ffbuf, long long *bcnt, const unsigned char *rcode, int nlanes,
 	float4 *dB, int prep)
 {
@@ -1076,7 +1252,7 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(6, 
 		const int ban = __float_as_int(R.nrm[r].w);
 		const SrcPatch &sp = s.split ? s.half[h] : s.whole;
 		Cnt w = {0, 0, 0, 0, 0, 0, 0};
-		const int hit = walk<F, 8>(S, px, py, pz, sp.c[0] - px, sp.c[1] - py, sp.c[2] - pz, ban, w, sub);
+		const int hit = walk_ahead<F>(S, px, py, pz, sp.c[0] - px, sp.c[1] - py, sp.c[2] - pz, ban, w, sub);
 		c.tests = w.tests;
 		if (sub == 0) {
 			c.rays = c.ref_rays = 1;
@@ -1513,7 +1689,9 @@ __global__ __launch_bounds__(kBlock) void k_cast(DScene S, const RayIn *rays, in
 	if (i >= n) return;  // a whole group: its lanes share i
 	const RayIn r = rays[i];
 	Cnt c = {0, 0, 0, 0, 0, 0, 0};
-	const int h = walk<F, L>(S, r.p[0], r.p[1], r.p[2], r.v[0], r.v[1], r.v[2], r.ban, c, sub);
+	int h;
+	if constexpr (L == 8) h = walk_ahead<F>(S, r.p[0], r.p[1], r.p[2], r.v[0], r.v[1], r.v[2], r.ban, c, sub);
+	else h = walk<F, L>(S, r.p[0], r.p[1], r.p[2], r.v[0], r.v[1], r.v[2], r.ban, c, sub);
 	int t = c.tests;
 	for (int o = 1; o < L; o <<= 1) t += __shfl_xor(t, o);
 	if (sub == 0) {
