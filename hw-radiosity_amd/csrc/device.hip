@@ -161,6 +161,12 @@ struct Loop {
 	unsigned rng[34];
 	SrcDesc src[kMaxSrc];
 	int v3_range[2][2];  // V3: the slots [r0, r1) of the pass of each parity
+	// V3: the pass's plan (k_v3_plan): its entries and their groups of sample
+	// points, the first receiver past them, the first entry with a departing
+	// sample (INT_MAX: none)
+	int v3_nent, v3_nsub, v3_rest, v3_first;
+	int v3_resume;  // V3: the receiver a pass goes on from with a new plan (0: the pass is over)
+	int v3_short;   // V3: that plan follows one that a departure ended early
 };
 
 struct Cnt {
@@ -205,10 +211,10 @@ __device__ __forceinline__ unsigned long long wave_max(unsigned long long k)
 	}
 	return k;
 }
-// sum over the wave, in every lane: prefix sums within rows of 16 lanes (DPP
-// row_shr 1, 2, 4, 8; lanes without a source add 0), then across the rows
-// (row_bcast 15 and 31), and lane 63's total read back
-__device__ __forceinline__ int wave_sum(int x)
+// prefix sums over the wave, a lane's own value included: within rows of 16
+// lanes (DPP row_shr 1, 2, 4, 8; lanes without a source add 0), then across
+// the rows (row_bcast 15 and 31)
+__device__ __forceinline__ int wave_scan(int x)
 {
 	x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
 	x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
@@ -216,8 +222,10 @@ __device__ __forceinline__ int wave_sum(int x)
 	x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
 	x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
 	x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
-	return __builtin_amdgcn_readlane(x, 63);
+	return x;
 }
+// sum over the wave, in every lane
+__device__ __forceinline__ int wave_sum(int x) { return __builtin_amdgcn_readlane(wave_scan(x), 63); }
 // (int)(((double)q - G0) / MinGridLen) of TreeNodeNum (raycast.cpp:263),
 // from the product with the reciprocal unless its fraction is within 1e-9
 // of an integer; there the exact quotient decides.  The division sits
@@ -771,28 +779,6 @@ template <bool F, bool LOWEST> __global__ void k_prep(DRecv R, Loop *L)
 	L->nsrc = 1;
 	L->shots++;
 	L->ncand = 0;
-}
-
-// k_prep for -variant v3: nothing while a split is still being shaded
-// (v3_pending: the pass of parity par continues it); else the next source
-// and a first pass over every slot in use
-template <bool F> __global__ void k_v3_prep(DRecv R, Loop *L, int par)
-{
-	if (threadIdx.x != 0 || L->done || L->v3_error || L->v3_pending) return;
-	const unsigned long long key = L->key;
-	L->key = 0;
-	if (key == 0) {
-		L->done = 1;
-		return;
-	}
-	const int idx = key_slot<false>(key);
-	make_source<F>(R, idx, L->src[0]);
-	R.dB[idx] = make_float4(0.f, 0.f, 0.f, 0.f);
-	L->nsrc = 1;
-	L->shots++;
-	L->ncand = 0;
-	L->v3_range[par][0] = 0;
-	L->v3_range[par][1] = L->trinum;
 }
 
 // Multi-source selection (-parallel_src k > 1): collect candidate keys, then
@@ -1753,13 +1739,25 @@ __global__ __launch_bounds__(kBlock) void k_ff_pairs(DScene S, DRecv R, const in
 // rand() (GetPointInTriangle, shade.cpp:49-68), is split at its centroid into
 // three (PartitionTriangleWithCenterAndStore, shade.cpp:261-306); the new
 // slots are shaded in further passes (rad.cpp:406-451).  On the device:
-// k_v3_gen computes every receiver's form factors (its vertices and centroid)
-// in parallel; k_v3_commit walks the receivers in order on one block, keeping
-// the pool count and the rand() state, drawing each receiver's samples 64 at
-// a time across the lanes, and writing the splits; k_v3_apply then runs
-// CalRadiosity (shade.cpp:244-259) for the receivers that keep their form
-// factors.  A split only changes its own slot and new ones, so the form
-// factors of the later receivers of a pass are those the reference computes.
+//  k_v3_gen    every receiver's form factors (its vertices and centroid), and
+//              the next kV3Ahead values of rand()
+//  k_v3_plan   the receivers of the pass that the reference would sample or
+//              split, in order, and where in rand()'s sequence each one's
+//              samples lie if none before it departs (a sample that departs
+//              ends its receiver's, and moves all later ones)
+//  k_v3_spec   those samples, in parallel
+//  k_v3_commit on one block: the splits up to the first departure, with their
+//              slots by prefix sums; the receivers after it (or past what was
+//              planned) in order, drawing each one's samples 64 at a time
+//  k_v3_finish CalRadiosity (shade.cpp:244-259) for the receivers that keep
+//              their form factors, and the next source's selection
+// A split only changes its own slot and new ones, so the form factors of the
+// later receivers of a pass are those the reference computes.  A sample departs at one
+// receiver in 70 (a room of 576 to 2200 slots, 7 receivers sampled a pass of
+// some 36 points each): what bounds a pass is a chain of ray walks, 12 us each.
+// Drawn and tested receiver by receiver on one block the steps after k_v3_gen
+// took 82 us a pass; now k_v3_plan, k_v3_spec and k_v3_commit 5, 6 and 7 us, and
+// the solve 45.2 -> 14.7 ms.
 enum { V3_NONE = 0, V3_APPLY = 1 };
 
 struct V3Dev {
@@ -1769,30 +1767,45 @@ struct V3Dev {
 	int cap;             // slots available (min(MaxTri, -triangle))
 	int n_orig;
 	float adapt_area, sample_area, delta_ff;
+	unsigned *rnd;  // rand()'s state (34 values), then the next kV3Ahead
+	int4 *ent;      // plan: receiver, samples (0: split without), samples before it, its first group
+	int2 *sub;      // group of kV3Sub points: its entry, its first point
+	int2 *out;      // its first departing point (-1: none), and that one's (or the last one's) |g - fs|
+	int *cnt;       // its counters, 8 each
+	int *f3;        // slots whose third corner the commit shades anew
 };
+// values of rand() made ahead: kV3Runs waves, kV3Run each
+constexpr int kV3Run = 16 * 31, kV3Runs = 64, kV3Ahead = kV3Run * kV3Runs;
+constexpr int kV3RunBlocks = kV3Runs / kWavesPerBlock;
+constexpr int kV3Sub = 16;      // sample points per block of k_v3_spec, 16 lanes each
+constexpr int kV3Subs = 4096;   // groups planned at most
+constexpr int kV3Wide = 5120;   // slots of a pass up to which a form factor takes 16 lanes
 
 // AdaptCalFF(CalFF(..)) at a point of a receiver with normal n
 // (shade.cpp:141-168): the whole source's form factor, or, for a split
 // source, the discarded whole one and then the sum of the two halves'.  On
-// the four lanes q = 0..3 of an aligned group: lanes 0-1 walk the first half
-// (or the whole source), lanes 2-3 the second half, two lanes sharing each
-// ray's lists (walk<F, 2>); every lane of the group returns the form
-// factor, the halves summed in AdaptCalFF's order.  Tests
-// are counted by every lane, the rest once per ray (its first lane).  The
-// four lanes call it together.
-template <bool F>
-__device__ float adapt_ff4(const DScene &S, const SrcDesc &s, float nx, float ny, float nz, float nlen, int logdst,
-                           float px, float py, float pz, int q, Cnt &c)
+// the 2 L lanes q of an aligned group: the first L walk the first half (or the
+// whole source), the others the second half, sharing each ray (walk<F, 2> or
+// walk_ahead); every lane of the group returns the form factor, the halves
+// summed in AdaptCalFF's order.  Tests are counted by every lane, the rest
+// once per ray (its first lane).  The group calls it together.
+template <bool F, int L>
+__device__ float adapt_ff(const DScene &S, const SrcDesc &s, float nx, float ny, float nz, float nlen, int logdst,
+                          float px, float py, float pz, int q, Cnt &c)
 {
-	const int h = q >> 1, sub = q & 1;
+	static_assert(L == 2 || L == 8, "lanes per ray");
+	const int h = q / L, sub = q % L;
 	float f = 0.0f;
 	if (s.split || h == 0) {
 		const SrcPatch &sp = s.split ? s.half[h] : s.whole;
-		if (s.split && q == 0 && ff_prefix<F>(s.whole, nx, ny, nz, nlen, px, py, pz) != 0.0f) c.ref_rays++;
+		if (s.split && q == 0 && ff_prefix_nonzero<F>(s.whole, nx, ny, nz, nlen, px, py, pz)) c.ref_rays++;
 		const float ff = ff_prefix<F>(sp, nx, ny, nz, nlen, px, py, pz);
 		if (ff != 0.0f) {
 			Cnt w = {0, 0, 0, 0, 0, 0, 0};
-			const int hit = walk<F, 2>(S, px, py, pz, sp.c[0] - px, sp.c[1] - py, sp.c[2] - pz, logdst, w, sub);
+			const float vx = sp.c[0] - px, vy = sp.c[1] - py, vz = sp.c[2] - pz;
+			int hit;
+			if constexpr (L == 8) hit = walk_ahead<F>(S, px, py, pz, vx, vy, vz, logdst, w, sub);
+			else hit = walk<F, L>(S, px, py, pz, vx, vy, vz, logdst, w, sub);
 			c.tests += w.tests;
 			if (sub == 0) {
 				c.rays++;
@@ -1805,8 +1818,8 @@ __device__ float adapt_ff4(const DScene &S, const SrcDesc &s, float nx, float ny
 			f = hit == s.log ? ff : 0.0f;
 		}
 	}
-	const int g0 = (int)(threadIdx.x & 63) & ~3;
-	const float fa = __shfl(f, g0), fb = __shfl(f, g0 + 2);
+	const int g0 = (int)(threadIdx.x & 63) & ~(2 * L - 1);
+	const float fa = __shfl(f, g0), fb = __shfl(f, g0 + L);
 	return s.split ? fa + fb : fa;
 }
 
@@ -1843,72 +1856,383 @@ __device__ void v3_store(const V3Dev &V, const DRecv &R, int r, const Patch &t)
 	R.dB[r] = make_float4(t.deltaB[0], t.deltaB[1], t.deltaB[2], 0.f);
 }
 
-// Form factors of receivers [r0, r1): 4 lanes per receiver, the vertices'
-// (shade.cpp:442-450) and, where area >= -adapt_area, the centroid's
-// (shade.cpp:469-470); act = V3_APPLY for each receiver the reference
-// shades (parent >= 0, not the source, not saturated: rad.cpp:419-428).
+// A triangle's sample point and the vertices' form factors interpolated there
+// (GetPointInTriangle, shade.cpp:49-68), from three values of rand()
 template <bool F>
-__global__ __launch_bounds__(kBlock) void k_v3_gen(DScene S, DRecv R, V3Dev V, Loop *L, int par, long long *bcnt)
+__device__ __forceinline__ void v3_point(const unsigned *o, const float (&P)[3][3], float f0, float f1, float f2,
+                                         float (&x)[3], float &g)
 {
-	Cnt c = {0, 0, 0, 0, 0, 0, 0};
-	const int r0 = L->v3_range[par][0], r1 = L->v3_range[par][1];
-	// four lanes per form factor (adapt_ff4), four form factors per receiver;
-	// the grid strides over the pass's slots
-	for (int t = blockIdx.x * kBlock + threadIdx.x; !L->done && t < 16 * (r1 - r0); t += gridDim.x * kBlock) {
-		const int r = r0 + t / 16, w = (t / 4) % 4, g4 = t % 4;
-		const SrcDesc &s = L->src[0];
-		const float4 nr = R.nrm[r];
-		const int parent = __float_as_int(nr.w);
-		bool sat = true;
-		for (int v = 0; v < 3; v++) {
-			const float4 a = R.acc[3 * r + v];
-			sat = sat && !(a.x < 255.0f || a.y < 255.0f || a.z < 255.0f);
-		}
-		const bool live = parent >= 0 && r != s.phys && !sat;
-		if (w == 0 && g4 == 0) V.act[r] = live ? V3_APPLY : V3_NONE;
-		float f = 0.0f;
-		const float4 ca = R.cA[r];
-		if (live && (w < 3 || ca.w >= V.adapt_area)) {
-			const float nlen = __builtin_sqrtf(dot3<F>(nr.x, nr.y, nr.z, nr.x, nr.y, nr.z));
-			float px, py, pz;
-			if (w < 3) {
-				px = R.vx[3 * r + w];
-				py = R.vy[3 * r + w];
-				pz = R.vz[3 * r + w];
-			} else {
-				px = ca.x;
-				py = ca.y;
-				pz = ca.z;
-			}
-			f = adapt_ff4<F>(S, s, nr.x, nr.y, nr.z, nlen, parent, px, py, pz, g4, c);
-		}
-		if (g4 == 0) V.ff[4 * (size_t)r + w] = f;
+	float w1 = (float)(int)(o[0] >> 1), w2 = (float)(int)(o[1] >> 1), w3 = (float)(int)(o[2] >> 1);
+	const float tot = w1 + w2 + w3;
+	w1 /= tot;
+	w2 /= tot;
+	w3 /= tot;
+	for (int k = 0; k < 3; k++) x[k] = dot3<F>(w1, w2, w3, P[0][k], P[1][k], P[2][k]);
+	g = dot3<F>(w1, w2, w3, f0, f1, f2);
+}
+
+// Form factors of one slot of the pass: the vertices' (shade.cpp:442-450) and,
+// where area >= -adapt_area, the centroid's (shade.cpp:469-470), 2 L lanes
+// each; act = V3_APPLY for a receiver the reference shades (parent >= 0, not
+// the source, not saturated: rad.cpp:419-428).
+template <bool F, int L>
+__device__ __forceinline__ void v3_corner(const DScene &S, const DRecv &R, const V3Dev &V, const SrcDesc &s, int r,
+                                          int w, int q, Cnt &c)
+{
+	const float4 nr = R.nrm[r];
+	const int parent = __float_as_int(nr.w);
+	bool sat = true;
+	for (int v = 0; v < 3; v++) {
+		const float4 a = R.acc[3 * r + v];
+		sat = sat && !(a.x < 255.0f || a.y < 255.0f || a.z < 255.0f);
 	}
+	const bool live = parent >= 0 && r != s.phys && !sat;
+	if (w == 0 && q == 0) V.act[r] = live ? V3_APPLY : V3_NONE;
+	float f = 0.0f;
+	const float4 ca = R.cA[r];
+	if (live && (w < 3 || ca.w >= V.adapt_area)) {
+		const float nlen = __builtin_sqrtf(dot3<F>(nr.x, nr.y, nr.z, nr.x, nr.y, nr.z));
+		float px, py, pz;
+		if (w < 3) {
+			px = R.vx[3 * r + w];
+			py = R.vy[3 * r + w];
+			pz = R.vz[3 * r + w];
+		} else {
+			px = ca.x;
+			py = ca.y;
+			pz = ca.z;
+		}
+		f = adapt_ff<F, L>(S, s, nr.x, nr.y, nr.z, nlen, parent, px, py, pz, q, c);
+	}
+	if (q == 0) V.ff[4 * (size_t)r + w] = f;
+}
+
+// glibc rand() (TYPE_3): r[i] = r[i - 3] + r[i - 31] (mod 2^32), output
+// r[i] >> 1.  The value n ahead is a fixed combination of the 31 before it:
+// with x^n = sum_k c_k x^k (mod x^31 - x^28 - 1), r[i + n] = sum_k c_k r[i + k].
+// c for n = 0, kV3Run, 2 kV3Run, ..: where each wave's run of values starts.
+struct V3Jump {
+	unsigned c[kV3Runs][31];
+};
+constexpr V3Jump v3_jump()
+{
+	V3Jump j{};
+	unsigned step[31] = {1};
+	for (int n = 0; n < kV3Run; n++) {  // times x
+		const unsigned top = step[30];
+		for (int k = 30; k > 0; k--) step[k] = step[k - 1];
+		step[0] = top;
+		step[28] += top;
+	}
+	j.c[0][0] = 1;
+	for (int w = 1; w < kV3Runs; w++) {
+		unsigned p[61] = {};
+		for (int a = 0; a < 31; a++)
+			for (int b = 0; b < 31; b++) p[a + b] += j.c[w - 1][a] * step[b];
+		for (int k = 60; k >= 31; k--) {
+			p[k - 3] += p[k];
+			p[k - 31] += p[k];
+		}
+		for (int k = 0; k < 31; k++) j.c[w][k] = p[k];
+	}
+	return j;
+}
+__device__ const V3Jump kV3Jump = v3_jump();
+
+// a value of the next block of 31, lane t's, from the last 31: every r[i - 31]
+// is known, so r[b + t] = r[b + t % 3 - 3] + (the sum of r[b + u - 31] over
+// u <= t, u = t mod 3): three interleaved prefix sums, four shuffle steps
+__device__ __forceinline__ unsigned v3_next31(unsigned cur, int lane)
+{
+	unsigned x = cur;
+	for (int d = 3; d < 31; d <<= 1) {  // 3, 6, 12, 24: within a residue class
+		const unsigned y = __shfl_up(x, d);
+		if (lane >= d) x += y;
+	}
+	return x + __shfl(cur, 28 + lane % 3);
+}
+// one wave: run w of V.rnd
+__device__ void v3_rand(const V3Dev &V, const Loop *L, unsigned (&s)[64], int w, int lane)
+{
+	const unsigned old = lane < 34 ? L->rng[(L->rng_k + lane) % 34] : 0u;  // oldest first
+	if (w == 0 && lane < 34) V.rnd[lane] = old;
+	unsigned cur = __shfl(old, lane < 31 ? lane + 3 : 0);
+	// the 62 values from the state's last 31 on: what the combinations read
+	const unsigned nx = v3_next31(cur, lane);
+	if (lane < 31) {
+		s[lane] = cur;
+		s[lane + 31] = nx;
+	}
+	__builtin_amdgcn_wave_barrier();
+	unsigned x = 0;
+	for (int k = 0; k < 31; k++) x += kV3Jump.c[w][k] * s[(lane < 31 ? lane : 0) + k];
+	cur = x;
+	unsigned *o = V.rnd + 34 + (size_t)w * kV3Run;
+	for (int b = 0; b < kV3Run; b += 31) {
+		cur = v3_next31(cur, lane);
+		if (lane < 31) o[b + lane] = cur;
+	}
+}
+
+// The form factors of the pass's slots, the grid striding over them; and, on
+// the last kV3RunBlocks blocks, the random numbers, which no form factor needs
+// (they are done before the walks are).  A form factor takes 16 lanes
+// (walk_ahead) while the pass's rays leave the machine mostly idle, else 4:
+// a shot of 576 slots takes 32 us against 41 with four, of 2236 39 and 49, of
+// 3414 67 and 75, of 4800 53 and 62, of 5874 107 to 114 and 108.
+template <bool F>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_v3_gen(
+	DScene S, DRecv R, V3Dev V, Loop *L, int par, long long *bcnt)
+{
+	__shared__ unsigned rs[kWavesPerBlock][64];
+	__shared__ SrcDesc s;
+	if (L->done || L->v3_error) return;
+	// no pass under way: a new source, and a first pass over every slot in use
+	const bool fresh = !L->v3_pending;
+	const unsigned long long key = L->key;
+	if (fresh && key == 0) return;  // nothing left to shoot: k_v3_plan ends the solve
+	const int nb = gridDim.x - kV3RunBlocks;
+	if ((int)blockIdx.x >= nb) {
+		const int wv = threadIdx.x >> 6;
+		v3_rand(V, L, rs[wv], (blockIdx.x - nb) * kWavesPerBlock + wv, threadIdx.x & 63);
+		return;
+	}
+	Cnt c = {0, 0, 0, 0, 0, 0, 0};
+	const int r0 = fresh ? 0 : L->v3_range[par][0], n = (fresh ? L->trinum : L->v3_range[par][1]) - r0;
+	const bool wide = n <= kV3Wide;
+	if (L->v3_resume || (long long)blockIdx.x * kBlock >= (wide ? 64LL : 16LL) * n) return;
+	// the source: each block makes its own (a launch less), block 0 keeps it
+	if (threadIdx.x == 0) {
+		if (fresh) make_source<F>(R, key_slot<false>(key), s);
+		else s = L->src[0];
+		if (fresh && blockIdx.x == 0) L->src[0] = s;
+	}
+	__syncthreads();
+	const long long t0 = (long long)blockIdx.x * kBlock + threadIdx.x, dt = (long long)nb * kBlock;
+	if (wide)
+		for (long long t = t0; t < 64LL * n; t += dt) v3_corner<F, 8>(S, R, V, s, r0 + (int)(t / 64), (int)(t / 16) % 4, (int)(t % 16), c);
+	else
+		for (long long t = t0; t < 16LL * n; t += dt) v3_corner<F, 2>(S, R, V, s, r0 + (int)(t / 16), (int)(t / 4) % 4, (int)(t % 4), c);
 	const int vals[8] = {c.rays, c.ref_rays, c.cells, c.tests, c.levels, c.precision, c.stalled, 0};
 	add_block_counters(vals, bcnt);
 }
 
-// glibc rand() (TYPE_3): r[i] = r[i - 3] + r[i - 31] (mod 2^32), output
-// r[i] >> 1; the state is the last 34 values, the oldest at st[k].
-//
-// v3_draw: the next n (<= 3 kWave) values, drawn by the block's first wave
-// into seq[34 .. 34 + n), after the state's 34 in order in seq[0, 34).  In
-// a block of 31 consecutive values every r[i - 31] is already known, so
-// within the block r[b + t] = r[b + t % 3 - 3] + (the sum of known_u over
-// u <= t, u = t mod 3): three interleaved prefix sums, four shuffle steps.
+// blocks of k_v3_gen's form factors for a pool of n slots in use
+inline int v3_gen_blocks(size_t n)
+{
+	const size_t lanes = std::max(64 * std::min(n, (size_t)kV3Wide), 16 * n);
+	return (int)std::min<size_t>((lanes + kBlock - 1) / kBlock, 4096);
+}
+constexpr int kV3SpecBlocks = 512;
+// A new plan (five launches, 45 us) against the ordered steps' 18 us a receiver:
+// taken where more than this many receivers go by without a departure.  The
+// room's longest commit was 1552 us without it, 46 us with it; all of them
+// together 5.2 and 2.7 ms.
+constexpr int kV3Again = 2;
+
+// exclusive prefix sums of x over a block of kV3Commit threads, and the total
+constexpr int kV3Commit = 1024;
+__device__ __forceinline__ int v3_scan(int x, int (&part)[kV3Commit / kWave], int &total)
+{
+	const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+	const int inc = wave_scan(x);
+	__syncthreads();  // part is free
+	if (lane == 63) part[wv] = inc;
+	__syncthreads();
+	int before = 0;
+	total = 0;
+	for (int w = 0; w < kV3Commit / kWave; w++) {
+		before += w < wv ? part[w] : 0;
+		total += part[w];
+	}
+	return before + inc - x;
+}
+
+// whether the vertices' form factors do not predict the centroid's
+// (shade.cpp:469-473): |mean - centre|
+__device__ __forceinline__ float v3_centre_diff(const V3Dev &V, int r)
+{
+	const float f0 = V.ff[4 * (size_t)r], f1 = V.ff[4 * (size_t)r + 1], f2 = V.ff[4 * (size_t)r + 2];
+	const float groud = (float)((double)(f0 + f1 + f2) / 3.0);
+	return ffabs(groud - V.ff[4 * (size_t)r + 3]);
+}
+
+// The source of a new pass is taken; then the pass's entries in receiver order,
+// on one block: the receivers that are split at once, or sampled first
+// (shade.cpp:455-473), from v3_resume on.  What cannot be sampled ahead (past
+// kV3Ahead values or kV3Subs groups) is left to the commit.
+__global__ __launch_bounds__(kV3Commit) void k_v3_plan(DRecv R, V3Dev V, Loop *L, int par)
+{
+	__shared__ int part[2][kV3Commit / kWave];
+	__shared__ int rest, ents, subs;
+	if (L->done || L->v3_error) return;
+	const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+	const bool fresh = !L->v3_pending;
+	const unsigned long long key = L->key;
+	if (fresh && key == 0) {
+		__syncthreads();
+		if (tid == 0) L->done = 1;
+		return;
+	}
+	const int trinum = L->trinum;
+	const int r1 = fresh ? trinum : L->v3_range[par][1];
+	const int start = max(L->v3_resume, fresh ? 0 : L->v3_range[par][0]);
+	int nent = 0, noff = 0, nsub = 0;
+	if (tid == 0) rest = r1;
+	bool more = trinum + 4 < V.cap;  // else every receiver keeps its form factors (shade.cpp:463)
+	for (int base = start; base < r1 && more; base += kV3Commit) {
+		const int r = base + tid;
+		bool is = false;
+		int n = 0;
+		if (r < r1 && V.act[r] == V3_APPLY) {
+			const float area = R.cA[r].w;
+			if (area >= V.adapt_area && !((double)area < 1e-8)) {
+				is = true;
+				if (v3_centre_diff(V, r) < V.delta_ff) {
+					n = (int)(area / V.sample_area);
+					is = n > 0;  // without a sample: not split
+					n = min(max(n, 0), kV3Ahead);
+				}
+			}
+		}
+		// prefix sums of the entries and (above 11 bits) their groups, and of the samples
+		const int g = (n + kV3Sub - 1) / kV3Sub;
+		static_assert(kV3Commit < 2048 && (long long)kV3Commit * ((kV3Ahead + kV3Sub - 1) / kV3Sub) < (1 << 21) &&
+		                  (long long)kV3Commit * kV3Ahead < (1 << 30),
+		              "packed prefix sums");
+		const unsigned a = (unsigned)is | (unsigned)g << 11;
+		unsigned ia = (unsigned)wave_scan((int)a);
+		int in = wave_scan(n);
+		if (lane == 63) part[0][wv] = (int)ia, part[1][wv] = in;
+		if (tid == 0) ents = subs = 0;
+		__syncthreads();
+		ia -= a;
+		in -= n;
+		unsigned ta = 0;
+		int tn = 0;
+		for (int w = 0; w < kV3Commit / kWave; w++) {
+			ia += w < wv ? (unsigned)part[0][w] : 0u;
+			in += w < wv ? part[1][w] : 0;
+			ta += (unsigned)part[0][w];
+			tn += part[1][w];
+		}
+		const int e = nent + (int)(ia & 2047u), off = noff + in, g0 = nsub + (int)(ia >> 11);
+		if (is) {
+			// what fits is the entries up to the first that does not
+			if (3 * (off + n) <= kV3Ahead && g0 + g <= kV3Subs) {
+				V.ent[e] = make_int4(r, n, off, g0);
+				for (int k = 0; k < n; k += kV3Sub) V.sub[g0 + k / kV3Sub] = make_int2(e, k);
+				atomicMax(&ents, e + 1 - nent);
+				atomicMax(&subs, g0 + g - nsub);
+			} else {
+				atomicMin(&rest, r);
+			}
+		}
+		__syncthreads();
+		more = ents == (int)(ta & 2047u);
+		nent += ents;
+		nsub += subs;
+		noff += tn;
+		__syncthreads();
+	}
+	__syncthreads();
+	if (tid == 0) {
+		L->v3_nent = nent;
+		L->v3_nsub = nsub;
+		L->v3_rest = rest;
+		L->v3_first = INT_MAX;
+		if (fresh) {
+			R.dB[key_slot<false>(key)] = make_float4(0.f, 0.f, 0.f, 0.f);
+			L->key = 0;
+			L->ncand = 0;
+			L->nsrc = 1;
+			L->shots++;
+			L->v3_range[par][0] = 0;
+			L->v3_range[par][1] = trinum;
+		}
+	}
+}
+
+// The plan's sample points, kV3Sub to a block and 16 lanes each; a group whose
+// entry lies past one known to depart is not needed.  A group's counters are
+// kept apart, for the commit to add those the ordered walk makes.
+template <bool F>
+__global__ __launch_bounds__(kV3Sub * 16) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_v3_spec(DScene S, DRecv R,
+                                                                                                     V3Dev V, Loop *L)
+{
+	__shared__ float pdff[kV3Sub];
+	__shared__ int pbrk[kV3Sub];
+	__shared__ int wcnt[kV3Sub / 4][8];
+	__shared__ bool skip;
+	if (L->done || L->v3_error) return;
+	const int tid = threadIdx.x, lane = tid & 63, pt = tid >> 4, q = tid & 15;
+	const int nsub = L->v3_nsub;
+	const SrcDesc &s = L->src[0];
+	for (int b = blockIdx.x; b < nsub; b += gridDim.x) {
+		const int2 sb = V.sub[b];
+		__syncthreads();  // the last group's results are read
+		if (tid == 0) skip = __hip_atomic_load(&L->v3_first, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < sb.x;
+		__syncthreads();
+		if (skip) continue;
+		const int4 en = V.ent[sb.x];
+		const int r = en.x, m = min(kV3Sub, en.y - sb.y);
+		Cnt c = {0, 0, 0, 0, 0, 0, 0};
+		if (pt < m) {
+			const float4 nr = R.nrm[r];
+			const float nlen = __builtin_sqrtf(dot3<F>(nr.x, nr.y, nr.z, nr.x, nr.y, nr.z));
+			float P[3][3], x[3], g;
+			for (int v = 0; v < 3; v++) {
+				P[v][0] = R.vx[3 * r + v];
+				P[v][1] = R.vy[3 * r + v];
+				P[v][2] = R.vz[3 * r + v];
+			}
+			v3_point<F>(V.rnd + 34 + 3 * (size_t)(en.z + sb.y + pt), P, V.ff[4 * (size_t)r], V.ff[4 * (size_t)r + 1],
+			            V.ff[4 * (size_t)r + 2], x, g);
+			const float fs = adapt_ff<F, 8>(S, s, nr.x, nr.y, nr.z, nlen, __float_as_int(nr.w), x[0], x[1], x[2], q, c);
+			const float d = ffabs(g - fs);
+			if (q == 0) {
+				pdff[pt] = d;
+				pbrk[pt] = d > V.delta_ff;
+			}
+		}
+		const int vals[8] = {c.rays, c.ref_rays, c.cells, c.tests, c.levels, c.precision, c.stalled, 0};
+		int mine = 0;
+#pragma unroll
+		for (int k = 0; k < 8; k++) {
+			const int t = wave_sum(vals[k]);
+			mine = lane == k ? t : mine;
+		}
+		if (lane < 8) wcnt[tid >> 6][lane] = mine;
+		__syncthreads();
+		if (tid < kWave) {
+			const unsigned long long bal = __ballot(lane < m && pbrk[lane & (kV3Sub - 1)]);
+			const int j = bal ? __ffsll((long long)bal) - 1 : -1;
+			if (lane == 0) {
+				V.out[b] = make_int2(j, __float_as_int(pdff[j >= 0 ? j : m - 1]));
+				if (j >= 0) atomicMin(&L->v3_first, sb.x);
+			}
+			if (lane < 8) {
+				int t = 0;
+				for (int w = 0; w < kV3Sub / 4; w++) t += wcnt[w][lane];
+				V.cnt[8 * (size_t)b + lane] = t;
+			}
+		}
+	}
+}
+
+// The ordered steps' random numbers: the state is the last 34 values, the
+// oldest at st[sk].  v3_draw: the next n (<= 3 kWave) values, by the block's
+// first wave, into seq[34 .. 34 + n), after the state's 34 in order.
 constexpr int kV3Seq = 34 + 3 * kWave + 31;
 __device__ __forceinline__ void v3_draw(const unsigned *st, int sk, unsigned *seq, int n, int tid)
 {
 	if (tid < kWave) {  // one wave: its LDS accesses stay in order
 		const int lane = tid;
 		if (lane < 34) seq[lane] = st[(sk + lane) % 34];
+		unsigned cur = seq[3 + (lane < 31 ? lane : 0)];
 		for (int b = 34; b < 34 + n; b += 31) {
-			unsigned x = lane < 31 ? seq[b + lane - 31] : 0u;
-			for (int d = 3; d < 31; d <<= 1) {  // 3, 6, 12, 24: within a residue class
-				const unsigned y = __shfl_up(x, d);
-				if (lane >= d) x += y;
-			}
-			if (lane < 31) seq[b + lane] = x + seq[b + lane % 3 - 3];
+			cur = v3_next31(cur, lane);
+			if (lane < 31) seq[b + lane] = cur;
 		}
 	}
 	__syncthreads();
@@ -1941,31 +2265,147 @@ template <bool F> __device__ void v3_area(Patch &t)
 	t.area = __builtin_sqrtf(dot3<F>(t.n[0], t.n[1], t.n[2], t.n[0], t.n[1], t.n[2])) / 2;
 }
 
-// The receivers [r0, r1) in order (see above) on one block of four waves:
-// every wave follows the same decisions; a chunk's 64 sample points take
-// four lanes each (adapt_ff4), the first wave draws the random numbers,
-// thread 0 writes the splits.
+// What PartitionTriangleWithCenterAndStore (shade.cpp:261-306) would make of
+// slot r: the slots it adds (0: left whole), -1 where the split would rewrite
+// an original the octree lists (a slot pre-partition overwrote): the rays of
+// the later receivers would change mid-pass; not supported
+template <bool F> __device__ __forceinline__ int v3_split_size(const V3Dev &V, int r)
+{
+	const Patch &src = V.pool[r];
+	float maxl = 0.0f, minl = 1e+30f;
+	for (int v = 0; v < 3; v++) {
+		const int w = (v + 1) % 3;
+		const float lx = src.p[w][0] - src.p[v][0], ly = src.p[w][1] - src.p[v][1], lz = src.p[w][2] - src.p[v][2];
+		const float len = dot3<F>(lx, ly, lz, lx, ly, lz);
+		maxl = (maxl < len) ? len : maxl;
+		minl = (len < minl) ? len : minl;
+	}
+	if ((double)(minl / maxl) < 1e-1 || minl < 1) return 0;
+	if (src.parent == r) return 3;
+	return r < V.n_orig ? -1 : 2;
+}
+// The split of slot r into slots id, id + 1 and, for an original, id + 2: an
+// original becomes logical, its three parts shaded next pass; else slot r holds
+// the third part, its centroid corner shaded anew (shade.cpp:508-520).
+template <bool F> __device__ void v3_split(const V3Dev &V, const DRecv &R, int r, int id)
+{
+	Patch src;
+	v3_load(V, R, r, src);
+	const bool orig = src.parent == r;
+	for (int k = 0; k < 3; k++) {
+		Patch t = src;
+		for (int x = 0; x < 3; x++) t.p[k][x] = src.c[x];
+		v3_center<F>(t.p, t.c);
+		v3_area<F>(t);
+		if (k == 0) t.neighbor[0] = id + 2, t.neighbor[2] = id + 1;
+		if (k == 1) t.neighbor[1] = id, t.neighbor[0] = id + 2;
+		if (k == 2) t.neighbor[2] = id + 1, t.neighbor[1] = id;
+		v3_store(V, R, k == 2 && !orig ? r : id + k, t);
+	}
+	if (orig) {
+		src.parent = -1;
+		v3_store(V, R, r, src);
+		V.act[r] = V3_NONE;
+	}
+}
+
+// The pass's splits, on one block: those of the plan up to its first departing
+// sample in parallel, one entry per thread; the receivers after it, or past
+// the plan, in receiver order, a chunk's 64 sample points on 16 lanes each.
 template <bool F>
-__global__ __launch_bounds__(4 * kWave) void k_v3_commit(DScene S, DRecv R, V3Dev V, Loop *L, int par,
-                                                         long long *bcnt)
+__global__ __launch_bounds__(kV3Commit) void k_v3_commit(DScene S, DRecv R, V3Dev V, Loop *L, int par, long long *bcnt)
 {
 	__shared__ unsigned st[34], seq[kV3Seq];
 	__shared__ int sk;
-	__shared__ unsigned long long pmask[4];  // each wave's departing points (bit 4k: its point k)
-	__shared__ float pdff[kWave];            // each point's |g - fs|
-	const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-	const int pt = tid >> 2, q = tid & 3;  // a chunk's point and the lane in its group of four
+	__shared__ float pdff[kWave];  // each point's |g - fs|
+	__shared__ int pbrk[kWave];    // whether it departs
+	__shared__ int part[kV3Commit / kWave];
+	__shared__ int full_at, err_at, added, nf3;
+	const int tid = threadIdx.x, lane = tid & 63;
+	const int pt = tid >> 4, q = tid & 15;  // a chunk's point and the lane in its group
 	Cnt c = {0, 0, 0, 0, 0, 0, 0};
 	if (L->done || L->v3_error) return;
-	const int r0 = L->v3_range[par][0], r1 = L->v3_range[par][1];
-	if (tid < 34) st[tid] = L->rng[tid];
-	if (tid == 0) sk = L->rng_k;
-	__syncthreads();
+	const int r1 = L->v3_range[par][1];
 	const SrcDesc &s = L->src[0];
-	const int limit = V.cap;
+	const int limit = V.cap, nent = L->v3_nent, first = L->v3_first;
+	const int last = min(first, nent - 1);  // the last entry whose samples are where the plan put them
 	int trinum = L->trinum;
-	bool stop = false;
-	for (int base = r0; base < r1 && !stop; base += kWave) {
+	bool stop = trinum + 4 >= limit;  // the pool is full: every receiver keeps its form factors
+	int pos = 0;                      // values of rand() used
+	if (tid == 0) nf3 = 0;
+	for (int base = 0; base <= last && !stop; base += kV3Commit) {
+		const int i = base + tid;
+		if (tid == 0) full_at = err_at = INT_MAX, added = 0;
+		int4 en = make_int4(0, 0, 0, 0);
+		int size = 0;
+		if (i <= last) {
+			en = V.ent[i];
+			const int groups = (en.y + kV3Sub - 1) / kV3Sub;
+			// a sampled receiver is split when a sample departs, or the last one
+			// does not come to less than -delta_ff
+			if (groups == 0 || i == first || !(__int_as_float(V.out[en.w + groups - 1].y) < V.delta_ff))
+				size = v3_split_size<F>(V, en.x);
+		}
+		int total;
+		const int before = trinum + v3_scan(max(size, 0), part, total);
+		const bool room = before + 4 < limit;  // once it is full nothing is drawn or split
+		if (i <= last && !room) atomicMin(&full_at, i);
+		if (size < 0 && room) atomicMin(&err_at, i);
+		__syncthreads();
+		if (i <= last && room && i <= err_at) {
+			// the chunks of 64 points (four groups) the ordered steps would have cast
+			int g1 = (en.y + kV3Sub - 1) / kV3Sub;
+			if (i == first) {
+				int k = 0;
+				while (V.out[en.w + k].x < 0) k++;
+				g1 = min(g1, (k & ~3) + 4);
+			}
+			for (int g = en.w; g < en.w + g1; g++) {
+				const int4 a = reinterpret_cast<const int4 *>(V.cnt)[2 * g], b = reinterpret_cast<const int4 *>(V.cnt)[2 * g + 1];
+				c.rays += a.x, c.ref_rays += a.y, c.cells += a.z, c.tests += a.w;
+				c.levels += b.x, c.precision += b.y, c.stalled += b.z;
+			}
+			if (size > 0 && i < err_at) {
+				v3_split<F>(V, R, en.x, before);
+				atomicAdd(&added, size);
+				if (size == 2) V.f3[atomicAdd(&nf3, 1)] = en.x;
+			}
+		}
+		__syncthreads();
+		trinum += added;
+		if (err_at != INT_MAX) {
+			if (tid == 0) L->v3_error = V.ent[err_at].x + 1;
+			stop = true;
+		} else if (full_at != INT_MAX) {
+			pos = 3 * V.ent[full_at].z;
+			stop = true;
+		}
+		__syncthreads();
+	}
+	int rest = L->v3_rest;  // the first receiver left to the ordered steps
+	if (!stop) {
+		if (first < nent) {
+			const int4 en = V.ent[first];
+			int k = 0;
+			while (V.out[en.w + k].x < 0) k++;
+			pos = 3 * (en.z + k * kV3Sub + V.out[en.w + k].x + 1);
+			rest = en.x + 1;
+		} else if (nent > 0) {
+			const int4 en = V.ent[nent - 1];
+			pos = 3 * (en.z + en.y);
+		}
+	}
+	// Entries left after a departure are planned anew, at their samples' real
+	// place, unless few are left or two plans in a row got no further than a few.
+	const int at = first < nent ? first + 1 : nent;
+	const bool brief = at <= kV3Again;
+	bool again = !stop && trinum + 4 < limit && nent - at > kV3Again && !(brief && L->v3_short);
+	const bool ordered = !stop && !again && rest < r1;
+	int left = nent - at, calm = 0;  // ordered steps: entries left, receivers in a row without a departure
+	if (tid < 34) st[tid] = pos > 0 ? V.rnd[pos + tid] : L->rng[(L->rng_k + tid) % 34];
+	if (tid == 0) sk = 0;
+	__syncthreads();
+	for (int base = rest; ordered && base < r1 && !stop; base += kWave) {
 		// Once the pool is full every later receiver keeps its form factors
 		// (the first test below), so nothing is left to do in order.
 		if (trinum + 4 >= limit) break;
@@ -1978,15 +2418,20 @@ __global__ __launch_bounds__(4 * kWave) void k_v3_commit(DScene S, DRecv R, V3De
 		while (todo) {
 			const int r = base + (__ffsll((long long)todo) - 1);
 			todo &= todo - 1;
-			const float4 ca = R.cA[r];
-			const float area = ca.w;
+			const float area = R.cA[r].w;
 			if (trinum + 4 >= limit || (double)area < 1e-8) continue;   // shade.cpp:463-466
-			const float f0 = V.ff[4 * (size_t)r], f1 = V.ff[4 * (size_t)r + 1], f2 = V.ff[4 * (size_t)r + 2];
-			float groud = (float)((double)(f0 + f1 + f2) / 3.0);
-			float dff = ffabs(groud - V.ff[4 * (size_t)r + 3]);
+			if (left > kV3Again && calm > kV3Again) {  // worth a plan again
+				again = stop = true;
+				rest = r;
+				break;
+			}
+			left--;
+			calm++;
+			float dff = v3_centre_diff(V, r);
 			if (dff < V.delta_ff) {
 				// GetPointInTriangle samples until one departs by more than -delta_ff
 				const int samples = (int)(area / V.sample_area);
+				const float f0 = V.ff[4 * (size_t)r], f1 = V.ff[4 * (size_t)r + 1], f2 = V.ff[4 * (size_t)r + 2];
 				const float4 nr = R.nrm[r];
 				const float nlen = __builtin_sqrtf(dot3<F>(nr.x, nr.y, nr.z, nr.x, nr.y, nr.z));
 				const int logdst = __float_as_int(nr.w);
@@ -1996,37 +2441,25 @@ __global__ __launch_bounds__(4 * kWave) void k_v3_commit(DScene S, DRecv R, V3De
 					P[v][1] = R.vy[3 * r + v];
 					P[v][2] = R.vz[3 * r + v];
 				}
-				for (int base = 0; base < samples; base += kWave) {
-					const int m = min(kWave, samples - base);
+				for (int done = 0; done < samples; done += kWave) {
+					const int m = min(kWave, samples - done);
 					v3_draw(st, sk, seq, 3 * m, tid);
-					bool brk = false;
 					if (pt < m) {
-						const unsigned *o = seq + 34 + 3 * pt;
-						float w1 = (float)(int)(o[0] >> 1), w2 = (float)(int)(o[1] >> 1), w3 = (float)(int)(o[2] >> 1);
-						const float tot = w1 + w2 + w3;
-						w1 /= tot;
-						w2 /= tot;
-						w3 /= tot;
-						const float qx = dot3<F>(w1, w2, w3, P[0][0], P[1][0], P[2][0]);
-						const float qy = dot3<F>(w1, w2, w3, P[0][1], P[1][1], P[2][1]);
-						const float qz = dot3<F>(w1, w2, w3, P[0][2], P[1][2], P[2][2]);
-						const float g = dot3<F>(w1, w2, w3, f0, f1, f2);
-						const float fs = adapt_ff4<F>(S, s, nr.x, nr.y, nr.z, nlen, logdst, qx, qy, qz, q, c);
-						const float mydff = ffabs(g - fs);
-						brk = mydff > V.delta_ff;
-						if (q == 0) pdff[pt] = mydff;
+						float x[3], g;
+						v3_point<F>(seq + 34 + 3 * pt, P, f0, f1, f2, x, g);
+						const float fs = adapt_ff<F, 8>(S, s, nr.x, nr.y, nr.z, nlen, logdst, x[0], x[1], x[2], q, c);
+						if (q == 0) {
+							const float d = ffabs(g - fs);
+							pdff[pt] = d;
+							pbrk[pt] = d > V.delta_ff;
+						}
 					}
-					const unsigned long long bw = __ballot(brk && q == 0);
-					if (lane == 0) pmask[wv] = bw;
 					__syncthreads();
-					unsigned long long bal = 0;  // bit p: point p departs
-					for (int w = 0; w < 4; w++) {
-						const unsigned long long x = pmask[w];
-						for (int k = 0; k < 16; k++) bal |= ((x >> (4 * k)) & 1ull) << (16 * w + k);
-					}
+					const unsigned long long bal = __ballot(lane < m && pbrk[lane]);
 					if (bal) {
 						const int j = __ffsll((long long)bal) - 1;
 						dff = pdff[j];
+						calm = 0;
 						// the state after the 3 (j + 1) draws the reference made
 						v3_advance(st, sk, seq, 3 * (j + 1), tid);
 						break;
@@ -2036,78 +2469,40 @@ __global__ __launch_bounds__(4 * kWave) void k_v3_commit(DScene S, DRecv R, V3De
 				}
 				if (dff < V.delta_ff) continue;  // CalRadiosity with the vertices' form factors
 			}
-			// PartitionTriangleWithCenterAndStore (shade.cpp:261-306)
-			if (trinum + 4 >= limit || (double)area < 1e-8) continue;
-			Patch src;
-			v3_load(V, R, r, src);
-			float maxl = 0.0f, minl = 1e+30f;
-			for (int v = 0; v < 3; v++) {
-				const int w = (v + 1) % 3;
-				const float lx = src.p[w][0] - src.p[v][0], ly = src.p[w][1] - src.p[v][1], lz = src.p[w][2] - src.p[v][2];
-				const float len = dot3<F>(lx, ly, lz, lx, ly, lz);
-				maxl = (maxl < len) ? len : maxl;
-				minl = (len < minl) ? len : minl;
-			}
-			if ((double)(minl / maxl) < 1e-1 || minl < 1) continue;
-			if (src.parent != r && r < V.n_orig) {
-				// the split would rewrite an original the octree lists (a slot
-				// pre-partition overwrote): the rays of the later receivers
-				// would change mid-pass; not supported
+			const int size = v3_split_size<F>(V, r);
+			if (size < 0) {
 				if (tid == 0) L->v3_error = r + 1;
 				stop = true;
 				break;
 			}
-			const int id[3] = {trinum, trinum + 1, trinum + 2};
-			Patch t[3];
-			for (int k = 0; k < 3; k++) {
-				t[k] = src;
-				for (int x = 0; x < 3; x++) t[k].p[k][x] = src.c[x];
-				v3_center<F>(t[k].p, t[k].c);
-				v3_area<F>(t[k]);
+			if (tid == 0 && size > 0) {
+				v3_split<F>(V, R, r, trinum);
+				if (size == 2) V.f3[nf3++] = r;
 			}
-			t[0].neighbor[0] = id[2], t[0].neighbor[2] = id[1];
-			t[1].neighbor[1] = id[0], t[1].neighbor[0] = id[2];
-			t[2].neighbor[2] = id[1], t[2].neighbor[1] = id[0];
-			if (tid == 0) {
-				v3_store(V, R, id[0], t[0]);
-				v3_store(V, R, id[1], t[1]);
-			}
-			if (src.parent == r) {
-				// an original becomes logical; its three parts are shaded next pass
-				if (tid == 0) {
-					v3_store(V, R, id[2], t[2]);
-					src.parent = -1;
-					v3_store(V, R, r, src);
-				}
-				trinum += 3;
-				V.act[r] = V3_NONE;
-			} else {
-				// slot r holds the third part (the last slot is given back), its
-				// centroid corner shaded anew (shade.cpp:508-520)
-				if (tid == 0) v3_store(V, R, r, t[2]);
-				trinum += 2;
-				const Patch &t3 = t[2];
-				const float nlen = __builtin_sqrtf(dot3<F>(t3.n[0], t3.n[1], t3.n[2], t3.n[0], t3.n[1], t3.n[2]));
-				float f3 = 0.0f;
-				if (tid < 4)
-					f3 = adapt_ff4<F>(S, s, t3.n[0], t3.n[1], t3.n[2], nlen, src.parent, t3.p[2][0], t3.p[2][1], t3.p[2][2],
-					                  q, c);
-				if (tid == 0) V.ff[4 * (size_t)r + 2] = f3;
-			}
-			__syncthreads();
+			trinum += size;
 		}
 	}
 	__syncthreads();
+	for (int i = tid >> 4; i < nf3; i += kV3Commit / 16) {
+		const int r = V.f3[i];
+		const Patch &t = V.pool[r];
+		const float nlen = __builtin_sqrtf(dot3<F>(t.n[0], t.n[1], t.n[2], t.n[0], t.n[1], t.n[2]));
+		const float f =
+			adapt_ff<F, 8>(S, s, t.n[0], t.n[1], t.n[2], nlen, t.parent, t.p[2][0], t.p[2][1], t.p[2][2], q, c);
+		if (q == 0) V.ff[4 * (size_t)r + 2] = f;
+	}
 	if (tid < 34) L->rng[tid] = st[tid];
 	if (tid == 0) {
-		L->rng_k = sk;
+		L->rng_k = 0;
 		L->trinum = trinum;
-		// the next pass: the slots this one made
-		L->v3_range[par ^ 1][0] = r1;
-		L->v3_range[par ^ 1][1] = trinum;
+		// the next pass: the slots this one made, or the rest of this one
+		L->v3_resume = again ? rest : 0;
+		L->v3_short = again && brief && !ordered;
+		L->v3_range[par ^ 1][0] = again ? L->v3_range[par][0] : r1;
+		L->v3_range[par ^ 1][1] = again ? r1 : trinum;
 	}
 	const int vals[8] = {c.rays, c.ref_rays, c.cells, c.tests, c.levels, c.precision, c.stalled, 0};
-	add_block_counters<4>(vals, bcnt);
+	add_block_counters<kV3Commit / kWave>(vals, bcnt);
 }
 
 // CalRadiosity (shade.cpp:244-259) of receiver r with its form factors V.ff
@@ -2135,31 +2530,26 @@ __device__ __forceinline__ void v3_receive(const DRecv &R, const V3Dev &V, const
 }
 
 // ... for the receivers of the pass that keep their form factors, one lane
-// each
-__global__ __launch_bounds__(kBlock) void k_v3_apply(DRecv R, V3Dev V, Loop *L, int par)
-{
-	if (L->done || L->v3_error) return;
-	const int r0 = L->v3_range[par][0], r1 = L->v3_range[par][1];
-	for (int r = r0 + blockIdx.x * kBlock + threadIdx.x; r < r1; r += gridDim.x * kBlock)
-		if (V.act[r] == V3_APPLY) v3_receive(R, V, L->src[0], r);
-}
-
-// the best candidate over the slots in use (listCanditate with one source,
-// rad.cpp:387-404: the highest slot on ties), once the passes are over: the
-// next pass (parity par) has no slot; else v3_pending makes the next
-// iteration's k_v3_prep leave the source as it is, for that pass
-__global__ __launch_bounds__(kBlock) void k_v3_select(DRecv R, Loop *L, float converge, int par)
+// each; and, once the passes are over (the next one, of parity par ^ 1, has no
+// slot), the best candidate over the slots in use (listCanditate with one
+// source, rad.cpp:387-404: the highest slot on ties), a slot's own lane having
+// updated it; else v3_pending makes the next launches keep the source, for
+// that pass
+__global__ __launch_bounds__(kBlock) void k_v3_finish(DRecv R, V3Dev V, Loop *L, float converge, int par)
 {
 	__shared__ unsigned long long wmax[kWavesPerBlock];
 	__shared__ int wn[kWavesPerBlock];
 	if (L->done || L->v3_error) return;
-	const bool pending = L->v3_range[par][0] < L->v3_range[par][1];
+	const int r0 = L->v3_range[par][0], r1 = L->v3_range[par][1];
+	const bool pending = L->v3_range[par ^ 1][0] < L->v3_range[par ^ 1][1];
 	if (blockIdx.x == 0 && threadIdx.x == 0) L->v3_pending = pending;
-	if (pending) return;
+	if (L->v3_resume) return;  // the pass goes on
 	unsigned long long key = 0;
 	int n = 0;
-	for (int r = blockIdx.x * kBlock + threadIdx.x; r < L->trinum; r += gridDim.x * kBlock) {
-		if (__float_as_int(R.nrm[r].w) < 0) continue;
+	const int lo = pending ? r0 : 0, hi = pending ? r1 : L->trinum;
+	for (int r = lo + blockIdx.x * kBlock + threadIdx.x; r < hi; r += gridDim.x * kBlock) {
+		if (r >= r0 && r < r1 && V.act[r] == V3_APPLY) v3_receive(R, V, L->src[0], r);
+		if (pending || __float_as_int(R.nrm[r].w) < 0) continue;
 		const float4 db = R.dB[r];
 		const float sum = db.x + db.y + db.z;
 		if (sum > converge) {
@@ -2412,6 +2802,7 @@ struct DeviceEngine::Impl {
 	bool v3 = false;
 	V3Dev V = {};
 	DevBuf<float> v3ff;
+	DevBuf<int> v3plan;
 	DevBuf<unsigned char> v3act;
 	hipEvent_t ev0 = nullptr, ev1 = nullptr;
 	Stage stage;
@@ -2625,7 +3016,7 @@ int DeviceEngine::upload(const HostScene &s, const FlatOctree &t, std::string &e
 	}
 	const int grid = ((d.nblocks + 7) / 8) * 8;  // a whole number of blocks per XCD
 	const int tgrid = ((d.trace_nblocks + 7) / 8) * 8;
-	const int v3grid = d.v3 ? (int)(((size_t)cap * 4 + kBlock - 1) / kBlock) : 0;
+	const int v3grid = d.v3 ? v3_gen_blocks((size_t)std::max(cap, 1)) : 0;
 	std::vector<long long> zeros((size_t)std::max(std::max(grid, tgrid), v3grid) * 8, 0);
 	if (d.bcnt.put(zeros.data(), zeros.size(), st, err)) return -1;
 	if (!d.lowest && d.parallel_src > 1 && d.cand.alloc((size_t)n + 1, err)) return -1;
@@ -2636,9 +3027,17 @@ int DeviceEngine::upload(const HostScene &s, const FlatOctree &t, std::string &e
 	d.host_loop->trinum = n;
 	glibc_rand_start(d.host_loop->rng);  // rand() is first called in the solve (shade.cpp:53)
 	if (d.v3) {
-		if (d.v3ff.alloc((size_t)cap * 4 + 4, err) || d.v3act.alloc((size_t)cap + 1, err)) return -1;
+		const size_t nplan = (size_t)cap + 1;  // a word list: plan entries, groups, their results and counters, slots, rand()
+		if (d.v3ff.alloc((size_t)cap * 4 + 4, err) || d.v3act.alloc((size_t)cap + 1, err) ||
+		    d.v3plan.alloc(nplan * 5 + (size_t)kV3Subs * 12 + 34 + kV3Ahead, err))
+			return -1;
+		int *w = d.v3plan.p;
+		int4 *ent = (int4 *)w;
+		int *cnt = w + 4 * nplan;
+		int2 *sub = (int2 *)(cnt + 8 * (size_t)kV3Subs), *out = sub + kV3Subs;
+		int *f3 = (int *)(out + kV3Subs);
 		d.V = V3Dev{d.pool.p, d.v3ff.p, d.v3act.p, std::min(s.o.max_tri, s.o.triangle), n0, s.o.adapt_area,
-		            s.o.sample_area, s.o.delta_ff};
+		            s.o.sample_area, s.o.delta_ff, (unsigned *)(f3 + nplan), ent, sub, out, cnt, f3};
 	}
 	// -parallel_src 0: listCanditate returns no source (rad.cpp:400), so the
 	// first iteration finds nothing to shoot
@@ -2696,19 +3095,20 @@ int DeviceEngine::shoot(int max_shots, int *shots, int *converged, std::string &
 		auto slot = [&]() {
 			const int p = d.v3_par;
 			const size_t nt = (size_t)std::max(d.host_loop->trinum, 1);  // as last read back
-			const dim3 g((unsigned)std::min<size_t>((nt * 16 + kBlock - 1) / kBlock, 4096));
-			const dim3 ga((unsigned)std::min<size_t>((nt + kBlock - 1) / kBlock, 1024)), blk(kBlock);
+			const dim3 g((unsigned)v3_gen_blocks(nt) + kV3RunBlocks), one(kV3Commit), blk(kBlock);
+			const dim3 gs(kV3SpecBlocks), gf((unsigned)std::min<size_t>((nt + kBlock - 1) / kBlock, 1024));
 			if (d.fma) {
-				hipLaunchKernelGGL(k_v3_prep<true>, dim3(1), dim3(64), 0, st, d.R, d.loop.p, p);
 				hipLaunchKernelGGL(k_v3_gen<true>, g, blk, 0, st, d.S, d.R, d.V, d.loop.p, p, d.bcnt.p);
-				hipLaunchKernelGGL(k_v3_commit<true>, dim3(1), dim3(4 * kWave), 0, st, d.S, d.R, d.V, d.loop.p, p, d.bcnt.p);
+				hipLaunchKernelGGL(k_v3_plan, dim3(1), one, 0, st, d.R, d.V, d.loop.p, p);
+				hipLaunchKernelGGL(k_v3_spec<true>, gs, dim3(kV3Sub * 16), 0, st, d.S, d.R, d.V, d.loop.p);
+				hipLaunchKernelGGL(k_v3_commit<true>, dim3(1), one, 0, st, d.S, d.R, d.V, d.loop.p, p, d.bcnt.p);
 			} else {
-				hipLaunchKernelGGL(k_v3_prep<false>, dim3(1), dim3(64), 0, st, d.R, d.loop.p, p);
 				hipLaunchKernelGGL(k_v3_gen<false>, g, blk, 0, st, d.S, d.R, d.V, d.loop.p, p, d.bcnt.p);
-				hipLaunchKernelGGL(k_v3_commit<false>, dim3(1), dim3(4 * kWave), 0, st, d.S, d.R, d.V, d.loop.p, p, d.bcnt.p);
+				hipLaunchKernelGGL(k_v3_plan, dim3(1), one, 0, st, d.R, d.V, d.loop.p, p);
+				hipLaunchKernelGGL(k_v3_spec<false>, gs, dim3(kV3Sub * 16), 0, st, d.S, d.R, d.V, d.loop.p);
+				hipLaunchKernelGGL(k_v3_commit<false>, dim3(1), one, 0, st, d.S, d.R, d.V, d.loop.p, p, d.bcnt.p);
 			}
-			hipLaunchKernelGGL(k_v3_apply, ga, blk, 0, st, d.R, d.V, d.loop.p, p);
-			hipLaunchKernelGGL(k_v3_select, ga, blk, 0, st, d.R, d.loop.p, d.converge, p ^ 1);
+			hipLaunchKernelGGL(k_v3_finish, gf, blk, 0, st, d.R, d.V, d.loop.p, d.converge, p);
 			d.v3_par = p ^ 1;
 		};
 		auto read_back = [&]() -> int {
