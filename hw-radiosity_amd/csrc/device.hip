@@ -23,8 +23,9 @@
 //             block's ray count;
 //   k_compact the rays as a dense list in the receivers' spatial order,
 //             grouped by origin key within a block; it also clears the
-//             source's deltaB and the key (at most 8192 slots: no list,
-//             k_trace_direct traces each ray position in place);
+//             source's deltaB and the key (at most 8192 slots: no list;
+//             k_shoot does k_gen's work and traces each ray position in
+//             place, k_trace_direct with several sources);
 //   k_trace   two lanes per ray (four and eight over the end of each XCD's
 //             share, or for few rays): RayHitted (raycast.cpp:335-360); a
 //             ray that misses the source zeroes its form factor;
@@ -160,6 +161,10 @@ struct Loop {
 	int v3_pending;  // the last pass made new slots: another pass before the selection
 	unsigned rng[34];
 	SrcDesc src[kMaxSrc];
+	// k_shoot: the sources taken, and as k_update last saw it; the key of an odd
+	// one (key: an even one's)
+	int taken, updated;
+	unsigned long long key_odd;
 	int v3_range[2][2];  // V3: the slots [r0, r1) of the pass of each parity
 	// V3: the pass's plan (k_v3_plan): its entries and their groups of sample
 	// points, the first receiver past them, the first entry with a departing
@@ -203,13 +208,23 @@ template <bool LOWEST> __device__ __forceinline__ int key_slot(unsigned long lon
 	return LOWEST ? (int)(0xffffffffu - lo) : (int)lo;
 }
 
+// maximum over the wave, in every lane: as wave_scan below (lanes without a
+// source give 0), the upper halves and then the lower ones of the lanes that
+// have the largest upper half
+__device__ __forceinline__ unsigned wave_max(unsigned x)
+{
+	x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, false));
+	x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, false));
+	x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, false));
+	x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, false));
+	x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x142, 0xa, 0xf, false));
+	x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x143, 0xc, 0xf, false));
+	return (unsigned)__builtin_amdgcn_readlane((int)x, 63);
+}
 __device__ __forceinline__ unsigned long long wave_max(unsigned long long k)
 {
-	for (int off = 32; off > 0; off >>= 1) {
-		const unsigned long long o = __shfl_xor(k, off);
-		k = o > k ? o : k;
-	}
-	return k;
+	const unsigned hi = (unsigned)(k >> 32), top = wave_max(hi);
+	return (unsigned long long)top << 32 | wave_max(hi == top ? (unsigned)k : 0u);
 }
 // prefix sums over the wave, a lane's own value included: within rows of 16
 // lanes (DPP row_shr 1, 2, 4, 8; lanes without a source add 0), then across
@@ -475,7 +490,7 @@ __device__ int walk(const DScene &S, float px, float py, float pz, float vx, flo
 //    is tested;
 //  - the hits are combined by DPP, and only where a lane has one.
 // The 2120-slot room, 5 leaves a ray and up to 17 in a launch: k_trace_direct
-// 24.2 -> 17.2 us with it (that needs its 90 VGPRs: held to 80 it spills and
+// (now in k_shoot) 24.2 -> 17.2 us with it (that needs its 90 VGPRs: held to 80 it spills and
 // gains nothing), 3001 rays cast 23.7 -> 16.9 us. Where waves enough are in
 // flight to hide the chain it gives nothing: the hall's k_trace 195 us with
 // walk, 198 with this, 98000 rays there at four lanes 91 and 100 us.
@@ -1114,7 +1129,7 @@ __global__ __launch_bounds__(kBlock) void k_ray_keys(DScene S, DRecv R, int nv, 
 // hall against one lane per ray (242 us) and four (239 us), two take 227 us,
 // the list loop's lanes being busier than the walk's doubled steps cost; on
 // the 2120-slot room eight lanes took an iteration from 49.4 to 48.4 us (its
-// launches now go to k_trace_direct).
+// launches now go to k_shoot).
 __host__ __device__ __forceinline__ int lanes_per_ray(int nr)
 {
 	return 8LL * nr <= kTraceSlots ? 8 : 4LL * nr <= kTraceSlots ? 4 : 2;
@@ -1215,20 +1230,14 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(6, 
 // positions fits the machine at eight lanes per ray (48 n <= kTraceSlots):
 // lane group q (eight lanes) takes position q of k_compact's order, lane
 // i = 6 order[q / 6] + q % 6, and traces it if rcode marks a ray there.
-// There are lane groups to spare, so the list and its launch buy nothing;
-// what k_compact does besides (the key and the source's deltaB with PREP)
-// block 0 does here.
+// There are lane groups to spare, so the list and its launch buy nothing.
+// For several sources per iteration; one goes to k_shoot.
 template <bool F>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_trace_direct(
-	DScene S, DRecv R, Loop *L, int k, float *ffbuf, long long *bcnt, const unsigned char *rcode, int nlanes,
-	float4 *dB, int prep)
+	DScene S, DRecv R, Loop *L, int k, float *ffbuf, long long *bcnt, const unsigned char *rcode, int nlanes)
 {
 	if (L->done || k >= L->nsrc) return;
 	const SrcDesc &s = L->src[k];
-	if (prep && blockIdx.x == 0 && threadIdx.x == 0) {
-		L->key = 0;
-		dB[s.phys] = make_float4(0.f, 0.f, 0.f, 0.f);
-	}
 	const int q = blockIdx.x * (kTraceBlock / 8) + (int)threadIdx.x / 8, sub = (int)threadIdx.x & 7;
 	Cnt c = {0, 0, 0, 0, 0, 0, 0};
 	if (q < nlanes && ((rcode[q >> 1] >> (q & 1)) & 1)) {
@@ -1253,13 +1262,88 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4, 
 	add_block_counters<kTraceBlock / kWave>(vals, bcnt);
 }
 
+// k_gen and k_trace_direct in one launch, for one source per iteration: each
+// lane group selects the source (its loads are the same everywhere), takes its
+// own position's form-factor prefix (k_gen's, above) and traces its ray.  The
+// key it reads is zeroed, and the source's deltaB with it, by k_update, which
+// collects the next key beside it (by the parity of the sources taken).
+// What bounds it is one chain: the key, the source, the prefix, the walk.
+// The 2120-slot room, us per iteration: 26.5 in two launches, 22.4 in one.
+template <bool F, bool LOWEST>
+__global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_shoot(
+	DScene S, DRecv R, Loop *L, unsigned char *live, float *ffbuf, long long *bcnt, int nlanes)
+{
+	if (L->done) return;
+	const int before = L->updated;
+	const unsigned long long key = before & 1 ? L->key_odd : L->key;
+	const int q = blockIdx.x * (kTraceBlock / 8) + (int)threadIdx.x / 8, sub = (int)threadIdx.x & 7;
+	const bool valid = q < nlanes;
+	const int i = valid ? 6 * R.order[q / 6] + q % 6 : 0;
+	const int sv = i >> 1, h = i & 1, r = sv / 3;
+	const float4 nr = R.nrm[r];
+	const float px = R.vx[sv], py = R.vy[sv], pz = R.vz[sv];
+	const float4 acc = R.acc[3 * r + min(sub, 2)];
+	if (key == 0) {
+		if (blockIdx.x == 0 && threadIdx.x == 0) L->done = 1;
+		return;
+	}
+	const int src = __builtin_amdgcn_readfirstlane(key_slot<LOWEST>(key));
+	SrcDesc s;
+	make_source<F>(R, src, s);
+	if (blockIdx.x == 0 && threadIdx.x == 0) {
+		L->src[0] = s;
+		L->nsrc = 1;
+		L->shots++;
+		L->ncand = 0;
+		L->taken = before + 1;
+	}
+	const int parent = __float_as_int(nr.w);
+	const unsigned long long sat = __ballot(!(acc.x < 255.0f || acc.y < 255.0f || acc.z < 255.0f));
+	const bool full = ((sat >> ((int)threadIdx.x & ~7)) & 7) == 7;
+	const bool lv = valid && parent >= 0 && r != src && !full;
+	Cnt c = {0, 0, 0, 0, 0, 0, 0};
+	float f = 0.0f;
+	if (lv && (h == 0 || s.split)) {
+		SrcPatch sp = s.whole;
+		const float nlen = __builtin_sqrtf(dot3<F>(nr.x, nr.y, nr.z, nr.x, nr.y, nr.z));
+		if (s.split) {
+			// the full-source ray AdaptCalFF computes and then discards
+			if (h == 0 && sub == 0 && ff_prefix_nonzero<F>(s.whole, nr.x, nr.y, nr.z, nlen, px, py, pz)) c.ref_rays++;
+			sp.area = h ? s.half[1].area : s.half[0].area;
+			for (int x = 0; x < 3; x++) sp.c[x] = h ? s.half[1].c[x] : s.half[0].c[x];
+		}
+		f = ff_prefix<F>(sp, nr.x, nr.y, nr.z, nlen, px, py, pz);
+		if (f != 0.0f) {
+			Cnt w = {0, 0, 0, 0, 0, 0, 0};
+			const int hit = walk_ahead<F>(S, px, py, pz, sp.c[0] - px, sp.c[1] - py, sp.c[2] - pz, parent, w, sub);
+			c.tests = w.tests;
+			if (sub == 0) {
+				c.rays = 1;
+				c.ref_rays++;
+				c.cells = w.cells;
+				c.levels = w.levels;
+				c.precision = w.precision;
+				c.stalled = w.stalled;
+			}
+			f = hit == s.log ? f : 0.0f;
+		}
+	}
+	if (valid && sub == 0) {
+		ffbuf[i] = f;
+		if (q % 6 == 0) live[r] = (unsigned char)(lv | (parent >= 0) << 1);
+	}
+	const int vals[8] = {c.rays, c.ref_rays, c.cells, c.tests, c.levels, c.precision, c.stalled, 0};
+	add_block_counters<kTraceBlock / kWave>(vals, bcnt);
+}
+
 // Source k, part 3: CalRadiosity (shade.cpp:244-259) per receiver, its
 // three vertex lanes combined by shuffles in the reference's order; after
 // the last source the next iteration's candidate key (listCanditate,
 // rad.cpp:387-404) by wave, block and one 64-bit atomicMax per block.
 template <bool F, bool FUSED_SELECT, bool LOWEST, int G>
 __global__ __launch_bounds__(kBlock) void k_update(DRecv R, Loop *L, int k, const unsigned char *live,
-                                                   const float *ffbuf, float converge, long long *bcnt, int nblocks)
+                                                   const float *ffbuf, float converge, long long *bcnt, int nblocks,
+                                                   bool shoot)
 {
 	if (L->done || k >= L->nsrc) return;
 	__shared__ unsigned long long wmax[kWavesPerBlock];
@@ -1289,7 +1373,9 @@ __global__ __launch_bounds__(kBlock) void k_update(DRecv R, Loop *L, int k, cons
 		const float r1 = __shfl(dr, m.base + 1), g1 = __shfl(dg, m.base + 1), b1 = __shfl(dbb, m.base + 1);
 		const float r2 = __shfl(dr, m.base + 2), g2 = __shfl(dg, m.base + 2), b2 = __shfl(dbb, m.base + 2);
 		float4 db = make_float4(0.f, 0.f, 0.f, 0.f);
-		if (valid && m.v == 0) db = R.dB[r];
+		const bool own = shoot && valid && m.v == 0 && r == s.phys;  // the source's unshot energy, as k_shoot left it
+		if (valid && m.v == 0 && !own) db = R.dB[r];
+		if (own) R.dB[r] = db;
 		if (lv) {
 			float4 acc = R.acc[sv];
 			acc.x += dr;
@@ -1329,8 +1415,14 @@ __global__ __launch_bounds__(kBlock) void k_update(DRecv R, Loop *L, int k, cons
 			key = wmax[w] > key ? wmax[w] : key;
 			ncand += wn[w];
 		}
-		if (FUSED_SELECT && key) atomicMax(&L->key, key);
+		// after k_shoot the next key goes beside the one it took, zeroed here
+		const bool odd = shoot && (L->taken & 1);
+		if (FUSED_SELECT && key) atomicMax(odd ? &L->key_odd : &L->key, key);
 		if (ncand) atomicAdd(&L->ncand, ncand);
+		if (shoot && blockIdx.x == 0) {
+			*(odd ? &L->key : &L->key_odd) = 0;
+			L->updated = L->taken;
+		}
 	}
 }
 
@@ -3163,6 +3255,7 @@ int DeviceEngine::shoot(int max_shots, int *shots, int *converged, std::string &
 	// every ray position fits the machine at eight lanes per ray: no dense list
 	const bool direct = 48LL * d.R.nslots <= kTraceSlots;
 	const int dgrid = (int)((6LL * d.R.nslots + kTraceBlock / 8 - 1) / (kTraceBlock / 8));
+	const bool shoot = direct && prep;  // one source, too few rays for a list: k_gen and the trace in one launch
 	auto iteration = [&](int ev) {
 		if (multi) {
 			hipLaunchKernelGGL(k_collect, dim3(cb > 0 ? cb : 1), dim3(kBlock), 0, st, d.R, d.loop.p, d.cand.p, d.converge);
@@ -3191,13 +3284,22 @@ int DeviceEngine::shoot(int max_shots, int *shots, int *converged, std::string &
 					hipLaunchKernelGGL(k_compact<G>, dim3(d.nblocks), blk, 0, st, d.loop.p, k, d.rcode.p, d.order.p,
 					                   6 * d.R.nslots, d.raycnt.p, d.nblocks, d.rays.p, d.dB.p, prep);
 			};
-			if (d.groups == 1) gen(std::integral_constant<int, 1>{});
-			else gen(std::integral_constant<int, 2>{});
+			if (shoot) {
+			} else if (d.groups == 1) {
+				gen(std::integral_constant<int, 1>{});
+			} else {
+				gen(std::integral_constant<int, 2>{});
+			}
 			if (ev >= 0 && k == 0) (void)hipEventRecord(d.kev[2 * ev], st);
-			if (direct) {
-				const dim3 dg((unsigned)dgrid);
-				if (d.fma) hipLaunchKernelGGL(k_trace_direct<true>, dg, dim3(kTraceBlock), 0, st, d.S, d.R, d.loop.p, k, d.ffbuf.p, d.bcnt.p, d.rcode.p, 6 * d.R.nslots, d.dB.p, prep);
-				else hipLaunchKernelGGL(k_trace_direct<false>, dg, dim3(kTraceBlock), 0, st, d.S, d.R, d.loop.p, k, d.ffbuf.p, d.bcnt.p, d.rcode.p, 6 * d.R.nslots, d.dB.p, prep);
+			const dim3 dg((unsigned)dgrid), db(kTraceBlock);
+			if (shoot) {
+#define SHOOT(F, LO) hipLaunchKernelGGL((k_shoot<F, LO>), dg, db, 0, st, d.S, d.R, d.loop.p, d.live.p, d.ffbuf.p, d.bcnt.p, 6 * d.R.nslots)
+				if (d.fma) { if (prep == 2) SHOOT(true, true); else SHOOT(true, false); }
+				else { if (prep == 2) SHOOT(false, true); else SHOOT(false, false); }
+#undef SHOOT
+			} else if (direct) {
+				if (d.fma) hipLaunchKernelGGL(k_trace_direct<true>, dg, db, 0, st, d.S, d.R, d.loop.p, k, d.ffbuf.p, d.bcnt.p, d.rcode.p, 6 * d.R.nslots);
+				else hipLaunchKernelGGL(k_trace_direct<false>, dg, db, 0, st, d.S, d.R, d.loop.p, k, d.ffbuf.p, d.bcnt.p, d.rcode.p, 6 * d.R.nslots);
 			} else if (d.fma) {
 				hipLaunchKernelGGL(k_trace<true>, tg, dim3(kTraceBlock), 0, st, d.S, d.R, d.loop.p, k, d.ffbuf.p, d.bcnt.p, d.rays.p);
 			} else {
@@ -3206,7 +3308,7 @@ int DeviceEngine::shoot(int max_shots, int *shots, int *converged, std::string &
 			if (ev >= 0 && k == 0) (void)hipEventRecord(d.kev[2 * ev + 1], st);
 			auto update = [&](auto gc) {
 				constexpr int G = decltype(gc)::value;
-#define UPD(F, FS, LO) hipLaunchKernelGGL((k_update<F, FS, LO, G>), g, blk, 0, st, d.R, d.loop.p, k, d.live.p, d.ffbuf.p, d.converge, d.bcnt.p, d.nblocks)
+#define UPD(F, FS, LO) hipLaunchKernelGGL((k_update<F, FS, LO, G>), g, blk, 0, st, d.R, d.loop.p, k, d.live.p, d.ffbuf.p, d.converge, d.bcnt.p, d.nblocks, shoot)
 				if (multi) { if (d.fma) UPD(true, false, false); else UPD(false, false, false); }
 				else if (d.lowest) { if (d.fma) UPD(true, true, true); else UPD(false, true, true); }
 				else { if (d.fma) UPD(true, true, false); else UPD(false, true, false); }
