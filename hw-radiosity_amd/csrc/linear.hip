@@ -239,16 +239,36 @@ __global__ __launch_bounds__(512) void k_gemm_dma(const E *__restrict__ A, const
 			}
 }
 
-// The sweep's second half after k_gemm_dma: its split-K partials summed in order
-template <typename E> __global__ void k_finish(const float *part, int S, int ld, int rp, SweepOut<E> o)
+// The element-wise kernels take R rows of one column per thread, columns across
+// the lanes (unit u -> rows [i, i + R) of column c).  R = 8 from 2^19 elements
+// up: the row-major arrays are read a line at a time, and a column's rows, 16
+// bytes of a fragment (frag_index) or 64 of the FP64 iterate, are one access
+// where an element per thread touches as many lines as lanes.  Below, one: there
+// it is threads that are short.  us at (n, columns), one row and eight: k_resid
+// (1000, 6) 5.5, 7.8; (4000, 96) 9.8, 9.4; (6000, 192) 27.5, 22.6; k_finish
+// (1000, 96) 4.1, 4.8; (4000, 96) 4.8, 4.8; (6000, 192) 14.8, 10.3; k_scale
+// (20000, 3) 2.9, 4.3; (4000, 96) 3.6, 5.2; (6000, 192) 7.2, 6.1.
+constexpr size_t kWide = (size_t)1 << 19;
+constexpr size_t row_units(int R, int n, int nrhs) { return (size_t)((n + R - 1) / R) * nrhs; }
+
+// The sweep's second half after k_gemm_dma: its split-K partials summed in
+// order.  Bound by the partials' and vectors' traffic: n = 7777, 192 columns, 8
+// partials, 17.2 us with one row, 11.8 (5.3 TB/s) with eight.
+template <typename E, int R>
+__global__ __launch_bounds__(kB) void k_finish(const float *part, int S, int ld, int rp, SweepOut<E> o)
 {
-	const size_t total = (size_t)o.n * o.nrhs;
-	for (size_t t = blockIdx.x * (size_t)kB + threadIdx.x; t < total; t += (size_t)gridDim.x * kB) {
-		const int i = (int)(t / o.nrhs), c = (int)(t % o.nrhs);
-		float y = 0.f;
-		for (int s = 0; s < S; s++) y += part[((size_t)s * ld + i) * rp + c];
-		o.put(i, c, ld, y);
-	}
+	const size_t u = blockIdx.x * (size_t)kB + threadIdx.x;
+	if (u >= row_units(R, o.n, o.nrhs)) return;
+	const int i = (int)(u / o.nrhs) * R, c = (int)(u % o.nrhs), m = min(R, o.n - i);
+	float y[R] = {};
+	const float *p = part + (size_t)i * rp + c;  // whole row groups: ld is a multiple of 256
+	for (int s = 0; s < S; s++)
+#pragma unroll
+		for (int r = 0; r < R; r++) y[r] += p[((size_t)s * ld + r) * rp];
+	E x[R];
+#pragma unroll
+	for (int r = 0; r < R; r++) x[r] = r < m ? o.value(i + r, c, ld, y[r]) : (E)0.f;
+	if (!o.y) put_frag<R>(o.XTn, c, i, ld, x);
 }
 
 // Split-K partials part[s][row][col] (FP64) of F X, summed in a fixed order
@@ -363,21 +383,32 @@ __global__ __launch_bounds__(kB) void k_fx64v(const float *__restrict__ F, const
 // out[i][c] = base[i][c] + rho[i][c] * y - xT[c][i], y = the split-K sum of
 // part (FP64, fixed order); base, rho and xT may be null (0, 1 and 0).  Per
 // block: sum of squares and max |out|.
+template <int R>
 __global__ __launch_bounds__(kB) void k_resid(const double *part, int S, int ld, int rp, int n, int nrhs,
                                               const double *xT, const double *base, const double *rho, double *out,
                                               double *blk)
 {
-	const size_t total = (size_t)n * nrhs;
-	const size_t t = blockIdx.x * (size_t)kB + threadIdx.x;
+	const size_t u = blockIdx.x * (size_t)kB + threadIdx.x;
 	double ss = 0.0, mx = 0.0;
-	if (t < total) {
-		const int i = (int)(t / nrhs), c = (int)(t % nrhs);
-		double y = 0.0;
-		for (int q = 0; q < S; q++) y += part[((size_t)q * ld + i) * rp + c];
-		const double v = (base ? base[t] : 0.0) + (rho ? rho[t] : 1.0) * y - (xT ? xT[(size_t)c * ld + i] : 0.0);
-		out[t] = v;
-		ss = v * v;
-		mx = fabs(v);
+	if (u < row_units(R, n, nrhs)) {
+		const int i = (int)(u / nrhs) * R, c = (int)(u % nrhs), m = min(R, n - i);
+		double y[R] = {}, x[R] = {};
+		const double *p = part + (size_t)i * rp + c;
+		for (int q = 0; q < S; q++)
+#pragma unroll
+			for (int r = 0; r < R; r++) y[r] += p[((size_t)q * ld + r) * rp];
+		if (xT)
+#pragma unroll
+			for (int r = 0; r < R; r++) x[r] = xT[(size_t)c * ld + i + r];
+#pragma unroll
+		for (int r = 0; r < R; r++) {
+			if (r >= m) break;
+			const size_t t = (size_t)(i + r) * nrhs + c;
+			const double v = (base ? base[t] : 0.0) + (rho ? rho[t] : 1.0) * y[r] - x[r];
+			out[t] = v;
+			ss += v * v;
+			mx = fmax(mx, fabs(v));
+		}
 	}
 	for (int off = 32; off > 0; off >>= 1) {
 		ss += __shfl_xor(ss, off);
@@ -395,16 +426,23 @@ __global__ __launch_bounds__(kB) void k_resid(const double *part, int S, int ld,
 	}
 }
 
-// r32 = r64 / s; XT (if given) <- r32 in fragment order
-template <typename E>
-__global__ void k_scale(const double *r64, double inv_s, size_t total, int nrhs, int ld, float *r32, E *XT,
-                        const float *rho_in = nullptr)
+// r32 = r64 / s; XT <- r32 (times rho_in, if given) in fragment order
+template <typename E, int R>
+__global__ __launch_bounds__(kB) void k_scale(const double *r64, double inv_s, int n, int nrhs, int ld, float *r32, E *XT,
+                                              const float *rho_in)
 {
-	for (size_t t = blockIdx.x * (size_t)kB + threadIdx.x; t < total; t += (size_t)gridDim.x * kB) {
+	const size_t u = blockIdx.x * (size_t)kB + threadIdx.x;
+	if (u >= row_units(R, n, nrhs)) return;
+	const int i = (int)(u / nrhs) * R, c = (int)(u % nrhs), m = min(R, n - i);
+	E x[R];
+#pragma unroll
+	for (int r = 0; r < R; r++) {
+		const size_t t = (size_t)min(i + r, n - 1) * nrhs + c;
 		const float v = (float)(r64[t] * inv_s);
-		r32[t] = v;
-		if (XT) XT[frag_index((int)(t % nrhs), (int)(t / nrhs), ld)] = (E)(rho_in ? rho_in[t] * v : v);
+		if (r < m) r32[t] = v;
+		x[r] = r < m ? (E)(rho_in ? rho_in[t] * v : v) : (E)0.f;
 	}
+	put_frag<R>(XT, c, i, ld, x);
 }
 
 // rho32 <- rho and per block (grid-stride): sum of squares and max of |E|, the
@@ -844,6 +882,22 @@ int pick_ct(int nrhs)
 	return -1;
 }
 
+// go(integral constant R, grid) for an element-wise kernel over n x nrhs
+template <typename Go> void launch_rows(int n, int nrhs, Go go)
+{
+	auto grid = [&](int R) { return dim3((unsigned)((row_units(R, n, nrhs) + kB - 1) / kB)); };
+	if ((size_t)n * nrhs >= kWide) go(std::integral_constant<int, 8>{}, grid(8));
+	else go(std::integral_constant<int, 1>{}, grid(1));
+}
+template <typename E>
+void launch_scale(const double *r64, double inv_s, int n, int nrhs, int ld, float *r32, E *XT, const float *rho_in,
+                  hipStream_t st)
+{
+	launch_rows(n, nrhs, [&](auto r, dim3 g) {
+		hipLaunchKernelGGL((k_scale<E, decltype(r)::value>), g, dim3(kB), 0, st, r64, inv_s, n, nrhs, ld, r32, XT, rho_in);
+	});
+}
+
 // the wide kernels' tiles: split-K over blocks, partials in part
 bool dma_tile(int rt, int ct) { return ct >= 8 && rt >= 2; }
 
@@ -880,7 +934,9 @@ int launch_sweep(int rt, int ct, int S, const E *A, const E *XT, float *part, in
 		else if (rt == 4 && ct == 12) hipLaunchKernelGGL((k_gemm_dma<E, 12, 4, 2>), grid, blk, 0, st, A, XT, part, ld, rp, kchunk);
 		else return -1;
 		if (finish)
-			hipLaunchKernelGGL(k_finish<E>, dim3(grid_for((size_t)o.n * o.nrhs)), dim3(kB), 0, st, part, S, ld, rp, o);
+			launch_rows(o.n, o.nrhs, [&](auto r, dim3 g) {
+				hipLaunchKernelGGL((k_finish<E, decltype(r)::value>), g, dim3(kB), 0, st, part, S, ld, rp, o);
+			});
 		return 0;
 	}
 	const int wr = kSweepWaves / S * rt;  // row tiles per block
@@ -957,7 +1013,7 @@ struct Fx64 {
 			nblk = (size_t)ld / 32 * ks;
 		} else {
 			tile();
-			nblk = ((size_t)n * nrhs + kB - 1) / kB;
+			launch_rows(n, nrhs, [&](auto, dim3 g) { nblk = g.x; });
 			if (part.alloc((size_t)S * ld * rp, err)) return -1;
 		}
 		if (stage.stat_room(std::max<size_t>(nblk * 2, 3 * kStatBlocks), err)) return -1;
@@ -1022,8 +1078,10 @@ struct Fx64 {
 			else if (W == 4) hipLaunchKernelGGL((k_fx64m<1, 4, 4>), grid, threads, 0, st, F, wT, part.p, ld, rp, kchunk);
 			else if (rt == 1) hipLaunchKernelGGL((k_fx64m<1, 4, 8>), grid, threads, 0, st, F, wT, part.p, ld, rp, kchunk);
 			else hipLaunchKernelGGL((k_fx64m<2, 4, 8>), grid, threads, 0, st, F, wT, part.p, ld, rp, kchunk);
-			hipLaunchKernelGGL(k_resid, dim3((unsigned)nblk), dim3(kB), 0, st, part.p, S, ld, rp, n, nrhs, xT, base, rho,
-			                   out, blk);
+			launch_rows(n, nrhs, [&](auto r, dim3 g) {
+				hipLaunchKernelGGL(k_resid<decltype(r)::value>, g, dim3(kB), 0, st, part.p, S, ld, rp, n, nrhs, xT, base, rho,
+				                   out, blk);
+			});
 		}
 		HIP_OK(hipGetLastError(), "FP64 product");
 		ss = mx = 0.0;
@@ -1253,7 +1311,7 @@ struct LinearSystem::Impl {
 		if (begin(err) || iterates(x, xts, err) || w.r32.alloc(total, err) || w.E64.alloc(total, err) ||
 		    (dma_tile(rt, ct) && w.part.alloc((size_t)S * ld * rp, err)) || stage.up(w.E64.p, X, total * 8, st, err))
 			return -1;
-		hipLaunchKernelGGL(k_scale<E>, dim3(grid_for(total)), dim3(kB), 0, st, w.E64.p, 1.0, total, nrhs, ld, w.r32.p, x[0].p);
+		launch_scale(w.E64.p, 1.0, n, nrhs, ld, w.r32.p, x[0].p, nullptr, st);
 		SweepOut<E> o{};
 		o.n = n, o.nrhs = nrhs, o.inv = inv, o.y = w.r32.p;
 		if (launch_sweep<E>(rt, ct, S, A, x[0].p, w.part.p, ld, rp, o, st)) {
@@ -1533,8 +1591,7 @@ int LinearSystem::gather(int prec, int nrhs, const double *rho, const double *E,
 		int rc;
 		auto refine = [&](const auto *A, auto &X) {
 			typedef std::remove_cv_t<std::remove_pointer_t<decltype(A)>> T;
-			hipLaunchKernelGGL(k_scale<T>, dim3(g), dim3(kB), 0, st, outer ? w.r64.p : w.E64.p, 1.0 / s, total, nrhs, ld,
-			                   w.r32.p, X[0].p);
+			launch_scale(outer ? w.r64.p : w.E64.p, 1.0 / s, n, nrhs, ld, w.r32.p, X[0].p, nullptr, st);
 			SweepOut<T> o{};
 			o.n = n, o.nrhs = nrhs, o.inv = inv, o.rhs = w.r32.p, o.rho = w.rho32.p;
 			o.xT = w.xT.p, o.s = s, o.first = outer == 0;
@@ -1756,8 +1813,7 @@ int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const do
 		rel = enorm > 0 ? std::sqrt(ss) / enorm : 0.0;
 		if (rel <= tol || outer >= max_outer || mx == 0.0) break;
 		// d <- r (scaled), then sweeps d <- r + F^T (rho o d) with XT = rho o d
-		hipLaunchKernelGGL(k_scale<_Float16>, dim3(g), dim3(kB), 0, st, outer ? w.r64.p : w.E64.p, 1.0 / mx, total, nrhs,
-		                   ld, w.r32.p, w.X16[0].p, w.rho32.p);
+		launch_scale(outer ? w.r64.p : w.E64.p, 1.0 / mx, n, nrhs, ld, w.r32.p, w.X16[0].p, w.rho32.p, st);
 		SweepOut<_Float16> o{};
 		o.n = n, o.nrhs = nrhs, o.inv = inv, o.rho_in = true, o.rhs = w.r32.p, o.rho = w.rho32.p;
 		o.xT = w.xT.p, o.s = mx, o.first = outer == 0, o.wT = w.wT.p, o.rho64 = w.rho64.p;
