@@ -3444,16 +3444,29 @@ int DeviceEngine::run_cast(int n, const RayIn *rays, void *dray, int *o, int *hi
 	Impl &d = *d_;
 	hipStream_t st = d.stream;
 	RayIn *dr = static_cast<RayIn *>(dray);
+	const size_t b = (size_t)n * sizeof(int);
 	HIP_OK(hipStreamSynchronize(st), "cast");  // nothing of an earlier call is in flight
 	d.stage.begin();
-	if (d.stage.up(dr, rays, (size_t)n * sizeof(RayIn), st, err, grow)) return -1;
+	// few rays: the kernel reads them from, and writes its results to, pinned memory
+	unsigned char *hin = d.stage.room((size_t)n * sizeof(RayIn)), *hout = hin ? d.stage.room(3 * b) : nullptr;
+	if (hout) {
+		std::memcpy(hin, rays, (size_t)n * sizeof(RayIn));
+		dr = reinterpret_cast<RayIn *>(hin);
+		o = reinterpret_cast<int *>(hout);
+	} else if (d.stage.up(dr, rays, (size_t)n * sizeof(RayIn), st, err, grow)) {
+		return -1;
+	}
 	HIP_OK(hipEventRecord(d.ev0, st), "event");
 	if (d.fma) launch_cast<true>(st, d.S, dr, n, o, o + n, o + 2 * (size_t)n);
 	else launch_cast<false>(st, d.S, dr, n, o, o + n, o + 2 * (size_t)n);
 	HIP_OK(hipGetLastError(), "cast launch");
 	HIP_OK(hipEventRecord(d.ev1, st), "event");
-	const size_t b = (size_t)n * sizeof(int);
-	if (cells && tests) {
+	if (hout) {
+		HIP_OK(hipStreamSynchronize(st), "cast");
+		std::memcpy(hit, o, b);
+		if (cells) std::memcpy(cells, o + n, b);
+		if (tests) std::memcpy(tests, o + 2 * (size_t)n, b);
+	} else if (cells && tests) {
 		const Stage::Part parts[3] = {{hit, b}, {cells, b}, {tests, b}};
 		if (d.stage.down_parts(o, parts, 3, st, err, grow)) return -1;
 	} else if (d.stage.down(hit, o, b, st, err, grow) || (cells && d.stage.down(cells, o + n, b, st, err, grow)) ||

@@ -446,15 +446,19 @@ __global__ __launch_bounds__(kB) void k_scale(const double *r64, double inv_s, i
 }
 
 // rho32 <- rho and per block (grid-stride): sum of squares and max of |E|, the
-// power sum_i area_i E_i
+// power sum_i area_i E_i; rho and E go to rho64 and E64 where those are others
 constexpr int kStatBlocks = 1024;
 __global__ __launch_bounds__(kB) void k_prep(const double *rho, const double *E, const float *area, unsigned total,
-                                             unsigned nrhs, float *rho32, double *stat)
+                                             unsigned nrhs, float *rho32, double *stat, double *rho64, double *E64)
 {
 	double ss = 0.0, mx = 0.0, pw = 0.0;
 	for (unsigned t = blockIdx.x * kB + threadIdx.x; t < total; t += gridDim.x * kB) {
-		const double e = E[t];
-		rho32[t] = (float)rho[t];
+		const double e = E[t], p = rho[t];
+		rho32[t] = (float)p;
+		if (rho64 != rho) {
+			rho64[t] = p;
+			E64[t] = e;
+		}
 		ss += e * e;
 		mx = fmax(mx, fabs(e));
 		pw += (double)area[t / nrhs] * e;
@@ -1116,6 +1120,7 @@ struct LinearSystem::Impl {
 	Buf<_Float16> F16, FT16;  // FT16: s16 * F^T in fragment order (the adjoint's sweeps)
 	Buf<__bf16> FB16;
 	Buf<unsigned> umax;
+	const double *in[2] = {};  // inputs()
 	float s16 = 1.f, sb16 = 1.f;
 	bool have16 = false, haveb16 = false, havet = false, havet16 = false;
 	std::map<std::pair<int, int>, std::pair<int, int>> tiles;  // (ct, prec) -> (rt, S)
@@ -1201,6 +1206,22 @@ struct LinearSystem::Impl {
 		HIP_OK(hipStreamSynchronize(st), "stream");
 		stage.begin();
 		return 0;
+	}
+	// rho and E (total each) where k_prep reads them: in pinned memory, or copied
+	// to work.rho64 and E64
+	int inputs(const double *rho, const double *E, size_t total, std::string &err)
+	{
+		double *h = (double *)stage.room(2 * total * 8);
+		if (h) {
+			std::memcpy(h, rho, total * 8);
+			std::memcpy(h + total, E, total * 8);
+			in[0] = h;
+			in[1] = h + total;
+			return 0;
+		}
+		in[0] = work.rho64.p;
+		in[1] = work.E64.p;
+		return stage.up(work.rho64.p, rho, total * 8, st, err) || stage.up(work.E64.p, E, total * 8, st, err) ? -1 : 0;
 	}
 	// room for count elements, zero where it was allocated anew
 	template <typename T> int zeroed(Buf<T> &b, size_t count, std::string &err)
@@ -1538,14 +1559,14 @@ int LinearSystem::gather(int prec, int nrhs, const double *rho, const double *E,
 	    (dma_tile(rt, ct) && w.part.alloc((size_t)S * ld * rp, err)) || w.rho64.alloc(total, err) ||
 	    w.E64.alloc(total, err) || d.zeroed(w.xT, (size_t)w.fx.rp * ld, err) || w.r64.alloc(total, err) ||
 	    w.out.alloc(total, err) || (prec == PREC_F16 ? d.iterates(w.X16, xts, err) : d.iterates(w.Xb, xts, err)) ||
-	    d.stage.up(w.rho64.p, rho, total * 8, st, err) || d.stage.up(w.E64.p, E, total * 8, st, err))
+	    d.inputs(rho, E, total, err))
 		return -1;
 	if (Bref && (w.Bref64.alloc(total, err) || w.blk.alloc(8192 * 2, err) ||
 	             d.stage.up(w.Bref64.p, Bref, total * 8, st, err)))
 		return -1;
 	const int g = grid_for(total), gs = std::min(g, kStatBlocks);
-	hipLaunchKernelGGL(k_prep, dim3(gs), dim3(kB), 0, st, w.rho64.p, w.E64.p, d.area.p, (unsigned)total, (unsigned)nrhs,
-	                   w.rho32.p, d.stage.stats);
+	hipLaunchKernelGGL(k_prep, dim3(gs), dim3(kB), 0, st, d.in[0], d.in[1], d.area.p, (unsigned)total, (unsigned)nrhs,
+	                   w.rho32.p, d.stage.stats, w.rho64.p, w.E64.p);
 	HIP_OK(hipGetLastError(), "upload");
 	HIP_OK(hipStreamSynchronize(st), "upload");
 	// x = 0 at the start, so the first residual is E itself
@@ -1609,9 +1630,16 @@ int LinearSystem::gather(int prec, int nrhs, const double *rho, const double *E,
 	const dim3 tg = turn_grid(n, nrhs);
 	const size_t blocks = (size_t)tg.x * tg.y;
 	if (d.stage.stat_room(blocks, err)) return -1;  // the residual's were read
-	hipLaunchKernelGGL(k_rows, tg, dim3(kB), 0, st, w.xT.p, ld, n, nrhs, nullptr, w.out.p, d.area.p, d.stage.stats);
+	double *out = (double *)d.stage.room(total * 8);
+	hipLaunchKernelGGL(k_rows, tg, dim3(kB), 0, st, w.xT.p, ld, n, nrhs, nullptr, out ? out : w.out.p, d.area.p,
+	                   d.stage.stats);
 	HIP_OK(hipGetLastError(), "download");
-	if (d.stage.down(B, w.out.p, total * 8, st, err)) return -1;
+	if (out) {
+		HIP_OK(hipStreamSynchronize(st), "download");
+		std::memcpy(B, out, total * 8);
+	} else if (d.stage.down(B, w.out.p, total * 8, st, err)) {
+		return -1;
+	}
 	if (info) {
 		info[INFO_OUTER] = outer;
 		info[INFO_SWEEPS] = total_sweeps;
@@ -1783,11 +1811,10 @@ int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const do
 	// out: lambda, then dL/drho
 	if (w.rho64.alloc(total, err) || w.E64.alloc(total, err) || d.zeroed(w.xT, xtn, err) || d.zeroed(w.wT, xtn, err) ||
 	    w.r64.alloc(total, err) || w.out.alloc(2 * total, err) || w.rho32.alloc(total, err) || w.r32.alloc(total, err) ||
-	    w.fb.alloc(total, err) || d.iterates(w.X16, (size_t)rp * ld, err) ||
-	    d.stage.up(w.rho64.p, rho, total * 8, st, err) || d.stage.up(w.E64.p, gin, total * 8, st, err))
+	    w.fb.alloc(total, err) || d.iterates(w.X16, (size_t)rp * ld, err) || d.inputs(rho, gin, total, err))
 		return -1;
-	hipLaunchKernelGGL(k_prep, dim3(gs), dim3(kB), 0, st, w.rho64.p, w.E64.p, d.area.p, (unsigned)total, (unsigned)nrhs,
-	                   w.rho32.p, d.stage.stats);
+	hipLaunchKernelGGL(k_prep, dim3(gs), dim3(kB), 0, st, d.in[0], d.in[1], d.area.p, (unsigned)total, (unsigned)nrhs,
+	                   w.rho32.p, d.stage.stats, w.rho64.p, w.E64.p);
 	HIP_OK(hipGetLastError(), "upload");
 	HIP_OK(hipStreamSynchronize(st), "upload");
 	const auto t0 = std::chrono::steady_clock::now();
@@ -1824,18 +1851,27 @@ int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const do
 	if (outer == 0)  // no refinement: lambda is the zero it started from
 		hipLaunchKernelGGL(k_fill<double>, dim3(grid_for(w.xT.n)), dim3(kB), 0, st, w.xT.p, w.xT.n, 0.0);
 	// dL/drho = lambda o (F B), F B in FP64 (wT takes B)
-	if (d.stage.up(w.r64.p, B, total * 8, st, err)) return -1;
+	double *hB = (double *)d.stage.room(total * 8);
+	if (hB) std::memcpy(hB, B, total * 8);
+	else if (d.stage.up(w.r64.p, B, total * 8, st, err)) return -1;
 	const dim3 tg = turn_grid(n, nrhs);
-	hipLaunchKernelGGL(k_cols, tg, dim3(kB), 0, st, w.r64.p, ld, n, nrhs, w.wT.p);
+	hipLaunchKernelGGL(k_cols, tg, dim3(kB), 0, st, hB ? hB : w.r64.p, ld, n, nrhs, w.wT.p);
 	{
 		double ss, mx;
 		if (w.fx.run(d.F32.p, w.wT.p, nullptr, nullptr, nullptr, w.fb.p, st, ss, mx, false, err)) return -1;
 	}
-	hipLaunchKernelGGL(k_rows, tg, dim3(kB), 0, st, w.xT.p, ld, n, nrhs, nullptr, w.out.p, nullptr, nullptr);
-	hipLaunchKernelGGL(k_rows, tg, dim3(kB), 0, st, w.xT.p, ld, n, nrhs, w.fb.p, w.out.p + total, nullptr, nullptr);
+	double *out = (double *)d.stage.room(2 * total * 8), *o = out ? out : w.out.p;
+	hipLaunchKernelGGL(k_rows, tg, dim3(kB), 0, st, w.xT.p, ld, n, nrhs, nullptr, o, nullptr, nullptr);
+	hipLaunchKernelGGL(k_rows, tg, dim3(kB), 0, st, w.xT.p, ld, n, nrhs, w.fb.p, o + total, nullptr, nullptr);
 	HIP_OK(hipGetLastError(), "adjoint");
-	const Stage::Part parts[2] = {{lambda, total * 8}, {drho, total * 8}};
-	if (d.stage.down_parts(w.out.p, parts, 2, st, err)) return -1;
+	if (out) {
+		HIP_OK(hipStreamSynchronize(st), "adjoint");
+		std::memcpy(lambda, out, total * 8);
+		std::memcpy(drho, out + total, total * 8);
+	} else {
+		const Stage::Part parts[2] = {{lambda, total * 8}, {drho, total * 8}};
+		if (d.stage.down_parts(w.out.p, parts, 2, st, err)) return -1;
+	}
 	const double ms = ms_since(t0);
 	if (info) {
 		for (int k = 0; k < INFO_N; k++) info[k] = -1;

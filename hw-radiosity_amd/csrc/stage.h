@@ -14,6 +14,13 @@
 
 struct Stage {
 	static constexpr size_t kSmall = (size_t)1 << 20;  // pinned bytes for small copies
+	// Arrays up to this many bytes, in the pinned memory for small copies, are
+	// read and written over the link by the kernels that use them, where a copy's
+	// launch and the wait for it cost more than the slower access.  us, copied and
+	// direct: a gather of n = 1000, 2000, 4000, 8000 with 3 columns 202, 212, 284,
+	// 756 and 160, 180, 262, 733, of n = 2000 with 24 (750 KB in) 275 and 270; 10,
+	// 3000, 16000 rays cast 44, 50, 71 and 32, 36, 51.
+	static constexpr size_t kDirect = (size_t)768 << 10;
 	static constexpr size_t kChunk = (size_t)1 << 20;  // of a large copy
 	static constexpr int kDepth = 4;                   // chunks on their way
 	unsigned char *p = nullptr, *q = nullptr;
@@ -92,6 +99,15 @@ struct Stage {
 			HIP_OK(hipEventRecord(ev[c % kDepth], st), "upload");
 		}
 		return 0;
+	}
+	// room for bytes that kernels read or write in the pinned memory themselves,
+	// or null where a copy is the better way
+	unsigned char *room(size_t bytes)
+	{
+		if (bytes > kDirect || off + bytes > kSmall) return nullptr;
+		unsigned char *h = p + off;
+		off += (bytes + 255) / 256 * 256;
+		return h;
 	}
 	// copies src's bytes from the device into consecutive parts of the host's;
 	// they are complete on return (the stream is synchronised up to the copy)
