@@ -913,11 +913,24 @@ bool dma_tile(int rt, int ct) { return ct >= 8 && rt >= 2; }
 // 8) 12.5; 9216 (2, 8) 30.7, (4, 8) 24.7; four column tiles: 20224 (4, 8)
 // 205.3, (4, 4) 197.6).  Past 16384 rows one column tile does better with more
 // blocks of 32 rows (20224: 136.3 against 142.2).
+// Wide (ct 8 and 12): up to 4096 rows and eight column tiles 16 rows a block as
+// above; else k_gemm_dma's 256 rows, K split as often as the blocks still fit the
+// CUs in one round (twelve column tiles below 1280 rows: four ways, as each
+// partial is then a sixth of the work).  Of the twelve tiles at 17 sizes from 512
+// to 20224 rows, both precisions, the fastest or within 5 % of it, with k_finish
+// (us: eight column tiles, 4096 (1, 8) 16.9, (4, 8) 20.1; 5120 (1, 8) 36.6, (4, 8)
+// 23.5; twelve, 7936 (2, 8) 44.4, (2, 4) 54.1; 10240 (2, 8) 78.2, (2, 4) 68.1;
+// 20224 (2, 4) 222, (2, 2) 211).  Timing them on the first solve took 9 ms at
+// 7777 rows.
 void sweep_tile(int ct, int ld, int &rt, int &S)
 {
 	rt = ld <= 4096 ? 1 : ld <= 8192 ? 2 : 4;
 	S = 8;
-	if (ld > 16384) {
+	if (ct > 4 && (ct > 8 || ld > 4096)) {
+		rt = ct > 8 ? 2 : 4;
+		while (S > 1 && ld / 256 * S > 256) S /= 2;
+		if (ld < 1280) S = 4;
+	} else if (ld > 16384) {
 		rt = ct == 1 ? 2 : 4;
 		S = ct == 1 ? 8 : 4;
 	}
@@ -1183,20 +1196,16 @@ struct LinearSystem::Impl {
 		return 0;
 	}
 
-	// the tile of a solve: tuned or forced, else by rule, tuned here for the
-	// wide tiles
-	int solve_tile(LinearSystem &L, int nrhs, int prec, int &rt, int &S, std::string &err)
+	// the tile of a solve: tuned or forced, else by rule
+	void solve_tile(int nrhs, int prec, int ld, int &rt, int &S) const
 	{
-		const int ct = pick_ct(nrhs);
-		if (!tiles.count({ct, prec})) {
-			if (ct <= 4) {
-				sweep_tile(ct, L.ld(), rt, S);
-				return 0;
-			}
-			if (L.autotune(nrhs, prec, err)) return -1;
+		const auto t = tiles.find({pick_ct(nrhs), prec});
+		if (t == tiles.end()) {
+			sweep_tile(pick_ct(nrhs), ld, rt, S);
+		} else {
+			rt = t->second.first;
+			S = t->second.second;
 		}
-		L.tile_config(nrhs, prec, &rt, &S);
-		return 0;
 	}
 
 	// the start of a call: nothing of an earlier one (which may have ended in
@@ -1548,7 +1557,7 @@ int LinearSystem::gather(int prec, int nrhs, const double *rho, const double *E,
 	}
 	if (d.ensure_lowp(prec, np_, err)) return -1;
 	int rt, S;
-	if (d.solve_tile(*this, nrhs, prec, rt, S, err)) return -1;
+	d.solve_tile(nrhs, prec, np_, rt, S);
 	const int n = n_, ld = np_, rp = ct * 16;
 	const size_t total = (size_t)n * nrhs;
 	const float inv = 1.0f / (prec == PREC_F16 ? d.s16 : d.sb16);
@@ -1802,7 +1811,7 @@ int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const do
 	const int ct = pick_ct(nrhs), rp = ct * 16;
 	if (d.ensure_t16(ld, err)) return -1;
 	int rt, Sg;
-	if (d.solve_tile(*this, nrhs, PREC_F16, rt, Sg, err)) return -1;
+	d.solve_tile(nrhs, PREC_F16, ld, rt, Sg);
 	const float inv = 1.0f / d.s16;
 	const int g = grid_for(total), gs = std::min(g, kStatBlocks);
 	Work &w = d.work;

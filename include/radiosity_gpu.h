@@ -210,8 +210,8 @@ rad_status rad_lin_get_matrix(rad_lin *lin, float *F);
 rad_status rad_lin_set_areas(rad_lin *lin, const double *area); /* power sums and shooting's source order */
 
 /* Picks the MFMA tile (rows per wave rt*16, split-K factor) for nrhs columns
- * by timing every candidate on this matrix; gather does it on first use for
- * more than 64 columns and goes by the matrix size up to 64. */
+ * by timing every candidate on this matrix; without it the solves go by the
+ * matrix size. */
 rad_status rad_lin_autotune(rad_lin *lin, int nrhs, int prec, int *rt, int *splitk);
 /* Forces the tile for nrhs columns instead of the autotuner's choice:
  * rt in {1, 2, 4} (rt = 4 with more than 64 columns shares the right-hand
