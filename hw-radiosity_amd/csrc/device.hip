@@ -174,6 +174,12 @@ struct Loop {
 	int v3_short;   // V3: that plan follows one that a departure ended early
 };
 
+// Values of the loop's state that a kernel's first branches and loads depend on:
+// read together, before the first of them is tested, for one round trip to
+// memory (the last launch wrote them) instead of one after another.
+template <typename T> __device__ __forceinline__ void read_now(T x) { asm volatile("" : : "s"(x)); }
+template <typename... T> __device__ __forceinline__ void together(T... x) { (read_now(x), ...); }
+
 struct Cnt {
 	int rays, ref_rays, cells, tests, levels, precision, stalled;
 };
@@ -1273,9 +1279,11 @@ template <bool F, bool LOWEST>
 __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) void k_shoot(
 	DScene S, DRecv R, Loop *L, unsigned char *live, float *ffbuf, long long *bcnt, int nlanes)
 {
-	if (L->done) return;
-	const int before = L->updated;
-	const unsigned long long key = before & 1 ? L->key_odd : L->key;
+	const int done = L->done, before = L->updated;
+	const unsigned long long even = L->key, odd = L->key_odd;
+	together(done, before, even, odd);
+	if (done) return;
+	const unsigned long long key = before & 1 ? odd : even;
 	const int q = blockIdx.x * (kTraceBlock / 8) + (int)threadIdx.x / 8, sub = (int)threadIdx.x & 7;
 	const bool valid = q < nlanes;
 	const int i = valid ? 6 * R.order[q / 6] + q % 6 : 0;
@@ -1340,31 +1348,47 @@ __global__ __launch_bounds__(kTraceBlock) __attribute__((amdgpu_waves_per_eu(4, 
 // three vertex lanes combined by shuffles in the reference's order; after
 // the last source the next iteration's candidate key (listCanditate,
 // rad.cpp:387-404) by wave, block and one 64-bit atomicMax per block.
-template <bool F, bool FUSED_SELECT, bool LOWEST, int G>
+// SHOOT: after k_shoot, whose scenes are so small that a launch is a chain of
+// loads: everything a receiver may need is read at once (the 2120-slot room 21.9
+// -> 21.2 us per iteration).  Larger ones are bound by the traffic and read what
+// they turn out to need.
+template <bool F, bool FUSED_SELECT, bool LOWEST, int G, bool SHOOT>
 __global__ __launch_bounds__(kBlock) void k_update(DRecv R, Loop *L, int k, const unsigned char *live,
-                                                   const float *ffbuf, float converge, long long *bcnt, int nblocks,
-                                                   bool shoot)
+                                                   const float *ffbuf, float converge, long long *bcnt, int nblocks)
 {
-	if (L->done || k >= L->nsrc) return;
+	const int done = L->done, nsrc = L->nsrc, taken = L->taken;
+	together(done, nsrc, taken);
+	if (done || k >= nsrc) return;
 	__shared__ unsigned long long wmax[kWavesPerBlock];
 	__shared__ int wn[kWavesPerBlock];
 	const RecvMap<G> m(nblocks);
 	const SrcDesc &s = L->src[k];
-	const bool last = k == L->nsrc - 1;
+	const bool last = k == nsrc - 1;
 	unsigned long long key = 0;
 	int recv = 0, ncand = 0;
 #pragma unroll
 	for (int g = 0; g < G; g++) {
 		const int r = m.slot(g);
 		const bool valid = m.valid(g, R.nslots, nblocks);
-		const int lb = valid ? live[r] : 0;  // bit 0: takes part; bit 1: parent >= 0
-		const bool lv = lb & 1;
+		int lb = valid ? live[r] : 0;  // bit 0: takes part; bit 1: parent >= 0
 		const int sv = 3 * r + m.v;
-		float ff = 0.f;
-		float4 rho = make_float4(0.f, 0.f, 0.f, 0.f);
-		if (lv) {
-			ff = s.split ? ffbuf[2 * sv] + ffbuf[2 * sv + 1] : ffbuf[2 * sv];
+		float4 rho = make_float4(0.f, 0.f, 0.f, 0.f), acc = rho, db = rho;
+		float2 f = make_float2(0.f, 0.f);
+		if (SHOOT && valid) {
+			f = *(const float2 *)(ffbuf + 2 * sv);
 			rho = R.rho[r];
+			acc = R.acc[sv];
+			if (m.v == 0) db = R.dB[r];
+			asm volatile("" : "+v"(lb), "+v"(f.x), "+v"(rho.x), "+v"(acc.x), "+v"(db.x));  // read here
+		}
+		const bool lv = lb & 1;
+		float ff = 0.f;
+		if (lv) {
+			if (!SHOOT) {
+				f = *(const float2 *)(ffbuf + 2 * sv);
+				rho = R.rho[r];
+			}
+			ff = s.split ? f.x + f.y : f.x;
 		}
 		const float kr = (float)(0.5 / 255.0);
 		const float dr = rho.x * kr * s.dB[0] / 3 * ff;
@@ -1372,17 +1396,19 @@ __global__ __launch_bounds__(kBlock) void k_update(DRecv R, Loop *L, int k, cons
 		const float dbb = rho.z * kr * s.dB[2] / 3 * ff;
 		const float r1 = __shfl(dr, m.base + 1), g1 = __shfl(dg, m.base + 1), b1 = __shfl(dbb, m.base + 1);
 		const float r2 = __shfl(dr, m.base + 2), g2 = __shfl(dg, m.base + 2), b2 = __shfl(dbb, m.base + 2);
-		float4 db = make_float4(0.f, 0.f, 0.f, 0.f);
-		const bool own = shoot && valid && m.v == 0 && r == s.phys;  // the source's unshot energy, as k_shoot left it
-		if (valid && m.v == 0 && !own) db = R.dB[r];
-		if (own) R.dB[r] = db;
+		const bool own = SHOOT && valid && m.v == 0 && r == s.phys;  // the source's unshot energy, as k_shoot left it
+		if (!SHOOT && valid && m.v == 0 && !own) db = R.dB[r];
+		if (own) {
+			db = make_float4(0.f, 0.f, 0.f, 0.f);
+			R.dB[r] = db;
+		}
 		if (lv) {
 			// Adding zeros leaves a sum as it is (none is -0): most vertices do
 			// not see the source, and their radiosities stay in memory (the
 			// hall's launch, bound by that traffic, 12.7 -> 9.4 us)
 			const bool some = dr != 0.0f || dg != 0.0f || dbb != 0.0f;
 			if (some) {
-				float4 acc = R.acc[sv];
+				if (!SHOOT) acc = R.acc[sv];
 				acc.x += dr;
 				acc.y += dg;
 				acc.z += dbb;
@@ -1422,12 +1448,12 @@ __global__ __launch_bounds__(kBlock) void k_update(DRecv R, Loop *L, int k, cons
 			ncand += wn[w];
 		}
 		// after k_shoot the next key goes beside the one it took, zeroed here
-		const bool odd = shoot && (L->taken & 1);
+		const bool odd = SHOOT && (taken & 1);
 		if (FUSED_SELECT && key) atomicMax(odd ? &L->key_odd : &L->key, key);
 		if (ncand) atomicAdd(&L->ncand, ncand);
-		if (shoot && blockIdx.x == 0) {
+		if (SHOOT && blockIdx.x == 0) {
 			*(odd ? &L->key : &L->key_odd) = 0;
-			L->updated = L->taken;
+			L->updated = taken;
 		}
 	}
 }
@@ -2084,10 +2110,13 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
 {
 	__shared__ unsigned rs[kWavesPerBlock][64];
 	__shared__ SrcDesc s;
-	if (L->done || L->v3_error) return;
-	// no pass under way: a new source, and a first pass over every slot in use
-	const bool fresh = !L->v3_pending;
+	const int done = L->done, error = L->v3_error, pending = L->v3_pending, resume = L->v3_resume;
+	const int slots = L->trinum, p0 = L->v3_range[par][0], p1 = L->v3_range[par][1];
 	const unsigned long long key = L->key;
+	together(done, error, pending, resume, slots, p0, p1, key);
+	if (done || error) return;
+	// no pass under way: a new source, and a first pass over every slot in use
+	const bool fresh = !pending;
 	if (fresh && key == 0) return;  // nothing left to shoot: k_v3_plan ends the solve
 	const int nb = gridDim.x - kV3RunBlocks;
 	if ((int)blockIdx.x >= nb) {
@@ -2096,9 +2125,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4, 8))) 
 		return;
 	}
 	Cnt c = {0, 0, 0, 0, 0, 0, 0};
-	const int r0 = fresh ? 0 : L->v3_range[par][0], n = (fresh ? L->trinum : L->v3_range[par][1]) - r0;
+	const int r0 = fresh ? 0 : p0, n = (fresh ? slots : p1) - r0;
 	const bool wide = n <= kV3Wide;
-	if (L->v3_resume || (long long)blockIdx.x * kBlock >= (wide ? 64LL : 16LL) * n) return;
+	if (resume || (long long)blockIdx.x * kBlock >= (wide ? 64LL : 16LL) * n) return;
 	// the source: each block makes its own (a launch less), block 0 keeps it
 	if (threadIdx.x == 0) {
 		if (fresh) make_source<F>(R, key_slot<false>(key), s);
@@ -2163,18 +2192,20 @@ __global__ __launch_bounds__(kV3Commit) void k_v3_plan(DRecv R, V3Dev V, Loop *L
 {
 	__shared__ int part[2][kV3Commit / kWave];
 	__shared__ int rest, ents, subs;
-	if (L->done || L->v3_error) return;
-	const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-	const bool fresh = !L->v3_pending;
+	const int done = L->done, error = L->v3_error, pending = L->v3_pending, resume = L->v3_resume;
+	const int trinum = L->trinum, p0 = L->v3_range[par][0], p1 = L->v3_range[par][1];
 	const unsigned long long key = L->key;
+	together(done, error, pending, resume, trinum, p0, p1, key);
+	if (done || error) return;
+	const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+	const bool fresh = !pending;
 	if (fresh && key == 0) {
 		__syncthreads();
 		if (tid == 0) L->done = 1;
 		return;
 	}
-	const int trinum = L->trinum;
-	const int r1 = fresh ? trinum : L->v3_range[par][1];
-	const int start = max(L->v3_resume, fresh ? 0 : L->v3_range[par][0]);
+	const int r1 = fresh ? trinum : p1;
+	const int start = max(resume, fresh ? 0 : p0);
 	int nent = 0, noff = 0, nsub = 0;
 	if (tid == 0) rest = r1;
 	bool more = trinum + 4 < V.cap;  // else every receiver keeps its form factors (shade.cpp:463)
@@ -2262,9 +2293,10 @@ __global__ __launch_bounds__(kV3Sub * 16) __attribute__((amdgpu_waves_per_eu(4, 
 	__shared__ int pbrk[kV3Sub];
 	__shared__ int wcnt[kV3Sub / 4][8];
 	__shared__ bool skip;
-	if (L->done || L->v3_error) return;
+	const int done = L->done, error = L->v3_error, nsub = L->v3_nsub;
+	together(done, error, nsub);
+	if (done || error) return;
 	const int tid = threadIdx.x, lane = tid & 63, pt = tid >> 4, q = tid & 15;
-	const int nsub = L->v3_nsub;
 	const SrcDesc &s = L->src[0];
 	for (int b = blockIdx.x; b < nsub; b += gridDim.x) {
 		const int2 sb = V.sub[b];
@@ -2422,12 +2454,14 @@ __global__ __launch_bounds__(kV3Commit) void k_v3_commit(DScene S, DRecv R, V3De
 	const int tid = threadIdx.x, lane = tid & 63;
 	const int pt = tid >> 4, q = tid & 15;  // a chunk's point and the lane in its group
 	Cnt c = {0, 0, 0, 0, 0, 0, 0};
-	if (L->done || L->v3_error) return;
-	const int r1 = L->v3_range[par][1];
+	const int done = L->done, error = L->v3_error, r0 = L->v3_range[par][0], r1 = L->v3_range[par][1];
+	const int nent = L->v3_nent, first = L->v3_first, made = L->trinum, after = L->v3_rest, brief0 = L->v3_short;
+	together(done, error, r0, r1, nent, first, made, after, brief0);
+	if (done || error) return;
 	const SrcDesc &s = L->src[0];
-	const int limit = V.cap, nent = L->v3_nent, first = L->v3_first;
+	const int limit = V.cap;
 	const int last = min(first, nent - 1);  // the last entry whose samples are where the plan put them
-	int trinum = L->trinum;
+	int trinum = made;
 	bool stop = trinum + 4 >= limit;  // the pool is full: every receiver keeps its form factors
 	int pos = 0;                      // values of rand() used
 	if (tid == 0) nf3 = 0;
@@ -2480,7 +2514,7 @@ __global__ __launch_bounds__(kV3Commit) void k_v3_commit(DScene S, DRecv R, V3De
 		}
 		__syncthreads();
 	}
-	int rest = L->v3_rest;  // the first receiver left to the ordered steps
+	int rest = after;  // the first receiver left to the ordered steps
 	if (!stop) {
 		if (first < nent) {
 			const int4 en = V.ent[first];
@@ -2497,7 +2531,7 @@ __global__ __launch_bounds__(kV3Commit) void k_v3_commit(DScene S, DRecv R, V3De
 	// place, unless few are left or two plans in a row got no further than a few.
 	const int at = first < nent ? first + 1 : nent;
 	const bool brief = at <= kV3Again;
-	bool again = !stop && trinum + 4 < limit && nent - at > kV3Again && !(brief && L->v3_short);
+	bool again = !stop && trinum + 4 < limit && nent - at > kV3Again && !(brief && brief0);
 	const bool ordered = !stop && !again && rest < r1;
 	int left = nent - at, calm = 0;  // ordered steps: entries left, receivers in a row without a departure
 	if (tid < 34) st[tid] = pos > 0 ? V.rnd[pos + tid] : L->rng[(L->rng_k + tid) % 34];
@@ -2596,7 +2630,7 @@ __global__ __launch_bounds__(kV3Commit) void k_v3_commit(DScene S, DRecv R, V3De
 		// the next pass: the slots this one made, or the rest of this one
 		L->v3_resume = again ? rest : 0;
 		L->v3_short = again && brief && !ordered;
-		L->v3_range[par ^ 1][0] = again ? L->v3_range[par][0] : r1;
+		L->v3_range[par ^ 1][0] = again ? r0 : r1;
 		L->v3_range[par ^ 1][1] = again ? r1 : trinum;
 	}
 	const int vals[8] = {c.rays, c.ref_rays, c.cells, c.tests, c.levels, c.precision, c.stalled, 0};
@@ -2637,14 +2671,16 @@ __global__ __launch_bounds__(kBlock) void k_v3_finish(DRecv R, V3Dev V, Loop *L,
 {
 	__shared__ unsigned long long wmax[kWavesPerBlock];
 	__shared__ int wn[kWavesPerBlock];
-	if (L->done || L->v3_error) return;
-	const int r0 = L->v3_range[par][0], r1 = L->v3_range[par][1];
-	const bool pending = L->v3_range[par ^ 1][0] < L->v3_range[par ^ 1][1];
+	const int done = L->done, error = L->v3_error, r0 = L->v3_range[par][0], r1 = L->v3_range[par][1];
+	const int n0 = L->v3_range[par ^ 1][0], n1 = L->v3_range[par ^ 1][1], resume = L->v3_resume, slots = L->trinum;
+	together(done, error, r0, r1, n0, n1, resume, slots);
+	if (done || error) return;
+	const bool pending = n0 < n1;
 	if (blockIdx.x == 0 && threadIdx.x == 0) L->v3_pending = pending;
-	if (L->v3_resume) return;  // the pass goes on
+	if (resume) return;  // the pass goes on
 	unsigned long long key = 0;
 	int n = 0;
-	const int lo = pending ? r0 : 0, hi = pending ? r1 : L->trinum;
+	const int lo = pending ? r0 : 0, hi = pending ? r1 : slots;
 	for (int r = lo + blockIdx.x * kBlock + threadIdx.x; r < hi; r += gridDim.x * kBlock) {
 		if (r >= r0 && r < r1 && V.act[r] == V3_APPLY) v3_receive(R, V, L->src[0], r);
 		if (pending || __float_as_int(R.nrm[r].w) < 0) continue;
@@ -3312,16 +3348,18 @@ int DeviceEngine::shoot(int max_shots, int *shots, int *converged, std::string &
 				hipLaunchKernelGGL(k_trace<false>, tg, dim3(kTraceBlock), 0, st, d.S, d.R, d.loop.p, k, d.ffbuf.p, d.bcnt.p, d.rays.p);
 			}
 			if (ev >= 0 && k == 0) (void)hipEventRecord(d.kev[2 * ev + 1], st);
-			auto update = [&](auto gc) {
+			auto update = [&](auto gc, auto sh) {
 				constexpr int G = decltype(gc)::value;
-#define UPD(F, FS, LO) hipLaunchKernelGGL((k_update<F, FS, LO, G>), g, blk, 0, st, d.R, d.loop.p, k, d.live.p, d.ffbuf.p, d.converge, d.bcnt.p, d.nblocks, shoot)
+				constexpr bool SH = decltype(sh)::value;
+#define UPD(F, FS, LO) hipLaunchKernelGGL((k_update<F, FS, LO, G, SH>), g, blk, 0, st, d.R, d.loop.p, k, d.live.p, d.ffbuf.p, d.converge, d.bcnt.p, d.nblocks)
 				if (multi) { if (d.fma) UPD(true, false, false); else UPD(false, false, false); }
 				else if (d.lowest) { if (d.fma) UPD(true, true, true); else UPD(false, true, true); }
 				else { if (d.fma) UPD(true, true, false); else UPD(false, true, false); }
 #undef UPD
 			};
-			if (d.groups == 1) update(std::integral_constant<int, 1>{});
-			else update(std::integral_constant<int, 2>{});
+			if (shoot) update(std::integral_constant<int, 1>{}, std::true_type{});
+			else if (d.groups == 1) update(std::integral_constant<int, 1>{}, std::false_type{});
+			else update(std::integral_constant<int, 2>{}, std::false_type{});
 		}
 	};
 	// With -graph 1 and without kernel timing, runs of kGraphIters
