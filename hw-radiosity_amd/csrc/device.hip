@@ -3493,6 +3493,7 @@ int DeviceEngine::run_cast(int n, const RayIn *rays, void *dray, int *o, int *hi
 	d.stage.begin();
 	// few rays: the kernel reads them from, and writes its results to, pinned memory
 	unsigned char *hin = d.stage.room((size_t)n * sizeof(RayIn)), *hout = hin ? d.stage.room(3 * b) : nullptr;
+	if (!hout) d.stage.begin();
 	if (hout) {
 		std::memcpy(hin, rays, (size_t)n * sizeof(RayIn));
 		dr = reinterpret_cast<RayIn *>(hin);

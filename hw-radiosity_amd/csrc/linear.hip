@@ -1578,6 +1578,7 @@ int LinearSystem::gather(int prec, int nrhs, const double *rho, const double *E,
 	                   w.rho32.p, d.stage.stats, w.rho64.p, w.E64.p);
 	HIP_OK(hipGetLastError(), "upload");
 	HIP_OK(hipStreamSynchronize(st), "upload");
+	d.stage.begin();  // the inputs were read
 	// x = 0 at the start, so the first residual is E itself
 	double ss0 = 0.0, mx0 = 0.0, power_E = 0.0;
 	for (int k = 0; k < gs; k++) {
@@ -1826,6 +1827,7 @@ int LinearSystem::adjoint(int nrhs, const double *rho, const double *B, const do
 	                   w.rho32.p, d.stage.stats, w.rho64.p, w.E64.p);
 	HIP_OK(hipGetLastError(), "upload");
 	HIP_OK(hipStreamSynchronize(st), "upload");
+	d.stage.begin();  // the inputs were read
 	const auto t0 = std::chrono::steady_clock::now();
 	double enorm = -1.0, rel = 0.0;
 	int outer = 0, total_sweeps = 0;

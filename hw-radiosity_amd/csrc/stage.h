@@ -24,7 +24,7 @@ struct Stage {
 	static constexpr size_t kChunk = (size_t)1 << 20;  // of a large copy
 	static constexpr int kDepth = 4;                   // chunks on their way
 	unsigned char *p = nullptr, *q = nullptr;
-	size_t off = 0;
+	size_t off = 0, keep = 0;  // bytes of p in use; those of room(), which copies leave alone
 	hipEvent_t ev[kDepth] = {};
 	// per-block statistics that kernels write to host memory directly (read
 	// after the stream is synchronised: no copy to wait for)
@@ -66,18 +66,19 @@ struct Stage {
 		return 0;
 	}
 	// the next calls' copies start at the buffer's beginning: none of the
-	// earlier ones may be in flight (the stream was synchronised)
-	void begin() { off = 0; }
+	// earlier ones may be in flight (the stream was synchronised), and what
+	// room() gave out is done with
+	void begin() { off = keep = 0; }
 	// queues a copy to the device; src may be reused at once.  grow = false
 	// (callers that must not allocate): a large copy goes directly where the
 	// chunks are not there yet, and src is free once the stream is synchronised
 	int up(void *dst, const void *src, size_t bytes, hipStream_t st, std::string &err, bool grow = true)
 	{
 		if (bytes == 0) return 0;
-		if (bytes <= kSmall) {
+		if (bytes <= kSmall - keep) {
 			if (off + bytes > kSmall) {
 				HIP_OK(hipStreamSynchronize(st), "upload");
-				off = 0;
+				off = keep;
 			}
 			std::memcpy(p + off, src, bytes);
 			HIP_OK(hipMemcpyAsync(dst, p + off, bytes, hipMemcpyHostToDevice, st), "upload");
@@ -100,13 +101,13 @@ struct Stage {
 		}
 		return 0;
 	}
-	// room for bytes that kernels read or write in the pinned memory themselves,
-	// or null where a copy is the better way
+	// room for bytes that kernels read or write in the pinned memory themselves
+	// (until begin()), or null where a copy is the better way
 	unsigned char *room(size_t bytes)
 	{
 		if (bytes > kDirect || off + bytes > kSmall) return nullptr;
 		unsigned char *h = p + off;
-		off += (bytes + 255) / 256 * 256;
+		keep = off = std::min(kSmall, off + (bytes + 255) / 256 * 256);
 		return h;
 	}
 	// copies src's bytes from the device into consecutive parts of the host's;
@@ -135,10 +136,10 @@ struct Stage {
 				done += b;
 			}
 		};
-		if (bytes <= kSmall) {
+		if (bytes <= kSmall - keep) {
 			if (off + bytes > kSmall) {
 				HIP_OK(hipStreamSynchronize(st), "download");
-				off = 0;
+				off = keep;
 			}
 			HIP_OK(hipMemcpyAsync(p + off, src, bytes, hipMemcpyDeviceToHost, st), "download");
 			HIP_OK(hipStreamSynchronize(st), "download");

@@ -56,3 +56,18 @@ def test_solves_around_the_line(n, nrhs):
             dE, drho, _ = lin.adjoint(rho, B, E, tol=1e-10, max_outer=60, sweeps=6)
             assert np.linalg.norm(E + F64.T @ (rho * dE) - dE) <= 1.01e-10 * np.linalg.norm(E)
             assert np.abs(drho - dE * (F64 @ B)).max() <= 1e-12 * np.abs(drho).max()
+
+
+@pytest.mark.parametrize("n,nrhs", [(300, 3), (900, 48), (1000, 48), (1024, 48), (1025, 48), (1400, 48)])
+def test_reference_copied_beside_direct_inputs(n, nrhs):
+    """A solve's B does not depend on the values it is compared with, whose copy
+    shares the pinned memory with inputs that no kernel has read yet."""
+    print(n, nrhs, flush=True)
+    rng = np.random.default_rng(n)
+    F = (rng.random((n, n)) / n).astype(np.float32)
+    rho, E = rng.uniform(0.2, 0.7, (n, nrhs)), rng.random((n, nrhs))
+    with radgpu.LinearSystem(n) as lin:
+        lin.set_matrix(F)
+        B, _ = lin.gather(rho, E, prec="f16", tol=1e-10, max_outer=60, sweeps=6)
+        C, info = lin.gather(rho, E, prec="f16", tol=1e-10, max_outer=60, sweeps=6, Bref=B, target=1e-6)
+    assert np.array_equal(B, C) and info["err"] == 0.0
