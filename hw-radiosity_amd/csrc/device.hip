@@ -2152,9 +2152,10 @@ inline int v3_gen_blocks(size_t n)
 }
 constexpr int kV3SpecBlocks = 512;
 // A new plan (five launches, 45 us) against the ordered steps' 18 us a receiver:
-// taken where more than this many receivers go by without a departure.  The
-// room's longest commit was 1552 us without it, 46 us with it; all of them
-// together 5.2 and 2.7 ms.
+// taken where more than this many receivers go by without a departure, and past
+// a plan's end.  The room's longest commit was 1552 us without it, 46 us with
+// it, all of them together 5.2 and 2.7 ms; with -delta_ff 2e-5 and 800 receivers
+// to sample a pass, past a plan's end in order 37.7 ms a solve, planned 26.6.
 constexpr int kV3Again = 2;
 
 // exclusive prefix sums of x over a block of kV3Commit threads, and the total
@@ -2527,13 +2528,14 @@ __global__ __launch_bounds__(kV3Commit) void k_v3_commit(DScene S, DRecv R, V3De
 			pos = 3 * (en.z + en.y);
 		}
 	}
-	// Entries left after a departure are planned anew, at their samples' real
-	// place, unless few are left or two plans in a row got no further than a few.
+	// What is left after a departure, or past the plan, is planned anew, unless
+	// that is little or two plans in a row got no further than a few entries.
 	const int at = first < nent ? first + 1 : nent;
 	const bool brief = at <= kV3Again;
-	bool again = !stop && trinum + 4 < limit && nent - at > kV3Again && !(brief && brief0);
+	int left = after < r1 ? INT_MAX : nent - at;  // entries left; past the plan: many
+	int calm = 0;                                 // ordered receivers in a row without a departure
+	bool again = !stop && trinum + 4 < limit && at > 0 && left > kV3Again && !(brief && brief0);
 	const bool ordered = !stop && !again && rest < r1;
-	int left = nent - at, calm = 0;  // ordered steps: entries left, receivers in a row without a departure
 	if (tid < 34) st[tid] = pos > 0 ? V.rnd[pos + tid] : L->rng[(L->rng_k + tid) % 34];
 	if (tid == 0) sk = 0;
 	__syncthreads();
