@@ -2909,9 +2909,10 @@ struct DeviceEngine::Impl {
 	SegIndex seg;                      // segment visibility of the explicit matrix, on the host
 	DevBuf<unsigned> seg_mask;         // ... and on the device
 	DevBuf<int> seg_begin, pos;        // pos: each slot's position in order
+	DevBuf<int> seg_order;             // order with the slots that V3 splits added
 	DevBuf<unsigned long long> vis;    // pair visibility bits of the explicit matrix
 	DevBuf<float4> seg_nc, seg_se;
-	bool have_seg = false;
+	bool have_seg = false, seg_split = false;  // seg_split: seg holds for slots that V3 splits added too
 	float seg_cl = 0.f;                // bound on |c|_1 of the records with a cull radius
 	DevBuf<Loop> loop;
 	DevBuf<long long> bcnt;
@@ -3060,7 +3061,7 @@ int DeviceEngine::warm(std::string &err)
 
 int DeviceEngine::upload(const HostScene &s, const FlatOctree &t, std::string &err)
 {
-	d_->have_seg = false;
+	d_->have_seg = d_->seg_split = false;
 	d_->drop_graph();  // its launches name the buffers of the previous upload
 	Impl &d = *d_;
 	const int n0 = s.n_orig, n = s.trinum;
@@ -3622,10 +3623,13 @@ int DeviceEngine::form_factors(float *dF, int n, int ld, int vis, FlatOctree &t,
 		return -1;
 	}
 	hipStream_t st = d.stream;
-	if (vis == VIS_SEGMENT && !d.have_seg) {
+	// V3 splits after the upload cut triangles out of the originals, whose own
+	// records keep their geometry
+	const bool split = s.trinum != s.n_orig;
+	if (vis == VIS_SEGMENT && (!d.have_seg || (split && !d.seg_split))) {
 		// the segment test reads the originals' planes; pre-partition
 		// rewrites originals in place when it splits, so it needs none
-		if (s.trinum != s.n_orig) {
+		if (!d.have_seg && split) {
 			err = "segment visibility needs a scene that pre-partition did not split (" + std::to_string(s.trinum) +
 			      " slots, " + std::to_string(s.n_orig) + " originals)";
 			return -1;
@@ -3633,7 +3637,7 @@ int DeviceEngine::form_factors(float *dF, int n, int ld, int vis, FlatOctree &t,
 		// originals only: upload's cull radii are theirs
 		std::vector<float> rad((size_t)s.n_orig + 1);
 		d.seg_cl = cull_radii(s, rad.data());
-		build_segment_index(d.seg, s.pool.data(), s.n_orig, rad.data());
+		build_segment_index(d.seg, s.pool.data(), s.n_orig, rad.data(), split);
 		const size_t ne = d.seg.items.size();
 		if (ne >= ((size_t)1 << 29)) {
 			err = "segment index too large for 32-bit record indices";  // the walk indexes in int
@@ -3655,6 +3659,15 @@ int DeviceEngine::form_factors(float *dF, int n, int ld, int vis, FlatOctree &t,
 			return -1;
 		HIP_OK(hipStreamSynchronize(st), "segment index upload");
 		d.have_seg = true;
+		d.seg_split = split;
+	}
+	DRecv R = d.R;
+	if (vis == VIS_SEGMENT && (size_t)n > d.order.n) {  // the uploaded order ends before the added slots
+		std::vector<int> order(n);
+		spatial_order(s.pool.data(), n, s.G0, s.G1, order.data());
+		if (d.seg_order.put(order.data(), order.size(), st, err)) return -1;
+		HIP_OK(hipStreamSynchronize(st), "segment order upload");
+		R.order = d.seg_order.p;
 	}
 	// rows of a 64 x 64 tile per block: fewer than 64 while that leaves less
 	// than eight blocks per CU
@@ -3687,21 +3700,21 @@ int DeviceEngine::form_factors(float *dF, int n, int ld, int vis, FlatOctree &t,
 			G.inv[k] = 1.0f / g.h[k];
 		}
 		if (d.vis.alloc((size_t)n * nt, err) || d.pos.alloc(n, err)) return -1;
-		hipLaunchKernelGGL(k_positions, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, d.order.p, n, d.pos.p);
+		hipLaunchKernelGGL(k_positions, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, st, R.order, n, d.pos.p);
 		const dim3 vg((unsigned)(tiles * (64 / rb)));
 		const size_t lds = (size_t)G.words * sizeof(unsigned);
 #define VIS(RB)                                                                                                        \
 	if (rb == RB) {                                                                                                    \
-		if (d.fma) hipLaunchKernelGGL((k_vis_tiles<true, RB>), vg, dim3(kBlock), lds, st, G, d.R, n, nt, (unsigned char *)d.vis.p, d.bcnt.p); \
-		else hipLaunchKernelGGL((k_vis_tiles<false, RB>), vg, dim3(kBlock), lds, st, G, d.R, n, nt, (unsigned char *)d.vis.p, d.bcnt.p);      \
+		if (d.fma) hipLaunchKernelGGL((k_vis_tiles<true, RB>), vg, dim3(kBlock), lds, st, G, R, n, nt, (unsigned char *)d.vis.p, d.bcnt.p); \
+		else hipLaunchKernelGGL((k_vis_tiles<false, RB>), vg, dim3(kBlock), lds, st, G, R, n, nt, (unsigned char *)d.vis.p, d.bcnt.p);      \
 	}
 		VIS(64) VIS(32) VIS(16) VIS(8)
 #undef VIS
-		if (d.fma) hipLaunchKernelGGL(k_ff_seg<true>, dim3(n), dim3(kBlock), (size_t)nt * 8, st, d.R, n, ld, nt, d.vis.p, d.pos.p, dF);
-		else hipLaunchKernelGGL(k_ff_seg<false>, dim3(n), dim3(kBlock), (size_t)nt * 8, st, d.R, n, ld, nt, d.vis.p, d.pos.p, dF);
+		if (d.fma) hipLaunchKernelGGL(k_ff_seg<true>, dim3(n), dim3(kBlock), (size_t)nt * 8, st, R, n, ld, nt, d.vis.p, d.pos.p, dF);
+		else hipLaunchKernelGGL(k_ff_seg<false>, dim3(n), dim3(kBlock), (size_t)nt * 8, st, R, n, ld, nt, d.vis.p, d.pos.p, dF);
 	} else {
-		if (d.fma) hipLaunchKernelGGL(k_ff_rows<true>, dim3(n), dim3(kBlock), 0, st, d.S, d.R, n, ld, dF, d.bcnt.p);
-		else hipLaunchKernelGGL(k_ff_rows<false>, dim3(n), dim3(kBlock), 0, st, d.S, d.R, n, ld, dF, d.bcnt.p);
+		if (d.fma) hipLaunchKernelGGL(k_ff_rows<true>, dim3(n), dim3(kBlock), 0, st, d.S, R, n, ld, dF, d.bcnt.p);
+		else hipLaunchKernelGGL(k_ff_rows<false>, dim3(n), dim3(kBlock), 0, st, d.S, R, n, ld, dF, d.bcnt.p);
 	}
 	HIP_OK(hipGetLastError(), "form factor launch");
 	HIP_OK(hipEventRecord(d.ev1, st), "event");

@@ -5,20 +5,23 @@
 
 namespace rgpu {
 
-void build_segment_index(SegIndex &g, const Patch *pool, int n, const float *radius)
+void build_segment_index(SegIndex &g, const Patch *pool, int n, const float *radius, bool split)
 {
 	float lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
 	for (int i = 0; i < n; i++)
 		for (int k = 0; k < 3; k++) {
-			lo[k] = i ? std::min(lo[k], pool[i].c[k]) : pool[i].c[k];
-			hi[k] = i ? std::max(hi[k], pool[i].c[k]) : pool[i].c[k];
+			const float (&p)[3][3] = pool[i].p;
+			const float c = pool[i].c[k];
+			const float mn = split ? std::min({p[0][k], p[1][k], p[2][k]}) : c, mx = split ? std::max({p[0][k], p[1][k], p[2][k]}) : c;
+			lo[k] = i ? std::min(lo[k], mn) : mn;
+			hi[k] = i ? std::max(hi[k], mx) : mx;
 		}
 	std::vector<int> cand;
 	double area = 0.0;
 	for (int i = 0; i < n; i++) {
 		const Patch &t = pool[i];
 		bool never = false;
-		for (int k = 0; k < 3; k++)
+		for (int k = 0; k < 3 && !split; k++)
 			never |= t.n[(k + 1) % 3] == 0.0f && t.n[(k + 2) % 3] == 0.0f && (t.c[k] == lo[k] || t.c[k] == hi[k]);
 		if (never) continue;
 		cand.push_back(i);

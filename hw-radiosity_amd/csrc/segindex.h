@@ -24,12 +24,14 @@ struct SegIndex {
 constexpr int kSegCells = 1 << 18;
 
 // The index of the originals [0, n) of pool, whose slots are whole (no
-// pre-partition); radius: their cull radii (infinite: no bound).
+// pre-partition); radius: their cull radii (infinite: no bound).  split: the
+// segments also run between centroids of triangles cut out of the originals;
+// the grid then covers the originals' corners, and none is left out.
 //
-// Left out are triangles that no test of any segment between two centroids
-// accepts: those whose normal has one component only, in a plane that holds
-// the least or the greatest centroid coordinate of its axis (the walls of a
-// room).  With X that coordinate, p and q the segment's ends, v = fl(q - p):
+// Left out otherwise are triangles that no test of any segment between two
+// centroids accepts: those whose normal has one component only, in a plane that
+// holds the least or the greatest centroid coordinate of its axis (the walls of
+// a room).  With X that coordinate, p and q the segment's ends, v = fl(q - p):
 // rounding is monotonic, so fl(q - p) is not less than fl(X - p) (not more, for
 // the greatest), and the test's quotient fl(fl(X - p) n) / fl(v n) is zero, not
 // positive, at least one, or not a number, and so outside (1e-4, 1 - 1e-4).
@@ -37,6 +39,6 @@ constexpr int kSegCells = 1 << 18;
 // grown by 4e-3 of a cell and by 2^-18 of the coordinates (the walk's and the
 // tests' rounding), by a whole cell without a cull radius (slivers, whose side
 // planes' rounding reaches further).
-void build_segment_index(SegIndex &g, const Patch *pool, int n, const float *radius);
+void build_segment_index(SegIndex &g, const Patch *pool, int n, const float *radius, bool split = false);
 
 }  // namespace rgpu

@@ -1,0 +1,59 @@
+"""Calls on one engine that follow each other where a later one meets what an
+earlier one left: slots, grids and buffers made for another size."""
+import numpy as np
+import pytest
+
+import oracle_lib as ol
+import radgpu
+from radgpu import scenes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("fma", ["1", "0"])
+@pytest.mark.parametrize("pieces", [(2,), (1, 3)])
+def test_matrix_after_splits(pieces, fma):
+    """-variant v3 adds slots to a scene that the upload had whole: the matrix
+    of all of them (300 rows), which entries are open and their values, against a test of every
+    original."""
+    opts = ["-variant", "v3", "-adapt_area", "0.5", "-converge", "300", "-delta_ff", "5e-6", "-quiet", "1", "-fma", fma,
+            "-triangle", "50000"]
+    sc = scenes.v3_room(4, 1.05)
+    with radgpu.Engine(*opts) as eng:
+        eng.set_scene(sc).prepare_host().upload()
+        n0 = len(eng.records()[0])
+        assert n0 == sc.n
+        with radgpu.LinearSystem(n0) as lin:
+            lin.from_scene(eng)
+        o = ol.Oracle(*(opts + ["-jobs", "16"]))
+        o.load(sc)
+        o.build_tree()
+        o.init_radiosity()
+        o.prepartition()
+        n = n0
+        for k in pieces:
+            assert eng.shoot(k)[0] == k
+            rec, _ = eng.records()
+            o.iterate(k)
+            assert rec.tobytes() == o.dump()[0].tobytes()
+            assert len(rec) > n
+            n = len(rec)
+            print(fma, pieces, n0, "->", n, flush=True)
+            with radgpu.LinearSystem(n) as lin:
+                lin.from_scene(eng)
+                F = lin.matrix()
+            rows = np.sort(np.random.default_rng(n).choice(n, 300, replace=False))
+            pairs = np.stack([np.repeat(rows, n), np.tile(np.arange(n), len(rows))], axis=1).astype(np.int32)
+            want = o.ff_centroid(pairs, ol.VIS_BRUTE).reshape(len(rows), n)
+            F = F[rows]
+            assert np.array_equal(F != 0, want != 0)
+            s = want.astype(np.float64).sum(axis=1)
+            scaled = want.astype(np.float64) / np.maximum(s, 1.0)[:, None]
+            # a row's scale and its product are rounded once each
+            assert np.all(np.abs(F - scaled) <= 3 * 2.0 ** -24 * np.abs(scaled))
+    with radgpu.Engine(*opts) as eng:  # first asked for after the splits: refused, as ever
+        eng.set_scene(sc).prepare_host().upload()
+        eng.shoot(pieces[0])
+        n = len(eng.records()[0])
+        with radgpu.LinearSystem(n) as lin, pytest.raises(radgpu.RadError, match="did not split"):
+            lin.from_scene(eng)
