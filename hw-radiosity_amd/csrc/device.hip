@@ -2842,6 +2842,15 @@ template <typename T> struct DevBuf {
 	}
 };
 
+// adds the blocks' counters to out
+void add_counters(const DevBuf<long long> &cnt, long long *out)
+{
+	if (!cnt.p || cnt.n == 0) return;
+	std::vector<long long> h(cnt.n);
+	if (hipMemcpy(h.data(), cnt.p, h.size() * sizeof(long long), hipMemcpyDeviceToHost) != hipSuccess) return;
+	for (size_t i = 0; i < h.size(); i++) out[i % CNT_N] += h[i];
+}
+
 float smallest_float_at_least(double x)
 {
 	float f = (float)x;
@@ -2915,7 +2924,8 @@ struct DeviceEngine::Impl {
 	bool have_seg = false, seg_split = false;  // seg_split: seg holds for slots that V3 splits added too
 	float seg_cl = 0.f;                // bound on |c|_1 of the records with a cull radius
 	DevBuf<Loop> loop;
-	DevBuf<long long> bcnt;
+	DevBuf<long long> bcnt;            // the shooting kernels' counters, eight per block
+	DevBuf<long long> ffcnt;           // the explicit matrix's
 	DevBuf<unsigned long long> cand;
 	DevBuf<unsigned char> live;
 	DevBuf<float> ffbuf;
@@ -3156,6 +3166,7 @@ int DeviceEngine::upload(const HostScene &s, const FlatOctree &t, std::string &e
 	const int v3grid = d.v3 ? v3_gen_blocks((size_t)std::max(cap, 1)) : 0;
 	std::vector<long long> zeros((size_t)std::max(std::max(grid, tgrid), v3grid) * 8, 0);
 	if (d.bcnt.put(zeros.data(), zeros.size(), st, err)) return -1;
+	d.ffcnt.n = 0;  // counted anew, as those
 	if (!d.lowest && d.parallel_src > 1 && d.cand.alloc((size_t)n + 1, err)) return -1;
 	if (d.live.alloc((size_t)n + 1, err) || d.ffbuf.alloc((size_t)n * 6 + 2, err) ||
 	    d.raycnt.alloc((size_t)d.nblocks + 1, err) || d.rays.alloc((size_t)n * 6 + 1, err))
@@ -3676,9 +3687,14 @@ int DeviceEngine::form_factors(float *dF, int n, int ld, int vis, FlatOctree &t,
 	int rb = 64;
 	while (rb > 8 && tiles * (64 / rb) < 2048) rb /= 2;
 	const size_t nblk_ff = std::max<size_t>((size_t)n, (size_t)tiles * (64 / rb));
-	if (d.bcnt.n < nblk_ff * 8) {  // the largest grid of the two kernels indexes bcnt
-		std::vector<long long> zeros(nblk_ff * 8, 0);
-		if (d.bcnt.put(zeros.data(), zeros.size(), st, err)) return -1;
+	// the form factors' own counters: the shooting kernels' keep their place, which
+	// a captured graph names.  Grown, they start from the sums so far.
+	if (!d.ffcnt.p || d.ffcnt.n < nblk_ff * 8) {
+		long long sums[CNT_N] = {};
+		add_counters(d.ffcnt, sums);
+		if (d.ffcnt.alloc(nblk_ff * 8, err)) return -1;
+		hipLaunchKernelGGL(k_fill_n<long long>, dim3(1024), dim3(kBlock), 0, st, d.ffcnt.p, d.ffcnt.n, 0LL);
+		HIP_OK(hipMemcpyAsync(d.ffcnt.p, sums, sizeof sums, hipMemcpyHostToDevice, st), "counter upload");
 		HIP_OK(hipStreamSynchronize(st), "counter upload");
 	}
 	HIP_OK(hipEventRecord(d.ev0, st), "event");
@@ -3705,16 +3721,16 @@ int DeviceEngine::form_factors(float *dF, int n, int ld, int vis, FlatOctree &t,
 		const size_t lds = (size_t)G.words * sizeof(unsigned);
 #define VIS(RB)                                                                                                        \
 	if (rb == RB) {                                                                                                    \
-		if (d.fma) hipLaunchKernelGGL((k_vis_tiles<true, RB>), vg, dim3(kBlock), lds, st, G, R, n, nt, (unsigned char *)d.vis.p, d.bcnt.p); \
-		else hipLaunchKernelGGL((k_vis_tiles<false, RB>), vg, dim3(kBlock), lds, st, G, R, n, nt, (unsigned char *)d.vis.p, d.bcnt.p);      \
+		if (d.fma) hipLaunchKernelGGL((k_vis_tiles<true, RB>), vg, dim3(kBlock), lds, st, G, R, n, nt, (unsigned char *)d.vis.p, d.ffcnt.p); \
+		else hipLaunchKernelGGL((k_vis_tiles<false, RB>), vg, dim3(kBlock), lds, st, G, R, n, nt, (unsigned char *)d.vis.p, d.ffcnt.p);      \
 	}
 		VIS(64) VIS(32) VIS(16) VIS(8)
 #undef VIS
 		if (d.fma) hipLaunchKernelGGL(k_ff_seg<true>, dim3(n), dim3(kBlock), (size_t)nt * 8, st, R, n, ld, nt, d.vis.p, d.pos.p, dF);
 		else hipLaunchKernelGGL(k_ff_seg<false>, dim3(n), dim3(kBlock), (size_t)nt * 8, st, R, n, ld, nt, d.vis.p, d.pos.p, dF);
 	} else {
-		if (d.fma) hipLaunchKernelGGL(k_ff_rows<true>, dim3(n), dim3(kBlock), 0, st, d.S, R, n, ld, dF, d.bcnt.p);
-		else hipLaunchKernelGGL(k_ff_rows<false>, dim3(n), dim3(kBlock), 0, st, d.S, R, n, ld, dF, d.bcnt.p);
+		if (d.fma) hipLaunchKernelGGL(k_ff_rows<true>, dim3(n), dim3(kBlock), 0, st, d.S, R, n, ld, dF, d.ffcnt.p);
+		else hipLaunchKernelGGL(k_ff_rows<false>, dim3(n), dim3(kBlock), 0, st, d.S, R, n, ld, dF, d.ffcnt.p);
 	}
 	HIP_OK(hipGetLastError(), "form factor launch");
 	HIP_OK(hipEventRecord(d.ev1, st), "event");
@@ -3726,12 +3742,9 @@ int DeviceEngine::form_factors(float *dF, int n, int ld, int vis, FlatOctree &t,
 
 void DeviceEngine::counters(long long *out)
 {
-	Impl &d = *d_;
 	for (int k = 0; k < CNT_N; k++) out[k] = 0;
-	if (!d.bcnt.p) return;
-	std::vector<long long> h(d.bcnt.n);
-	if (hipMemcpy(h.data(), d.bcnt.p, h.size() * sizeof(long long), hipMemcpyDeviceToHost) != hipSuccess) return;
-	for (size_t i = 0; i < h.size(); i++) out[i % 8] += h[i];
+	add_counters(d_->bcnt, out);
+	add_counters(d_->ffcnt, out);
 }
 
 }  // namespace rgpu

@@ -57,3 +57,34 @@ def test_matrix_after_splits(pieces, fma):
         n = len(eng.records()[0])
         with radgpu.LinearSystem(n) as lin, pytest.raises(radgpu.RadError, match="did not split"):
             lin.from_scene(eng)
+
+
+@pytest.mark.parametrize("n", [2000, 8192])
+@pytest.mark.parametrize("vis", ["segment", "reference"])
+def test_matrix_between_shots(n, vis):
+    """A matrix asked for between two runs of shots, whose replayed graph names
+    the engine's buffers: the same records as without it, and the counters of
+    both; a second upload counts from zero."""
+    sc = scenes.patch_room(3, n)
+
+    def counts(opts, shots, matrices):
+        with radgpu.Engine("-triangle", str(n), "-quiet", "1", "-converge", "60", *opts) as eng, radgpu.LinearSystem(n) as lin:
+            eng.set_scene(sc).prepare_host().upload()
+            for k in range(2):
+                if shots:
+                    assert eng.shoot(16)[0] == 16
+                for _ in range(matrices[k]):
+                    lin.from_scene(eng, vis)
+            c, rec = eng.counters(), eng.records()[0].tobytes()
+            eng.upload()
+            assert not any(eng.counters().values())
+        return c, rec
+
+    plain, want = counts((), True, (0, 0))
+    only, _ = counts((), False, (1, 1))
+    assert plain["rays"] > 0 and only["rays"] > 0
+    for opts in ((), ("-graph", "1")):
+        print(n, vis, opts, flush=True)
+        both, rec = counts(opts, True, (1, 1))
+        assert rec == want
+        assert all(both[k] == plain[k] + only[k] for k in both)
