@@ -937,7 +937,10 @@ void sweep_tile(int ct, int ld, int &rt, int &S)
 }
 
 // One product with the tile (rt, S) and what follows it (o).  finish = false:
-// the wide tiles' product only (for timing it alone).
+// the wide tiles' product only (for timing it alone).  ld is a multiple of 256,
+// so rt 1, 2 and 4 and S 1, 2, 4 and 8 go with every size: k_sweep clamps its
+// rows and k-blocks, and k_gemm_dma's 256 rows and S chunks of at least 32 k
+// divide it.
 template <typename E>
 int launch_sweep(int rt, int ct, int S, const E *A, const E *XT, float *part, int ld, int rp, const SweepOut<E> &o,
                  hipStream_t st, bool finish = true)
@@ -969,17 +972,6 @@ int launch_sweep(int rt, int ct, int S, const E *A, const E *XT, float *part, in
 	G(4, 1) G(4, 2) G(4, 4)
 #undef G
 	return -1;
-}
-
-// tiles set_tile takes: whole blocks of 64 rt rows (256 for the wide kernels),
-// whole chunks of 32 k, and per chunk a multiple of 8 k-blocks (4 for 8 or 12
-// column tiles at rt = 1; any for the wide kernels)
-bool valid_tile(int rt, int ct, int S, int ld)
-{
-	const bool dma = dma_tile(rt, ct);
-	const int u2 = dma ? 1 : 2 * (ct <= 4 ? 4 : 2);
-	const int rows = dma ? 256 : 64 * rt;
-	return ld % rows == 0 && ld % (32 * S) == 0 && (ld / 32 / S) % u2 == 0 && ld / 32 / S >= 1;
 }
 
 double power_sum(const std::vector<float> &a, const double *v, int n, int nrhs)
@@ -1275,7 +1267,6 @@ struct LinearSystem::Impl {
 		int brt = 0, bs = 0;
 		for (int rt : {1, 2, 4}) {
 			for (int S : {1, 2, 4, 8}) {
-				if (dma_tile(rt, ct) && !valid_tile(rt, ct, S, ld)) continue;
 				if (launch_sweep<E>(rt, ct, S, A, X[0].p, part.p, ld, rp, o, st)) continue;  // warm-up
 				HIP_OK(hipEventRecord(e0, st), "event");
 				for (int k = 0; k < 3; k++) launch_sweep<E>(rt, ct, S, A, X[0].p, part.p, ld, rp, o, st);
@@ -1473,16 +1464,16 @@ int LinearSystem::set_tile(int nrhs, int prec, int rt, int splitk, std::string &
 {
 	const int ct = pick_ct(nrhs);
 	if (nrhs <= 0 || ct < 0 || (prec != PREC_F16 && prec != PREC_BF16) || (rt != 1 && rt != 2 && rt != 4) ||
-	    (splitk != 1 && splitk != 2 && splitk != 4 && splitk != 8) || !valid_tile(rt, ct, splitk, np_)) {
-		err = "set_tile: no kernel for this tile at this size";
+	    (splitk != 1 && splitk != 2 && splitk != 4 && splitk != 8)) {
+		err = "set_tile: nrhs 1..192, precision FP16 or BF16, rt 1, 2 or 4, splitk 1, 2, 4 or 8";
 		return -1;
 	}
 	d_->tiles[{ct, prec}] = {rt, splitk};
 	return 0;
 }
 
-// Times one sweep (GEMM + Jacobi epilogue) for every valid (rows per wave,
-// split-K) and keeps the fastest for (nrhs column tiles, precision).
+// Times one sweep for every (rows per wave, split-K) and keeps the fastest for
+// (nrhs column tiles, precision).
 int LinearSystem::autotune(int nrhs, int prec, std::string &err)
 {
 	Impl &d = *d_;
