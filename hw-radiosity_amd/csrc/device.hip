@@ -906,10 +906,17 @@ template <int W = kWavesPerBlock> __device__ void add_block_counters(const int (
 	if (threadIdx.x < 8 && mine != 0) bcnt[(size_t)blockIdx.x * 8 + threadIdx.x] += mine;
 }
 
+__device__ __forceinline__ bool has_minus_zero(const float4 &a)
+{
+	const unsigned z = 0x80000000u;
+	return __float_as_uint(a.x) == z || __float_as_uint(a.y) == z || __float_as_uint(a.z) == z;
+}
+
 // Source k's rays, part 1: which receivers take part (fixed at the first
 // source: parent >= 0, not a source, not all nine accB >= 255,
 // rad.cpp:420-428; bit 0 of live[slot], bit 1 holding parent >= 0 alone,
-// which k_update's candidate test needs) and CalFF up to the ray (shade.cpp:107-123) for each
+// which k_update's candidate test needs, and bit 2 whether one of its
+// radiosities is -0) and CalFF up to the ray (shade.cpp:107-123) for each
 // (receiver, vertex, half) into ffbuf[2 * (3 * slot + vertex) + half]; 0
 // where no ray is cast.  For k_compact, per receiver vertex in position
 // order (rcode[3 p + vertex], p the receiver's position in R.order): bit h
@@ -965,14 +972,15 @@ __global__ __launch_bounds__(kBlock) void k_gen(DRecv R, Loop *L, int k, unsigne
 				parent = __float_as_int(R.nrm[r].w);
 				acc = R.acc[3 * r + m.v];
 			}
-			const int vfull = !(acc.x < 255.0f || acc.y < 255.0f || acc.z < 255.0f);
-			const bool full = __shfl(vfull, m.base) && __shfl(vfull, m.base + 1) && __shfl(vfull, m.base + 2);
+			const int q = (int)!(acc.x < 255.0f || acc.y < 255.0f || acc.z < 255.0f) | (int)has_minus_zero(acc) << 2;
+			const int q0 = __shfl(q, m.base), q1 = __shfl(q, m.base + 1), q2 = __shfl(q, m.base + 2);
+			const bool full = q0 & q1 & q2 & 1;
 			bool chosen = false;
 			if (PREP) chosen = sd.phys == r;
 			else
 				for (int j = 0; j < L->nsrc; j++) chosen |= (L->src[j].phys == r);
 			lv = valid && parent >= 0 && !chosen && !full;
-			if (valid && m.v == 0) live[r] = (unsigned char)(lv | (parent >= 0) << 1);
+			if (valid && m.v == 0) live[r] = (unsigned char)(lv | (parent >= 0) << 1 | ((q0 | q1 | q2) & 4));
 		} else {
 			lv = valid && (live[r] & 1);
 		}
@@ -1370,7 +1378,7 @@ __global__ __launch_bounds__(kBlock) void k_update(DRecv R, Loop *L, int k, cons
 	for (int g = 0; g < G; g++) {
 		const int r = m.slot(g);
 		const bool valid = m.valid(g, R.nslots, nblocks);
-		int lb = valid ? live[r] : 0;  // bit 0: takes part; bit 1: parent >= 0
+		int lb = valid ? live[r] : 0;  // bit 0: takes part; 1: parent >= 0; 2 (not after k_shoot): a radiosity is -0
 		const int sv = 3 * r + m.v;
 		float4 rho = make_float4(0.f, 0.f, 0.f, 0.f), acc = rho, db = rho;
 		float2 f = make_float2(0.f, 0.f);
@@ -1403,10 +1411,11 @@ __global__ __launch_bounds__(kBlock) void k_update(DRecv R, Loop *L, int k, cons
 			R.dB[r] = db;
 		}
 		if (lv) {
-			// Adding zeros leaves a sum as it is (none is -0): most vertices do
-			// not see the source, and their radiosities stay in memory (the
-			// hall's launch, bound by that traffic, 12.7 -> 9.4 us)
-			const bool some = dr != 0.0f || dg != 0.0f || dbb != 0.0f;
+			// Adding zeros leaves a sum as it is, unless that is -0 (a negative
+			// -light times 0): most vertices do not see the source, and their
+			// radiosities stay in memory (the hall's launch, bound by that
+			// traffic, 12.7 -> 9.4 us)
+			const bool some = dr != 0.0f || dg != 0.0f || dbb != 0.0f || (SHOOT ? has_minus_zero(acc) : (lb & 4) != 0);
 			if (some) {
 				if (!SHOOT) acc = R.acc[sv];
 				acc.x += dr;
