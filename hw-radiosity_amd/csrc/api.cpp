@@ -5,6 +5,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <string>
 #include <thread>
 #include <vector>
@@ -28,6 +29,7 @@ struct rad_ctx {
 	std::string err;
 	bool loaded = false, prepared = false, uploaded = false, device_newer = false;
 	double ms_setup = 0, ms_upload = 0;
+	std::mutex cast_lock;  // casts on one context take turns: they share its ray buffers and pinned memory
 	// device start-up on its own thread while the host prepares (rad_run):
 	// the engine it made, or the error; read only after the join
 	std::thread starter;
@@ -43,6 +45,7 @@ struct rad_ctx {
 struct rad_lin {
 	std::unique_ptr<rgpu::LinearSystem> sys;
 	std::string err;
+	std::mutex lock;  // calls on one system take turns: they share its work buffers and pinned memory
 };
 
 struct rad_batch {
@@ -371,6 +374,7 @@ rad_status rad_cast(rad_ctx *c, int n, const void *rays, int *hit, int *cells, i
 {
 	if (!c || n < 0 || (n > 0 && (!rays || !hit))) return RAD_EINVAL;
 	if (!c->uploaded) return fail(c, RAD_ESTATE, "rad_upload first");
+	std::lock_guard<std::mutex> turn(c->cast_lock);
 	if (c->dev->cast(n, (const RayIn *)rays, hit, cells, tests, c->err)) return RAD_EDEVICE;
 	return RAD_OK;
 }
@@ -384,6 +388,7 @@ rad_status rad_cast_static(rad_ctx *c, int n, const void *rays, int *hit, int *c
 		         std::to_string(RAD_CAST_STATIC_MAX) + " per call";
 		return RAD_EINVAL;
 	}
+	std::lock_guard<std::mutex> turn(c->cast_lock);
 	if (c->dev->cast_static(n, (const RayIn *)rays, hit, cells, tests, c->err)) return RAD_EDEVICE;
 	return RAD_OK;
 }
@@ -446,6 +451,7 @@ rad_status rad_lin_from_scene(rad_lin *l, rad_ctx *c, int visibility, double *ms
 	if (visibility != RAD_VIS_SEGMENT && visibility != RAD_VIS_REFERENCE)
 		return lfail(l, RAD_EINVAL, "unknown visibility mode");
 	if (!c->uploaded) return lfail(l, RAD_ESTATE, "rad_upload the scene first");
+	std::lock_guard<std::mutex> turn(l->lock);
 	const HostScene &s = c->scene;
 	if (s.trinum != l->sys->n())
 		return lfail(l, RAD_EINVAL, "matrix size " + std::to_string(l->sys->n()) + " != scene slots " +
@@ -462,18 +468,21 @@ rad_status rad_lin_from_scene(rad_lin *l, rad_ctx *c, int visibility, double *ms
 rad_status rad_lin_set_matrix(rad_lin *l, const float *F)
 {
 	if (!l || !F) return RAD_EINVAL;
+	std::lock_guard<std::mutex> turn(l->lock);
 	return l->sys->set_matrix(F, l->err) ? RAD_EDEVICE : RAD_OK;
 }
 
 rad_status rad_lin_get_matrix(rad_lin *l, float *F)
 {
 	if (!l || !F) return RAD_EINVAL;
+	std::lock_guard<std::mutex> turn(l->lock);
 	return l->sys->get_matrix(F, l->err) ? RAD_EDEVICE : RAD_OK;
 }
 
 rad_status rad_lin_set_areas(rad_lin *l, const double *area)
 {
 	if (!l || !area) return RAD_EINVAL;
+	std::lock_guard<std::mutex> turn(l->lock);
 	return l->sys->set_areas(area, l->err) ? RAD_EDEVICE : RAD_OK;
 }
 
@@ -481,6 +490,7 @@ rad_status rad_lin_autotune(rad_lin *l, int nrhs, int prec, int *rt, int *splitk
 {
 	if (!l || nrhs <= 0 || nrhs > 192 || (prec != RAD_PREC_F16 && prec != RAD_PREC_BF16))
 		return l ? lfail(l, RAD_EINVAL, "autotune: nrhs 1..192, precision FP16 or BF16") : RAD_EINVAL;
+	std::lock_guard<std::mutex> turn(l->lock);
 	if (l->sys->autotune(nrhs, prec, l->err)) return RAD_EDEVICE;
 	int a, b;
 	l->sys->tile_config(nrhs, prec, &a, &b);
@@ -492,6 +502,7 @@ rad_status rad_lin_autotune(rad_lin *l, int nrhs, int prec, int *rt, int *splitk
 rad_status rad_lin_set_tile(rad_lin *l, int nrhs, int prec, int rt, int splitk)
 {
 	if (!l) return RAD_EINVAL;
+	std::lock_guard<std::mutex> turn(l->lock);
 	return l->sys->set_tile(nrhs, prec, rt, splitk, l->err) ? RAD_EINVAL : RAD_OK;
 }
 
@@ -499,6 +510,7 @@ rad_status rad_lin_gemm_ms(rad_lin *l, int nrhs, int prec, int reps, double *ms)
 {
 	if (!l || !ms || nrhs <= 0 || nrhs > 192 || reps <= 0 || (prec != RAD_PREC_F16 && prec != RAD_PREC_BF16))
 		return l ? lfail(l, RAD_EINVAL, "gemm_ms: bad arguments") : RAD_EINVAL;
+	std::lock_guard<std::mutex> turn(l->lock);
 	return l->sys->gemm_ms(nrhs, prec, reps, ms, l->err) ? RAD_EDEVICE : RAD_OK;
 }
 
@@ -506,6 +518,7 @@ rad_status rad_lin_multiply(rad_lin *l, int prec, int nrhs, const double *X, dou
 {
 	if (!l || !X || !Y || nrhs <= 0 || nrhs > 192 || prec < RAD_PREC_F32 || prec > RAD_PREC_BF16)
 		return l ? lfail(l, RAD_EINVAL, "multiply: bad arguments") : RAD_EINVAL;
+	std::lock_guard<std::mutex> turn(l->lock);
 	return l->sys->multiply(prec, nrhs, X, Y, l->err) ? RAD_EDEVICE : RAD_OK;
 }
 
@@ -515,6 +528,7 @@ rad_status rad_lin_gather(rad_lin *l, int prec, int nrhs, const double *rho, con
 	if (!l || !rho || !E || !B || nrhs <= 0 || nrhs > 192 || sweeps <= 0 || max_outer < 0 ||
 	    (prec != RAD_PREC_F16 && prec != RAD_PREC_BF16))
 		return l ? lfail(l, RAD_EINVAL, "gather: bad arguments") : RAD_EINVAL;
+	std::lock_guard<std::mutex> turn(l->lock);
 	return l->sys->gather(prec, nrhs, rho, E, tol, max_outer, sweeps, Bref, target, B, info, l->err) ? RAD_EDEVICE
 	                                                                                                    : RAD_OK;
 }
@@ -524,6 +538,7 @@ rad_status rad_lin_shoot(rad_lin *l, int nrhs, const double *rho, const double *
 {
 	if (!l || !rho || !E || !B || nrhs <= 0 || nrhs > 16 || max_shots < 0)
 		return l ? lfail(l, RAD_EINVAL, "shoot: bad arguments") : RAD_EINVAL;
+	std::lock_guard<std::mutex> turn(l->lock);
 	return l->sys->shoot(nrhs, rho, E, Bref, target, max_shots, B, info, l->err) ? RAD_EDEVICE : RAD_OK;
 }
 
@@ -532,6 +547,7 @@ rad_status rad_lin_adjoint(rad_lin *l, int nrhs, const double *rho, const double
 {
 	if (!l || !rho || !B || !dLdB || !dLdE || !dLdrho || nrhs <= 0 || nrhs > 4 || sweeps <= 0 || max_outer < 0)
 		return l ? lfail(l, RAD_EINVAL, "adjoint: bad arguments") : RAD_EINVAL;
+	std::lock_guard<std::mutex> turn(l->lock);
 	return l->sys->adjoint(nrhs, rho, B, dLdB, tol, max_outer, sweeps, dLdE, dLdrho, info, l->err) ? RAD_EDEVICE
 	                                                                                                : RAD_OK;
 }

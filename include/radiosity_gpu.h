@@ -9,7 +9,8 @@
  * returns a status, and the library never exits the process.
  *
  * Threading: one context per host thread.  A context owns one HIP stream
- * and its device buffers; host arrays belong to the caller.
+ * and its device buffers; host arrays belong to the caller.  Ray casts on one
+ * context, and calls on one rad_lin, from several threads take turns.
  */
 #ifndef RADIOSITY_GPU_H
 #define RADIOSITY_GPU_H
