@@ -38,14 +38,21 @@ void build_segment_index(SegIndex &g, const Patch *pool, int n, const float *rad
 	}
 	double side = cand.empty() ? ext : 1.5 * std::sqrt(2.0 * area / cand.size());
 	if (!(side > 0.0) || !std::isfinite(side)) side = ext > 0.0 ? ext : 1.0;
+	// ... nor less than twice what the lists are grown by (below), so that scenes
+	// far from the origin, whose coordinates round by much of a cell, do not list
+	// each triangle in all the cells around it
+	const double grow = 0x1p-18 * (mag + ext);
+	side = std::max(side, 2.0 * grow);
+	// the grid's extent along an axis: that of the centroids and their rounding
+	auto extent = [&](int k) { return ((double)hi[k] - lo[k]) * (1.0 + 2e-3) + mag * 0x1p-20 + 1e-30; };
 	auto cells = [&](double s) {
 		double p = 1.0;
-		for (int k = 0; k < 3; k++) p *= std::ceil(((double)hi[k] - lo[k]) * (1.0 + 2e-3) / s) + 3.0;
+		for (int k = 0; k < 3; k++) p *= std::ceil(extent(k) / s) + 3.0;
 		return p;
 	};
 	while (cells(side) > kSegCells) side *= 1.05;
 	for (int k = 0; k < 3; k++) {
-		const double e = ((double)hi[k] - lo[k]) * (1.0 + 2e-3) + mag * 0x1p-20 + 1e-30;
+		const double e = extent(k);
 		const int inner = std::max(1, (int)std::ceil(e / side));
 		g.r[k] = inner + 2;
 		g.h[k] = (float)(e / inner);
@@ -55,7 +62,6 @@ void build_segment_index(SegIndex &g, const Patch *pool, int n, const float *rad
 	// the cells [a, b] of every axis that candidate i touches; false: none
 	auto range = [&](int i, int (&a)[3], int (&b)[3]) {
 		const Patch &t = pool[i];
-		const double grow = 0x1p-18 * (mag + ext);
 		const bool wide = !std::isfinite(radius[i]);
 		for (int k = 0; k < 3; k++) {
 			const double mn = std::min({t.p[0][k], t.p[1][k], t.p[2][k]}), mx = std::max({t.p[0][k], t.p[1][k], t.p[2][k]});

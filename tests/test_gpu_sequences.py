@@ -1,5 +1,6 @@
 """Calls on one engine that follow each other where a later one meets what an
-earlier one left: slots, grids and buffers made for another size."""
+earlier one left (slots, grids and buffers made for another size), and the
+matrix of scenes at the edge of what its index is made for."""
 import numpy as np
 import pytest
 
@@ -88,3 +89,25 @@ def test_matrix_between_shots(n, vis):
         both, rec = counts(opts, True, (1, 1))
         assert rec == want
         assert all(both[k] == plain[k] + only[k] for k in both)
+
+
+@pytest.mark.parametrize("off", [1e4, 1e6])
+def test_matrix_far_from_the_origin(off):
+    """Coordinates that round by a cell of the segment grid or more: which
+    entries are open, against a test of every original."""
+    sc = scenes.patch_room(5, 700)
+    p = (sc.p.astype(np.float64) + [off, -off / 3, 0.1]).astype(np.float32)
+    opts = ["-triangle", str(sc.n), "-quiet", "1"]
+    sc = scenes.Scene(p, sc.frgb, sc.brgb)
+    with radgpu.Engine(*opts) as eng, radgpu.LinearSystem(sc.n) as lin:
+        eng.set_scene(sc).prepare_host().upload()
+        lin.from_scene(eng)
+        F = lin.matrix()
+    o = ol.Oracle(*(opts + ["-jobs", "16"]))
+    o.load(sc)
+    o.build_tree()
+    o.init_radiosity()
+    o.prepartition()
+    i, j = np.meshgrid(np.arange(sc.n), np.arange(sc.n), indexing="ij")
+    want = o.ff_centroid(np.stack([i.ravel(), j.ravel()], axis=1).astype(np.int32), ol.VIS_BRUTE)
+    assert np.array_equal(F != 0, want.reshape(sc.n, sc.n) != 0)
