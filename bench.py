@@ -443,8 +443,8 @@ def linear_leg(n=32768, n_adj=16384):
     log("batched 192: %s" % info)
     lin.close()
     eng.close()
-    # many scenes: 256 rooms of log-uniform size in one graph launch vs the
-    # same kernels launched scene after scene
+    # many scenes: 256 rooms of log-uniform size, a graph launch per refinement of
+    # all of them, vs the same kernels launched scene after scene
     out["batched_scenes"] = batch_leg()
     # adjoint at n_adj
     sc = scenes.patch_room(5, n_adj)

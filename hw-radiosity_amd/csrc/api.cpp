@@ -456,7 +456,7 @@ rad_status rad_lin_from_scene(rad_lin *l, rad_ctx *c, int visibility, double *ms
 	if (s.trinum != l->sys->n())
 		return lfail(l, RAD_EINVAL, "matrix size " + std::to_string(l->sys->n()) + " != scene slots " +
 		                                std::to_string(s.trinum));
-	if (c->dev->form_factors(l->sys->matrix32(), s.trinum, l->sys->ld(), visibility, c->tree, s, l->err))
+	if (c->dev->form_factors(l->sys->matrix32(), s.trinum, l->sys->ld(), visibility, s, l->err))
 		return RAD_EDEVICE;
 	if (ms) *ms = c->dev->cast_ms();
 	std::vector<double> area(s.trinum);
@@ -596,7 +596,7 @@ rad_status rad_batch_from_scene(rad_batch *b, int scene, rad_ctx *c, int visibil
 		         std::to_string(s.trinum);
 		return RAD_EINVAL;
 	}
-	if (c->dev->form_factors(b->b->matrix32(scene), s.trinum, b->b->ld(scene), visibility, c->tree, s, b->err))
+	if (c->dev->form_factors(b->b->matrix32(scene), s.trinum, b->b->ld(scene), visibility, s, b->err))
 		return RAD_EDEVICE;
 	if (ms) *ms = c->dev->cast_ms();
 	return RAD_OK;

@@ -12,9 +12,10 @@
 
 namespace rgpu {
 
-// Schedule of the batched sweep: each wave owns 16*rt rows, a block's eight
-// waves split K into chunks of kc or more (at most eight) and take as many row
-// groups as that leaves, and grid persistent blocks walk the tile list.
+// Schedule of the batched sweep: each wave owns 16*rt rows; a block's eight
+// waves split K as many ways as the largest power of two that is neither above
+// eight nor above ld / kc rounded up, and take as many row groups as that
+// leaves; grid persistent blocks walk the tile list.
 struct BatchTile {
 	int rt, kc, grid;
 };
@@ -36,8 +37,7 @@ public:
 	int set_tile(const BatchTile &t, std::string &err);
 	// rho, E, B: (total() x 3) row-major, scenes concatenated in order.
 	// graph = true: a HIP graph launch per refinement of all scenes, until none
-	// is above tol; false: the same
-	// kernels launched scene after scene (the unbatched reference schedule,
+	// is above tol; false: the same kernels launched scene after scene (the unbatched reference schedule,
 	// bit-identical results).  rel_res[count] = each scene's final FP64
 	// relative residual.  info[4]: device ms of the solve, ms to build the
 	// graph (capture + instantiate, 0 when cached), kernel launches (graph

@@ -290,7 +290,7 @@ struct SceneBatch::Impl {
 		gtb.assign(count, 0);
 		gte.assign(count, 0);
 		for (const int s : ord) {
-			int S = kSweepWaves;  // K split: chunks of at least kc
+			int S = kSweepWaves;  // K split: the largest power of two up to 8 and ld / kc rounded up
 			while (g.kc && S > 1 && (S - 1) * g.kc >= ld[s]) S /= 2;
 			gtb[s] = (int)tl.size();
 			const int wr = kSweepWaves / S * g.rt;  // row tiles per block

@@ -67,8 +67,8 @@ public:
 	// each whole patch, times the visibility vis (VIS_SEGMENT: the segment
 	// between the centroids is clear, k_ff_seg; VIS_REFERENCE: RayHitted from
 	// the centroid returns the patch, k_ff_rows); rows scaled to sum <= 1.
-	// VIS_SEGMENT builds t's segment index on first use.
-	int form_factors(float *dF, int n, int ld, int vis, FlatOctree &t, const HostScene &s, std::string &err);
+	// VIS_SEGMENT builds its index (segindex.h) on first use.
+	int form_factors(float *dF, int n, int ld, int vis, const HostScene &s, std::string &err);
 	double shoot_ms() const { return shoot_ms_; }  // device time of the shooting kernels so far
 	double kernel_ms() const { return kernel_ms_; }  // device time of the fused shoot kernel alone
 	long long kernel_launches() const { return kernel_launches_; }

@@ -3631,7 +3631,7 @@ int DeviceEngine::ff_pairs(int n, const int *pairs, float *ff3, std::string &err
 }
 
 
-int DeviceEngine::form_factors(float *dF, int n, int ld, int vis, FlatOctree &t, const HostScene &s, std::string &err)
+int DeviceEngine::form_factors(float *dF, int n, int ld, int vis, const HostScene &s, std::string &err)
 {
 	Impl &d = *d_;
 	if (n <= 0 || n > d.R.nslots || ld < n) {

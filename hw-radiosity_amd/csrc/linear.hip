@@ -18,10 +18,10 @@
 // A[l%16][8*(l/16)+j] and B[8*(l/16)+j][l%16], j = 0..7, and receives
 // D[4*(l/16)+j][l%16], j = 0..3.  A wave owns 16*RT rows and all 16*CT
 // right-hand-side columns, so F is read from HBM once per sweep; split-K S
-// spreads the K loop over S waves of a block (over S blocks for 8 or 12 column
-// tiles), whose partial tiles are summed in a fixed order (results do not
-// depend on timing).  (RT, S) go by the size (sweep_tile); for 8 or 12 column
-// tiles the autotuner times a whole sweep for each candidate.
+// spreads the K loop over S waves of a block (k_sweep) or, with 8 or 12 column
+// tiles and RT 2 or 4, over S blocks (k_gemm_dma), whose partial tiles are
+// summed in a fixed order (results do not depend on timing).  (RT, S) go by the
+// size (sweep_tile), unless the caller had the tuner time every tile or set one.
 #include "linear.h"
 
 #include "pack.h"
@@ -1058,9 +1058,8 @@ struct Fx64 {
 				}
 		}
 	}
-	// at most 4 columns: the vector-unit kernel (ld is a multiple of 256:
-	// whole steps of 256 k, whole blocks of 32 rows)
-	bool vec() const { return nrhs <= 4 && ld % 256 == 0; }
+	// at most 4 columns: the vector-unit kernel
+	bool vec() const { return nrhs <= 4; }
 	template <int NC> void launch_vec(const float *F, const double *wT, const double *base, const double *rho,
 	                                  const double *xT, double *out, hipStream_t st)
 	{

@@ -21,6 +21,16 @@ struct SegIndex {
 	std::vector<uint32_t> mask;  // bit per cell: has items
 };
 
+// The bound on the cells also keeps the walk within what the lists are grown by
+// (4e-3 of a cell, below).  The walk adds the parameter of an axis's next wall up
+// from the last, so that a wall's place is off by 0.004 of a cell after 512 cells
+// and by 0.06 after 2048 (measured).  Along its own axis that only moves the
+// moment of a step, and the end of the walk by 3e-5 of the segment, where tests
+// stop 1e-4 short of it; a cell skipped for it is one whose part of the segment
+// lies within that error of a wall of another axis: in that axis's cells, the
+// error times the ratio of the two axes' cells.  An axis of 2048 leaves at most
+// 2^18 / (3 * 2048) = 42 for another: 0.06 * 42 / 2048 = 1.2e-3; one of 512, 170:
+// 1.3e-3.  With a larger bound the lists would have to grow with it.
 constexpr int kSegCells = 1 << 18;
 
 // The index of the originals [0, n) of pool, whose slots are whole (no

@@ -5,7 +5,7 @@ and 192 right-hand sides, 2000 plain shots; with --gemm, the same matrix and
 five FP16 sweeps with 192 right-hand sides at the tile RT = 2 (the LDS DMA
 kernel), split-K 2;
 with --batch, 256 rooms of 500-8000 patches, the autotuned FP16 batch solve
-twice in one graph launch; with --adjoint, the 16384-patch room's FP16
+twice, a graph launch per refinement; with --adjoint, the 16384-patch room's FP16
 adjoint solve twice), then a plain 256 MiB device copy that calibrates the
 FETCH_SIZE / WRITE_SIZE counters in the same run.
 

@@ -11,6 +11,16 @@
  * Threading: one context per host thread.  A context owns one HIP stream
  * and its device buffers; host arrays belong to the caller.  Ray casts on one
  * context, and calls on one rad_lin, from several threads take turns.
+ *
+ * Memory: handles keep what their calls work in until they are destroyed, so
+ * that a repeated gather, adjoint, product, batch solve or cast allocates
+ * nothing.  Each has 1 MB of pinned host memory, 4 MB more after a copy above
+ * 1 MB, and its per-block statistics (24 KB to a few MB).  A rad_lin of n patches
+ * keeps on the device, per column of its widest solve (counted in whole
+ * sixteens), up to about 100 n bytes, above 4 columns up to 96 n more (split
+ * products); its low-precision copies (2 n^2 bytes each) and, after an adjoint
+ * or plain shooting, the transposed matrix (4 n^2).  A context keeps the buffers
+ * of its largest rad_cast up to 4,194,304 rays (44 bytes each).
  */
 #ifndef RADIOSITY_GPU_H
 #define RADIOSITY_GPU_H
@@ -269,8 +279,9 @@ const char *rad_batch_last_error(const rad_batch *batch);
 rad_status rad_batch_from_scene(rad_batch *batch, int scene, rad_ctx *ctx, int visibility, double *ms);
 rad_status rad_batch_set_matrix(rad_batch *batch, int scene, const float *F);
 /* Picks the schedule of the batched sweep product -- rows per wave rt*16
- * (rt in {1, 2, 4}), k per tile kc (1024..8192) and the persistent grid
- * (512..4096 blocks) -- by timing one sweep of every candidate on this
+ * (rt in {1, 2, 4}), kc (1024..8192: a scene's k range is split the largest
+ * power of two ways that is neither above 8 nor above n / kc rounded up) and the
+ * persistent grid (512..4096 blocks) -- by timing one sweep of every candidate on this
  * batch; without it solve goes by the batch's size. */
 rad_status rad_batch_autotune(rad_batch *batch, int prec, int *rt, int *kc, int *grid);
 /* Forces that schedule instead (rt in {1, 2, 4}, kc in {1024, 2048, 4096,

@@ -32,3 +32,19 @@ def test_every_tile_is_taken_and_solves(n, nrhs, prec):
         for bad in ((3, 1), (1, 3), (8, 1), (1, 16), (0, 0)):
             with pytest.raises(radgpu.RadError):
                 lin.set_tile(nrhs, prec, *bad)
+
+
+@pytest.mark.parametrize("nrhs", [65, 129])
+def test_rule_with_a_partly_filled_last_column_tile(nrhs):
+    n = 8193
+    print(n, nrhs, flush=True)
+    rng = np.random.default_rng(n)
+    k = 8
+    U, W = rng.random((n, k), np.float32), rng.random((k, n), np.float32)
+    F = (U / (U @ W.sum(1)).max()) @ W
+    rho, E = rng.uniform(0.2, 0.7, (n, nrhs)), rng.random((n, nrhs))
+    with radgpu.LinearSystem(n) as lin:
+        lin.set_matrix(F)
+        B, _ = lin.gather(rho, E, prec="f16", tol=1e-10, max_outer=60, sweeps=6)
+    FB = np.concatenate([F[i:i + 1024].astype(np.float64) @ B for i in range(0, n, 1024)])
+    assert np.linalg.norm(E + rho * FB - B) <= 1.01e-10 * np.linalg.norm(E)
