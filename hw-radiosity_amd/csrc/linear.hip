@@ -276,11 +276,12 @@ __global__ __launch_bounds__(kB) void k_finish(const float *part, int S, int ld,
 // A[l%16][l/16] and B[l/16][l%16], receives D[l/16 + 4*j][l%16], j = 0..3 --
 // rows interleaved, unlike the 16-bit MFMAs).  A block is W waves of 16 RT rows
 // each over the same 16 CT columns, whose 32 k per step they stage in LDS (two
-// buffers, columns 34 doubles apart: a lane's 16-byte reads of 16 columns fall
-// on all 64 banks); a lane loads 8 consecutive F entries of its row per step
+// buffers, columns 34 doubles apart: the 16-byte reads of 16 columns fall on all
+// 64 banks; 3.5 conflict cycles an instruction are left); a lane loads 8 consecutive F entries of its row per step
 // (converted exactly to FP64), the next step's on their way, and step s pairs
 // k = kk + 8*(l/16) + s in both operands, so every k is summed once.
-// Bound by the FP64 matrix units (73 TFLOP/s in a large library product); with
+// Bound by the FP64 matrix units (busy 0.81 of the cycles at n = 7777, 192 columns;
+// 73 TFLOP/s in a large library product); with
 // each wave reading its own X from L2 it was that traffic (12 TB/s).  us at n =
 // 7936, 16, 32, 64, 192 columns: 67, 103, 172, 486 -> 45, 75, 131, 382 (63
 // TFLOP/s); n = 1024, 16 and 64: 9.2, 13.2 -> 4.6, 9.2; n = 16384, 192: 1850 ->
@@ -602,9 +603,9 @@ __device__ __forceinline__ void block_record(unsigned long long key, const float
 // sets by parity: one barrier a shot), and every wave takes the block's
 // largest from there.  The runner-up's column is loaded while the source's is
 // on its way: mostly it is the next source.
-// Bound by that dependent chain (an HBM or cache latency where the guess
-// fails, two reductions, a barrier) and, from about 4000 patches, by one CU's
-// loads and updates.  us per shot for 3 columns, a launch per shot -> now: n =
+// Bound by one CU's VALU issue (n = 4000, 3 columns: 0.86 of its cycles, 190
+// instructions a wave and shot), below about 2000 patches by the dependent chain
+// (an HBM or cache latency where the guess fails, two reductions, a barrier).  us per shot for 3 columns, a launch per shot -> now: n =
 // 500 4.00 -> 0.85, 2000 4.23 -> 1.16, 4000 4.32 -> 1.55, 8000 4.41 -> 2.87;
 // 1 column, n = 12000 3.71 -> 2.25.  16 patches a thread (1 column, n = 16000)
 // spill: 4.82 against 3.74, so twelve is the most.
