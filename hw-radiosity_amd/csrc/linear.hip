@@ -603,12 +603,14 @@ __device__ __forceinline__ void block_record(unsigned long long key, const float
 // sets by parity: one barrier a shot), and every wave takes the block's
 // largest from there.  The runner-up's column is loaded while the source's is
 // on its way: mostly it is the next source.
-// Bound by one CU's VALU issue (n = 4000, 3 columns: 0.86 of its cycles, 190
-// instructions a wave and shot), below about 2000 patches by the dependent chain
-// (an HBM or cache latency where the guess fails, two reductions, a barrier).  us per shot for 3 columns, a launch per shot -> now: n =
-// 500 4.00 -> 0.85, 2000 4.23 -> 1.16, 4000 4.32 -> 1.55, 8000 4.41 -> 2.87;
-// 1 column, n = 12000 3.71 -> 2.25.  16 patches a thread (1 column, n = 16000)
-// spill: 4.82 against 3.74, so twelve is the most.
+// Bound by one CU's VALU issue, 0.85 of its cycles at n = 4000 with 3 columns (191
+// instructions a wave and shot) and 0.88 at 12000 with 1, and by the dependent
+// chain (a latency where the guess fails, two reductions, a barrier), whose share
+// is larger in small systems (issue 0.61 at n = 500, 0.69 at 2000) and where the
+// columns no longer stay in cache (0.72 at 8000).  us per shot for 3 columns, a
+// launch per shot -> now: n = 500 4.00 -> 0.85, 2000 4.23 -> 1.16, 4000 4.32 ->
+// 1.55, 8000 4.41 -> 2.87; 1 column, n = 12000 3.71 -> 2.25.  16 patches a thread
+// (1 column, n = 16000) spill: 4.82 against 3.74, so twelve is the most.
 constexpr int kOneThreads = 1024;
 constexpr int kOneState = 100;
 
