@@ -1,6 +1,5 @@
 #include "pack.h"
 
-#include <omp.h>
 #include <parallel/algorithm>
 
 #include <cmath>
@@ -43,20 +42,6 @@ void spatial_order(const Patch *pool, int n, const float *G0, const float *G1, i
 	for (int i = 0; i < n; i++) order[i] = (int)(uint32_t)key[i];
 }
 
-// The team that the engine's other loops use, so that none changes its size: that
-// ends and starts threads.  us, 16 threads on 16 CPUs, a team of one thread per
-// slice (at most eight), of eight, of all: 1.5 MB to the device 104, 68, 69, 4 MB
-// back 222, 154, 155; 65536 rays cast 260, 180, 179 (240 by the runtime's own
-// copies); the scene read between two casts, which has to start the threads
-// again, 1445 after eight, 1335 after all, as without any copy.  Where that team
-// is wide, or larger than the CPUs, eight: 64 threads on 16 CPUs took 284 us for
-// the first 1.1 MB (62).
-static int copy_team()
-{
-	const int all = omp_get_max_threads(), cpus = omp_get_num_procs();
-	return all <= 32 && all <= cpus ? all : cpus < 8 ? cpus : 8;
-}
-
 void copy_bytes(void *dst, const void *src, size_t bytes)
 {
 	constexpr size_t kSlice = (size_t)128 << 10;
@@ -65,7 +50,16 @@ void copy_bytes(void *dst, const void *src, size_t bytes)
 		return;
 	}
 	const long slices = (long)((bytes + kSlice - 1) / kSlice);
-#pragma omp parallel for schedule(static) num_threads(copy_team())
+	// always the same number of threads: a team that changes its size ends and
+	// starts threads, 30 us and more a call.  With a thread per slice instead, us:
+	// 1.5 MB to the device 104 (68 so), 4 MB back 222 (154); 65536 rays cast 260
+	// (180), where copies by the runtime itself take 240.  Eight, not the 16 of
+	// the engine's other loops, though the scene read after a copy then has to
+	// start threads (1445 us, 1335 after 16): beside torch's own team, 16 threads
+	// took 1980 us for a cast of 10^6 rays (1840), 4560 for 192 columns on 7777
+	// patches (4200).  Eight of the engine's own, asleep between calls, read that
+	// scene in 1400 but cast 100000 rays after it in 400 to 740 (285)
+#pragma omp parallel for schedule(static) num_threads(8)
 	for (long k = 0; k < slices; k++) {
 		const size_t o = (size_t)k * kSlice;
 		std::memcpy((char *)dst + o, (const char *)src + o, bytes - o < kSlice ? bytes - o : kSlice);
